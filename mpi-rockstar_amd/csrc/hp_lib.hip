@@ -202,12 +202,15 @@ struct SubBufs {
     // (counts, then the list)
     DevBuf edges, deg, adj, kmin, par, first_label, lab, root, v0, v1, x0, x1, rng0, rng1, rsmall,
         ssum, ecnt, evt;
+    // for the searches: each slot's leaf and packed vector; the boxes of each 64 slots and of each 64 such chunks
+    DevBuf slot_leaf, pk, chunks, cblocks;
     void release() {
         for (DevBuf *b : {&groups, &tiles, &qtiles, &ltiles, &drawn, &qidx, &psum, &mean, &pcorr, &sig, &pbox,
                           &gerr, &w, &w2, &rk, &bpos, &spos, &nodes, &act0, &act1, &counters,
                           &slot_group, &dist, &sel, &sel2, &target, &csize, &emit, &fused,
                           &edges, &deg, &adj, &kmin, &par, &first_label, &lab, &root, &v0, &v1,
-                          &x0, &x1, &rng0, &rng1, &rsmall, &ssum, &ecnt, &evt})
+                          &x0, &x1, &rng0, &rng1, &rsmall, &ssum, &ecnt, &evt, &slot_leaf, &pk,
+                          &chunks, &cblocks})
             b->release();
     }
 };
@@ -2209,8 +2212,6 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
             ndrawn += ns;
         }
         sg.seed = seed;  // advanced past the draws below for the drawn groups
-        for (int64_t off = 0; off < n; off += kWave)
-            ltiles.push_back(SubTile{(int32_t)g, (int32_t)off});
         sg.k = (int32_t)(int64_t)((float)ns * thresh);  // src/groupies.c:771
         if (ns > 0 && sg.k >= ns)
             return set_error(HP_EINVAL, "hp_find_subfofs: FOF_FRACTION selects past the sample");
@@ -2218,10 +2219,20 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
         for (int64_t off = 0; off < n; off += kSubTile)
             tiles.push_back(SubTile{(int32_t)g, (int32_t)off});
         sg.ntiles = (int32_t)(tiles.size() - sg.tile0);
-        for (int64_t off = 0; off < ns; off += kWave)
-            qtiles.push_back(SubTile{(int32_t)g, (int32_t)off});
         M += n;
         S += ns;
+    }
+    // the searches' wavefronts, those of the largest groups first: they go
+    // through the most chunks, and the last ones started bound the launch
+    std::vector<int32_t> by_size((size_t)ngroups);
+    for (int64_t g = 0; g < ngroups; g++) by_size[(size_t)g] = (int32_t)g;
+    std::stable_sort(by_size.begin(), by_size.end(), [&](int32_t a, int32_t b) {
+        return G[(size_t)a].n > G[(size_t)b].n;
+    });
+    for (int32_t g : by_size) {
+        const SubGroup &sg = G[(size_t)g];
+        for (int32_t off = 0; off < sg.n; off += kWave) ltiles.push_back(SubTile{g, off});
+        for (int32_t off = 0; off < sg.nsample; off += kWave) qtiles.push_back(SubTile{g, off});
     }
     // src/groupies.c:300-304 for each drawn group: the sample positions in
     // draw order (seed = num_p), then sorted by position (counting sort,
@@ -2302,6 +2313,11 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
     HP_ENSURE(B.sel2, sizeof(float) * (S + 1));
     HP_ENSURE(B.target, sizeof(float) * ng);
     HP_ENSURE(B.csize, sizeof(int32_t) * (M + 1));
+    const int32_t nchunk = Engine::blocks(M, kWave);
+    HP_ENSURE(B.slot_leaf, sizeof(int32_t) * (M + 1));
+    HP_ENSURE(B.pk, sizeof(PackPoint) * kWave * (nchunk + 1));
+    HP_ENSURE(B.chunks, sizeof(Box6) * (nchunk + 1));
+    HP_ENSURE(B.cblocks, sizeof(Box6) * (nchunk / kWave + 2));
     HP_ENSURE(B.emit, sizeof(int4) * cap_emit);
     // the linking's pair list starts at 8 per particle and grows to what the
     // walk reports
@@ -2407,7 +2423,17 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
         nn = (int32_t)std::min<int64_t>(nn, node_cap);
         if (nn > 0) {
             k_sub_collect<<<(uint32_t)nn, kWave, 0, s>>>(B.nodes.as<Node6>(), B.w.as<SParticle>(),
-                                                         B.w2.as<SParticle>());
+                                                         B.w2.as<SParticle>(),
+                                                         B.slot_leaf.as<int32_t>());
+            HP_LAUNCHED();
+        }
+        if (nchunk > 0) {
+            k_sub_pack<<<(uint32_t)nchunk, kWave, 0, s>>>(
+                (int32_t)M, B.slot_group.as<int32_t>(), B.nodes.as<Node6>(), B.w.as<SParticle>(),
+                B.pk.as<PackPoint>(), B.chunks.as<Box6>());
+            HP_LAUNCHED();
+            k_sub_blocks<<<Engine::blocks(nchunk, kWave), kWave, 0, s>>>(
+                nchunk, B.chunks.as<Box6>(), B.cblocks.as<Box6>());
             HP_LAUNCHED();
         }
     }
@@ -2415,7 +2441,9 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
     if (!qtiles.empty()) {
         k_sub_next_closest<<<(uint32_t)qtiles.size(), kWave, 0, s>>>(
             dg, B.qtiles.as<SubTile>(), B.drawn.as<int32_t>(), B.qidx.as<int32_t>(),
-            B.w.as<SParticle>(), B.nodes.as<Node6>(), B.dist.as<float>(), cfg.ordered_search);
+            B.w.as<SParticle>(), B.nodes.as<Node6>(), B.slot_leaf.as<int32_t>(),
+            B.pk.as<PackPoint>(), B.chunks.as<Box6>(), B.cblocks.as<Box6>(),
+            B.dist.as<float>(), cfg.ordered_search);
         HP_LAUNCHED();
         HP_TRY(hipMemcpyAsync(B.sel.p, B.dist.p, sizeof(float) * S, hipMemcpyDeviceToDevice, s));
     }
@@ -2443,7 +2471,9 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
             HP_LAUNCHED();
             k_sub_link<<<(uint32_t)ltiles.size(), kWave, 0, s>>>(
                 dg, B.ltiles.as<SubTile>(), B.target.as<float>(), B.w.as<SParticle>(),
-                B.nodes.as<Node6>(), B.edges.as<EdgeRec>(), cap_edges, deg, cnt);
+                B.nodes.as<Node6>(), B.pk.as<PackPoint>(),
+                B.chunks.as<Box6>(), B.cblocks.as<Box6>(), B.edges.as<EdgeRec>(), cap_edges, deg,
+                cnt);
             HP_LAUNCHED();
             HP_TRY(hipMemcpyAsync(&ne, cnt + kSfEdges, sizeof ne, hipMemcpyDeviceToHost, s));
             HP_TRY(hipStreamSynchronize(s));

@@ -790,13 +790,18 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
 }
 
 // after the build: the leaves whose points the last write left in the
-// second buffer copy them to the first, which the searches read
+// second buffer copy them to the first, which the searches read; each slot's
+// leaf
 __global__ __launch_bounds__(kWave) void k_sub_collect(const Node6 *__restrict__ nodes,
                                                        SParticle *__restrict__ wa,
-                                                       const SParticle *__restrict__ wb) {
+                                                       const SParticle *__restrict__ wb,
+                                                       int32_t *__restrict__ slot_leaf) {
     const Node6 nd = nodes[blockIdx.x];
-    if (nd.div >= 0 || !nd.where) return;
-    for (int32_t p = lane_id(); p < nd.n; p += kWave) wa[nd.start + p] = wb[nd.start + p];
+    if (nd.div >= 0) return;
+    for (int32_t p = lane_id(); p < nd.n; p += kWave) {
+        if (nd.where) wa[nd.start + p] = wb[nd.start + p];
+        slot_leaf[nd.start + p] = blockIdx.x;
+    }
 }
 
 // ---------------------------------------------------------- tree searches
@@ -835,18 +840,15 @@ __device__ __forceinline__ int32_t near_child(const Node6 &nd, const float (&c)[
 }
 
 // The reference's own-leaf step (src/fast3tree.c:999-1025): the leaf the
-// query descends to, climbed while its parent's split dimension is flat
-// there (that subtree, `skip`, is left out of the search), and the start
-// value: the smallest nonzero squared distance in it, or its squared
-// diagonal.
-__device__ __forceinline__ float nc_start(const float (&c)[6], int32_t root,
+// query descends to (the one that holds its slot: a point lies on the side
+// of every plane its node went to), climbed while its parent's split
+// dimension is flat there (that subtree, `skip`, is left out of the search),
+// and the start value: the smallest nonzero squared distance in it, or its
+// squared diagonal.
+__device__ __forceinline__ float nc_start(const float (&c)[6], int32_t root, int32_t own,
                                           const SParticle *__restrict__ w,
                                           const Node6 *__restrict__ nodes, int32_t *skip) {
-    int32_t nd = root;
-    while (nodes[nd].div >= 0) {
-        const Node6 &x = nodes[nd];
-        nd = acoord(c, x.div) <= acoord(nodes[x.left].hi, x.div) ? x.left : x.right;
-    }
+    int32_t nd = own;
     while (nd != root) {
         const int pd = nodes[nodes[nd].parent].div;
         if (acoord(nodes[nd].lo, pd) != acoord(nodes[nd].hi, pd)) break;
@@ -905,15 +907,311 @@ __device__ float nc_ordered(const float (&c)[6], int32_t root, int32_t skip, flo
     return r;
 }
 
-// a node whose box is at least thr (squared) from c: every point in it is
-__device__ __forceinline__ bool box_far(const Node6 &nd, const float (&c)[6], float thr) {
-    float d = 0.0f, e;
-#pragma unroll
-    for (int i = 0; i < 6; i++) {
-        if ((e = c[i] - nd.lo[i]) < 0) d += e * e;
-        else if ((e = c[i] - nd.hi[i]) > 0) d += e * e;
+// ------------------------------------------------- pairs on matrix cores
+//
+// Both searches below test a wavefront's 64 queries against chunks of 64
+// consecutive slots.  In six dimensions a sphere reaches the boxes of a third
+// of a group's leaves while nearly all of their points lie outside it, so the
+// time goes into pairs that are not close; a chunk's squared distances are
+// therefore bounded with matrix instructions first: d^2 = |a|^2 + |b|^2 -
+// 2 a.b (a the query, b the point, group-centred by norm_sd) is a product of
+// vectors: the six dimensions, |a|^2 by 1 and 1 by |b|^2.  Each entry, scaled
+// by powers of two, is held as two halves (hi + lo, 22 bits; k_sub_pack), and
+// one 16x16x32 product takes hi.hi, hi.lo, lo.hi and lo.lo of 16 points by 16
+// queries: lane l holds row (column) l % 16 and the eight k of quarter
+// l / 16; quarters 0 and 1 of the points are hi, 2 and 3 lo, of the queries 0
+// and 2 hi, 1 and 3 lo.  The result's lane l holds rows 4 (l / 16) + i of
+// column l % 16.
+//
+// The error of that value is below kPairEps (|a|^2 + |b|^2) (2^-22 of each
+// product for the split, 32 sums in FP32, each to 2^-23) plus 1.5e-4 (2 |a| +
+// |b|) + 1 for lo parts below the smallest normal half, 2^-14, taken as zero.
+// With |b| <= |a| + d the thresholds leave that much room on both sides of a
+// radius: a pair above `may` is certainly not closer, one below `sure`
+// certainly is, and the few between are decided by the reference's own float
+// expression.  Values and thresholds are compared as integers: the order of
+// floats where either is positive.
+//
+// Bound by vector issue: a chunk costs 16 products of 16 cycles, beside about
+// 75 vector instructions to test them and 25 more per tile that holds a pair,
+// where the float expression alone takes 14 per point and 64 queries (900 per
+// chunk).  4,000 FOF groups of 7.34M particles: next-closest 12.6 ms with a
+// tree walk of scalar leaf points, 7.8 with each leaf (18 points) multiplied
+// about the wavefront's centre, 3.9 with whole chunks packed once; linking
+// 12.1, 6.8 and 3.3 ms.
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+constexpr float kPairEps = 1.5258789e-5f;  // 2^-16
+constexpr float kPairUnit = 8192.0f;       // |b|^2 / kPairUnit fits a half
+
+struct PackPoint {
+    half8 hi, lo;
+};
+
+// a box of points; the boxes of each 64 slots and of each 64 such chunks
+struct Box6 {
+    float lo[6], hi[6];
+};
+
+// The power of two that brings a group's largest coordinate into [4096,
+// 8192), so that twice a coordinate fits a half.
+__device__ __forceinline__ float pair_scale(const Node6 &root) {
+    float m = 0.0f;
+    for (int k = 0; k < 6; k++)
+        m = fmaxf(m, fmaxf(__builtin_fabsf(root.lo[k]), __builtin_fabsf(root.hi[k])));
+    if (!(m > 0.0f && m < __builtin_inff())) return 1.0f;
+    return __builtin_ldexpf(1.0f, min(13 - __builtin_amdgcn_frexp_expf(m), 100));
+}
+
+// Each slot's vector in halves (as a point: the six dimensions, 1 and |b|^2),
+// and the box of each 64 slots.
+__global__ __launch_bounds__(kWave) void k_sub_pack(int32_t m, const int32_t *__restrict__ slot_group,
+                                                    const Node6 *__restrict__ nodes,
+                                                    const SParticle *__restrict__ w,
+                                                    PackPoint *__restrict__ pk,
+                                                    Box6 *__restrict__ chunks) {
+    const int32_t i = blockIdx.x * kWave + lane_id();
+    const bool in = i < m;
+    float x[6];
+    PackPoint p = {};
+    for (int k = 0; k < 6; k++) x[k] = 0.0f;
+    if (in) {
+        const SParticle q = w[i];
+        const float S = pair_scale(nodes[slot_group[i]]);
+        float n2 = 0.0f;
+        for (int k = 0; k < 6; k++) {
+            x[k] = q.pos[k];
+            const float v = x[k] * S;
+            p.hi[k] = (_Float16)v;
+            p.lo[k] = (_Float16)(v - (float)p.hi[k]);
+            n2 = __builtin_fmaf(v, v, n2);
+        }
+        n2 *= 1.0f / kPairUnit;
+        p.hi[6] = (_Float16)kPairUnit;
+        p.hi[7] = (_Float16)n2;
+        p.lo[7] = (_Float16)(n2 - (float)p.hi[7]);
     }
-    return d >= thr;
+    pk[i] = p;
+    Box6 b;
+    for (int k = 0; k < 6; k++) {
+        b.lo[k] = wave_min(in ? x[k] : __builtin_inff());
+        b.hi[k] = wave_max(in ? x[k] : -__builtin_inff());
+    }
+    if (lane_id() == 0) chunks[blockIdx.x] = b;
+}
+
+// the box of each 64 chunks
+__global__ __launch_bounds__(kWave) void k_sub_blocks(int32_t nc, const Box6 *__restrict__ chunks,
+                                                      Box6 *__restrict__ blocks) {
+    const int32_t i = blockIdx.x * kWave + lane_id();
+    Box6 b;
+    for (int k = 0; k < 6; k++) {
+        b.lo[k] = wave_min(i < nc ? chunks[i].lo[k] : __builtin_inff());
+        b.hi[k] = wave_max(i < nc ? chunks[i].hi[k] : -__builtin_inff());
+    }
+    if (lane_id() == 0) blocks[blockIdx.x] = b;
+}
+
+// The squared distance of a box and the box [lo, hi], a lower bound (in
+// float, term by term) of every pair's float distance between them.
+__device__ __forceinline__ float box_gap2(const Box6 &x, const float *lo, const float *hi) {
+    float d = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        const float e = fmaxf(fmaxf(x.lo[k] - hi[k], lo[k] - x.hi[k]), 0.0f);
+        d += e * e;
+    }
+    return d;
+}
+
+// v reduced over the lane's row of 16 (all lanes active)
+template <typename T, typename Op>
+__device__ __forceinline__ T row_reduce(T v, Op op) {
+    v = op(v, dpp_move<0xB1>(v));   // quad_perm [1, 0, 3, 2]
+    v = op(v, dpp_move<0x4E>(v));   // quad_perm [2, 3, 0, 1]
+    v = op(v, dpp_move<0x141>(v));  // row_half_mirror
+    return op(v, dpp_move<0x140>(v));  // row_mirror
+}
+
+// A wavefront's queries: four rows of 16 lanes, one per column tile of the
+// products, each with its box and its largest squared radius (consecutive
+// slots share leaves, so a row's box is about a leaf's).
+constexpr int kRows = kWave / 16;
+struct PairLds {
+    float lo[kRows][6], hi[kRows][6], far[kRows];
+    int32_t t[kWave];
+    uint32_t may[kWave][2], sure[kWave][2];  // per query, a bit per point of the chunk
+};
+
+struct PairSearch {
+    half8 b[kRows];
+    int32_t may[kRows], sure[kRows];  // thresholds of this lane's column, per column tile
+    float S, na;                      // the scale; this lane's query: |a|^2
+    half8 a[4];                       // the points of chunk `have`, read ahead
+    int32_t have;
+
+    // lane = query: its slot (any slot of the group where it is not valid)
+    __device__ __forceinline__ void init(int32_t slot, bool valid, const float (&c)[6], float scale,
+                                         const PackPoint *__restrict__ pk, PairLds &L) {
+        const int lane = lane_id(), col = lane & 15, q = lane >> 4;
+        S = scale;
+        na = 0.0f;
+        have = -1;
+        for (int k = 0; k < 6; k++) {
+            na = __builtin_fmaf(c[k] * S, c[k] * S, na);
+            const float lo = row_reduce(valid ? c[k] : __builtin_inff(), [](float a, float b) { return b < a ? b : a; });
+            const float hi = row_reduce(valid ? c[k] : -__builtin_inff(), [](float a, float b) { return b > a ? b : a; });
+            if (col == 0) {
+                L.lo[q][k] = lo;
+                L.hi[q][k] = hi;
+            }
+        }
+        L.may[lane][0] = L.may[lane][1] = 0;
+        L.sure[lane][0] = L.sure[lane][1] = 0;
+        L.t[lane] = slot;
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < kRows; t++) {
+            const PackPoint *p = pk + L.t[16 * t + col];
+            b[t] = ((q & 1) ? p->lo : p->hi) * (_Float16)-2.0f;
+            b[t][6] = (q & 1) ? p->lo[7] : p->hi[7];  // |a|^2, against the points' 1
+            b[t][7] = (q & 1) ? (_Float16)0.0f : (_Float16)kPairUnit;
+        }
+    }
+
+    // This lane's query takes pairs closer than the squared radius r2 (none
+    // where it is not valid).
+    __device__ __forceinline__ void radius(float r2, bool valid, PairLds &L) {
+        const int lane = lane_id(), col = lane & 15, q = lane >> 4;
+        const float s2 = (r2 * S) * S;
+        const float room = 3.0f * kPairEps * na + 1.0e-3f * sqrtf(na) + 1.5f;
+        const float up = s2 * 1.001f + room, dn = s2 * 0.999f - room;
+        const float f = row_reduce(valid ? r2 : 0.0f, [](float a, float b) { return b > a ? b : a; });
+        __syncthreads();
+        if (col == 0) L.far[q] = f;
+        L.t[lane] = valid ? __float_as_int(up) : INT32_MIN;
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < kRows; t++) may[t] = L.t[16 * t + col];
+        __syncthreads();
+        L.t[lane] = valid && dn > 0.0f ? __float_as_int(dn) : INT32_MIN;
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < kRows; t++) sure[t] = L.t[16 * t + col];
+    }
+
+    __device__ __forceinline__ void points(const PackPoint *__restrict__ pk, int32_t k,
+                                           half8 (&x)[4]) const {
+        const int lane = lane_id(), col = lane & 15, q = lane >> 4;
+#pragma unroll
+        for (int r = 0; r < 4; r++) x[r] = (&pk[k * kWave + 16 * r + col].hi)[q >> 1];
+    }
+
+    // The slots of chunk k against the queries of the rows in `rows`: per
+    // query the bits of the points that may be, and that certainly are,
+    // closer.  The points of chunk `next` are read meanwhile.
+    template <bool SURE>
+    __device__ __forceinline__ void chunk(const PackPoint *__restrict__ pk, int32_t k, int32_t next,
+                                          uint32_t rows, PairLds &L, uint64_t &m_may,
+                                          uint64_t &m_sure) {
+        const int lane = lane_id(), col = lane & 15, q = lane >> 4;
+        if (have != k) points(pk, k, a);
+        half8 ahead[4];
+        points(pk, next, ahead);
+#pragma unroll
+        for (int t = 0; t < kRows; t++) {
+            if (!(rows >> t & 1)) continue;
+            const floatx4 zero = {};
+            floatx4 v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                v[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[r], b[t], zero, 0, 0, 0);
+            int32_t low[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                low[r] = min(min(min(__float_as_int(v[r][0]), __float_as_int(v[r][1])),
+                                 __float_as_int(v[r][2])), __float_as_int(v[r][3]));
+            if (!ballot(min(min(low[0], low[1]), min(low[2], low[3])) < may[t])) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (!ballot(low[r] < may[t])) continue;
+                uint32_t nm = 0, ns = 0;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    nm |= __float_as_int(v[r][i]) < may[t] ? 1u << i : 0u;
+                    if constexpr (SURE) ns |= __float_as_int(v[r][i]) < sure[t] ? 1u << i : 0u;
+                }
+                const int sh = 16 * (r & 1) + 4 * q;
+                if (nm) {
+                    atomicOr(&L.may[16 * t + col][r >> 1], nm << sh);
+                    if constexpr (SURE) atomicOr(&L.sure[16 * t + col][r >> 1], ns << sh);
+                }
+            }
+        }
+        __syncthreads();
+        m_may = ((uint64_t)L.may[lane][1] << 32) | L.may[lane][0];
+        L.may[lane][0] = L.may[lane][1] = 0;
+        m_sure = 0;
+        if constexpr (SURE) {
+            m_sure = ((uint64_t)L.sure[lane][1] << 32) | L.sure[lane][0];
+            L.sure[lane][0] = L.sure[lane][1] = 0;
+        }
+        for (int r = 0; r < 4; r++) a[r] = ahead[r];
+        have = next;
+    }
+};
+
+// Calls f(chunk, next, rows) for the chunks [k0, k1) that lie within a row's
+// radius of its box (rows: which), in array order: 64 blocks of 64 chunks,
+// then 64 chunks, are tested at a time, one per lane.  next: the chunk of the
+// call after this one, where it is known, else the same.
+template <class F>
+__device__ __forceinline__ void near_chunks(const Box6 *__restrict__ chunks,
+                                            const Box6 *__restrict__ blocks, int32_t k0,
+                                            int32_t k1, const PairLds &L, F &&f) {
+    const int lane = lane_id();
+    for (int32_t b0 = k0 / kWave; b0 * kWave < k1; b0 += kWave) {
+        uint64_t mb = 1;
+        if ((b0 + 1) * kWave < k1) {  // more than one block is left
+            const int32_t bi = b0 + lane;
+            const Box6 x = blocks[min(bi, (k1 - 1) / kWave)];
+            bool near = false;
+#pragma unroll
+            for (int t = 0; t < kRows; t++) near |= box_gap2(x, L.lo[t], L.hi[t]) < L.far[t];
+            mb = ballot(bi * kWave < k1 && near);
+        }
+        while (mb) {
+            const int32_t base = (b0 + __builtin_ctzll(mb)) * kWave;
+            mb &= mb - 1;
+            const int32_t ki = base + lane;
+            const bool in = ki >= k0 && ki < k1;
+            const Box6 x = chunks[in ? ki : k0];
+            uint64_t mr[kRows], ml = 0;
+#pragma unroll
+            for (int t = 0; t < kRows; t++) {
+                mr[t] = ballot(in && box_gap2(x, L.lo[t], L.hi[t]) < L.far[t]);
+                ml |= mr[t];
+            }
+            while (ml) {
+                const int k = __builtin_ctzll(ml);
+                ml &= ml - 1;
+                uint32_t rows = 0;
+#pragma unroll
+                for (int t = 0; t < kRows; t++) rows |= (uint32_t)(mr[t] >> k & 1) << t;
+                f(base + k, base + (ml ? __builtin_ctzll(ml) : k), rows);
+            }
+        }
+    }
+}
+
+// bits of the slots of the chunk from `base` that lie in [lo, hi)
+__device__ __forceinline__ uint64_t slot_bits(int32_t base, int32_t lo, int32_t hi) {
+    const int32_t a = lo - base, b = hi - base;
+    const uint64_t from = a <= 0 ? ~0ull : (a >= 64 ? 0ull : ~0ull << a);
+    const uint64_t to = b <= 0 ? 0ull : (b >= 64 ? ~0ull : (1ull << b) - 1ull);
+    return from & to;
 }
 
 // fast3tree_find_next_closest_distance (src/fast3tree.c:992-1030) for 64
@@ -926,67 +1224,66 @@ __device__ __forceinline__ bool box_far(const Node6 &nd, const float (&c)[6], fl
 // when D >= T and sqrt(D) otherwise -- unless a value D' with
 // D < D' <= D (1 + 2^-21) was taken first, whose round trip
 // fl(fl(sqrt(D'))^2) can fall to D or below and reject it.  The wavefront
-// walks the tree once for all its lanes (a node is entered when any lane
-// may find a value below its bound there), each lane keeps the two smallest
-// distinct values, and a lane whose two are that close repeats the search
-// in the reference's own order.
+// goes through the chunks any of its lanes may find a value below its bound
+// in, each lane keeps the two smallest distinct values below it, and a lane
+// whose two are that close repeats the search in the reference's own order.
 __global__ __launch_bounds__(kWave) void k_sub_next_closest(
     const SubGroup *__restrict__ groups, const SubTile *__restrict__ qtiles,
     const int32_t *__restrict__ qpos, const int32_t *__restrict__ qidx,
-    const SParticle *__restrict__ w, const Node6 *__restrict__ nodes, float *__restrict__ dist,
-    int ordered) {
+    const SParticle *__restrict__ w, const Node6 *__restrict__ nodes,
+    const int32_t *__restrict__ slot_leaf, const PackPoint *__restrict__ pk,
+    const Box6 *__restrict__ chunks,
+    const Box6 *__restrict__ blocks, float *__restrict__ dist, int ordered) {
+    __shared__ PairLds L;
     const SubTile tl = qtiles[blockIdx.x];
     const SubGroup g = groups[tl.group];
     const int32_t q = tl.off + lane_id();
     const bool valid = q < g.nsample;
     const int32_t root = tl.group;
     float c[6] = {0, 0, 0, 0, 0, 0};
-    int32_t skip = -1, s_lo = 0, s_hi = 0;
+    int32_t skip = -1, s_lo = 0, s_hi = 0, slot = g.off;
     float r0 = 0.0f, T = 0.0f;
     if (valid) {
-        const SParticle me = w[g.off + (g.drawn ? qpos[g.draw_off + q] : q)];
+        slot = g.off + (g.drawn ? qpos[g.draw_off + q] : q);
+        const SParticle me = w[slot];
         for (int k = 0; k < 6; k++) c[k] = me.pos[k];
-        r0 = (float)sqrt((double)nc_start(c, root, w, nodes, &skip));
+        r0 = (float)sqrt((double)nc_start(c, root, slot_leaf[slot], w, nodes, &skip));
         T = r0 * r0;
         s_lo = nodes[skip].start;
         s_hi = s_lo + nodes[skip].n;
     }
     float m1 = __builtin_inff(), m2 = __builtin_inff();
     float thr = valid ? T : 0.0f;  // nothing at or above T is ever taken
-    int32_t cur = ordered ? -1 : root;
-    while (cur >= 0) {
-        cur = uniform(cur);
-        const Node6 x = load_const(nodes + cur);
-        const bool inside = x.start >= s_lo && x.start + x.n <= s_hi;  // the skipped subtree
-        const bool need = valid && !inside && !box_far(x, c, thr);
-        if (!ballot(need)) {
-            cur = x.skip;
-            continue;
-        }
-        if (x.div >= 0) {
-            cur = x.left;
-            continue;
-        }
-        // the leaf's points at wavefront-uniform addresses: scalar loads
-        const int32_t x0 = uniform(x.start), xn = uniform(x.n);
-        for (int32_t t = 0; t < xn; t++) {
-            const SParticle pt = load_const(w + x0 + t);
-            float d = 0.0f;
-            for (int k = 0; k < 6; k++) {
-                const float dx = c[k] - pt.pos[k];
-                d += dx * dx;
-            }
-            if (need) {
-                if (d < m1) {
-                    m2 = m1;
-                    m1 = d;
-                } else if (d > m1 && d < m2) {
-                    m2 = d;
+    if (!ordered) {
+        PairSearch P;
+        P.init(slot, valid, c, pair_scale(nodes[root]), pk, L);
+        P.radius(thr, valid, L);
+        near_chunks(chunks, blocks, g.off / kWave, (g.off + g.n + kWave - 1) / kWave, L,
+                    [&](int32_t k, int32_t next, uint32_t rows) {
+            const int32_t base = k * kWave;
+            uint64_t may, sure;
+            P.chunk<false>(pk, k, next, rows, L, may, sure);
+            // the group's slots outside the skipped subtree
+            may &= slot_bits(base, g.off, g.off + g.n) & ~slot_bits(base, s_lo, s_hi);
+            if (!valid) may = 0;
+            if (!ballot(may != 0)) return;
+            while (ballot(may != 0)) {
+                if (may) {
+                    const int t = __builtin_ctzll(may);
+                    may &= may - 1;
+                    const float d = dist6(c, w[base + t]);
+                    if (d < m1) {
+                        m2 = m1;
+                        m1 = d;
+                    } else if (d > m1 && d < m2) {
+                        m2 = d;
+                    }
                 }
             }
-        }
-        if (need && m1 < thr) thr = fminf(thr, m1 * 1.000002f);
-        cur = x.skip;
+            const float was = thr;
+            if (m1 < thr) thr = fminf(thr, m1 * 1.000002f);
+            if (ballot(thr < was)) P.radius(thr, valid, L);
+        });
     }
     if (!valid) return;
     float r;
@@ -1148,26 +1445,28 @@ __global__ void k_sub_init(int32_t m, int32_t *__restrict__ kmin, int32_t *__res
 
 // Each particle's sphere search over the later slots: the later particles
 // closer than the group's length, appended to `edges` in the order the
-// search lists them.  64 consecutive slots per wavefront walk the tree
-// together: a node is entered when some lane's sphere reaches it and it
-// holds slots after that lane's, and each leaf's points are loaded once and
-// passed lane to lane.  Every pair is tested with the reference's float
-// distance.  The append counter keeps counting past cap_edges (nothing is
-// written there), so the host can size the list and run again.
+// search lists them (array order).  64 consecutive slots per wavefront go
+// through the chunks from their own on; the pairs are decided on the matrix
+// cores, those near the length with the reference's float distance.  The
+// append counter keeps counting past cap_edges (nothing is written there), so
+// the host can size the list and run again.
 __global__ __launch_bounds__(kWave) void k_sub_link(const SubGroup *__restrict__ groups,
                                                     const SubTile *__restrict__ ltiles,
                                                     const float *__restrict__ target,
                                                     const SParticle *__restrict__ w,
                                                     const Node6 *__restrict__ nodes,
+                                                    const PackPoint *__restrict__ pk,
+                                                    const Box6 *__restrict__ chunks,
+                                                    const Box6 *__restrict__ blocks,
                                                     EdgeRec *__restrict__ edges, int64_t cap_edges,
                                                     int32_t *__restrict__ deg,
                                                     int32_t *__restrict__ counters) {
-    __shared__ float4 s_pts[kWave][2];
+    __shared__ PairLds L;
     __shared__ EdgeRec s_e[kLinkStage];
     const SubTile tl = ltiles[blockIdx.x];
     const SubGroup g = groups[tl.group];
-    const int32_t i = g.off + tl.off + lane_id();
-    const bool valid = tl.off + lane_id() < g.n;
+    const int32_t i = g.off + tl.off + lane_id(), end = g.off + g.n;
+    const bool valid = i < end;
     const float r = target[tl.group];
     const float r2 = r * r;
     float c[6] = {0, 0, 0, 0, 0, 0};
@@ -1189,76 +1488,54 @@ __global__ __launch_bounds__(kWave) void k_sub_link(const SubGroup *__restrict__
         __syncthreads();
         staged = 0;
     };
-    int32_t cur = tl.group;
-    while (cur >= 0) {
-        cur = uniform(cur);
-        const Node6 x = load_const(nodes + cur);
-        const bool need = valid && x.start + x.n > i + 1 && !box_apart(x, c, r);
-        if (!ballot(need)) {
-            cur = x.skip;
-            continue;
-        }
-        if (x.div >= 0) {
-            cur = x.left;
-            continue;
-        }
-        // the leaf's points, one per lane, staged in LDS and read back by
-        // every lane at the same address (a broadcast; a leaf whose split
-        // failed can hold more than a wavefront of points)
-        for (int32_t base = 0; base < x.n; base += kWave) {
-            const int32_t cnt = min(x.n - base, kWave);
-            if (lane_id() < cnt) {
-                const SParticle q = w[x.start + base + lane_id()];
-                s_pts[lane_id()][0] = make_float4(q.pos[0], q.pos[1], q.pos[2], q.pos[3]);
-                s_pts[lane_id()][1] = make_float4(q.pos[4], q.pos[5], 0.0f, 0.0f);
-            }
-            __syncthreads();
-            uint64_t hit = 0;
-            for (int32_t t = 0; t < cnt; t++) {
-                const float4 a = s_pts[t][0], b = s_pts[t][1];
-                const float pp[6] = {a.x, a.y, a.z, a.w, b.x, b.y};
-                float d = 0.0f;
-                for (int k = 0; k < 6; k++) {
-                    const float dx = c[k] - pp[k];
-                    d += dx * dx;
-                }
-                const int32_t j = x.start + base + t;
-                if (need && j > i && d < r2) hit |= 1ull << t;
-            }
-            __syncthreads();
-            // the chunk's pairs: lanes in order, each lane's in order, staged
-            // in LDS (appended directly when they alone overfill it)
-            const int32_t nh = __popcll(hit);
-            const int32_t incl = wave_scan_add(nh);
-            const int32_t tot = __builtin_amdgcn_readlane(incl, kWave - 1);
-            if (tot) {
-                if (staged + tot > kLinkStage) flush();
-                int32_t rank = listed;
-                if (tot > kLinkStage) {
-                    unsigned long long at = 0;
-                    if (lane_id() == 0) at = atomicAdd(ecount, (unsigned long long)tot);
-                    int64_t pos = (int64_t)read_lane(at, 0) + (incl - nh);
-                    while (hit) {
-                        const int t = __builtin_ctzll(hit);
-                        hit &= hit - 1;
-                        if (pos < cap_edges) edges[pos] = EdgeRec{i, x.start + base + t, rank};
-                        pos++;
-                        rank++;
-                    }
-                } else {
-                    int32_t at = staged + incl - nh;
-                    while (hit) {
-                        const int t = __builtin_ctzll(hit);
-                        hit &= hit - 1;
-                        s_e[at++] = EdgeRec{i, x.start + base + t, rank++};
-                    }
-                    staged += tot;
-                }
-                listed += nh;
+    PairSearch P;
+    P.init(valid ? i : g.off, valid, c, pair_scale(nodes[tl.group]), pk, L);
+    P.radius(r2, valid, L);
+    near_chunks(chunks, blocks, (g.off + tl.off) / kWave, (end + kWave - 1) / kWave, L,
+                [&](int32_t k, int32_t next, uint32_t rows) {
+        const int32_t base = k * kWave;
+        uint64_t may, hit;
+        P.chunk<true>(pk, k, next, rows, L, may, hit);
+        const uint64_t later = valid ? slot_bits(base, i + 1, end) : 0ull;
+        hit &= later;
+        uint64_t amb = may & later & ~hit;
+        if (!ballot((hit | amb) != 0)) return;
+        while (ballot(amb != 0)) {
+            if (amb) {
+                const int t = __builtin_ctzll(amb);
+                amb &= amb - 1;
+                if (dist6(c, w[base + t]) < r2) hit |= 1ull << t;
             }
         }
-        cur = x.skip;
-    }
+        // the chunk's pairs: lanes in order, each lane's in order, staged in
+        // LDS (appended directly when they alone overfill it)
+        const int32_t nh = __popcll(hit);
+        const int32_t incl = wave_scan_add(nh);
+        const int32_t tot = __builtin_amdgcn_readlane(incl, kWave - 1);
+        if (staged + tot > kLinkStage) flush();
+        int32_t rank = listed;
+        if (tot > kLinkStage) {
+            unsigned long long at = 0;
+            if (lane_id() == 0) at = atomicAdd(ecount, (unsigned long long)tot);
+            int64_t pos = (int64_t)read_lane(at, 0) + (incl - nh);
+            while (hit) {
+                const int t = __builtin_ctzll(hit);
+                hit &= hit - 1;
+                if (pos < cap_edges) edges[pos] = EdgeRec{i, base + t, rank};
+                pos++;
+                rank++;
+            }
+        } else {
+            int32_t at = staged + incl - nh;
+            while (hit) {
+                const int t = __builtin_ctzll(hit);
+                hit &= hit - 1;
+                s_e[at++] = EdgeRec{i, base + t, rank++};
+            }
+            staged += tot;
+        }
+        listed += nh;
+    });
     if (staged) flush();
     if (valid) deg[i] = listed;
 }

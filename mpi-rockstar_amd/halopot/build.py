@@ -6,6 +6,10 @@ Flags:
                       code are never fused; hot loops use explicit fmaf
   -Xclang -target-feature -Xclang -packed-fp32-ops
                       no packed FP32 instructions are generated
+  -mllvm -amdgpu-mfma-vgpr-form
+                      matrix products write vector registers (their results are
+                      compared at once: without it every one is first moved out
+                      of an accumulation register)
   -fvisibility=hidden only the C ABI of include/halopot.h is exported
 """
 from __future__ import annotations
@@ -32,7 +36,7 @@ def hipcc() -> str:
 def command(out: pathlib.Path = LIB, extra=()) -> list[str]:
     return [
         hipcc(), "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
-        "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+        "-ffp-contract=off", "-mllvm", "-amdgpu-mfma-vgpr-form", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
         "-fvisibility=hidden", "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
         f"-I{ROOT / 'include'}", *extra, "-o", str(out), str(CSRC / "hp_lib.hip"),
     ]

@@ -185,6 +185,35 @@ def test_gpu_subfof_empty_groups_and_mixed_levels(restatement):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("spread", [1.0, 3e3, 1e6])
+def test_gpu_subfof_chunk_edges(restatement, spread):
+    """The searches' chunks of 64 slots and blocks of 64 chunks: groups that
+    end on, before and after their edges, so that chunks hold the end of one
+    group and the start of the next; with outliers far outside the group along two axes (the
+    packed coordinates' common scale leaves the others few bits, so that more
+    pairs are decided by the float distance) and a lattice, whose distances
+    equal the linking length.  Coordinates are multiples of 2^-12, so that
+    norm_sd's sums of them are exact in any order, and the outliers leave its
+    smallest eigenvalues alone."""
+    rng = np.random.default_rng(11)
+    plist = []
+    for n in (41, 63, 64, 65, 127, 129, 1, 4031, 4096, 4097, 63, 8191):
+        x = rng.normal(size=(n, 6))
+        x[: n // 3] *= 0.05
+        if n > 40:
+            x[rng.integers(0, n, 2)[:, None], [1, 4]] *= spread
+        p = np.zeros(n, catalog.PARTICLE_DTYPE)
+        p["id"] = np.arange(n)
+        p["pos"] = np.round(x * 4096) / 4096
+        plist.append(p)
+    lat = np.stack(np.meshgrid(*[np.arange(4)] * 6, indexing="ij"), -1).reshape(-1, 6)
+    p = np.zeros(lat.shape[0], catalog.PARTICLE_DTYPE)
+    p["pos"] = lat
+    plist.append(p)
+    _check_batch(restatement, plist)
+
+
+@pytest.mark.gpu
 def test_gpu_subfof_exact_ll_and_lower_levels(restatement):
     fg = catalog.fof_groups(seed=5, n_groups=6, lo=300, hi=12000)
     plist = [fg.particles[f:f + n].copy() for f, n in fg.groups]
