@@ -1656,9 +1656,9 @@ constexpr int kTokThreads = 1024;
 constexpr int kTokLds = 12288;  // a group's numbers held in LDS up to this many
 constexpr int kTokHash = 1024;  // one chunk's root pairs, deduplicated
 
-// root of x with path halving, in the group's table u (LDS, or global when
-// the group has more than kTokLds numbers; one workgroup only)
-template <bool kLds>
+// root of x, in the group's table u (LDS, or global when the group has more
+// than kTokLds numbers; one workgroup only); kHalve: with path halving
+template <bool kLds, bool kHalve = true>
 __device__ __forceinline__ int32_t tok_find(int32_t *u, int32_t x) {
     if constexpr (kLds) {
         volatile int32_t *v = u;
@@ -1666,7 +1666,7 @@ __device__ __forceinline__ int32_t tok_find(int32_t *u, int32_t x) {
             const int32_t y = v[x];
             if (y == x) return x;
             const int32_t z = v[y];
-            if (z != y) v[x] = z;
+            if (kHalve && z != y) v[x] = z;
             x = z;
         }
     } else {
@@ -1674,7 +1674,8 @@ __device__ __forceinline__ int32_t tok_find(int32_t *u, int32_t x) {
             const int32_t y = __hip_atomic_load(u + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (y == x) return x;
             const int32_t z = __hip_atomic_load(u + y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (z != y) __hip_atomic_store(u + x, z, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (kHalve && z != y)
+                __hip_atomic_store(u + x, z, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             x = z;
         }
     }
@@ -1744,8 +1745,10 @@ __device__ void tok_group(int32_t *u, int32_t nl, int32_t q0, int32_t q1, int32_
             }
         __syncthreads();
     }
+    // a global table is the result itself, so the last finds leave it alone: a
+    // halving store could land on a number's root after its own thread's
     for (int32_t k = threadIdx.x; k < nl; k += kTokThreads) {
-        const int32_t rt = tok_find<kLds>(u, k);
+        const int32_t rt = tok_find<kLds, kLds>(u, k);
         __hip_atomic_store(root + L0 + k, rt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
