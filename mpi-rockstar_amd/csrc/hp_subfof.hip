@@ -1656,35 +1656,40 @@ constexpr int kTokThreads = 1024;
 constexpr int kTokLds = 12288;  // a group's numbers held in LDS up to this many
 constexpr int kTokHash = 1024;  // one chunk's root pairs, deduplicated
 
-// root of x, in the group's table u (LDS, or global when the group has more
-// than kTokLds numbers; one workgroup only); kHalve: with path halving
-template <bool kLds, bool kHalve = true>
-__device__ __forceinline__ int32_t tok_find(int32_t *u, int32_t x) {
-    if constexpr (kLds) {
-        volatile int32_t *v = u;
-        for (;;) {
-            const int32_t y = v[x];
-            if (y == x) return x;
-            const int32_t z = v[y];
-            if (kHalve && z != y) v[x] = z;
-            x = z;
-        }
-    } else {
-        for (;;) {
-            const int32_t y = __hip_atomic_load(u + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (y == x) return x;
-            const int32_t z = __hip_atomic_load(u + y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (kHalve && z != y)
-                __hip_atomic_store(u + x, z, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            x = z;
-        }
-    }
-}
-
+// A group's union-find table: in LDS, or global when the group has more than
+// kTokLds numbers (one workgroup only).  The LDS form keeps the address space
+// in its pointer: through a generic one its accesses would be flat ones.
 template <bool kLds>
-__device__ __forceinline__ void tok_set(int32_t *u, int32_t x, int32_t v) {
-    if constexpr (kLds) *(volatile int32_t *)(u + x) = v;
-    else __hip_atomic_store(u + x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+struct TokTable;
+
+template <>
+struct TokTable<true> {
+    volatile __attribute__((address_space(3))) int32_t *u;
+    __device__ __forceinline__ int32_t get(int32_t x) const { return u[x]; }
+    __device__ __forceinline__ void set(int32_t x, int32_t v) const { u[x] = v; }
+};
+
+template <>
+struct TokTable<false> {
+    int32_t *u;
+    __device__ __forceinline__ int32_t get(int32_t x) const {
+        return __hip_atomic_load(u + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void set(int32_t x, int32_t v) const {
+        __hip_atomic_store(u + x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+};
+
+// root of x; kHalve: with path halving
+template <bool kHalve = true, class Table>
+__device__ __forceinline__ int32_t tok_find(const Table &u, int32_t x) {
+    for (;;) {
+        const int32_t y = u.get(x);
+        if (y == x) return x;
+        const int32_t z = u.get(y);
+        if (kHalve && z != y) u.set(x, z);
+        x = z;
+    }
 }
 
 struct TokShared {
@@ -1697,21 +1702,25 @@ struct TokShared {
 // One group's merges, a chunk of kTokThreads pairs at a time.  Every thread
 // finds its pair's two roots as the chunk starts; a pair whose roots are
 // equal then, or equal as a set to an earlier pair's of the chunk, cannot
-// merge.  One thread replays the others in order: the root of step i's small
-// FOF under the root of the listed particle's.
+// merge.  One wavefront replays the others in order: the root of step i's
+// small FOF under the root of the listed particle's.  It finds the roots of 64
+// pairs at once and keeps them up to date in registers as the pairs merge, so
+// that a merge is a few lane moves and not a chain of dependent table reads
+// (4,000 groups: 1.55 -> 0.46 ms together with LDS accesses in place of flat
+// ones; one group of 11,000 particles 0.48 -> 0.11 ms).
 template <bool kLds>
-__device__ void tok_group(int32_t *u, int32_t nl, int32_t q0, int32_t q1, int32_t L0,
+__device__ void tok_group(const TokTable<kLds> &u, int32_t nl, int32_t q0, int32_t q1, int32_t L0,
                           const int2 *__restrict__ ev, int32_t *__restrict__ root,
                           TokShared &S) {
-    for (int32_t k = threadIdx.x; k < nl; k += kTokThreads) tok_set<kLds>(u, k, k);
+    for (int32_t k = threadIdx.x; k < nl; k += kTokThreads) u.set(k, k);
     __syncthreads();
     for (int32_t base = q0; base < q1; base += kTokThreads) {
         const int32_t q = base + threadIdx.x;
         int32_t ra = 0, rb = 0;
         if (q < q1) {
             const int2 p = ev[q];
-            ra = tok_find<kLds>(u, p.x - L0);
-            rb = tok_find<kLds>(u, p.y - L0);
+            ra = tok_find(u, p.x - L0);
+            rb = tok_find(u, p.y - L0);
         }
         for (int k = threadIdx.x; k < kTokHash; k += kTokThreads) {
             S.key[k] = 0ull;
@@ -1738,17 +1747,30 @@ __device__ void tok_group(int32_t *u, int32_t nl, int32_t q0, int32_t q1, int32_
         const int at = block_rank<kTokThreads>(keep, &tot, S.w);
         if (keep) S.pair[at] = make_int2(ra, rb);
         __syncthreads();
-        if (threadIdx.x == 0)
-            for (int k = 0; k < tot; k++) {
-                const int32_t a = tok_find<kLds>(u, S.pair[k].x), b = tok_find<kLds>(u, S.pair[k].y);
-                if (a != b) tok_set<kLds>(u, a, b);
+        if (threadIdx.x < kWave)
+            for (int32_t k0 = 0; k0 < tot; k0 += kWave) {
+                const int32_t n = min(tot - k0, kWave);
+                int32_t a = 0, b = 0;
+                if (lane_id() < n) {
+                    a = tok_find(u, S.pair[k0 + lane_id()].x);
+                    b = tok_find(u, S.pair[k0 + lane_id()].y);
+                }
+                for (int32_t k = 0; k < n; k++) {
+                    const int32_t x = __builtin_amdgcn_readlane(a, k);
+                    const int32_t y = __builtin_amdgcn_readlane(b, k);
+                    if (x == y) continue;
+                    if (lane_id() == 0) u.set(x, y);
+                    a = a == x ? y : a;
+                    b = b == x ? y : b;
+                }
+                if constexpr (!kLds) __threadfence();  // the next roots are read by other lanes
             }
         __syncthreads();
     }
     // a global table is the result itself, so the last finds leave it alone: a
     // halving store could land on a number's root after its own thread's
     for (int32_t k = threadIdx.x; k < nl; k += kTokThreads) {
-        const int32_t rt = tok_find<kLds, kLds>(u, k);
+        const int32_t rt = tok_find<kLds>(u, k);
         __hip_atomic_store(root + L0 + k, rt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
@@ -1768,8 +1790,11 @@ __global__ __launch_bounds__(kTokThreads) void k_sub_tokens(
     const int32_t nl = first_label[g.off + g.n] - L0;
     if (nl <= 0) return;
     const int32_t q0 = eoff[g.off], q1 = eoff[g.off + g.n];
-    if (nl <= kTokLds) tok_group<true>(s_u, nl, q0, q1, L0, ev, root, S);
-    else tok_group<false>(root + L0, nl, q0, q1, L0, ev, root, S);
+    if (nl <= kTokLds)
+        tok_group<true>({(volatile __attribute__((address_space(3))) int32_t *)s_u}, nl, q0, q1,
+                        L0, ev, root, S);
+    else
+        tok_group<false>({root + L0}, nl, q0, q1, L0, ev, root, S);
 }
 
 // each particle's sort value (its root's number in the group, -1 without a
