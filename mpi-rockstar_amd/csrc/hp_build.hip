@@ -26,10 +26,9 @@
 //             counter read.
 //   subtrees  every node of at most kSmallMax points is finished in one go:
 //             65..kSmallMax points by a workgroup (a kernel each for nodes of
-//             at most 256, 512 and 1,024 points), point-parallel per level
-//             (block prefix of the left flags, segmented DPP scans for the
-//             child boxes); at most 64 points by one wavefront, a point per
-//             lane.  Both keep the points and the node table in LDS, compute
+//             at most 256, 512 and 1,024 points), a thread per point down to
+//             nodes of at most 32 points, then by its wavefronts; at most 64
+//             points by one wavefront, a point per lane.  Both keep the points and the node table in LDS, compute
 //             centres of mass bottom-up and dmin over the final order, and
 //             write leaves straight into the final tree-order array.
 // Multipoles of the nodes made by the split levels (src/potential.c:71-124):
@@ -528,27 +527,33 @@ __device__ __forceinline__ int32_t group_pushes(const Sizes &s, int32_t nl, int3
 // ------------------------------------------------------------- subtrees
 //
 // A node of 65..kSmallMax points is finished by one workgroup, a node of at
-// most 64 points by one wavefront (below).  Both keep the points in LDS and
-// number the subtree's nodes locally in creation order: levels in order,
-// the two children of a split as a pair.
+// most 64 points by one wavefront.  Both keep the points in LDS.
 //
-// Workgroup subtrees are point-parallel per level over the whole subtree:
-// thread t takes positions t, t + 256, ...; a block-wide prefix of the
-// left flags (one 64-bit ballot per chunk of 64 positions) gives every
-// node's left count and every point's stable scatter position at once; the
-// children's tight boxes come from segmented scans over runs of lanes, one
-// LDS atomic per run and coordinate.  Per-node bookkeeping runs a thread per
-// node.  Local ids map onto a block of 2n - 2 global ids reserved with one
-// atomic when the subtree starts; ids it does not use are never referenced.
-// Centres of mass are combined bottom-up in LDS and dmin is computed over
-// the final order in LDS.
+// The workgroup has a thread per point and splits, level by level, only the
+// nodes of more than 32 points (at most 31 at a time); each level lists the
+// nodes' points by side, moves them to the in-place partition's order, and
+// takes the children's tight boxes from segmented scans over runs of lanes,
+// one LDS atomic per run and coordinate.  The nodes of at most 32 points are
+// then finished by its wavefronts, packed up to 64 points to a wavefront, as
+// the wavefront subtrees are, with no workgroup barrier: the deep levels, where most of a tree's nodes are,
+// cost a wavefront's own latency.  Last come the nodes above: centres of mass
+// bottom-up, dmin by a wavefront each over the final order.  (A workgroup of
+// 256 threads that split every node level by level took 13 us a level and
+// 162 us for a task of 1,024 points on its own; this one takes 72.  On the
+// one-GPU catalogue, 6.71M points: 796 -> 731, 320 -> 249 and 281 -> 227 us
+// for the three sizes, 160 -> 126 for the wavefront subtrees, whose segmented
+// scans are on integers now.)
+//
+// Nodes are numbered locally and mapped onto a block of 2n - 2 global ids
+// reserved for the subtree: the workgroup's levels first (2k ids for k
+// splits), then 2m - 2 for each of its k + 1 parts of m points, in position
+// order.  Ids that are not used are never referenced.
 
 constexpr int kWaveTask = 64;   // subtrees up to this size: one wavefront
 constexpr int kWaveMin = 32;    // the smallest wavefront/workgroup boundary (wave_max) used
 constexpr int kRootSkip = -2;   // local skip pointer: the subtree root's own skip
-constexpr int kSubThreads = 256;
-constexpr int kSubWaves = kSubThreads / kWave;
-constexpr uint8_t kNoEntry = 0xff;
+constexpr uint8_t kNone8 = 0xff;
+constexpr int kPart = 32;       // a workgroup splits nodes of more points than this level by level
 
 // The workgroup subtree kernel comes in three sizes, for nodes of at most
 // 256, 512 and 1,024 points: its LDS grows with the size, and the smaller
@@ -556,17 +561,6 @@ constexpr uint8_t kNoEntry = 0xff;
 // list per kernel (k_group_classes) before the kernels run.
 constexpr int kSubClasses = 3;
 __host__ __device__ constexpr int sub_class(int32_t n) { return n > 512 ? 2 : (n > 256 ? 1 : 0); }
-template <int kCap>
-struct SubSize {
-    static constexpr int chunks = kCap / kWave;                     // ballot chunks
-    static constexpr int list = 2 * (kCap / (kLeafPoints + 1)) + 2; // nodes of one level
-    static constexpr int nodes = 2 * kCap;                          // local ids (2n - 1 at most)
-    static constexpr int per_thread = nodes / kSubThreads;
-    static_assert(list < kNoEntry, "level entries fit a byte");
-    static_assert(kCap >= kSubThreads && kCap <= kSmallMax && kCap % kSubThreads == 0,
-                  "a whole number of positions per thread");
-};
-
 __device__ __forceinline__ uint64_t lanes_below(int i) {
     return i >= 64 ? ~0ull : ((1ull << i) - 1ull);
 }
@@ -579,10 +573,13 @@ __device__ __forceinline__ uint64_t lane_run(int lf, int n) {
 // Inclusive scan of v over this lane's run [seg, lane] of the wavefront
 // (seg <= lane; runs are contiguous), on DPP moves: row_shr 1, 2, 4, 8
 // within rows of 16, then row_bcast 15 and 31 across rows.
+// On integers (float_key), where a move and a minimum are one instruction.
+// (v_min_i32 with a lane move: 2 instructions a step against 6 on floats,
+// whose minimum first makes both operands canonical.)
 template <typename Op>
-__device__ __forceinline__ float seg_scan(float v, int seg, Op op) {
+__device__ __forceinline__ int seg_scan(int v, int seg, Op op) {
     const int lane = lane_id(), r = lane & 15;
-    float u;
+    int u;
     u = dpp_move<0x111>(v);
     if (r >= 1 && lane - 1 >= seg) v = op(v, u);
     u = dpp_move<0x112>(v);
@@ -598,14 +595,255 @@ __device__ __forceinline__ float seg_scan(float v, int seg, Op op) {
     return v;
 }
 
-struct SubEntry {       // a node of the level being split, 20 bytes
-    float lim;          // split plane, from the node's tight box
-    int16_t loc;        // local node id
-    int16_t lf, n, nl;  // first point (subtree-relative), points, left count
-    int16_t child;      // local id of the left child (splits), else -1
-    int16_t skip;       // local skip pointer
-    uint8_t kind, dim;  // 1: split; split dimension
+// ---- one wavefront, at most 64 points
+//
+// One point per lane, the points of one subtree or of several whose points
+// follow each other.  Each level, every lane tests its point against its
+// node's split plane; ballots give the left counts and the stable listing (a
+// node's points occupy a contiguous run of lanes), and the children's tight
+// boxes come from segmented scans across the lanes.  The node table stays in
+// LDS with local ids (the roots, then children in pairs, levels in order).
+// Centres of mass and dmin are computed with a lane per node, summing the
+// node's points in tree order, the order of the reference's loops.
+
+constexpr int kWaveNodes = 2 * kWaveTask;  // a tree over n points has at most 2n - 1 nodes
+constexpr int kSkipRoot = 128;             // skip >= this: that of root skip - kSkipRoot
+static_assert(kWaveNodes <= kSkipRoot && kSkipRoot + kWaveTask < kNone8, "local ids fit a byte");
+
+struct WaveTree {
+    union {
+        float lim[kWaveNodes];     // split planes, while the levels run
+        float com[3][kWaveNodes];  // then the centres of mass
+    };
+    float mass[kWaveNodes];
+    uint8_t dim[kWaveNodes], lf[kWaveNodes], cnt[kWaveNodes];
+    uint8_t left[kWaveNodes], skip[kWaveNodes];  // left: kNone8 for a leaf
+    uint8_t lev[kWaveNodes];     // each node's level
+    uint8_t st[kWaveTask];       // a level's points by side, node by node
 };
+
+// v, as a value that the compiler knows nothing about.
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// A wavefront's LDS accesses complete in order; the compiler has to keep
+// them so.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The subtrees of `nroots` nodes over the n points p of the lanes [0, n), in
+// tree order from position `first` on.  Root r (id(r), its skip pointer
+// skip(r)) holds the lanes from the r-th set bit of `heads` to the next; with
+// one root (kMany false) its split plane (dim, lim) is given.  Node ids [base, base + 2 (n - nroots)) (fits:
+// they are there; else the root stays a leaf and the error is flagged).  P: n
+// points of LDS.  Writes the points' order and leaves and every node's record
+// but the roots' boxes; the roots' centres and masses end in W.com[.][r],
+// W.mass[r].
+template <bool kMany, class Id, class Skip>
+__device__ __forceinline__ void wave_subtree(const BuildArgs &a, WaveTree &W, float4 *P, float4 p, int n,
+                             uint64_t heads, int nroots, int root_dim, float root_lim, int32_t first, int32_t base,
+                             bool fits, double particle_mass, Id &&root_id, Skip &&root_skip) {
+    const int lane = lane_id();
+    const bool v = lane < n;
+    const int root = kMany ? __popcll(heads & lanes_below(lane + 1)) - 1 : 0;
+    // this lane's node: its run of lanes [lf, lf + c)
+    int lf = 0, c = n, nid = root, M = nroots, nlev = 0;
+    if constexpr (kMany) {
+        lf = 63 - __builtin_clzll(heads & lanes_below(lane + 1));
+        const uint64_t after = heads & ~lanes_below(lane + 1);
+        c = (after ? __builtin_ctzll(after) : n) - lf;
+    }
+    auto gid = [&](int j) -> int32_t { return j < nroots ? root_id(j) : base + j - nroots; };
+    // the tight box of each run of the lanes `in`, in its last lane
+    auto boxes = [&](bool in, float (&lo)[3], float (&hi)[3]) {
+        auto mn = [](int x, int y) { return min(x, y); };
+        auto mx = [](int x, int y) { return max(x, y); };
+        const int seg = in ? lf : lane;
+        const int kx = float_key(p.x), ky = float_key(p.y), kz = float_key(p.z);
+        lo[0] = key_float(seg_scan(kx, seg, mn));
+        lo[1] = key_float(seg_scan(ky, seg, mn));
+        lo[2] = key_float(seg_scan(kz, seg, mn));
+        hi[0] = key_float(seg_scan(kx, seg, mx));
+        hi[1] = key_float(seg_scan(ky, seg, mx));
+        hi[2] = key_float(seg_scan(kz, seg, mx));
+    };
+    if constexpr (kMany) {
+        float lo[3], hi[3];
+        boxes(v, lo, hi);
+        if (v && lane == lf + c - 1) {
+            const int dm = split_dim(lo, hi);
+            W.lf[root] = (uint8_t)lf;
+            W.cnt[root] = (uint8_t)c;
+            W.dim[root] = (uint8_t)dm;
+            W.lim[root] = split_lim(lo, hi, dm);
+            W.left[root] = kNone8;
+            W.lev[root] = 0;
+            W.skip[root] = (uint8_t)(kSkipRoot + root);
+        }
+    } else if (lane == 0) {
+        W.lf[0] = 0;
+        W.cnt[0] = (uint8_t)n;
+        W.dim[0] = (uint8_t)root_dim;
+        W.lim[0] = root_lim;
+        W.left[0] = kNone8;
+        W.lev[0] = 0;
+        W.skip[0] = kSkipRoot;
+    }
+    wave_sync();
+    bool pend = v && c > kLeafPoints;
+    while (ballot(pend)) {
+        // src/fast3tree.c:751-774 (partition), 805-809 (failed split)
+        bool gl = false;
+        if (pend) gl = comp(p, W.dim[nid]) <= W.lim[nid];
+        const uint64_t mL = ballot(gl);
+        const uint64_t mN = pend ? lane_run(lf, c) : 0ull;
+        const int nl = __popcll(mL & mN);
+        const bool split = pend && nl > 0 && nl < c;
+        const uint64_t mH = ballot(split && lane == lf);
+        const int C = M + 2 * __popcll(mH & lanes_below(lf));
+        // the in-place partition's order (inplace_dest), from the node's
+        // points listed by side
+        const uint64_t below = mN & lanes_below(lane);
+        const int rank = gl ? __popcll(mL & below) : __popcll(~mL & below);
+        if (split) W.st[lf + (gl ? rank : nl + rank)] = (uint8_t)(lane - lf);
+        wave_sync();
+        if (split) {
+            P[lf + inplace_dest(lane - lf, gl, rank, c, nl,
+                                [&](int k) { return (int)W.st[lf + k]; })] = p;
+            if (lane == lf) {
+                W.lf[C] = (uint8_t)lf;
+                W.cnt[C] = (uint8_t)nl;
+                W.lf[C + 1] = (uint8_t)(lf + nl);
+                W.cnt[C + 1] = (uint8_t)(c - nl);
+                W.left[C] = W.left[C + 1] = kNone8;
+                W.lev[C] = W.lev[C + 1] = (uint8_t)(nlev + 1);
+                W.skip[C] = (uint8_t)(C + 1);
+                W.skip[C + 1] = W.skip[nid];
+                W.left[nid] = (uint8_t)C;
+            }
+        }
+        wave_sync();
+        if (split) {  // the point that came here, and its node
+            p = P[lane];
+            const bool right = lane - lf >= nl;
+            nid = C + (right ? 1 : 0);
+            lf += right ? nl : 0;
+            c = right ? c - nl : nl;
+        }
+        if (mH) {
+            M += 2 * __popcll(mH);
+            nlev++;
+        }
+        // tight boxes of the new children
+        float lo[3], hi[3];
+        boxes(split, lo, hi);
+        if (split && lane == lf + c - 1) {
+            const int dm = split_dim(lo, hi);
+            W.dim[nid] = (uint8_t)dm;
+            W.lim[nid] = split_lim(lo, hi, dm);
+            if (fits) {
+                Node *g = a.nodes + base + nid - nroots;
+                for (int d = 0; d < 3; d++) {
+                    g->lo[d] = lo[d];
+                    g->hi[d] = hi[d];
+                }
+            }
+        }
+        wave_sync();
+        pend = split && c > kLeafPoints;
+    }
+    // every lane's node is a leaf now (its box is there already)
+    if (M > nroots && !fits) {  // out of node ids: the root stays a leaf
+        if (lane == 0) {
+            atomicOr(&a.counters[kErrFlags], kErrCapacity);
+            W.left[0] = kNone8;
+        }
+        M = nroots;
+        nlev = 0;
+        nid = root;
+    }
+    if (v) {
+        P[lane] = p;
+        a.fin[first + lane] = p;
+        a.leaf_of[first + lane] = gid(nid);
+    }
+    wave_sync();
+    // leaf centres: f64 sums in tree order (src/potential.c:100-107)
+    for (int j = lane; j < M; j += kWave) {
+        if (W.left[j] != kNone8) continue;
+        const int lf = W.lf[j], c = W.cnt[j];
+        double sx = 0.0, sy = 0.0, sz = 0.0;
+#pragma unroll 5
+        for (int i = lf; i < lf + c; i++) {
+            const float4 q = P[i];
+            sx += (double)q.x;
+            sy += (double)q.y;
+            sz += (double)q.z;
+        }
+        const double dn = (double)c;
+        W.com[0][j] = sx != 0.0 ? (float)(sx / dn) : 0.0f;
+        W.com[1][j] = sy != 0.0 ? (float)(sy / dn) : 0.0f;
+        W.com[2][j] = sz != 0.0 ? (float)(sz / dn) : 0.0f;
+        W.mass[j] = (float)(particle_mass * dn);
+    }
+    wave_sync();
+    // internal centres, deepest level first (src/potential.c:115-122: float,
+    // right term first); a lane keeps its two nodes' places, so that a level
+    // is one round of table reads
+    const bool two = lane + kWave < M;
+    const int lev0 = lane < M ? W.lev[lane] : -1, lev1 = two ? W.lev[lane + kWave] : -1;
+    const int left0 = lane < M ? W.left[lane] : kNone8, left1 = two ? W.left[lane + kWave] : kNone8;
+    for (int L = nlev - 1; L >= 0; L--) {
+        for (int h = 0; h < 2; h++) {
+            const int cl = h ? left1 : left0;
+            if ((h ? lev1 : lev0) != L || cl == kNone8) continue;
+            const int j = lane + kWave * h;
+            const float ml = W.mass[cl], mr = W.mass[cl + 1];
+            const float m = ml + mr;
+            for (int d = 0; d < 3; d++) {
+                const float rr = W.com[d][cl + 1] * mr;
+                const float ll = W.com[d][cl] * ml;
+                W.com[d][j] = m != 0.0f ? (rr + ll) / m : 0.0f;
+            }
+            W.mass[j] = m;
+        }
+        wave_sync();
+    }
+    // dmin over each node's points in tree order (src/potential.c:71-82),
+    // then the node records: every field but the box (the root's is its
+    // creator's, the others were written with their level)
+    for (int j = lane; j < M; j += kWave) {
+        const int lf = W.lf[j], c = W.cnt[j];
+        const float com[3] = {W.com[0][j], W.com[1][j], W.com[2][j]};
+        double big = 0.0, sum = 0.0;
+#pragma unroll 4
+        for (int i = lf; i < lf + c; i++) {
+            const double d = d2_ref(com, P[i]);
+            big = d > big ? d : big;
+            sum += d;
+        }
+        Node nd;
+        finish_dmin(&nd, big, sum, c);
+        const int cl = W.left[j], sk = W.skip[j];
+        const int32_t id = gid(j);
+        Node *g = a.nodes + id;
+        for (int d = 0; d < 3; d++) g->com[d] = com[d];
+        g->mass = W.mass[j];
+        g->dmin2 = nd.dmin2;
+        g->first = first + lf;
+        g->count = c;
+        g->left = cl != kNone8 ? base + cl - nroots : -1;
+        g->skip = sk >= kSkipRoot ? root_skip(sk - kSkipRoot) : base + sk - nroots;
+        g->dmin = nd.dmin;
+        if (cl != kNone8)
+            a.parent[base + cl - nroots] = a.parent[base + cl + 1 - nroots] = id;
+    }
+    wave_sync();
+}
 
 // Splits the workgroup subtree tasks by size into the lists of the three
 // kernel sizes: list c at out + c * cap_group, counted in counters[kClassNext + c].
@@ -640,453 +878,432 @@ __global__ __launch_bounds__(256) void k_group_classes(const Task *__restrict__ 
     }
 }
 
-// One workgroup per task of the list `cls` (nodes of at most kCap points).
-// The two smaller sizes ask the compiler for 7 wavefronts per SIMD (72
-// VGPRs, a few values spilled outside the level loop): their LDS fits more
-// workgroups than their registers otherwise allowed, and the latency-bound
-// levels gain more from the extra wavefronts than the spills cost.
+// A node of more than kPart points of the workgroup's current level.
+struct SubEntry {
+    float lim;          // split plane, from the node's tight box
+    int16_t loc;        // local node id
+    int16_t lf, n, nl;  // first point (subtree-relative), points, left count
+    int16_t skip;       // local skip pointer
+    uint8_t split, dim; // whether both sides hold points; split dimension
+};
+
 template <int kCap>
-__global__ __launch_bounds__(kSubThreads, kCap <= 512 ? 7 : 1) void k_subtree(const float4 *__restrict__ A,
-                                                         const float4 *__restrict__ B,
-                                                         const Task *__restrict__ tasks,
-                                                         BuildArgs a, double particle_mass,
-                                                         int cls) {
-    constexpr int kSubChunks = SubSize<kCap>::chunks, kSubList = SubSize<kCap>::list,
-                  kSubNodes = SubSize<kCap>::nodes, kSubPerThread = SubSize<kCap>::per_thread;
-    // The points stay where they were loaded (P); the order is a 16-bit
-    // permutation, PM[buf][i] = the point at position i.  Once the levels are
-    // done, the final order is moved to PM[0] and the local nodes' centres of
-    // mass (CM) take the room of the level arrays: the LDS fits four
-    // workgroups per CU at 1,024 points.
-    struct Levels {
-        int16_t PM[2][kCap];
-        uint8_t Q[2][kCap];               // level entry of each position
-        SubEntry E[2][kSubList];
-        int32_t BOX[kSubList][6];         // next level's tight boxes, float keys
+struct SubLds {
+    static constexpr int kWaves = kCap / kWave;
+    static constexpr int kAct = kCap / (kPart + 1);  // nodes of more than kPart points at a time
+    static_assert(2 * kAct <= kWave, "a lane per child");
+    // local nodes whose table entries fit here
+    static constexpr int kTop = (3 * kCap / 16 + kWave - 1) / kWave * kWave;
+    float4 P[kCap];
+    WaveTree wt[kWaves];
+    union {
+        uint16_t st[kCap];      // a level's points by side, node by node
+        float4 cm[kTop];        // then the local nodes' centres of mass
     };
-    constexpr int kCM = (int)((sizeof(Levels) - sizeof(int16_t) * kCap) / sizeof(float4));
-    struct Centres {
-        int16_t PMF[kCap];                // the final order
-        float4 CM[kCM];                   // centres of mass of local nodes j < kCM
-    };
-    static_assert(sizeof(Centres) <= sizeof(Levels) && kCM >= kCap / 2, "centre room");
-    __shared__ float4 P[kCap];
-    __shared__ union Pool {
-        Levels lv;
-        Centres cm;
-    } pool;
-    auto &PM = pool.lv.PM;
-    auto &Q = pool.lv.Q;
-    auto &E = pool.lv.E;
-    auto &BOX = pool.lv.BOX;
-    __shared__ int16_t s_left[kSubNodes];     // left child of each local node, -1: leaf
-    __shared__ uint16_t s_lvl[kCap + 2]; // first local id of each level
-    __shared__ uint64_t s_mask[kSubChunks + 1];
-    __shared__ int32_t s_pre[kSubChunks + 1];
-    __shared__ int32_t s_nn[2], s_M, s_nlev, s_base, s_next;
-    const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
+    // a part (a node of at most kPart points, or a larger leaf), at its first
+    // position; n: of the leaves of more than 64 points, else 0
+    int16_t part_id[kCap], part_skip[kCap], wide_n[kCap];
+    uint16_t lvl[kCap + 2];     // first local id of each level
+    int16_t top_left[kTop], top_lf[kTop], top_n[kTop];
+    SubEntry e[2][kAct];
+    int32_t box[2 * kAct][6];   // the children's tight boxes, float keys
+    uint8_t map[2 * kAct];      // a child slot's place among the next level's nodes
+    uint64_t mask[kWaves], head[kWaves];
+    int32_t na[2], M, nlev, next;
+};
+
+// One workgroup per task of the list `cls` (nodes of at most kCap points), a
+// thread per point.  Bound by the latency of a task: LDS (77 KB at 1,024
+// points) and registers leave 8 wavefronts per SIMD at every size.
+template <int kCap>
+__global__ __launch_bounds__(kCap, 8) void k_subtree(const float4 *__restrict__ A,
+                                                     const float4 *__restrict__ B,
+                                                     const Task *__restrict__ tasks, BuildArgs a,
+                                                     double particle_mass, int cls) {
+    constexpr int kWaves = SubLds<kCap>::kWaves, kTop = SubLds<kCap>::kTop;
+    __shared__ SubLds<kCap> S;
+    const int tid = threadIdx.x, lane = lane_id(), w = uniform(tid / kWave);
     const int32_t ntasks = a.counters[kClassNext + cls];
-    const float inf = __int_as_float(0x7f800000), ninf = __int_as_float((int)0xff800000);
+    const float inf = __int_as_float(0x7f800000);
     // A dynamic queue over the list: thread 0 takes the workgroup's next
     // entry when it starts the current one.  Entries are taken from the end
     // of the list: the largest subtrees (children of the big nodes of the
     // last split levels) are queued last and should start first.
-    if (tid == 0) s_next = atomicAdd(&a.counters[kClassCursor + cls], 1);
+    if (tid == 0) S.next = atomicAdd(&a.counters[kClassCursor + cls], 1);
     __syncthreads();
-    for (int32_t k = s_next; k < ntasks; k = s_next) {
+    for (int32_t k = uniform(S.next); k < ntasks; k = uniform(S.next)) {
         int32_t k_after = 0;
         if (tid == 0) k_after = atomicAdd(&a.counters[kClassCursor + cls], 1);
-        const Task t = tasks[ntasks - 1 - k];
-        const int32_t first = t.pad[0], n = t.pad[1];
-        const int32_t root_skip = a.nodes[t.node].skip;
+        const Task t = load_const(tasks + (ntasks - 1 - k));
+        const int32_t first = t.pad[0], n = min(t.pad[1], kCap);
+        const int32_t root_skip = load_const(&a.nodes[t.node].skip);
         const float4 *src = (t.depth & 1) ? B : A;
-        for (int i = tid; i < n; i += kSubThreads) {
-            P[i] = src[first + i];
-            PM[0][i] = (int16_t)i;
-            Q[0][i] = 0;
-        }
-        if (tid <= kSubChunks) s_mask[tid] = 0;  // chunks past n stay empty
-        const int rounds = (n + kSubThreads - 1) / kSubThreads;
-        if (tid == 0) {
-            SubEntry e;
-            e.loc = 0;
-            e.lf = 0;
-            e.n = (int16_t)n;
-            e.nl = 0;
-            e.child = -1;
-            e.skip = kRootSkip;
-            e.kind = 0;
-            e.dim = (uint8_t)t.dim;
-            e.lim = t.lim;
-            E[0][0] = e;
-            s_nn[0] = 1;
-            s_M = 1;
-            s_nlev = 0;
-            s_lvl[0] = 0;
-            s_lvl[1] = 1;
-            s_left[0] = -1;
-            const int32_t R = 2 * n - 2;
-            int32_t base = t.tile0;  // R ids reserved by k_group_classes
-            if (base + R > a.cap_nodes) {  // out of node ids: the root stays a leaf
-                atomicOr(&a.counters[kErrFlags], kErrCapacity);
-                base = -1;
-                s_nn[0] = 0;
+        const bool in = tid < n;
+        const float4 p0 = in ? src[first + tid] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        const int32_t base = t.tile0;  // 2n - 2 ids reserved by k_group_classes
+        if (base + 2 * n - 2 > a.cap_nodes) {  // out of node ids: the root stays a leaf
+            if (tid == 0) atomicOr(&a.counters[kErrFlags], kErrCapacity);
+            if (in) {
+                a.fin[first + tid] = p0;
+                a.leaf_of[first + tid] = t.node;
             }
-            s_base = base;
+            if (tid == 0) S.next = k_after;
+            __syncthreads();
+            continue;
         }
-        __syncthreads();
-        const int32_t base = s_base;
         auto gid = [&](int j) { return j == 0 ? t.node : base + j - 1; };
         auto gskip = [&](int s) { return s == kRootSkip ? root_skip : gid(s); };
-        int cur = 0, buf = 0;
-        while (true) {
-            const int nn = s_nn[cur];
-            if (nn == 0) break;
+        if (in) S.P[tid] = p0;
+        if (tid < kWaves) S.head[tid] = 0;
+        __syncthreads();
+        if (tid == 0) {
+            S.M = 1;
+            S.nlev = 0;
+            S.lvl[0] = 0;
+            S.lvl[1] = 1;
+            S.top_left[0] = -1;
+            S.top_lf[0] = 0;
+            S.top_n[0] = (int16_t)n;
+            if (n > kPart) {
+                SubEntry e;
+                e.loc = 0;
+                e.lf = 0;
+                e.n = (int16_t)n;
+                e.nl = 0;
+                e.skip = kRootSkip;
+                e.split = 0;
+                e.dim = (uint8_t)t.dim;
+                e.lim = t.lim;
+                S.e[0][0] = e;
+                S.na[0] = 1;
+            } else {  // one part
+                S.na[0] = 0;
+                S.head[0] = 1;
+                S.part_id[0] = 0;
+                S.wide_n[0] = 0;
+                S.part_skip[0] = kRootSkip;
+            }
+        }
+        __syncthreads();
+        int cur = 0;
+        int q = in && n > kPart ? 0 : -1;  // this position's node among the level's, if any
+        for (int na; (na = uniform(S.na[cur])) > 0; cur ^= 1) {
             const int nxt = cur ^ 1;
-            const int c0 = s_M;  // first local id of the next level
-            // 1. left flags (src/fast3tree.c:751-774), one ballot per chunk
-            for (int r = 0; r < rounds; r++) {
-                const int i = r * kSubThreads + tid;
-                bool gl = false;
-                if (i < n) {
-                    const uint8_t e = Q[cur][i];
-                    if (e != kNoEntry && E[cur][e].n > kLeafPoints)
-                        gl = comp(P[PM[buf][i]], E[cur][e].dim) <= E[cur][e].lim;
-                }
-                const uint64_t m = ballot(gl);
-                if (lane == 0) s_mask[r * kSubWaves + w] = m;
+            // what follows from the thread's number is found anew each level
+            // (kept, it would not fit the registers)
+            const int tid = opaque((int)threadIdx.x), lane = opaque(lane_id());
+            SubEntry en;
+            en.lf = en.n = 0;
+            if (q >= 0) en = S.e[cur][q];
+            float4 p = S.P[tid];
+            // 1. left flags (src/fast3tree.c:751-774), one ballot per wavefront
+            const bool gl = q >= 0 && comp(p, en.dim) <= en.lim;
+            const uint64_t m = ballot(gl);
+            if (lane == 0) S.mask[w] = m;
+            for (int x = tid; x < 12 * na; x += kCap)
+                (&S.box[0][0])[x] = float_key(x % 6 < 3 ? inf : -inf);
+            __syncthreads();
+            // 2. left flags before a position: the wavefronts' counts, scanned
+            //    in every wavefront's lanes; the node's points by side
+            int cnt = lane < kWaves ? __popcll(S.mask[lane]) : 0;
+            const int excl = wave_scan_add(cnt) - cnt;  // lane kWaves: the total
+            auto before = [&](int x) {
+                const int c = x >> 6;
+                const uint64_t mk = S.mask[min(c, kWaves - 1)];
+                return __shfl(excl, c, 64) + (c < kWaves ? __popcll(mk & lanes_below(x & 63)) : 0);
+            };
+            const int s0 = before(en.lf), nl = before(en.lf + en.n) - s0;
+            const int sl = __builtin_amdgcn_readlane(excl, w) + __popcll(m & lanes_below(lane)) - s0;
+            // src/fast3tree.c:805-809: a split with an empty side is a leaf
+            const bool split = q >= 0 && nl > 0 && nl < en.n;
+            const int rel = tid - en.lf, rank = gl ? sl : rel - sl;
+            if (split) S.st[en.lf + (gl ? rank : nl + rank)] = (uint16_t)rel;
+            if (q >= 0 && rel == 0) {
+                S.e[cur][q].nl = (int16_t)nl;
+                S.e[cur][q].split = split ? 1 : 0;
             }
             __syncthreads();
-            // 2. wavefront 0: chunk prefix, left counts, splits, child ids
-            //    and the next level's entries
-            if (w == 0) {
-                const uint64_t mk = lane < kSubChunks ? s_mask[lane] : 0ull;
-                const int cnt = __popcll(mk);
-                int incl = cnt;
-                for (int o = 1; o < kSubChunks; o <<= 1) {
-                    const int u = __shfl_up(incl, o, 64);
-                    if (lane >= o) incl += u;
+            // 3. the points to the in-place partition's order (inplace_dest)
+            if (split) {
+                const int dst = en.lf + inplace_dest(rel, gl, rank, en.n, nl,
+                                                     [&](int x) { return (int)S.st[en.lf + x]; });
+                S.P[dst] = p;
+            }
+            __syncthreads();
+            // 4. tight boxes of the children
+            int slot = 0, lf = tid;
+            if (split) {  // the point that came here, and its child
+                p = S.P[tid];
+                slot = 2 * q + (rel >= nl ? 1 : 0);
+                lf = en.lf + ((slot & 1) ? nl : 0);
+            }
+            if (ballot(split)) {
+                const int chunk0 = tid - lane;
+                const int sg = split ? (lf > chunk0 ? lf - chunk0 : 0) : lane;
+                auto mn = [](int x, int y) { return min(x, y); };
+                auto mx = [](int x, int y) { return max(x, y); };
+                const int kx = float_key(p.x), ky = float_key(p.y), kz = float_key(p.z);
+                const int l0 = seg_scan(kx, sg, mn), l1 = seg_scan(ky, sg, mn),
+                          l2 = seg_scan(kz, sg, mn);
+                const int h0 = seg_scan(kx, sg, mx), h1 = seg_scan(ky, sg, mx),
+                          h2 = seg_scan(kz, sg, mx);
+                const int end = (slot & 1) ? en.lf + en.n : en.lf + nl;  // the child's
+                if (split && (lane == kWave - 1 || tid + 1 == end)) {
+                    atomicMin(&S.box[slot][0], l0);
+                    atomicMin(&S.box[slot][1], l1);
+                    atomicMin(&S.box[slot][2], l2);
+                    atomicMax(&S.box[slot][3], h0);
+                    atomicMax(&S.box[slot][4], h1);
+                    atomicMax(&S.box[slot][5], h2);
                 }
-                const int excl = incl - cnt;
-                const int total = __shfl(incl, kSubChunks - 1, 64);
-                if (lane < kSubChunks) s_pre[lane] = excl;
-                if (lane == kSubChunks) s_pre[kSubChunks] = total;
-                // left flags in [0, x)
-                auto S = [&](int x) {
-                    const int c = x >> 6;
-                    const int b = __shfl(excl, c < kSubChunks ? c : 0, 64);
-                    return (c < kSubChunks ? b : total) +
-                           __popcll(s_mask[c] & lanes_below(x & 63));
-                };
-                int M = c0;
-                for (int k0 = 0; k0 < nn; k0 += kWave) {
-                    const int kk = k0 + lane;
-                    const bool v = kk < nn;
-                    SubEntry en;
-                    en.lf = en.n = 0;
-                    if (v) en = E[cur][kk];
-                    const int s0 = S(en.lf), s1 = S(en.lf + en.n);
-                    const int nl = s1 - s0;
-                    // src/fast3tree.c:805-809: a split with an empty side is a leaf
-                    const bool split = v && en.n > kLeafPoints && nl > 0 && nl < en.n;
-                    const uint64_t ms = ballot(split);
-                    const int C = M + 2 * rank_below(ms);
-                    if (v) {
-                        E[cur][kk].nl = (int16_t)nl;
-                        E[cur][kk].kind = split ? 1 : 0;
-                        E[cur][kk].child = split ? (int16_t)C : (int16_t)-1;
-                        s_left[en.loc] = split ? (int16_t)C : (int16_t)-1;
+            }
+            __syncthreads();
+            // 5. wavefront 0, a lane per child: ids, records, the next level's
+            //    nodes and the parts
+            if (w == 0) {
+                const bool v = lane < 2 * na;
+                const int side = lane & 1;
+                SubEntry pe;
+                pe.split = 0;
+                if (v) pe = S.e[cur][lane >> 1];
+                const bool sp = v && pe.split;
+                const uint64_t ms = ballot(sp);
+                const int M = uniform(S.M), C = M + rank_below(ms);
+                const int cn = side ? pe.n - pe.nl : pe.nl;
+                const bool act = sp && cn > kPart;
+                const uint64_t ma = ballot(act);
+                if (sp) {
+                    const int clf = pe.lf + (side ? pe.nl : 0);
+                    const int skip = side ? pe.skip : C + 1;
+                    float lo[3], hi[3];
+                    for (int d = 0; d < 3; d++) {
+                        lo[d] = key_float(S.box[lane][d]);
+                        hi[d] = key_float(S.box[lane][3 + d]);
                     }
-                    if (split) {
-                        const int slot = C - c0;
-                        SubEntry L, R;
-                        L.loc = (int16_t)C;
-                        L.lf = en.lf;
-                        L.n = (int16_t)nl;
-                        L.skip = (int16_t)(C + 1);
-                        R.loc = (int16_t)(C + 1);
-                        R.lf = (int16_t)(en.lf + nl);
-                        R.n = (int16_t)(en.n - nl);
-                        R.skip = en.skip;
-                        L.nl = R.nl = 0;
-                        L.child = R.child = -1;
-                        L.kind = R.kind = 0;
-                        L.dim = R.dim = 0;
-                        L.lim = R.lim = 0.0f;
-                        E[nxt][slot] = L;
-                        E[nxt][slot + 1] = R;
-                        for (int d = 0; d < 3; d++) {
-                            BOX[slot][d] = BOX[slot + 1][d] = float_key(inf);
-                            BOX[slot][3 + d] = BOX[slot + 1][3 + d] = float_key(ninf);
-                        }
-                        a.nodes[gid(en.loc)].left = gid(C);
-                        a.parent[gid(C)] = a.parent[gid(C + 1)] = gid(en.loc);
+                    Node *g = a.nodes + gid(C);
+                    for (int d = 0; d < 3; d++) {
+                        g->lo[d] = lo[d];
+                        g->hi[d] = hi[d];
                     }
-                    M += 2 * __popcll(ms);
+                    a.parent[gid(C)] = gid(pe.loc);
+                    if (!side) {
+                        a.nodes[gid(pe.loc)].left = gid(C);
+                        if (pe.loc < kTop) S.top_left[pe.loc] = (int16_t)C;
+                    }
+                    if (C < kTop) {
+                        S.top_left[C] = -1;
+                        S.top_lf[C] = (int16_t)clf;
+                        S.top_n[C] = (int16_t)cn;
+                    }
+                    S.map[lane] = act ? (uint8_t)rank_below(ma) : kNone8;
+                    if (act) {
+                        g->first = first + clf;
+                        g->count = cn;
+                        g->skip = gskip(skip);
+                        SubEntry ne;
+                        ne.loc = (int16_t)C;
+                        ne.lf = (int16_t)clf;
+                        ne.n = (int16_t)cn;
+                        ne.nl = 0;
+                        ne.skip = (int16_t)skip;
+                        ne.split = 0;
+                        ne.dim = (uint8_t)split_dim(lo, hi);
+                        ne.lim = split_lim(lo, hi, ne.dim);
+                        S.e[nxt][rank_below(ma)] = ne;
+                    } else {
+                        S.part_id[clf] = (int16_t)C;
+                        S.wide_n[clf] = 0;
+                        S.part_skip[clf] = (int16_t)skip;
+                        atomicOr((unsigned long long *)&S.head[clf >> 6], 1ull << (clf & 63));
+                    }
+                } else if (v && !side) {  // a failed split: a leaf
+                    S.part_id[pe.lf] = pe.loc;
+                    S.wide_n[pe.lf] = pe.n > kWave ? pe.n : 0;
+                    S.part_skip[pe.lf] = pe.skip;
+                    atomicOr((unsigned long long *)&S.head[pe.lf >> 6], 1ull << (pe.lf & 63));
+                    if (pe.loc) a.nodes[gid(pe.loc)].left = -1;
                 }
                 if (lane == 0) {
-                    s_M = M;
-                    s_nn[nxt] = M - c0;
-                    if (M > c0) {
-                        s_nlev = s_nlev + 1;
-                        s_lvl[s_nlev + 1] = (uint16_t)M;
+                    S.na[nxt] = __popcll(ma);
+                    if (ms) {
+                        S.nlev = S.nlev + 1;
+                        S.M = M + __popcll(ms);
+                        S.lvl[S.nlev + 1] = (uint16_t)S.M;
                     }
                 }
             }
             __syncthreads();
-            // 3. scatter: split points to their child's place in the next
-            //    buffer, in the order of the reference's in-place partition
-            //    (inplace_dest); leaf points are in tree order already.  The
-            //    node's k-th left (right) point is the (Sx(lf) + k)-th set
-            //    (lf - Sx(lf) + k)-th clear bit of the left flags: a binary
-            //    search over the chunk prefixes, then a select in the word.
-            auto Sx = [&](int x) {
-                const int c = x >> 6;
-                return s_pre[c] + __popcll(s_mask[c] & lanes_below(x & 63));
-            };
-            // r-th set / clear bit overall, searched among chunks [lo, hi]
-            auto nth_left = [&](int r, int lo, int hi) {
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (s_pre[mid] <= r) lo = mid;
-                    else hi = mid - 1;
+            q = split && S.map[slot] != kNone8 ? (int)S.map[slot] : -1;
+        }
+        // The parts, packed: a wavefront takes consecutive parts of together
+        // at most 64 points.  A pack ends before the part that holds the 64th
+        // position after its start; every wavefront follows the chain of packs
+        // on the scalar unit and takes each kWaves-th.  Part i at position lf
+        // has its node ids from base + (M - 1) + 2 (lf - i) on.
+        const int M = uniform(S.M), nlev = uniform(S.nlev);
+        auto cm_put = [&](int j, float x, float y, float z, float mass) {
+            if (j < kTop) S.cm[j] = make_float4(x, y, z, mass);
+        };
+        const uint64_t hw = lane < kWaves ? S.head[lane] : 0ull;
+        int at = 0, i0 = 0;  // a pack's first position and part
+        for (int pk = 0; at < n; pk++) {
+            int end = at + kWave;
+            const int wide = uniform(S.wide_n[at]);
+            if (wide) end = at + wide;
+            if (end >= n) {
+                end = n;
+            } else if (!wide) {
+                const int c = end >> 6;
+                uint64_t hm = read_lane(hw, c) & lanes_below((end & 63) + 1);
+                end = 64 * c + 63;
+                if (!hm) {  // the part that holds it starts in the 64 positions before
+                    hm = read_lane(hw, c - 1);
+                    end -= 64;
                 }
-                return lo * 64 + select_bit(s_mask[lo], r - s_pre[lo]);
-            };
-            auto nth_right = [&](int r, int lo, int hi) {
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (64 * mid - s_pre[mid] <= r) lo = mid;
-                    else hi = mid - 1;
-                }
-                return lo * 64 + select_bit(~s_mask[lo], r - (64 * lo - s_pre[lo]));
-            };
-            for (int r = 0; r < rounds; r++) {
-                const int i = r * kSubThreads + tid;
-                if (i >= n) break;
-                const int16_t pi = PM[buf][i];
-                const float4 p = P[pi];
-                const uint8_t e = Q[cur][i];
-                int dst = i;
-                uint8_t q = kNoEntry;
-                if (e != kNoEntry) {
-                    const SubEntry en = E[cur][e];
-                    if (en.kind) {
-                        const bool gl = comp(p, en.dim) <= en.lim;
-                        const int lf = en.lf, s0 = Sx(lf), sl = Sx(i) - s0, nl = en.nl;
-                        const int clo = lf >> 6, chi = (lf + en.n - 1) >> 6;  // the node's chunks
-                        dst = lf + inplace_dest(i - lf, gl, gl ? sl : i - lf - sl, en.n, nl,
-                                                [&](int k) {
-                                                    return k < nl
-                                                        ? nth_left(s0 + k, clo, chi) - lf
-                                                        : nth_right(lf - s0 + k - nl, clo, chi) - lf;
-                                                });
-                        q = (uint8_t)(en.child - c0 + (gl ? 0 : 1));
-                    } else {
-                        a.fin[first + i] = p;
-                        a.leaf_of[first + i] = gid(en.loc);
-                    }
-                }
-                PM[buf ^ 1][dst] = pi;
-                Q[nxt][dst] = q;
+                end -= __builtin_clzll(hm);
             }
-            __syncthreads();
-            // 4. tight boxes of the next level's nodes
-            const int nn_next = s_nn[nxt];
-            if (nn_next > 0) {
-                for (int r = 0; r < rounds; r++) {
-                    const int i = r * kSubThreads + tid;
-                    const uint8_t q = i < n ? Q[nxt][i] : kNoEntry;
-                    const bool fresh = q != kNoEntry;
-                    if (!ballot(fresh)) continue;
-                    const float4 p = fresh ? P[PM[buf ^ 1][i]] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    const int lf = fresh ? E[nxt][q].lf : i;
-                    const int chunk0 = i - lane;
-                    const int seg = lf > chunk0 ? lf - chunk0 : 0;
-                    const int sg = fresh ? seg : lane;
-                    auto mn = [](float x, float y) { return fminf(x, y); };
-                    auto mx = [](float x, float y) { return fmaxf(x, y); };
-                    const float l0 = seg_scan(p.x, sg, mn), l1 = seg_scan(p.y, sg, mn),
-                                l2 = seg_scan(p.z, sg, mn);
-                    const float h0 = seg_scan(p.x, sg, mx), h1 = seg_scan(p.y, sg, mx),
-                                h2 = seg_scan(p.z, sg, mx);
-                    const int qn = __shfl_down((int)q, 1, 64);
-                    const bool last = fresh && (lane == kWave - 1 || i + 1 >= n || qn != (int)q);
-                    if (last) {
-                        atomicMin(&BOX[q][0], float_key(l0));
-                        atomicMin(&BOX[q][1], float_key(l1));
-                        atomicMin(&BOX[q][2], float_key(l2));
-                        atomicMax(&BOX[q][3], float_key(h0));
-                        atomicMax(&BOX[q][4], float_key(h1));
-                        atomicMax(&BOX[q][5], float_key(h2));
+            const int m = end - at, c = at >> 6, sh = at & 63;
+            // the pack's first positions, as a mask from `at` on
+            uint64_t heads = read_lane(hw, c) >> sh;
+            if (sh && c + 1 < kWaves) heads |= read_lane(hw, c + 1) << (64 - sh);
+            if (m < kWave) heads &= lanes_below(m);
+            const int nr = wide ? 1 : __popcll(heads);
+            if (pk % kWaves == w) {
+                if (!wide) {
+                    const float4 x = lane < m ? S.P[at + lane] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    wave_subtree<true>(
+                        a, S.wt[w], S.P + at, x, m, heads, nr, 0, 0.0f, first + at,
+                        base + (M - 1) + 2 * (at - i0), true, particle_mass,
+                        [&](int j) { return gid(S.part_id[at + S.wt[w].lf[j]]); },
+                        [&](int j) { return gskip(S.part_skip[at + S.wt[w].lf[j]]); });
+                    if (lane < nr)
+                        cm_put(S.part_id[at + S.wt[w].lf[lane]], S.wt[w].com[0][lane],
+                               S.wt[w].com[1][lane], S.wt[w].com[2][lane], S.wt[w].mass[lane]);
+                } else {  // a leaf whose split failed: f64 sums in tree order
+                    const int id = S.part_id[at];
+                    for (int j = lane; j < m; j += kWave) {
+                        a.fin[first + at + j] = S.P[at + j];
+                        a.leaf_of[first + at + j] = gid(id);
+                    }
+                    double sx = 0.0, sy = 0.0, sz = 0.0;
+                    for (int j = 0; j < m; j++) {
+                        const float4 x = S.P[at + j];
+                        sx += (double)x.x;
+                        sy += (double)x.y;
+                        sz += (double)x.z;
+                    }
+                    if (lane == 0) {
+                        const double dn = (double)m;
+                        const float cx = sx != 0.0 ? (float)(sx / dn) : 0.0f;
+                        const float cy = sy != 0.0 ? (float)(sy / dn) : 0.0f;
+                        const float cz = sz != 0.0 ? (float)(sz / dn) : 0.0f;
+                        const float mass = (float)(particle_mass * dn);
+                        Node *g = a.nodes + gid(id);
+                        g->com[0] = cx;
+                        g->com[1] = cy;
+                        g->com[2] = cz;
+                        g->mass = mass;
+                        cm_put(id, cx, cy, cz, mass);
                     }
                 }
             }
-            __syncthreads();
-            // 5. the next level's node records and split planes, a thread each
-            for (int c = tid; c < nn_next; c += kSubThreads) {
-                SubEntry &en = E[nxt][c];
-                float lo[3], hi[3];
-                for (int d = 0; d < 3; d++) {
-                    lo[d] = key_float(BOX[c][d]);
-                    hi[d] = key_float(BOX[c][3 + d]);
-                }
-                const int dim = split_dim(lo, hi);
-                en.dim = (uint8_t)dim;
-                en.lim = split_lim(lo, hi, dim);
-                write_node(a.nodes + gid(en.loc), lo, hi, first + en.lf, en.n, gskip(en.skip));
-            }
-            __syncthreads();
-            cur = nxt;
-            buf ^= 1;
+            at = end;
+            i0 += nr;
         }
-        if (base < 0) {  // the root stays a leaf over the points in input order
-            for (int i = tid; i < n; i += kSubThreads) {
-                a.fin[first + i] = P[i];
-                a.leaf_of[first + i] = t.node;
-            }
-        }
-        // centres of mass and dmin (src/potential.c:71-124): the final order
-        // to PM[0] (PMF), the rest of the level arrays' room for com (x, y,
-        // z) and mass
-        if (buf) {
-            for (int i = tid; i < n; i += kSubThreads) PM[0][i] = PM[1][i];
+        if (tid == 0) S.next = k_after;
+        if (M == 1 && n <= kWave) {  // one part: its wavefront did it all
             __syncthreads();
+            continue;
         }
-        const int M = s_M, nlev = s_nlev;
-        const int16_t *PMF = pool.cm.PMF;
-        float4 *CM = pool.cm.CM;
-        auto F = [&](int i) { return P[PMF[i]]; };
+        __threadfence_block();
+        __syncthreads();
+        // the nodes above the parts: centres of mass, deepest level first
+        // (src/potential.c:115-122: float, right term first), by one wavefront
+        // (a level reads what this wavefront wrote at deeper levels, or the
+        // parts' roots, made visible by the barrier above)
+        struct Top {
+            int left, lf, n;
+        };
+        auto top = [&](int j) {
+            if (j < kTop) return Top{S.top_left[j], S.top_lf[j], S.top_n[j]};
+            const Node *g = a.nodes + gid(j);
+            const int32_t l = g->left;
+            // a part's own children are not of the levels above
+            return Top{l >= base && l < base + M - 1 ? l - base + 1 : -1, g->first - first, g->count};
+        };
         auto cm_get = [&](int j) {
-            if (j < kCM) return CM[j];
-            const Node *np = a.nodes + gid(j);
-            return make_float4(np->com[0], np->com[1], np->com[2], np->mass);
+            if (j < kTop) return S.cm[j];
+            const Node *g = a.nodes + gid(j);
+            return make_float4(g->com[0], g->com[1], g->com[2], g->mass);
         };
-        auto cm_put = [&](int j, float4 v) {
-            if (j < kCM) CM[j] = v;
-            Node *np = a.nodes + gid(j);
-            np->com[0] = v.x;
-            np->com[1] = v.y;
-            np->com[2] = v.z;
-            np->mass = v.w;
+        auto combine = [&](int j, int cl) {
+            const float4 l = cm_get(cl), r = cm_get(cl + 1);
+            const float m = l.w + r.w;
+            float c[3];
+            const float lc[3] = {l.x, l.y, l.z}, rc[3] = {r.x, r.y, r.z};
+            for (int d = 0; d < 3; d++) {
+                const float rr = rc[d] * r.w;
+                const float ll = lc[d] * l.w;
+                c[d] = m != 0.0f ? (rr + ll) / m : 0.0f;
+            }
+            Node *g = a.nodes + gid(j);
+            for (int d = 0; d < 3; d++) g->com[d] = c[d];
+            g->mass = m;
+            cm_put(j, c[0], c[1], c[2], m);
         };
-        int32_t my_lf[kSubPerThread], my_n[kSubPerThread];
-#pragma unroll
-        for (int q = 0; q < kSubPerThread; q++) {
-            const int j = tid + q * kSubThreads;
-            my_lf[q] = my_n[q] = 0;
-            if (j < M) {
-                const Node *np = a.nodes + gid(j);
-                my_lf[q] = np->first - first;
-                my_n[q] = np->count;
-            }
-        }
-        // leaves: f64 sums in tree order (src/potential.c:100-107)
-#pragma unroll
-        for (int q = 0; q < kSubPerThread; q++) {
-            const int j = tid + q * kSubThreads;
-            if (j >= M || s_left[j] >= 0) continue;
-            double sx = 0.0, sy = 0.0, sz = 0.0;
-            for (int i = my_lf[q]; i < my_lf[q] + my_n[q]; i++) {
-                const float4 p = F(i);
-                sx += (double)p.x;
-                sy += (double)p.y;
-                sz += (double)p.z;
-            }
-            const double dn = (double)my_n[q];
-            cm_put(j, make_float4(sx != 0.0 ? (float)(sx / dn) : 0.0f,
-                                  sy != 0.0 ? (float)(sy / dn) : 0.0f,
-                                  sz != 0.0 ? (float)(sz / dn) : 0.0f, (float)(particle_mass * dn)));
-        }
-        __threadfence_block();
-        __syncthreads();
-        // internal nodes, deepest level first (src/potential.c:115-122:
-        // float, right term first).  One wavefront walks all levels: a level
-        // reads only values this wavefront wrote at deeper levels (or the
-        // leaves, made visible by the barrier above), so the levels need no
-        // workgroup barrier, only program order within the wavefront.
         if (w == 0) {
+            int left[kTop / kWave];  // a lane's nodes' children, read ahead
+            for (int h = 0; h < kTop / kWave; h++) {
+                const int j = lane + kWave * h;
+                left[h] = j < M ? S.top_left[j] : -1;
+            }
+            int l1 = M;
             for (int L = nlev; L >= 0; L--) {
-                const int l1 = s_lvl[L + 1];
-                for (int j = s_lvl[L] + lane; j < l1; j += kWave) {
-                    const int cl = s_left[j];
-                    if (cl < 0) continue;
-                    const float4 l = cm_get(cl), r = cm_get(cl + 1);
-                    const float m = l.w + r.w;
-                    float c[3];
-                    const float lc[3] = {l.x, l.y, l.z}, rc[3] = {r.x, r.y, r.z};
-                    for (int d = 0; d < 3; d++) {
-                        const float rr = rc[d] * r.w;
-                        const float ll = lc[d] * l.w;
-                        c[d] = m != 0.0f ? (rr + ll) / m : 0.0f;
-                    }
-                    cm_put(j, make_float4(c[0], c[1], c[2], m));
+                const int l0 = uniform(S.lvl[L]);
+                for (int h = 0; h < kTop / kWave; h++) {
+                    const int j = lane + kWave * h;
+                    if (j >= l0 && j < l1 && left[h] >= 0) combine(j, left[h]);
                 }
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                __builtin_amdgcn_wave_barrier();
+                for (int j = max(l0, kTop) + lane; j < l1; j += kWave) {
+                    const int cl = top(j).left;
+                    if (cl >= 0) combine(j, cl);
+                }
+                wave_sync();
+                l1 = l0;
             }
         }
         __threadfence_block();
         __syncthreads();
-        // dmin: nodes of at most 64 points a thread each, in tree order
-#pragma unroll
-        for (int q = 0; q < kSubPerThread; q++) {
-            const int j = tid + q * kSubThreads;
-            if (j >= M || my_n[q] > kWave) continue;
-            const float4 c4 = cm_get(j);
-            const float com[3] = {c4.x, c4.y, c4.z};
-            double big = 0.0, sum = 0.0;
-#pragma unroll 4
-            for (int i = my_lf[q]; i < my_lf[q] + my_n[q]; i++) {
-                const double d = d2_ref(com, F(i));
-                big = d > big ? d : big;
-                sum += d;
-            }
-            finish_dmin(a.nodes + gid(j), big, sum, my_n[q]);
-        }
-        // larger nodes a wavefront each: the wavefront takes the nodes of
-        // its lanes' chunk (j = tid + k * kSubThreads) that have more than
-        // 64 points, one after another, reading each node's range lane-parallel
-#pragma unroll
-        for (int k = 0; k < kSubPerThread; k++) {
-            const int j0 = w * kWave + k * kSubThreads;
-            if (j0 >= M) break;
-            uint64_t wide = ballot(tid + k * kSubThreads < M && my_n[k] > kWave);
-            while (wide) {
-                const int q = __builtin_ctzll(wide);
-                wide &= wide - 1;
-                const int32_t qn = read_lane(my_n[k], q), ql = read_lane(my_lf[k], q);
-                const float4 c4 = cm_get(j0 + q);
+        // their dmin (src/potential.c:71-82), a wavefront each
+        for (int j0 = w; j0 < M; j0 += kWaves * kWave) {
+            double my_big = 0.0, my_sum = 0.0;  // lane k's: of node j0 + k kWaves
+            int my_n = 0;
+            for (int k = 0; k < kWave; k++) {
+                const int j = j0 + k * kWaves;
+                if (j >= M) break;
+                const Top tp = top(j);
+                if (tp.left < 0 && tp.n <= kWave) continue;  // a part
+                const float4 c4 = cm_get(j);
                 const float com[3] = {c4.x, c4.y, c4.z};
                 double big = 0.0, sum = 0.0;
-                for (int32_t i = lane; i < qn; i += kWave) {
-                    const double d = d2_ref(com, F(ql + i));
+                for (int i = lane; i < tp.n; i += kWave) {
+                    const double d = d2_ref(com, S.P[tp.lf + i]);
                     big = d > big ? d : big;
                     sum += d;
                 }
                 big = wave_max(big);
                 sum = wave_sum(sum);
-                if (lane == 0) finish_dmin(a.nodes + gid(j0 + q), big, sum, qn);
+                if (lane == k) {
+                    my_big = big;
+                    my_sum = sum;
+                    my_n = tp.n;
+                }
             }
+            if (my_n > 0) finish_dmin(a.nodes + gid(j0 + lane * kWaves), my_big, my_sum, my_n);
         }
-        if (tid == 0) s_next = k_after;
         __syncthreads();
     }
 }
-
-// ---------------------------------------------------- wavefront subtrees
-//
-// A subtree of at most kWaveTask points is built by one wavefront, one point
-// per lane.  Each level, every lane tests its point against its node's split
-// plane; ballots give the left counts and the stable scatter positions (a
-// node's points occupy a contiguous run of lanes), and the children's tight
-// boxes come from segmented scans across the lanes.  The node table stays in
-// LDS with local ids (children in pairs, levels in order) until the subtree
-// is complete; then one atomic reserves exactly its node ids.  Centres of
-// mass and dmin are computed with a lane per node, summing the node's points
-// in tree order, the order of the reference's loops.
-
-constexpr int kWaveNodes = 2 * kWaveTask;  // a tree over n points has at most 2n - 1 nodes
 
 // Node ids of the wavefront subtrees, assigned before they are built: a
 // subtree of n points gets 2n - 2 ids (the most it can need; ids it does not
@@ -1110,22 +1327,17 @@ __global__ void k_wave_base(BuildArgs a, const int32_t *__restrict__ off) {
     a.counters[kNodeCount] = base0 + off[ntasks];
 }
 
-__global__ __launch_bounds__(kWave) void k_subtree_wave(const float4 *__restrict__ A,
+// One wavefront per task: subtrees of at most 64 points whose parent the
+// split levels made.  Under 5 KB of LDS, so that 8 wavefronts fit per SIMD:
+// the nodes' boxes go to their global records as they are found (only each
+// node's split plane stays), parents are written from the parent's side.
+__global__ __launch_bounds__(kWave, 8) void k_subtree_wave(const float4 *__restrict__ A,
                                                         const float4 *__restrict__ B,
                                                         const Task *__restrict__ tasks,
                                                         BuildArgs a, double particle_mass,
                                                         const int32_t *__restrict__ wave_off) {
-    // under 5 KB of LDS, so that 8 wavefronts fit per SIMD: the nodes' boxes
-    // go to their global records as they are found (only each node's split
-    // plane stays), parents are written from the parent's side
     __shared__ float4 P[kWaveTask];
-    __shared__ int16_t Q[kWaveTask];
-    __shared__ float s_lim[kWaveNodes];
-    __shared__ uint8_t s_dim[kWaveNodes];
-    __shared__ float s_com[3][kWaveNodes], s_mass[kWaveNodes];
-    __shared__ int16_t s_lf[kWaveNodes], s_cnt[kWaveNodes], s_left[kWaveNodes];
-    __shared__ int16_t s_skip[kWaveNodes];
-    __shared__ int16_t s_lvl[kWaveTask + 2];  // first local id of each level
+    __shared__ WaveTree W;
     const int lane = lane_id();
     const int32_t ntasks = min(a.counters[kSmallNext], a.cap_small);
     const int32_t id_base = a.counters[kWaveIdBase];
@@ -1141,200 +1353,14 @@ __global__ __launch_bounds__(kWave) void k_subtree_wave(const float4 *__restrict
         // the task carries the root's range and split plane, so the points
         // load at once; the root's node record is needed only at the end
         const float4 *src = (t.depth & 1) ? B : A;
-        const int32_t first = t.pad[0];
-        const bool v = lane < n;
-        float4 p = v ? src[first + lane] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        const Node root = a.nodes[t.node];
+        const float4 p = lane < n ? src[t.pad[0] + lane] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        const int32_t skip = a.nodes[t.node].skip;
         // the task's node ids (2n - 2 from the scan); a subtree that does not
         // fit keeps its root as a leaf (checked once the levels are done)
-        const int32_t base0 = id_base + wave_off[k];
-        const bool fits = base0 + wave_ids(n) <= a.cap_nodes;
-        if (lane == 0) {
-            s_lf[0] = 0;
-            s_cnt[0] = (int16_t)n;
-            s_left[0] = -1;
-            s_skip[0] = kRootSkip;
-            s_lvl[0] = 0;
-            s_lvl[1] = 1;
-        }
-        __syncthreads();
-        int nid = 0, M = 1, nlev = 0;
-        bool pend = v && n > kLeafPoints;
-        while (ballot(pend)) {
-            int lf = 0, c = 0, dim = 0;
-            float lim = 0.0f;
-            if (pend) {
-                lf = s_lf[nid];
-                c = s_cnt[nid];
-                if (nid == 0) {  // make_task's plane from the root's box
-                    dim = t.dim;
-                    lim = t.lim;
-                } else {
-                    dim = s_dim[nid];
-                    lim = s_lim[nid];
-                }
-            }
-            // src/fast3tree.c:751-774 (partition), 805-809 (failed split)
-            const bool gl = pend && comp(p, dim) <= lim;
-            const uint64_t mL = ballot(gl);
-            const uint64_t mN = pend ? lane_run(lf, c) : 0ull;
-            const int nl = __popcll(mL & mN);
-            const bool split = pend && nl > 0 && nl < c;
-            const uint64_t mH = ballot(split && lane == lf);
-            const int C = M + 2 * __popcll(mH & lanes_below(lf));
-            int dst = lane, nn = nid;
-            // the in-place partition's order (inplace_dest): the node's k-th
-            // left (right) point is the k-th set bit of its left (right)
-            // lanes' mask
-            const uint64_t below = mN & lanes_below(lane);
-            const int rank = gl ? __popcll(mL & below) : __popcll(~mL & below);
-            if (split) {
-                const uint64_t mLn = mL & mN, mRn = ~mL & mN;
-                dst = lf + inplace_dest(lane - lf, gl, rank, c, nl, [&](int k) {
-                    return (k < nl ? select_bit(mLn, k) : select_bit(mRn, k - nl)) - lf;
-                });
-                nn = gl ? C : C + 1;
-                if (lane == lf) {
-                    s_lf[C] = (int16_t)lf;
-                    s_cnt[C] = (int16_t)nl;
-                    s_lf[C + 1] = (int16_t)(lf + nl);
-                    s_cnt[C + 1] = (int16_t)(c - nl);
-                    s_left[C] = s_left[C + 1] = -1;
-                    s_skip[C] = (int16_t)(C + 1);
-                    s_skip[C + 1] = s_skip[nid];
-                    s_left[nid] = (int16_t)C;
-                }
-            }
-            if (v) {
-                P[dst] = p;
-                Q[dst] = nn;
-            }
-            __syncthreads();
-            if (v) {
-                p = P[lane];
-                nid = Q[lane];
-            }
-            const int M0 = M;
-            M += 2 * __popcll(mH);
-            // tight boxes of the new children: segmented scans over their runs
-            const bool fresh = v && nid >= M0;
-            const int seg = fresh ? s_lf[nid] : lane;
-            auto mn = [](float x, float y) { return fminf(x, y); };
-            auto mx = [](float x, float y) { return fmaxf(x, y); };
-            const float l0 = seg_scan(p.x, seg, mn), l1 = seg_scan(p.y, seg, mn),
-                        l2 = seg_scan(p.z, seg, mn);
-            const float h0 = seg_scan(p.x, seg, mx), h1 = seg_scan(p.y, seg, mx),
-                        h2 = seg_scan(p.z, seg, mx);
-            const int cnt_new = fresh ? s_cnt[nid] : 0;
-            if (fresh && lane == seg + cnt_new - 1) {
-                const float lo3[3] = {l0, l1, l2}, hi3[3] = {h0, h1, h2};
-                const int dm = split_dim(lo3, hi3);
-                s_dim[nid] = (uint8_t)dm;
-                s_lim[nid] = split_lim(lo3, hi3, dm);
-                if (fits) {
-                    Node *g = a.nodes + base0 + nid - 1;
-                    for (int d = 0; d < 3; d++) {
-                        g->lo[d] = lo3[d];
-                        g->hi[d] = hi3[d];
-                    }
-                }
-            }
-            if (M > M0) {
-                nlev++;
-                if (lane == 0) s_lvl[nlev + 1] = (int16_t)M;
-            }
-            __syncthreads();
-            pend = fresh && cnt_new > kLeafPoints;
-        }
-        // every lane's node is a leaf now; local id j > 0 is node base + j - 1
-        // of the ids reserved for the task (its box is there already)
-        int32_t base = base0;
-        if (M > 1 && !fits) {
-            if (lane == 0) atomicOr(&a.counters[kErrFlags], kErrCapacity);
-            base = -1;
-        }
-        if (base < 0) {  // out of node ids: the root stays a leaf
-            M = 1;
-            nlev = 0;
-            nid = 0;
-            if (lane == 0) s_left[0] = -1;
-        }
-        if (v) {
-            P[lane] = p;
-            a.fin[first + lane] = p;
-            a.leaf_of[first + lane] = nid ? base + nid - 1 : t.node;
-        }
-        __syncthreads();
-        // leaf centres: f64 sums in tree order (src/potential.c:100-107)
-        for (int j = lane; j < M; j += kWave) {
-            if (s_left[j] >= 0) continue;
-            const int lf = s_lf[j], c = s_cnt[j];
-            double sx = 0.0, sy = 0.0, sz = 0.0;
-            for (int i = lf; i < lf + c; i++) {
-                const float4 q = P[i];
-                sx += (double)q.x;
-                sy += (double)q.y;
-                sz += (double)q.z;
-            }
-            const double dn = (double)c;
-            s_com[0][j] = sx != 0.0 ? (float)(sx / dn) : 0.0f;
-            s_com[1][j] = sy != 0.0 ? (float)(sy / dn) : 0.0f;
-            s_com[2][j] = sz != 0.0 ? (float)(sz / dn) : 0.0f;
-            s_mass[j] = (float)(particle_mass * dn);
-        }
-        __syncthreads();
-        // internal centres, deepest level first (src/potential.c:115-122:
-        // float, right term first)
-        for (int L = nlev; L >= 0; L--) {
-            for (int j = s_lvl[L] + lane; j < s_lvl[L + 1]; j += kWave) {
-                const int cl = s_left[j];
-                if (cl < 0) continue;
-                const float ml = s_mass[cl], mr = s_mass[cl + 1];
-                const float m = ml + mr;
-                for (int d = 0; d < 3; d++) {
-                    const float rr = s_com[d][cl + 1] * mr;
-                    const float ll = s_com[d][cl] * ml;
-                    s_com[d][j] = m != 0.0f ? (rr + ll) / m : 0.0f;
-                }
-                s_mass[j] = m;
-            }
-            __syncthreads();
-        }
-        // dmin over each node's points in tree order (src/potential.c:71-82),
-        // then the node records
-        for (int j = lane; j < M; j += kWave) {
-            const int lf = s_lf[j], c = s_cnt[j];
-            const float com[3] = {s_com[0][j], s_com[1][j], s_com[2][j]};
-            double big = 0.0, sum = 0.0;
-            for (int i = lf; i < lf + c; i++) {
-                const double d = d2_ref(com, P[i]);
-                big = d > big ? d : big;
-                sum += d;
-            }
-            Node nd;
-            for (int d = 0; d < 3; d++) nd.com[d] = com[d];
-            nd.mass = s_mass[j];
-            nd.first = first + lf;
-            nd.count = c;
-            const int cl = s_left[j], sk = s_skip[j];
-            nd.left = cl >= 0 ? base + cl - 1 : -1;
-            nd.skip = sk == kRootSkip ? root.skip : base + sk - 1;
-            finish_dmin(&nd, big, sum, c);
-            const int32_t id = j ? base + j - 1 : t.node;
-            // every field but the box (the root's is the task's, the others
-            // were written with their level)
-            Node *g = a.nodes + id;
-            for (int d = 0; d < 3; d++) g->com[d] = nd.com[d];
-            g->mass = nd.mass;
-            g->dmin2 = nd.dmin2;
-            g->first = nd.first;
-            g->count = nd.count;
-            g->left = nd.left;
-            g->skip = nd.skip;
-            g->dmin = nd.dmin;
-            if (cl >= 0) a.parent[base + cl - 1] = a.parent[base + cl] = id;
-        }
-        __syncthreads();
+        const int32_t base = id_base + wave_off[k];
+        wave_subtree<false>(a, W, P, p, n, 1ull, 1, t.dim, t.lim, t.pad[0], base,
+                            base + wave_ids(n) <= a.cap_nodes, particle_mass,
+                            [&](int) { return t.node; }, [&](int) { return skip; });
     }
 }
 

@@ -160,9 +160,11 @@ __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirs
 // its row's result), then combine the four row results read from lanes 0,
 // 16, 32 and 48.  The result is wavefront-uniform.  Call with all 64 lanes
 // active, in wavefront-uniform control flow.
+// A lane move that reads no lane gives 0 (bound_ctrl, so that the compiler
+// can make the move part of the operation that uses it).
 template <int CTRL>
 __device__ __forceinline__ int dpp_i32(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
 }
 
 template <int CTRL, typename T>

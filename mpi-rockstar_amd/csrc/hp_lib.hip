@@ -443,11 +443,11 @@ struct Engine {
         // wavefront one at a fixed stride, until the lists are empty; their
         // grids are the workgroups that fit on the device at once.
         int per_cu = 0;
-        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<256>, kSubThreads, 0));
+        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<256>, 256, 0));
         sub_grid[0] = std::max(1, per_cu) * prop.multiProcessorCount;
-        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<512>, kSubThreads, 0));
+        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<512>, 512, 0));
         sub_grid[1] = std::max(1, per_cu) * prop.multiProcessorCount;
-        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<1024>, kSubThreads, 0));
+        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<1024>, 1024, 0));
         sub_grid[2] = std::max(1, per_cu) * prop.multiProcessorCount;
         HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree_wave, kWave, 0));
         wave_grid = std::max(1, per_cu) * prop.multiProcessorCount;
@@ -520,11 +520,11 @@ struct Engine {
             xcds = 1;
         }
         int per_cu = 0;
-        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<256>, kSubThreads, 0));
+        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<256>, 256, 0));
         sub_grid[0] = std::max(1, per_cu) * prop.multiProcessorCount;
-        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<512>, kSubThreads, 0));
+        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<512>, 512, 0));
         sub_grid[1] = std::max(1, per_cu) * prop.multiProcessorCount;
-        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<1024>, kSubThreads, 0));
+        HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree<1024>, 1024, 0));
         sub_grid[2] = std::max(1, per_cu) * prop.multiProcessorCount;
         HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree_wave, kWave, 0));
         wave_grid = std::max(1, per_cu) * prop.multiProcessorCount;
@@ -852,17 +852,17 @@ struct Engine {
             s3 = side[2];
         }
         if (gmax > 512) {
-            k_subtree<1024><<<sub_grid[2], kSubThreads, 0, s>>>(
+            k_subtree<1024><<<sub_grid[2], 1024, 0, s>>>(
                 A.as<float4>(), B.as<float4>(), groupc.as<Task>() + 2 * cap_group, ba, PARTICLE_MASS, 2);
             HP_LAUNCHED();
         }
         if (gmax > 256) {
-            k_subtree<512><<<sub_grid[1], kSubThreads, 0, s1>>>(
+            k_subtree<512><<<sub_grid[1], 512, 0, s1>>>(
                 A.as<float4>(), B.as<float4>(), groupc.as<Task>() + cap_group, ba, PARTICLE_MASS, 1);
             HP_LAUNCHED();
         }
         if (gmax > kWaveMin) {
-            k_subtree<256><<<sub_grid[0], kSubThreads, 0, s2>>>(A.as<float4>(), B.as<float4>(),
+            k_subtree<256><<<sub_grid[0], 256, 0, s2>>>(A.as<float4>(), B.as<float4>(),
                                                                groupc.as<Task>(), ba, PARTICLE_MASS, 0);
             HP_LAUNCHED();
         }

@@ -86,6 +86,41 @@ def test_tree_identical_small_calls(restatement, n):
     _compare_trees(gnodes, perm, onodes, opo)
 
 
+@pytest.mark.parametrize("shape", ["nfw", "chain1", "chain5", "clumps", "plane", "coincident"])
+@pytest.mark.parametrize("n", [65, 97, 255, 511, 767, 1023, 1024])
+def test_tree_identical_workgroup_subtrees(restatement, shape, n):
+    """One workgroup's subtree where its parts (nodes of at most 32 points,
+    packed 64 points to a wavefront) go to their limits: chains of splits that
+    take off one or five points each (hundreds of parts, more nodes above them
+    than the LDS table holds), clumps of 64 and 33 points, a flat set, and
+    leaves of more than 64 points whose split fails."""
+    prm = catalog.config1().params
+    halopot.set_config(prm)
+    rng = np.random.default_rng(n)
+    po = with_ids(catalog.config1().segment(0)[:n])
+    x = np.zeros((n, 3))
+    if shape == "nfw":
+        x = po["pos"][:, :3].astype(np.float64)
+    elif shape in ("chain1", "chain5"):
+        k = np.arange(n) // (1 if shape == "chain1" else 5)
+        x[:, 0] = np.ldexp(1.0 + 0.1 * rng.uniform(size=n), -(k % 110))
+        x[:, 1:] = np.ldexp(rng.uniform(size=(n, 2)), (-(k % 110) - 3)[:, None])
+    elif shape == "clumps":
+        c = np.where(np.arange(n) % 97 < 64, np.arange(n) // 97 * 2, np.arange(n) // 97 * 2 + 1)
+        x = rng.uniform(size=(n, 3))[c] + 1e-4 * rng.normal(size=(n, 3))
+    elif shape == "plane":
+        x[:, :2] = np.floor(rng.uniform(size=(n, 2)) * 8)  # few places: many equal coordinates
+    else:
+        x = rng.uniform(size=(n, 3))
+        x[n // 4:n // 4 + max(65, n // 3)] = x[0]
+        x = x[:n]
+    po["pos"][:, :3] = x[rng.permutation(n)]
+    gnodes, perm = halopot.debug_tree(po)
+    opo = po.copy()
+    onodes = restatement.build_tree(opo, prm)
+    _compare_trees(gnodes, perm, onodes, opo)
+
+
 def test_tree_identical_coincident_points(restatement):
     """31 of 40 points coincide: the split that cannot separate them leaves a
     31-point leaf (src/fast3tree.c:805-809), whose self term the walk skips
