@@ -653,6 +653,8 @@ struct Engine {
     int load_tables(const Tables &T) {
         int r;
         max_count = T.count.empty() ? 0 : *std::max_element(T.count.begin(), T.count.end());
+        loaded_n = T.nrec;
+        loaded_h = T.nhalos;
         if ((r = upload(hfirst, T.first))) return r;
         if ((r = upload(hcount, T.count))) return r;
         if ((r = upload(root_tiles, T.root_tiles))) return r;
@@ -728,6 +730,21 @@ struct Engine {
 
     static int blocks(int64_t n, int per) { return (int)((n + per - 1) / per); }
 
+    // A grid that fills the device, or what `units` workgroups' worth of work
+    // at most there can be: the kernels' lists are counted on the device, and
+    // on a small batch starting workgroups that find nothing to do would be
+    // most of a launch (2,048 workgroups on one queue counter, for one task:
+    // 45 us against 24; the centres of mass of one depth 4.5 against 3.3).
+    static int grid(int64_t units, int fill) {
+        return (int)std::min<int64_t>(std::max<int64_t>(units, 1), fill);
+    }
+    int64_t loaded_n = 0, loaded_h = 0;  // records and calls of the loaded tables
+    // nodes above their split size on one level, their tiles, and the tasks
+    // of one subtree kernel (more than `above` points each)
+    int64_t max_big() const { return loaded_n / (big_min() + 1) + 1; }
+    int64_t max_tiles() const { return loaded_n / kTile + max_big(); }
+    int64_t max_tasks(int64_t above) const { return loaded_n / (above + 1); }
+
     // ------------------------------------------------------ enqueue stages
     // Nothing below reads device memory back: every stage can be recorded
     // into a graph.  The eager driver (potential) checks the level state
@@ -776,19 +793,20 @@ struct Engine {
         if (first < 1 || first + n - 1 >= kMaxLevels)
             return set_error(HP_EINVAL, "split levels %d..%d out of range", first, first + n - 1);
         int32_t *lv = depth_buf.as<int32_t>();
+        const int lg = grid(max_tiles(), kLevelGrid);
         for (int level = first; level < first + n; level++) {
             float4 *src = (level & 1) ? A.as<float4>() : B.as<float4>();
             float4 *dst = (level & 1) ? B.as<float4>() : A.as<float4>();
             const BuildArgs ba = build_args(small0.as<Task>());
-            k_big_count<<<kLevelGrid, kTileThreads, 0, s>>>(src, tiles.as<int2>(), big.as<Task>(),
+            k_big_count<<<lg, kTileThreads, 0, s>>>(src, tiles.as<int2>(), big.as<Task>(),
                                                       nodes.as<Node>(), parts.as<TilePart>(), lv,
                                                       level);
             HP_LAUNCHED();
-            k_big_tiles<kSides><<<kLevelGrid, kTileThreads, 0, s>>>(
+            k_big_tiles<kSides><<<lg, kTileThreads, 0, s>>>(
                 src, dst, tiles.as<int2>(), big.as<Task>(), parts.as<TilePart>(),
                 splitres.as<BigSplit>(), ba, lv, level);
             HP_LAUNCHED();
-            k_big_tiles<kScatter><<<kLevelGrid, kTileThreads, 0, s>>>(
+            k_big_tiles<kScatter><<<lg, kTileThreads, 0, s>>>(
                 src, dst, tiles.as<int2>(), big.as<Task>(), parts.as<TilePart>(),
                 splitres.as<BigSplit>(), ba, lv, level);
             HP_LAUNCHED();
@@ -852,21 +870,21 @@ struct Engine {
             s3 = side[2];
         }
         if (gmax > 512) {
-            k_subtree<1024><<<sub_grid[2], 1024, 0, s>>>(
+            k_subtree<1024><<<grid(max_tasks(512), sub_grid[2]), 1024, 0, s>>>(
                 A.as<float4>(), B.as<float4>(), groupc.as<Task>() + 2 * cap_group, ba, PARTICLE_MASS, 2);
             HP_LAUNCHED();
         }
         if (gmax > 256) {
-            k_subtree<512><<<sub_grid[1], 512, 0, s1>>>(
+            k_subtree<512><<<grid(max_tasks(256), sub_grid[1]), 512, 0, s1>>>(
                 A.as<float4>(), B.as<float4>(), groupc.as<Task>() + cap_group, ba, PARTICLE_MASS, 1);
             HP_LAUNCHED();
         }
         if (gmax > kWaveMin) {
-            k_subtree<256><<<sub_grid[0], 256, 0, s2>>>(A.as<float4>(), B.as<float4>(),
+            k_subtree<256><<<grid(max_tasks(kWaveMin), sub_grid[0]), 256, 0, s2>>>(A.as<float4>(), B.as<float4>(),
                                                                groupc.as<Task>(), ba, PARTICLE_MASS, 0);
             HP_LAUNCHED();
         }
-        k_subtree_wave<<<wave_grid, kWave, 0, s3>>>(A.as<float4>(), B.as<float4>(), small0.as<Task>(),
+        k_subtree_wave<<<grid(max_tasks(kLeafPoints), wave_grid), kWave, 0, s3>>>(A.as<float4>(), B.as<float4>(), small0.as<Task>(),
                                               build_args(small0.as<Task>()), PARTICLE_MASS,
                                               wave_off.as<int32_t>());
         HP_LAUNCHED();
@@ -887,7 +905,7 @@ struct Engine {
             }
         }
         // the roots that stay leaves (at most 10 points, or as many finite)
-        k_leaf_com<<<2048, 256, 0, s>>>(nodes.as<Node>(), F.as<float4>(), cnt, PARTICLE_MASS);
+        k_leaf_com<<<grid((loaded_h + 2 * levels * max_big()) / 256 + 1, 2048), 256, 0, s>>>(nodes.as<Node>(), F.as<float4>(), cnt, PARTICLE_MASS);
         HP_LAUNCHED();
         // the calls without split levels have their whole trees now: their
         // walk on a branch beside the split levels' nodes (joined after the
@@ -904,18 +922,18 @@ struct Engine {
         // subtree kernels finished it (its root included): the fat leaves,
         // the internal nodes and dmin of the levels' nodes have no work.
         if (levels == 0) return HP_OK;
-        k_fat_leaf_com<<<256, 256, 0, s>>>(nodes.as<Node>(), fat.as<int32_t>(), cnt,
+        k_fat_leaf_com<<<grid(cap_fat / 4, 256), 256, 0, s>>>(nodes.as<Node>(), fat.as<int32_t>(), cnt,
                                            (int32_t)cap_fat, F.as<float4>(), PARTICLE_MASS);
         HP_LAUNCHED();
         for (int d = levels; d >= 0; d--) {
-            k_internal_com<<<512, 256, 0, s>>>(nodes.as<Node>(), depth_buf.as<int32_t>(), d);
+            k_internal_com<<<grid((loaded_h + 2 * max_big()) / 256 + 1, 512), 256, 0, s>>>(nodes.as<Node>(), depth_buf.as<int32_t>(), d);
             HP_LAUNCHED();
         }
-        k_dmin_tiles<<<1024, kTileThreads, 0, s>>>(nodes.as<Node>(), F.as<float4>(),
+        k_dmin_tiles<<<grid(levels * max_tiles(), 1024), kTileThreads, 0, s>>>(nodes.as<Node>(), F.as<float4>(),
                                                    tiles.as<int2>(), big.as<Task>(), cnt,
                                                    dparts.as<double2>());
         HP_LAUNCHED();
-        k_dmin_big<<<64, 256, 0, s>>>(nodes.as<Node>(), big.as<Task>(), cnt, dparts.as<double2>());
+        k_dmin_big<<<grid(levels * max_big() / 256 + 1, 64), 256, 0, s>>>(nodes.as<Node>(), big.as<Task>(), cnt, dparts.as<double2>());
         HP_LAUNCHED();
         return HP_OK;
     }
