@@ -286,7 +286,7 @@ static int make_tables(Tables &T, const int64_t *first, const int64_t *count, in
                          (long long)pos, (long long)kMaxRecords);
     T.nrec = pos;
     for (int64_t h = 0; h < nh; h++) {
-        for (int64_t off = 0; off < count[h]; off += kTile)
+        for (int64_t off = 0; off < count[h]; off += root_tile_records(count[h]))
             T.root_tiles.push_back(RootTile{(int32_t)h, (int32_t)off});
         const bool direct = method == HP_METHOD_DIRECT ||
                             (method == HP_METHOD_AUTO && count[h] <= T.direct_max);
@@ -933,7 +933,7 @@ struct Engine {
                                                    tiles.as<int2>(), big.as<Task>(), cnt,
                                                    dparts.as<double2>());
         HP_LAUNCHED();
-        k_dmin_big<<<grid(levels * max_big() / 256 + 1, 64), 256, 0, s>>>(nodes.as<Node>(), big.as<Task>(), cnt, dparts.as<double2>());
+        k_dmin_big<<<grid(levels * max_big() / 4 + 1, 2048), 256, 0, s>>>(nodes.as<Node>(), big.as<Task>(), cnt, dparts.as<double2>());
         HP_LAUNCHED();
         return HP_OK;
     }

@@ -661,6 +661,23 @@ __device__ __forceinline__ int32_t block_sum_i32(int32_t v) {
     return m;
 }
 
+// The per-call kernels run a thread per call.  A thread goes through at most
+// kFewTiles tiles by itself; the calls with more are taken one after another
+// by the whole wavefront, f(first tile, tiles, whether it is this lane's
+// call), a lane per tile: on a call of 2.1M records (1,115 tiles) the loops
+// of dependent reads were 74 to 288 us a kernel.  Called with all lanes
+// active.
+constexpr int32_t kFewTiles = 8;
+template <class F>
+__device__ __forceinline__ void for_large_calls(int32_t t0, int32_t nt, F &&f) {
+    uint64_t large = ballot(nt > kFewTiles);
+    while (large) {
+        const int l = __builtin_ctzll(large);
+        large &= large - 1;
+        f(__builtin_amdgcn_readlane(t0, l), __builtin_amdgcn_readlane(nt, l), lane_id() == l);
+    }
+}
+
 // rvir_max (src/properties.c:173-177): the largest j < kept with
 // j^2 > r2_j^3 (4pi/3 rho_vir)^2, r2^3 in float, the rest in double.
 // Per tile (k_rvir_vel_tiles, below), then per call.
@@ -670,11 +687,19 @@ __global__ void k_rvir_calls(const float4 *__restrict__ rv,
                              const int32_t *__restrict__ tile_rvir, int32_t nh,
                              CallInfo *__restrict__ ci) {
     const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    CallInfo c = ci[h];
+    const bool v = h < nh;
+    const int32_t t0 = v ? call_tile0[h] : 0, nt = v ? call_ntiles[h] : 0;
     int32_t rvm = -1;
-    for (int32_t t = call_tile0[h]; t < call_tile0[h] + call_ntiles[h]; t++)
-        rvm = tile_rvir[t] > rvm ? tile_rvir[t] : rvm;
+    if (nt <= kFewTiles)
+        for (int32_t t = t0; t < t0 + nt; t++) rvm = max(rvm, tile_rvir[t]);
+    for_large_calls(t0, nt, [&](int32_t a, int32_t n, bool mine) {
+        int32_t m = -1;
+        for (int32_t t = a + lane_id(); t < a + n; t += kWave) m = max(m, tile_rvir[t]);
+        m = wave_max(m);
+        if (mine) rvm = m;
+    });
+    if (!v) return;
+    CallInfo c = ci[h];
     c.rvir_max = rvm;
     if (rvm >= 1) {
         const float ref = rv[c.first + rvm].x;
@@ -741,18 +766,36 @@ __global__ void k_vel_prefix(const int32_t *__restrict__ call_tile0,
                              const int32_t *__restrict__ call_ntiles, int32_t nh,
                              Moments *__restrict__ tsum) {
     const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    double a[6] = {0, 0, 0, 0, 0, 0};
-    const int32_t t0 = call_tile0[h], nt = call_ntiles[h];
-    for (int32_t t = t0; t < t0 + nt; t++) {
-        const Moments m = tsum[t];
-        const double b[6] = {m.s1[0], m.s1[1], m.s1[2], m.s2[0], m.s2[1], m.s2[2]};
-        for (int k = 0; k < 3; k++) {
-            tsum[t].s1[k] = a[k];
-            tsum[t].s2[k] = a[3 + k];
+    const int32_t t0 = h < nh ? call_tile0[h] : 0, nt = h < nh ? call_ntiles[h] : 0;
+    if (nt <= kFewTiles) {
+        double a[6] = {0, 0, 0, 0, 0, 0};
+        for (int32_t t = t0; t < t0 + nt; t++) {
+            const Moments m = tsum[t];
+            const double b[6] = {m.s1[0], m.s1[1], m.s1[2], m.s2[0], m.s2[1], m.s2[2]};
+            for (int k = 0; k < 3; k++) {
+                tsum[t].s1[k] = a[k];
+                tsum[t].s2[k] = a[3 + k];
+            }
+            for (int k = 0; k < 6; k++) a[k] += b[k];
         }
-        for (int k = 0; k < 6; k++) a[k] += b[k];
     }
+    for_large_calls(t0, nt, [&](int32_t first, int32_t n, bool) {
+        double run[6] = {0, 0, 0, 0, 0, 0};
+        for (int32_t base = 0; base < n; base += kWave) {
+            const bool in = base + lane_id() < n;
+            Moments *me = tsum + first + base + (in ? lane_id() : 0);
+            const Moments m = *me;
+            const double b[6] = {m.s1[0], m.s1[1], m.s1[2], m.s2[0], m.s2[1], m.s2[2]};
+            for (int k = 0; k < 6; k++) {
+                const double y = wave_scan_add(in ? b[k] : 0.0) + run[k];
+                double before = __shfl_up(y, 1, kWave);
+                if (lane_id() == 0) before = run[k];
+                run[k] = read_lane(y, kWave - 1);
+                if (in && k < 3) me->s1[k] = before;
+                if (in && k >= 3) me->s2[k - 3] = before;
+            }
+        }
+    });
 }
 
 // Candidate prefix of the running-minimum selection: its normalised
@@ -882,8 +925,42 @@ __global__ void k_vel_finish(const float4 *__restrict__ rv,
                              const CallInfo *__restrict__ ci, const Cand *__restrict__ tcand,
                              hp_halo *__restrict__ halos, const int32_t *__restrict__ flags) {
     const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh || (*flags & kErrDeep)) return;
-    const CallInfo c = ci[h];
+    if (*flags & kErrDeep) return;
+    const bool v = h < nh;
+    CallInfo c;
+    c.rvir_max = -1;
+    if (v) c = ci[h];
+    // the best of the tiles' candidates, kept in scalars (a select of whole
+    // Cand records would go through scratch memory)
+    Cand a = no_cand(), b = no_cand();
+    auto take = [](Cand &x, const Cand &y) {
+        const bool t = y.val < x.val || (y.val == x.val && y.idx < x.idx);
+        x.val = t ? y.val : x.val;
+        x.idx = t ? y.idx : x.idx;
+#pragma unroll
+        for (int k = 0; k < 3; k++) x.s1[k] = t ? y.s1[k] : x.s1[k];
+    };
+    const bool has = v && c.rvir_max >= 1;
+    const int32_t t0 = has ? call_tile0[h] : 0, nt = has ? call_ntiles[h] : 0;
+    if (nt <= kFewTiles)
+        for (int32_t t = t0; t < t0 + nt; t++) {
+            take(a, tcand[2 * t]);
+            take(b, tcand[2 * t + 1]);
+        }
+    for_large_calls(t0, nt, [&](int32_t first, int32_t n, bool mine) {
+        Cand x = no_cand(), y = no_cand();
+        for (int32_t t = first + lane_id(); t < first + n; t += kWave) {
+            take(x, tcand[2 * t]);
+            take(y, tcand[2 * t + 1]);
+        }
+        x = wave_better(x);
+        y = wave_better(y);
+        if (mine) {
+            a = x;
+            b = y;
+        }
+    });
+    if (!v) return;
     // the fields are written one by one (a copy of the whole record would
     // sit in scratch)
     hp_halo *hh = halos + h;
@@ -892,23 +969,6 @@ __global__ void k_vel_finish(const float4 *__restrict__ rv,
     if (c.rvir_max >= 1) {
         const int32_t lim = c.rvir_max;
         const int32_t core_lim = min(c.core_max, lim);
-        // the best of the tiles' candidates, kept in scalars (a select of
-        // whole Cand records would go through scratch memory)
-        Cand a = no_cand(), b = no_cand();
-        for (int32_t t = call_tile0[h]; t < call_tile0[h] + call_ntiles[h]; t++) {
-            const Cand ca = tcand[2 * t], cb = tcand[2 * t + 1];
-            const bool ta = ca.val < a.val || (ca.val == a.val && ca.idx < a.idx);
-            const bool tb = cb.val < b.val || (cb.val == b.val && cb.idx < b.idx);
-            a.val = ta ? ca.val : a.val;
-            a.idx = ta ? ca.idx : a.idx;
-            b.val = tb ? cb.val : b.val;
-            b.idx = tb ? cb.idx : b.idx;
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                a.s1[k] = ta ? ca.s1[k] : a.s1[k];
-                b.s1[k] = tb ? cb.s1[k] : b.s1[k];
-            }
-        }
         // windows of at most 10 records: the last forced update wins
         if (core_lim <= 10) a = small_prefix(rv, c.first, core_lim - 1);
         if (lim <= 10) b = small_prefix(rv, c.first, lim - 1);
@@ -1014,10 +1074,18 @@ __global__ void k_nbound_calls(const int32_t *__restrict__ call_tile0,
                                const int32_t *__restrict__ tile_nb, int32_t nh,
                                hp_halo *__restrict__ halos, const int32_t *__restrict__ flags) {
     const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh || (*flags & kErrDeep)) return;
-    int64_t n = 0;
-    for (int32_t t = call_tile0[h]; t < call_tile0[h] + call_ntiles[h]; t++) n += tile_nb[t];
-    halos[h].n_bound = n;
+    if (*flags & kErrDeep) return;
+    const int32_t t0 = h < nh ? call_tile0[h] : 0, nt = h < nh ? call_ntiles[h] : 0;
+    int32_t n = 0;
+    if (nt <= kFewTiles)
+        for (int32_t t = t0; t < t0 + nt; t++) n += tile_nb[t];
+    for_large_calls(t0, nt, [&](int32_t first, int32_t m, bool mine) {
+        int32_t x = 0;
+        for (int32_t t = first + lane_id(); t < first + m; t += kWave) x += tile_nb[t];
+        x = wave_sum(x);
+        if (mine) n = x;
+    });
+    if (h < nh) halos[h].n_bound = n;
 }
 
 // the plain reference entry point: every record with ke >= 0, one centre
