@@ -27,6 +27,14 @@
 // Lane sets (active, inside, accepting, opening) are wavefront masks handled
 // by the scalar unit.
 //
+// What bounds it: issue.  Of the cycles of a 6.7M-record batch's walk 92% hold
+// a vector instruction (33 a node visit) and 77% a scalar one or a branch (29
+// a visit), of 93% and 79% before the accumulator and the loop's state were
+// kept in place (36 and 33 a visit, 1.64 ms; now 1.51).  Both units count: an
+// acceptance test in float with a scalar fallback (3 vector instructions
+// less, 8 scalar ones more) and a scalar test of the node's range (2 less, 4
+// more) made the walk 7 and 6% slower.
+//
 // Pair arithmetic is FP32 (rsqrt, clamp at FORCE_RES for particle pairs,
 // src/potential.c:31-36) with compensated accumulation: terms are summed in
 // short FP32 blocks (<= 16 terms) that are folded into a (hi, lo) pair by
@@ -53,17 +61,17 @@ struct Acc<HP_ACC_COMPENSATED> {
     float hi = 0.0f, lo = 0.0f, blk = 0.0f;
     __device__ __forceinline__ void add(float t) { blk += t; }
     __device__ __forceinline__ void fold() {
-        float s, e;
-        two_sum(hi, blk, s, e);
-        hi = s;
-        lo += e;
+        add_block(blk);
         blk = 0.0f;
     }
+    // hi and lo are updated where they are: left to itself the compiler
+    // gives the new pair registers of its own and moves it at every join of
+    // the walk's paths, two moves a visit
     __device__ __forceinline__ void add_block(float t) {
         float s, e;
         two_sum(hi, t, s, e);
-        hi = s;
-        lo += e;
+        asm("v_add_f32 %0, %0, %1" : "+v"(hi) : "v"(t));
+        asm("v_add_f32 %0, %0, %1" : "+v"(lo) : "v"(e));
     }
     __device__ __forceinline__ double value() const {
         return ((double)hi + (double)lo) + (double)blk;
@@ -151,7 +159,7 @@ struct Walker {
 
     // Node nd for the lanes of `act` (those whose walk reaches it): the
     // monopole where it is accepted, the leaf's particle pairs where a leaf
-    // is opened.  Returns the lanes that open nd (none for a leaf).  Lane
+    // is opened.  Returns the lanes that open nd (or sum its pairs).  Lane
     // sets are wavefront masks (the compares write them directly), combined
     // on the scalar unit.
     __device__ __forceinline__ uint64_t visit(const NodeHead &nd, uint64_t act) {
@@ -187,23 +195,25 @@ struct Walker {
                 }
             }
         }
-        // an internal node is opened by a lane whose leaf lies inside it or
-        // that does not accept it
-        if (nd.left >= 0) return act & (inr | ~ok);
-        // a leaf: particle pairs, softened (src/potential.c:38-55); the self
-        // leaf only up to 20 points (src/potential.c:144-146)
-        const uint64_t p2p = act & ((nd.count <= kDegenerate ? inr : 0ull) | (~inr & ~ok));
-        if (p2p) {
+        // the others open nd: their leaf lies inside it, or they don't accept
+        // it.  A leaf: particle pairs, softened (src/potential.c:38-55); the
+        // self leaf only up to 20 points (src/potential.c:144-146)
+        const uint64_t open = act & ~p2m;
+        if (nd.left < 0) {
+            const uint64_t p2p = nd.count <= kDegenerate ? open : open & ~inr;
+            const uint64_t self = p2p & inr;
             if constexpr (COUNT) {
                 n_p2p += (unsigned long long)__popcll(p2p) * (unsigned long long)nd.count -
-                         (unsigned long long)__popcll(p2p & inr);
+                         (unsigned long long)__popcll(self);
             }
+            // the self pair is left out only where a lane's own leaf is
+            // summed (two tests and not an else: behind an else the compiler
+            // keeps the accumulator from before it too, and moves it around)
             const bool mine = __builtin_amdgcn_inverse_ballot_w64(p2p);
-            // the self pair is left out only where a lane's own leaf is summed
-            if (p2p & inr) leaf_pairs<true>(nd, mine);
-            else leaf_pairs<false>(nd, mine);
+            if (self) leaf_pairs<true>(nd, mine);
+            if (self == 0 && p2p) leaf_pairs<false>(nd, mine);
         }
-        return 0;
+        return open;
     }
 
     // The pairs of this lane's sink with the leaf's points, added when p2p.
@@ -214,7 +224,8 @@ struct Walker {
         struct Batch {
             float4 q[kSrcBatch];
         };
-        for (int32_t j0 = 0; j0 < nd.count; j0 += kSrcBatch) {
+        int32_t j0 = 0;
+        do {  // at least once: a batch of no points adds 0
             const int32_t cnt = min(kSrcBatch, nd.count - j0);
             const Batch b = load_const(reinterpret_cast<const Batch *>(fin + nd.first + j0));
             // all of the batch's loads are issued before the first use (the
@@ -255,7 +266,8 @@ struct Walker {
                 }
                 acc.add_block(p2p ? pm * s : 0.0f);
             }
-        }
+            j0 += kSrcBatch;
+        } while (j0 < nd.count);
     }
 
     // Sibling-pair walk.  Both children of an opened node are decided in one
@@ -277,41 +289,46 @@ struct Walker {
         int32_t st_c = 0, st_lo = 0, st_hi = 0;
         int32_t sp = 0;
         uint64_t m = live;
-        int32_t c = rn.left;
-        int32_t guard = cap, fail = 0;
-        while (c >= 0) {
-            if (sp > kWave) break;  // a pending pair was lost: the caller walks node by node
-            --guard;
-            fail = (uint32_t)c >= (uint32_t)(nnodes - 1) ? kErrBadTree : (guard < 0 ? kErrWalkCap : 0);
-            if (fail != 0) break;
+        // A step is run while three numbers are below 0, tested by the sign
+        // of their and: c - lim (c is a node whose sibling exists), left
+        // (the steps left) and full (no pending pair was lost).  One
+        // exit, at the loop's end: every value that leaves the loop is
+        // defined there, and those of the wavefront stay scalar.
+        constexpr int32_t kEnd = INT32_MAX;  // no pair is left
+        const int32_t lim = nnodes - 1;
+        int32_t c = rn.left, left = -cap, full = -1;
+        while (((c - lim) & left & full) < 0) {
             const NodeHead n0 = load_const(reinterpret_cast<const NodeHead *>(nodes + c));
             const NodeHead n1 = load_const(reinterpret_cast<const NodeHead *>(nodes + c + 1));
             // both loads are issued before either node is used
             asm volatile("" ::"s"(n1.com[0]), "s"(n1.dmin2), "s"(n1.left), "s"(n0.com[0]));
-            const uint64_t m0 = visit(n0, m);
-            const uint64_t m1 = visit(n1, m);
+            uint64_t m0 = visit(n0, m);
+            uint64_t m1 = visit(n1, m);
+            if (n0.left < 0) m0 = 0;
+            if (n1.left < 0) m1 = 0;
             if (m1) {
                 // entry sp of the stack: lane sp of each register (a lane
-                // past 63 selects none, and the check above ends the walk)
+                // past 63 selects none, and `full` ends the walk)
                 write_lane(st_c, n1.left, sp);
                 write_lane(st_lo, (int32_t)(uint32_t)m1, sp);
                 write_lane(st_hi, (int32_t)(uint32_t)(m1 >> 32), sp);
                 sp++;
             }
+            full = sp - (kWave + 1);
             if (m0) {
                 c = n0.left;
                 m = m0;
-            } else if (sp > 0 && sp <= kWave) {
-                sp--;
-                c = __builtin_amdgcn_readlane(st_c, sp);
-                m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(st_hi, sp) << 32) |
-                    (uint32_t)__builtin_amdgcn_readlane(st_lo, sp);
             } else {
-                c = -1;
+                sp--;
+                const int32_t top = sp & (kWave - 1);
+                c = sp < 0 ? kEnd : __builtin_amdgcn_readlane(st_c, top);
+                m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(st_hi, top) << 32) |
+                    (uint32_t)__builtin_amdgcn_readlane(st_lo, top);
             }
+            left++;
         }
-        if (fail && lane == 0) atomicOr(err, fail);
-        return sp <= kWave;
+        if (full < 0 && c != kEnd && lane == 0) atomicOr(err, c >= lim ? kErrBadTree : kErrWalkCap);
+        return full < 0;
     }
 
     // Node-by-node walk.  The wavefront visits the union of the lanes'
@@ -337,7 +354,8 @@ struct Walker {
             }
             const Node nd = load_const(nodes + c);
             const uint64_t act = ballot(resume == c);
-            const uint64_t open = visit(*reinterpret_cast<const NodeHead *>(&nd), act);
+            uint64_t open = visit(*reinterpret_cast<const NodeHead *>(&nd), act);
+            if (nd.left < 0) open = 0;
             if (__builtin_amdgcn_inverse_ballot_w64(act))
                 resume = __builtin_amdgcn_inverse_ballot_w64(open) ? nd.left : nd.skip;
             c = open ? nd.left : nd.skip;
@@ -384,7 +402,7 @@ __global__ __launch_bounds__(64) void k_walk(WalkArgs a) {
     w.fin = a.fin;
     const Node *__restrict__ nodes = a.nodes;
     asm volatile("" ::"s"(w.pm), "s"(w.pm_d), "s"(w.fr_d), "s"(w.fin), "s"(nodes));
-    const int32_t cap = 2 * rn.count + 4;
+    const int32_t cap = uniform(2 * rn.count + 4);
     bool done = false;
     const uint64_t live_m = ballot(live);
     if (a.pairs) done = w.walk_pairs(nodes, rn, live_m, nnodes, cap, a.err);
