@@ -387,7 +387,7 @@ struct Engine {
     DevBuf seg_wave_l, seg_block_l, seg_tiles_l, seg_hist, seg_hsum, srt_rv;
     // halo properties
     DevBuf pcnt, pscan, pcall, psums, shape_st, shape_part, shape_cd, scale_calls, r_pe, pe_cnt,
-        fit_list, fit_n;
+        fit_list, fit_n, shape_one, shape_pairs, shape_windows;
     // record assembly
     DevBuf gsegs, gtiles, gcen;
     SubBufs sub;
@@ -487,7 +487,7 @@ struct Engine {
         DevBuf *all[] = {&hfirst, &hcount, &root_tiles, &groups, &direct_blocks,
                          &scan_tiles, &call_tile0, &call_ntiles, &box, &bad, &pot, &rkey, &badlist, &A, &B, &F,
                          &leaf_of, &sides, &nodes, &parent, &fat, &small0, &group0, &groupc, &wave_off, &wave_hsum, &big, &tiles,
-                         &parts, &splitres, &dparts, &counters, &work, &depth_buf, &pcnt, &pscan, &pcall, &psums, &shape_st, &shape_part, &shape_cd, &scale_calls, &r_pe, &pe_cnt, &fit_list, &fit_n, &gsegs, &gtiles, &gcen, &keys0, &keys1, &vals0,
+                         &parts, &splitres, &dparts, &counters, &work, &depth_buf, &pcnt, &pscan, &pcall, &psums, &shape_st, &shape_part, &shape_cd, &scale_calls, &r_pe, &pe_cnt, &fit_list, &fit_n, &shape_one, &shape_pairs, &shape_windows, &gsegs, &gtiles, &gcen, &keys0, &keys1, &vals0,
                          &vals1, &hist, &hsum, &srt, &callinfo, &tsum, &tcand, &tile_i32, &rec_call, &strip_cnt, &stage,
                          &seg_wave_l, &seg_block_l, &seg_tiles_l, &seg_hist, &seg_hsum, &srt_rv};
         for (DevBuf *b : all) f(*b);
@@ -1346,7 +1346,10 @@ struct Engine {
         HP_ENSURE(r_pe, sizeof(double) * (H + 1));
         HP_ENSURE(pe_cnt, sizeof(int32_t) * (nst + 1));
         HP_ENSURE(fit_list, sizeof(int32_t) * (H + 1));
-        HP_ENSURE(fit_n, sizeof(int32_t) * 2);
+        HP_ENSURE(fit_n, sizeof(int32_t) * (1 + kShapeLists));
+        HP_ENSURE(shape_one, sizeof(int32_t) * 2 * (H + 1));
+        HP_ENSURE(shape_pairs, sizeof(int32_t) * 2 * (nst + 1));
+        HP_ENSURE(shape_windows, sizeof(int32_t) * 2 * (H + 1));
         PropArgs pa;
         const double four_thirds_pi = 4.0 * M_PI / 3.0;  // src/properties.c:393-398
         pa.dens_thresh = md.thresh_dens[0] * four_thirds_pi;
@@ -1397,19 +1400,33 @@ struct Engine {
                                                shape_cd.as<float4>());
             HP_LAUNCHED();
         }
-        for (int it = 0; it < kShapeIterations; it++) {
-            if (nst > 0) {
-                k_shape_tiles<<<std::min(nst, 8192), kWave, 0, s>>>(
-                    tl, nst, hf, ss, shape_cd.as<float4>(), shape_part.as<ShapePart>());
+        // the windows of few records in one launch, the large ones an
+        // iteration at a time
+        int32_t *cnts = fit_n.as<int32_t>();
+        k_fill_i32<<<1, 64, 0, s>>>(cnts, 0, 1 + kShapeLists);
+        HP_LAUNCHED();
+        if (nst > 0) {
+            const ShapeLists sl = {shape_one.as<int32_t>(), shape_pairs.as<int32_t>(),
+                                   shape_windows.as<int32_t>(), cnts + 1};
+            k_shape_list<<<blocks(nst, kListThreads), kListThreads, 0, s>>>(tl, nst, ss, sl);
+            HP_LAUNCHED();
+            // few windows: four to a workgroup, so that they spread over the GPU
+            k_shape_small<<<kOneTileGroups + std::min<int>(blocks(2 * (int64_t)H, 4), kShapeGroups),
+                            kShapeThreads, 0, s>>>(H, hf, shape_cd.as<float4>(), sl.one,
+                                                   sl.counts + kOneTile, ss);
+            HP_LAUNCHED();
+            for (int it = 0; it < kShapeIterations; it++) {
+                k_shape_tiles<<<std::min(2 * nst, 8192), kWave, 0, s>>>(
+                    sl.pairs, sl.counts + kPairs, tl, hf, ss, shape_cd.as<float4>(),
+                    shape_part.as<ShapePart>());
+                HP_LAUNCHED();
+                k_shape_large<<<std::min(2 * H, 2048), kWave, 0, s>>>(
+                    sl.windows, sl.counts + kLarge, it, t0, tn, shape_part.as<ShapePart>(),
+                    ss);
                 HP_LAUNCHED();
             }
-            k_shape_calls<<<blocks(2 * (int64_t)H, 128), 128, 0, s>>>(
-                H, it, t0, tn, shape_part.as<ShapePart>(), ss);
-            HP_LAUNCHED();
         }
         // calc_scale_radius and the pseudo-evolution masses
-        k_fill_i32<<<1, 64, 0, s>>>(fit_n.as<int32_t>(), 0, 1);
-        HP_LAUNCHED();
         k_scale_init<<<blocks(H, 256), 256, 0, s>>>(H, d_po, hf, t0, tn, pcall.as<PropCall>(),
                                                     psums.as<PropSums>(),
                                                     scale_calls.as<ScaleCall>(),

@@ -459,8 +459,11 @@ __global__ void k_props_final(const struct potential *__restrict__ srt,
 // [0, dens_tot) with the final h->r.  Each iteration is a tile pass (the
 // weighted second moments of the bound records inside the current
 // ellipsoid) and a per-(call, window) step: normalise, Jacobi, axis ratios,
-// convergence.  The host runs SHAPE_ITERATIONS iterations; a window that has
-// stopped is skipped.  The records' offsets from the centre (float
+// convergence.  Windows of one tile run all of their iterations in one
+// launch (k_shape_small); the others take two launches an iteration, a
+// window that has stopped being skipped.  On 50,000 calls (6.7M records) ten
+// tile passes over everything and their per-window steps were 1.67 ms; now
+// 0.68 ms in the one launch and 0.24 in the twenty.  The records' offsets from the centre (float
 // differences, as the reference takes them) and bound flags are compacted
 // once into 16 bytes per record.
 
@@ -474,18 +477,13 @@ struct ShapeState {
     float b_to_a, c_to_a, A[3];
     float inertia[6];
     int32_t n;         // records [0, n)
-    int32_t limit;     // iterations to run; -1 until the first pass counted
     int32_t done;
     int32_t assigned;  // inertia written by this window
     int32_t nbound;    // bound records in [0, n)
-    int32_t pad;
 };
 
 struct ShapePart {
-    double w;
-    double t[6];       // xx, yy, zz, yx, zx, zy
-    int32_t cnt;       // bound records of the window in the tile
-    int32_t pad;
+    double v[8];       // weight, xx, yy, zz, yx, zx, zy, unused
 };
 
 __global__ void k_shape_init(int32_t nh, const hp_halo *__restrict__ halos,
@@ -510,11 +508,9 @@ __global__ void k_shape_init(int32_t nh, const hp_halo *__restrict__ halos,
             for (int l = 0; l < 3; l++) s.orth[k][l] = k == l ? 1.0 : 0.0;
             s.eig[k] = (double)(s.r * s.r) * 1e-6;
         }
-        s.limit = -1;
         s.done = !(s.r > 0) || s.n <= 0;
         s.assigned = 0;
         s.nbound = 0;
-        s.pad = 0;
         st[2 * h + w] = s;
     }
 }
@@ -561,114 +557,116 @@ __device__ __forceinline__ bool shape_exact(const ShapeState &s) {
     return s.n <= kShapeExactRecords || s.nbound < kShapeExactBound;
 }
 
-// src/properties.c:243-268 for one tile, both windows
-__global__ __launch_bounds__(kWave) void k_shape_tiles(const ScanTile *__restrict__ tiles,
-                                                       int32_t ntiles,
+// one record's terms (src/properties.c:243-268): the weight 1 / r and the
+// weighted second moments, or false where the ellipsoid does not hold it
+__device__ __forceinline__ bool shape_terms(double r, double min_r, const double (&d)[3],
+                                            double (&v)[7]) {
+    if (r < min_r) r = min_r;
+    if (!(r > 0 && r <= 1)) return false;
+    const double tw = 1.0 / r;  // WEIGHTED_SHAPES = 1
+    v[0] = tw;
+    v[1] = d[0] * d[0] * tw;
+    v[2] = d[1] * d[1] * tw;
+    v[3] = d[2] * d[2] * tw;
+    v[4] = d[0] * d[1] * tw;
+    v[5] = d[0] * d[2] * tw;
+    v[6] = d[1] * d[2] * tw;
+    return true;
+}
+
+// The windows too large to be summed record by record: those of one tile,
+// and those of several as (tile, window) pairs 2 tile + window for
+// k_shape_tiles and as windows for k_shape_large.  The lists' order does not
+// reach the results: a pair's sums have a place of their own and are added
+// in tile order.  A workgroup takes its places in one atomic a list (one a
+// wavefront took 36 us on 50,000 calls, all on three addresses).
+constexpr int kListThreads = 1024;
+enum { kOneTile, kPairs, kLarge, kShapeLists };
+struct ShapeLists {
+    int32_t *one;      // windows
+    int32_t *pairs;
+    int32_t *windows;
+    int32_t *counts;   // of each
+};
+
+__global__ __launch_bounds__(kListThreads) void k_shape_list(const ScanTile *__restrict__ tiles,
+                                                             int32_t ntiles,
+                                                             const ShapeState *__restrict__ st,
+                                                             ShapeLists out) {
+    __shared__ int32_t s_n[kShapeLists], s_base[kShapeLists];
+    const int32_t tid = threadIdx.x, t = blockIdx.x * kListThreads + tid;
+    if (tid < kShapeLists) s_n[tid] = 0;
+    __syncthreads();
+    const ScanTile tl = t < ntiles ? tiles[t] : ScanTile{};
+    int32_t at[2][kShapeLists];  // place in the workgroup's part of each list, or -1
+    for (int w = 0; w < 2; w++) {
+        bool use = false, one = false;
+        if (t < ntiles) {
+            const ShapeState &s = st[2 * tl.call + w];
+            use = !s.done && !shape_exact(s) && tl.off < s.n;
+            one = use && s.n <= kScanTile;
+        }
+        at[w][kOneTile] = one ? atomicAdd(&s_n[kOneTile], 1) : -1;
+        at[w][kPairs] = use && !one ? atomicAdd(&s_n[kPairs], 1) : -1;
+        at[w][kLarge] = use && !one && tl.off == 0 ? atomicAdd(&s_n[kLarge], 1) : -1;
+    }
+    __syncthreads();
+    if (tid < kShapeLists) s_base[tid] = s_n[tid] ? atomicAdd(&out.counts[tid], s_n[tid]) : 0;
+    __syncthreads();
+    for (int w = 0; w < 2; w++) {
+        if (at[w][kOneTile] >= 0) out.one[s_base[kOneTile] + at[w][kOneTile]] = 2 * tl.call + w;
+        if (at[w][kPairs] >= 0) out.pairs[s_base[kPairs] + at[w][kPairs]] = 2 * t + w;
+        if (at[w][kLarge] >= 0) out.windows[s_base[kLarge] + at[w][kLarge]] = 2 * tl.call + w;
+    }
+}
+
+// The sums of a window's records [off, end), lanes strided, in the ellipsoid
+// of orth (by rows) and eig
+__device__ __forceinline__ void shape_sums(const double *orth, const double *eig, double min_r,
+                                           const float4 *__restrict__ rec, int32_t off,
+                                           int32_t end, double (&acc)[7]) {
+    double o[3][3], ie[3];
+    for (int k = 0; k < 7; k++) acc[k] = 0.0;
+    for (int k = 0; k < 3; k++) {
+        ie[k] = 1.0 / eig[k];  // the reference divides per record; within 1 ulp
+        for (int l = 0; l < 3; l++) o[k][l] = orth[3 * k + l];
+    }
+    for (int32_t j = off + lane_id(); j < end; j += kWave) {
+        const float4 q = rec[j];
+        if (q.w == 0.0f) continue;
+        const double d[3] = {(double)q.x, (double)q.y, (double)q.z};
+        double r = 0;
+        for (int k = 0; k < 3; k++) {
+            double dr = 0;
+            for (int l = 0; l < 3; l++) dr += o[k][l] * d[l];
+            r += dr * dr * ie[k];
+        }
+        double v[7];
+        if (!shape_terms(r, min_r, d, v)) continue;
+        for (int k = 0; k < 7; k++) acc[k] += v[k];
+    }
+    for (int k = 0; k < 7; k++) acc[k] = wave_sum(acc[k]);
+}
+
+// src/properties.c:243-268 for the pairs of a large window and a tile
+__global__ __launch_bounds__(kWave) void k_shape_tiles(const int32_t *__restrict__ pairs,
+                                                       const int32_t *__restrict__ npairs,
+                                                       const ScanTile *__restrict__ tiles,
                                                        const int64_t *__restrict__ hfirst,
                                                        const ShapeState *__restrict__ st,
                                                        const float4 *__restrict__ cd,
                                                        ShapePart *__restrict__ part) {
-    __shared__ double s_term[kWave][8];
-    for (int32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const ScanTile tl = tiles[t];
-    const int64_t first = hfirst[tl.call];
-    for (int w = 0; w < 2; w++) {
-        const ShapeState &s = st[2 * tl.call + w];
-        double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-        int32_t cnt = 0;
-        if (!s.done && shape_exact(s)) {
-            // the window's first tile sums the whole window in record order
-            // (src/properties.c:243-268: r with the divisions by eig, then
-            // the running sums); the other tiles add nothing
-            if (tl.off == 0) {
-                const int lane = lane_id();
-                for (int32_t base = 0; base < s.n; base += kWave) {
-                    const int32_t j = base + lane;
-                    bool take = false;
-                    if (j < s.n) {
-                        const float4 q = cd[first + j];
-                        if (q.w != 0.0f) {
-                            cnt++;
-                            const double d[3] = {(double)q.x, (double)q.y, (double)q.z};
-                            double r = 0;
-                            for (int k = 0; k < 3; k++) {
-                                double dr = 0;
-                                for (int l = 0; l < 3; l++) dr += s.orth[k][l] * d[l];
-                                r += dr * dr / s.eig[k];
-                            }
-                            if (r < (double)s.min_r) r = s.min_r;
-                            if (r > 0 && r <= 1) {
-                                take = true;
-                                const double tw = 1.0 / r;  // WEIGHTED_SHAPES = 1
-                                s_term[lane][0] = tw;
-                                s_term[lane][1] = d[0] * d[0] * tw;
-                                s_term[lane][2] = d[1] * d[1] * tw;
-                                s_term[lane][3] = d[2] * d[2] * tw;
-                                s_term[lane][4] = d[0] * d[1] * tw;
-                                s_term[lane][5] = d[0] * d[2] * tw;
-                                s_term[lane][6] = d[1] * d[2] * tw;
-                            }
-                        }
-                    }
-                    uint64_t m = ballot(take);
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    while (m) {  // every lane keeps the same running sums
-                        const int i = __builtin_ctzll(m);
-                        m &= m - 1;
-                        for (int k = 0; k < 7; k++) acc[k] += s_term[i][k];
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                }
-            }
-            ShapePart pt;
-            pt.w = acc[0];
-            for (int k = 0; k < 6; k++) pt.t[k] = acc[k + 1];
-            pt.cnt = wave_sum(cnt);
-            pt.pad = 0;
-            if (lane_id() == 0) part[2 * t + w] = pt;
-            continue;
-        }
-        if (!s.done) {
-            const int32_t end = min(tl.off + kScanTile, s.n);
-            double o[3][3], ie[3];
-            for (int k = 0; k < 3; k++) {
-                ie[k] = 1.0 / s.eig[k];  // the reference divides per record; within 1 ulp
-                for (int l = 0; l < 3; l++) o[k][l] = s.orth[k][l];
-            }
-            for (int32_t j = tl.off + lane_id(); j < end; j += kWave) {
-                const float4 q = cd[first + j];
-                if (q.w == 0.0f) continue;
-                cnt++;
-                const double d[3] = {(double)q.x, (double)q.y, (double)q.z};
-                double r = 0;
-                for (int k = 0; k < 3; k++) {
-                    double dr = 0;
-                    for (int l = 0; l < 3; l++) dr += o[k][l] * d[l];
-                    r += dr * dr * ie[k];
-                }
-                if (r < (double)s.min_r) r = s.min_r;
-                if (!(r > 0 && r <= 1)) continue;
-                const double tw = 1.0 / r;  // WEIGHTED_SHAPES = 1
-                acc[0] += tw;
-                acc[1] += d[0] * d[0] * tw;
-                acc[2] += d[1] * d[1] * tw;
-                acc[3] += d[2] * d[2] * tw;
-                acc[4] += d[0] * d[1] * tw;
-                acc[5] += d[0] * d[2] * tw;
-                acc[6] += d[1] * d[2] * tw;
-            }
-        }
-        ShapePart pt;
-        pt.w = wave_sum(acc[0]);
-        for (int k = 0; k < 6; k++) pt.t[k] = wave_sum(acc[k + 1]);
-        pt.cnt = wave_sum(cnt);
-        pt.pad = 0;
-        if (lane_id() == 0) part[2 * t + w] = pt;
-    }
+    for (int32_t i = blockIdx.x; i < *npairs; i += gridDim.x) {
+        const int32_t e = pairs[i];
+        const ScanTile tl = tiles[e >> 1];
+        const int64_t first = hfirst[tl.call];
+        const ShapeState &s = st[2 * tl.call + (e & 1)];
+        if (s.done) continue;
+        double acc[7];
+        shape_sums(&s.orth[0][0], s.eig, (double)s.min_r, cd + first, tl.off,
+                   min(tl.off + kScanTile, s.n), acc);
+        if (lane_id() == 0)
+            for (int k = 0; k < 7; k++) part[e].v[k] = acc[k];
     }
 }
 
@@ -685,135 +683,93 @@ __device__ __forceinline__ double add_sqrt_ext(double a_abs, double x) {
 }
 
 // The cyclic Jacobi eigenvalue iteration of src/jacobi.c:8-135 (largest
-// off-diagonal element first, each row's largest column cached, stop when
-// no eigenvalue changes by more than 1e-6 of itself).  orth's rows are the
-// eigenvectors; m is left symmetric.  With three rows the pivot (k, l) is
-// (0, 1), (0, 2) or (1, 2); each case is spelled out with constant indices
-// so that the matrices stay in registers.
+// off-diagonal element first, each row's largest column cached, stop when no
+// eigenvalue changes by more than 1e-6 of itself) for three rows.  orth's
+// rows are the eigenvectors.  The pivot (k, l) is (0, 1), (0, 2) or (1, 2),
+// with n the third row: the lanes of a wavefront take different ones, so one
+// rotation serves all, on operands taken and put back by selects (a branch
+// per pivot ran the some 250 instructions of a rotation up to three times).
 struct Jacobi3 {
-    double m[3][3], eig[3], orth[3][3];
-    int max_col[3], changed[3], state;
-    double c, s;
+    double m01, m02, m12, eig[3], orth[3][3];
 
-    template <int W, int X, int Y, int Z, bool R>
-    __device__ __forceinline__ void rot(double (&M)[3][3]) {
-        const double tt = M[W][X], uu = M[Y][Z];
-        M[W][X] = tt * c - s * uu;
-        M[Y][Z] = s * tt + c * uu;
-        if (R) {
-            if (fabs(M[W][X]) > fabs(col(M, W))) max_col[W] = X;
-            if (Y < 3 && fabs(M[Y][Z]) > fabs(col(M, Y))) max_col[Y] = Z;
-        }
-    }
-    // M[w][max_col[w]] for the rows that hold a cached column (0 and 1)
-    __device__ __forceinline__ double col(const double (&M)[3][3], int w) const {
-        const int j = max_col[w];
-        return w == 0 ? (j == 1 ? M[0][1] : M[0][2]) : M[1][2];
-    }
-    __device__ __forceinline__ void update(int x, double y) {
-        double &e = x == 0 ? eig[0] : (x == 1 ? eig[1] : eig[2]);
-        int &ch = x == 0 ? changed[0] : (x == 1 ? changed[1] : changed[2]);
-        e += y;
-        if (ch && fabs(y) < 1e-6 * fabs(e)) {
-            ch = 0;
-            state--;
-        } else if (!ch && fabs(y) > 1e-6 * fabs(e)) {
-            ch = 1;
-            state++;
-        }
-    }
-    template <int K, int L>
-    __device__ __forceinline__ bool step() {
-        const double v = m[K][L];
-        if (v == 0.0) return false;
-        const double a = (eig[L] - eig[K]) * 0.5;
-        double t = add_sqrt_ext(fabs(a), v * v + a * a);
-        s = add_sqrt_ext(0.0, v * v + t * t);
-        c = t / s;
-        s = v / s;
-        t = v * v / t;
-        if (a < 0) {
-            s = -s;
-            t = -t;
-        }
-        update(K, -t);
-        update(L, t);
-        m[K][L] = 0.0;
-        // src/jacobi.c:113-124: rows before k, between k and l, after l
-        if (K == 1) rot<0, 1, 0, L, true>(m);
-        if (K == 0 && L == 2) rot<0, 1, 1, 2, true>(m);
-        if (K == 0 && L == 1) rot<0, 2, 1, 2, true>(m);
-        rot<K, 0, L, 0, false>(orth);
-        rot<K, 1, L, 1, false>(orth);
-        rot<K, 2, L, 2, false>(orth);
-        return true;
-    }
-    __device__ void run() {
-        max_col[0] = fabs(m[0][2]) > fabs(m[0][1]) ? 2 : 1;  // ties keep the first column
-        max_col[1] = 2;
-        max_col[2] = 3;
+    // from the matrix's diagonal in eig
+    __device__ __forceinline__ void run() {
         for (int i = 0; i < 3; i++)
             for (int j = 0; j < 3; j++) orth[i][j] = i == j ? 1.0 : 0.0;
-        state = 0;
-        for (int i = 0; i < 3; i++) {
-            eig[i] = m[i][i];
-            changed[i] = 1;
+        bool col2 = fabs(m02) > fabs(m01);  // row 0's largest column: 2, else 1 (also on ties)
+        // rows whose eigenvalue still changes
+        bool ch[3] = {m01 != 0.0 || m02 != 0.0, m01 != 0.0 || m12 != 0.0, m02 != 0.0 || m12 != 0.0};
+        for (int guard = 0; (ch[0] || ch[1] || ch[2]) && guard < 1000; guard++) {
+            const bool row1 = fabs(m12) > fabs(col2 ? m02 : m01);
+            const bool p02 = !row1 && col2, p01 = !row1 && !col2;
+            const double v = row1 ? m12 : (p02 ? m02 : m01);
+            if (v == 0.0) break;
+            // k = 1 in row 1, else 0; l = 1 for (0, 1), else 2
+            double ek = row1 ? eig[1] : eig[0], el = p01 ? eig[1] : eig[2];
+            const double a = (el - ek) * 0.5;
+            double t = add_sqrt_ext(fabs(a), v * v + a * a);
+            double s = add_sqrt_ext(0.0, v * v + t * t);
+            const double c = t / s;
+            s = v / s;
+            t = v * v / t;
+            if (a < 0) {
+                s = -s;
+                t = -t;
+            }
+            ek += -t;
+            el += t;
+            const bool ck = changes(row1 ? ch[1] : ch[0], t, ek);
+            const bool cl = changes(p01 ? ch[1] : ch[2], t, el);
+            if (row1) eig[1] = ek, ch[1] = ck;
+            else eig[0] = ek, ch[0] = ck;
+            if (p01) eig[1] = el, ch[1] = cl;
+            else eig[2] = el, ch[2] = cl;
+            // src/jacobi.c:113-124: elements (k, n) and (l, n)
+            const double p = p02 || row1 ? m01 : m02, q = row1 ? m02 : m12;
+            const double p2 = p * c - s * q, q2 = s * p + c * q;
+            m01 = p01 ? 0.0 : p2;
+            m02 = p02 ? 0.0 : (row1 ? q2 : p2);
+            m12 = row1 ? 0.0 : q2;
+            col2 = col2 ? !(fabs(m01) > fabs(m02)) : fabs(m02) > fabs(m01);
+            for (int x = 0; x < 3; x++) {
+                const double ok = row1 ? orth[1][x] : orth[0][x];
+                const double ol = p01 ? orth[1][x] : orth[2][x];
+                const double ok2 = ok * c - s * ol, ol2 = s * ok + c * ol;
+                orth[0][x] = row1 ? orth[0][x] : ok2;
+                orth[1][x] = row1 ? ok2 : (p01 ? ol2 : orth[1][x]);
+                orth[2][x] = p01 ? orth[2][x] : ol2;
+            }
         }
-        if (m[0][1] == 0.0 && m[0][2] == 0.0) { state--; changed[0] = 0; }
-        if (m[1][0] == 0.0 && m[1][2] == 0.0) { state--; changed[1] = 0; }
-        if (m[2][0] == 0.0 && m[2][1] == 0.0) { state--; changed[2] = 0; }
-        state += 3;
-        for (int guard = 0; state && guard < 1000; guard++) {
-            const bool row1 = fabs(m[1][2]) > fabs(col(m, 0));
-            bool go;
-            if (row1) go = step<1, 2>();
-            else if (max_col[0] == 1) go = step<0, 1>();
-            else go = step<0, 2>();
-            if (!go) break;
-        }
-        m[0][1] = m[1][0];
-        m[0][2] = m[2][0];
-        m[1][2] = m[2][1];
+    }
+    // whether an eigenvalue changed by y still counts as changing
+    static __device__ __forceinline__ bool changes(bool ch, double y, double e) {
+        return ch ? !(fabs(y) < 1e-6 * fabs(e)) : fabs(y) > 1e-6 * fabs(e);
     }
 };
 
-// src/properties.c:270-325 for each (call, window) still running
-__global__ void k_shape_calls(int32_t nh, int32_t it, const int32_t *__restrict__ call_tile0,
-                              const int32_t *__restrict__ call_ntiles,
-                              const ShapePart *__restrict__ part, ShapeState *__restrict__ st) {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 2 * nh) return;
-    ShapeState &s = st[i];
-    if (s.done) return;
-    const int32_t h = i >> 1, w = i & 1;
-    double wt = 0.0, t6[6] = {0, 0, 0, 0, 0, 0};
-    int64_t cnt = 0;
-    for (int32_t t = call_tile0[h]; t < call_tile0[h] + call_ntiles[h]; t++) {
-        const ShapePart &pt = part[2 * t + w];
-        wt += pt.w;
-        for (int k = 0; k < 6; k++) t6[k] += pt.t[k];
-        cnt += pt.cnt;
-    }
-    if (s.limit < 0) {  // src/properties.c:228-236
-        if (cnt < 3) {
-            s.done = 1;
-            return;
-        }
-        s.limit = (int32_t)min((int64_t)kShapeIterations, cnt);
-    }
-    if (it >= s.limit || !(wt != 0.0)) {
-        s.done = 1;
-        return;
-    }
+// A window's running values; its other results go to its ShapeState as they
+// are found.
+struct ShapeRun {
+    float r, b_to_a, c_to_a;
+    int32_t it, limit;
+};
+
+// src/properties.c:270-325: the window's next ellipsoid (orth by rows, eig)
+// from its sums (the weight and the six moments).  Returns false where the
+// window stops.
+__device__ __forceinline__ bool shape_step(ShapeRun &s, const double (&sum)[7],
+                                           ShapeState *__restrict__ out, double *orth,
+                                           double *eig) {
+    const double wt = sum[0];
+    const double *t6 = sum + 1;
+    if (s.it >= s.limit || !(wt != 0.0)) return false;
     Jacobi3 jb;
-    jb.m[0][0] = t6[0] / wt;
-    jb.m[1][1] = t6[1] / wt;
-    jb.m[2][2] = t6[2] / wt;
-    jb.m[0][1] = jb.m[1][0] = t6[3] / wt;
-    jb.m[0][2] = jb.m[2][0] = t6[4] / wt;
-    jb.m[1][2] = jb.m[2][1] = t6[5] / wt;
-    const float inert[6] = {(float)jb.m[0][0], (float)jb.m[1][1], (float)jb.m[2][2],
-                            (float)jb.m[0][1], (float)jb.m[1][2], (float)jb.m[2][0]};
+    for (int k = 0; k < 3; k++) jb.eig[k] = t6[k] / wt;
+    jb.m01 = t6[3] / wt;
+    jb.m02 = t6[4] / wt;
+    jb.m12 = t6[5] / wt;
+    const float inert[6] = {(float)jb.eig[0], (float)jb.eig[1], (float)jb.eig[2],
+                            (float)jb.m01,    (float)jb.m12,    (float)jb.m02};
     jb.run();
     const double e0 = jb.eig[0], e1 = jb.eig[1], e2 = jb.eig[2];
     auto E = [&](int q) { return q == 0 ? e0 : (q == 1 ? e1 : e2); };
@@ -832,34 +788,233 @@ __global__ void k_shape_calls(int32_t nh, int32_t it, const int32_t *__restrict_
         b = q;
     }
     const double ea = E(a), eb = E(b), ec = E(c);
-    for (int k = 0; k < 3; k++) {
-        s.eig[k] = jb.eig[k];
-        for (int l = 0; l < 3; l++) s.orth[k][l] = jb.orth[k][l];
-    }
-    if (!(ea != 0.0) || !(eb != 0.0) || !(ec != 0.0)) {
-        s.done = 1;
-        return;
-    }
+    if (!(ea != 0.0) || !(eb != 0.0) || !(ec != 0.0)) return false;
     const float b_to_a = (float)sqrt(eb / ea);
     const float c_to_a = (float)sqrt(ec / ea);
     if ((fabs((double)(b_to_a - s.b_to_a)) < 0.01 * (double)s.b_to_a) &&
-        (fabs((double)(c_to_a - s.c_to_a)) < 0.01 * (double)s.c_to_a)) {
-        s.done = 1;
-        return;
-    }
+        (fabs((double)(c_to_a - s.c_to_a)) < 0.01 * (double)s.c_to_a))
+        return false;
     s.b_to_a = b_to_a > 0 ? b_to_a : 0.0f;
     s.c_to_a = c_to_a > 0 ? c_to_a : 0.0f;
     const double r = sqrt(ea);
-    const double oa[3] = {a == 0 ? jb.orth[0][0] : (a == 1 ? jb.orth[1][0] : jb.orth[2][0]),
-                          a == 0 ? jb.orth[0][1] : (a == 1 ? jb.orth[1][1] : jb.orth[2][1]),
-                          a == 0 ? jb.orth[0][2] : (a == 1 ? jb.orth[1][2] : jb.orth[2][2])};
     const double sc = ((double)(s.r * s.r) * 1e-6) / (r * r);
     for (int k = 0; k < 3; k++) {
-        s.A[k] = (float)(1e3 * r * oa[k]);
-        s.eig[k] = jb.eig[k] * sc;
+        const double oa = a == 0 ? jb.orth[0][k] : (a == 1 ? jb.orth[1][k] : jb.orth[2][k]);
+        out->A[k] = (float)(1e3 * r * oa);
+        eig[k] = jb.eig[k] * sc;
+        for (int l = 0; l < 3; l++) orth[3 * k + l] = jb.orth[k][l];
     }
-    for (int k = 0; k < 6; k++) s.inertia[k] = inert[k];
-    s.assigned = 1;
+    for (int k = 0; k < 6; k++) out->inertia[k] = inert[k];
+    out->b_to_a = s.b_to_a;
+    out->c_to_a = s.c_to_a;
+    out->assigned = 1;
+    return ++s.it < s.limit;
+}
+
+// The windows summed in the reference's order (shape_exact), all iterations
+// in one launch.  A workgroup holds 64 windows at a time of a range of its
+// own; a window that stops makes room for the range's next one, so that the
+// steps stay full though windows take 1 to 10 iterations.  Every iteration
+//   * the windows' records are laid end to end and gone through 256 at a
+//     time, a thread per record: windows hold 25 records on average, and a
+//     wavefront per window left most lanes idle;
+//   * each window's seven sums are added up in record order by four lanes,
+//     from the terms in LDS (0 for a record outside the ellipsoid: the
+//     running sums start at 0, so they never are -0 and keep their bits);
+//   * one lane per window takes the step.
+// What bounds it is the chain through the three, above all the last: some
+// 2,000 dependent double instructions of the Jacobi rotations, on one of the
+// four wavefronts (53% of the cycles hold a vector instruction).  So as many
+// workgroups as fit are kept on a compute unit: what a window carries from
+// step to step is held down to a few registers, and six workgroups with a few
+// registers spilled are 0.68 ms against 0.73 with four.
+constexpr int kShapeWindows = 64;
+constexpr int kShapeThreads = 4 * kShapeWindows;
+constexpr int kShapeResident = 6;                     // workgroups on a compute unit
+constexpr int kComputeUnits = 256;
+constexpr int kShapeGroups = kComputeUnits * kShapeResident;  // all that run at once
+
+// The first kOneTileGroups workgroups take the one-tile windows instead, a
+// wavefront each through all of its iterations: both kinds are chains of
+// dependent double operations and fill each other's waits.
+constexpr int kOneTileGroups = 256;
+
+// ell: 12 doubles in LDS of this wavefront's own; every lane writes and reads
+// the same values
+__device__ void shape_one_tile(const int32_t *__restrict__ list, int32_t n, int32_t first,
+                               int32_t stride, const int64_t *__restrict__ hfirst,
+                               const float4 *__restrict__ cd, ShapeState *__restrict__ st,
+                               double *ell) {
+    for (int32_t i = first; i < n; i += stride) {
+        const int32_t sw = uniform(list[i]);
+        const ShapeState &s = st[sw];
+        ShapeRun run = {s.r, s.b_to_a, s.c_to_a, 0, kShapeIterations};
+        for (int k = 0; k < 9; k++) ell[k] = s.orth[k / 3][k % 3];
+        for (int k = 0; k < 3; k++) ell[9 + k] = s.eig[k];
+        const float4 *rec = cd + hfirst[sw >> 1];
+        const int32_t end = s.n;
+        const double min_r = (double)s.min_r;
+        double sum[7];
+        do shape_sums(ell, ell + 9, min_r, rec, 0, end, sum);
+        while (shape_step(run, sum, st + sw, ell, ell + 9));
+    }
+}
+
+__global__ __launch_bounds__(kShapeThreads, kShapeResident) void k_shape_small(
+    int32_t nh, const int64_t *__restrict__ hfirst, const float4 *__restrict__ cd,
+    const int32_t *__restrict__ one, const int32_t *__restrict__ none,
+    ShapeState *__restrict__ st) {
+    static_assert(kShapeWindows == kWave, "a lane of the leading wavefront per window");
+    __shared__ double s_term[kShapeThreads][7];
+    __shared__ double s_ell[kShapeWindows][13];  // orth, eig, min_r
+    __shared__ double s_sum[kShapeWindows][7];
+    __shared__ int64_t s_first[kShapeWindows];
+    __shared__ int32_t s_n[kShapeWindows];       // records; 0: no window
+    const int32_t tid = threadIdx.x, lane = lane_id();
+    const uint32_t wave0 = (uint32_t)uniform(tid & ~(kWave - 1));
+    constexpr int kWaves = kShapeThreads / kWave;
+    if (blockIdx.x < kOneTileGroups) {
+        shape_one_tile(one, *none, blockIdx.x * kWaves + uniform(tid / kWave),
+                       kOneTileGroups * kWaves, hfirst, cd, st, s_ell[tid / kWave]);
+        return;
+    }
+    const int64_t groups = gridDim.x - kOneTileGroups;
+    const int64_t per = (2 * (int64_t)nh + groups - 1) / groups;
+    int64_t next = (blockIdx.x - kOneTileGroups) * per;  // the range's next window
+    const int64_t last = min(next + per, 2 * (int64_t)nh);
+    const bool leads = tid < kWave;  // the wavefront that takes the steps
+    ShapeRun run = {};    // of the window of this lane of that wavefront
+    int64_t cur = -1;     // that window
+    const int task = tid >> 2, comp = 2 * (tid & 3), comp2 = min(comp + 1, 6);
+    if (leads) s_n[lane] = 0;
+    while (true) {
+        if (leads) {
+            while (next < last) {
+                const bool want = cur < 0;
+                const uint64_t m = ballot(want);
+                if (!m) break;
+                const int64_t i = next + __popcll(m & ((1ull << lane) - 1));
+                next += __popcll(m);
+                if (want && i < last) {
+                    const ShapeState &s = st[i];
+                    // src/properties.c:228-236: none with fewer than 3
+                    if (!s.done && shape_exact(s) && s.nbound >= 3) {
+                        cur = i;
+                        run = ShapeRun{s.r, s.b_to_a, s.c_to_a, 0, min(kShapeIterations, s.nbound)};
+                        s_n[lane] = s.n;
+                        s_first[lane] = hfirst[i >> 1];
+                        for (int k = 0; k < 9; k++) s_ell[lane][k] = s.orth[k / 3][k % 3];
+                        for (int k = 0; k < 3; k++) s_ell[lane][9 + k] = s.eig[k];
+                        s_ell[lane][12] = (double)s.min_r;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        // lane l of every wavefront: the end of window l's records
+        const uint32_t nl = (uint32_t)s_n[lane];
+        const uint32_t ends = (uint32_t)wave_scan_add((int32_t)nl);
+        const uint32_t total = (uint32_t)read_lane((int32_t)ends, kWave - 1);
+        if (total == 0) break;  // the same in every wavefront
+        const uint32_t hi = (uint32_t)__shfl((int32_t)ends, task, 64);
+        const uint32_t lo = hi - (uint32_t)__shfl((int32_t)nl, task, 64);
+        double acc = 0.0, acc2 = 0.0;
+        for (uint32_t base = 0;; base += kShapeThreads) {
+            const uint32_t f0 = base + wave0;  // of this wavefront
+            if (f0 < total) {
+                const uint32_t f = f0 + (uint32_t)lane;
+                // the window of f: those ended by f0, and by each end after it
+                int32_t w = __popcll(ballot(ends <= f0));
+                uint64_t m = ballot(ends > f0 && ends - f0 < (uint32_t)kWave);
+                while (m) {
+                    const int b = __builtin_ctzll(m);
+                    m &= m - 1;
+                    w += f >= (uint32_t)read_lane((int32_t)ends, b) ? 1 : 0;
+                }
+                const uint32_t w_lo = (uint32_t)__shfl((int32_t)(ends - nl), w, 64);
+                if (f < total) {
+                    const float4 q = cd[s_first[w] + (int64_t)(f - w_lo)];
+                    double v[7] = {0, 0, 0, 0, 0, 0, 0};
+                    if (q.w != 0.0f) {
+                        const double *e = s_ell[w];
+                        const double d[3] = {(double)q.x, (double)q.y, (double)q.z};
+                        double r = 0;
+                        for (int k = 0; k < 3; k++) {
+                            double dr = 0;
+                            for (int l = 0; l < 3; l++) dr += e[3 * k + l] * d[l];
+                            r += dr * dr / e[9 + k];
+                        }
+                        if (!shape_terms(r, e[12], d, v))
+                            for (int k = 0; k < 7; k++) v[k] = 0.0;
+                    }
+                    for (int k = 0; k < 7; k++) s_term[tid][k] = v[k];
+                }
+            }
+            __syncthreads();
+            const int32_t a = lo > base ? (int32_t)min(lo - base, (uint32_t)kShapeThreads) : 0;
+            const int32_t b = hi > base ? (int32_t)min(hi - base, (uint32_t)kShapeThreads) : 0;
+            int32_t i = a;
+            for (; i + 8 <= b; i += 8) {
+                double v[8], v2[8];
+                for (int k = 0; k < 8; k++) {
+                    v[k] = s_term[i + k][comp];
+                    v2[k] = s_term[i + k][comp2];
+                }
+                for (int k = 0; k < 8; k++) {
+                    acc += v[k];
+                    acc2 += v2[k];
+                }
+            }
+            for (; i < b; i++) {
+                acc += s_term[i][comp];
+                acc2 += s_term[i][comp2];
+            }
+            __syncthreads();
+            if (total - base <= kShapeThreads) break;
+        }
+        s_sum[task][comp] = acc;
+        if (comp < 6) s_sum[task][comp2] = acc2;
+        __syncthreads();
+        if (cur >= 0) {
+            double sum[7];
+            for (int k = 0; k < 7; k++) sum[k] = s_sum[lane][k];
+            if (!shape_step(run, sum, st + cur, s_ell[lane], s_ell[lane] + 9)) {
+                cur = -1;
+                s_n[lane] = 0;
+            }
+        }
+    }
+}
+
+// The step of the large windows still running, a wavefront each: eight tiles'
+// sums are read at a time (lane 8 i + k: sum k of tile i) and added in tile
+// order, lane k holding sum k.
+__global__ __launch_bounds__(kWave) void k_shape_large(
+    const int32_t *__restrict__ windows, const int32_t *__restrict__ nwindows, int32_t it,
+    const int32_t *__restrict__ call_tile0, const int32_t *__restrict__ call_ntiles,
+    const ShapePart *__restrict__ part, ShapeState *__restrict__ st) {
+    const int lane = lane_id();
+    for (int32_t i = blockIdx.x; i < *nwindows; i += gridDim.x) {
+        const int32_t sw = uniform(windows[i]);
+        if (st[sw].done) continue;
+        const int32_t h = sw >> 1, w = sw & 1;
+        // the tiles that hold records of the window
+        const int32_t t0 = call_tile0[h];
+        const int32_t nt = min(call_ntiles[h], (st[sw].n + kScanTile - 1) / kScanTile);
+        double acc = 0.0;
+        for (int32_t b = 0; b < nt; b += 8) {
+            const int32_t t = b + (lane >> 3);
+            const double v = t < nt ? part[2 * (t0 + t) + w].v[lane & 7] : 0.0;
+            for (int k = 0; k < 8; k++) acc += __shfl(v, 8 * k + (lane & 7), 64);
+        }
+        double sum[7];
+        for (int k = 0; k < 7; k++) sum[k] = __shfl(acc, k, 64);
+        ShapeState &s = st[sw];
+        // at least 64 bound records, so all of the iterations
+        ShapeRun run = {s.r, s.b_to_a, s.c_to_a, it, kShapeIterations};
+        const bool go = shape_step(run, sum, &s, &s.orth[0][0], s.eig);
+        if (lane == 0 && !go) s.done = 1;
+    }
 }
 
 // ------------------------------------------- scale radius, pseudo-evolution

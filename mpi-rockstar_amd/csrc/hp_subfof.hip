@@ -194,8 +194,10 @@ __global__ __launch_bounds__(kWave) void k_sub_centre(const SubGroup *__restrict
 // src/jacobi.c:137-151: sqrt of the smallest eigenvalue, or of the trace
 __device__ double set_eig(const double (&in)[3][3]) {
     Jacobi3 jb;
-    for (int i = 0; i < 3; i++)
-        for (int j = 0; j < 3; j++) jb.m[i][j] = in[i][j];
+    for (int i = 0; i < 3; i++) jb.eig[i] = in[i][i];
+    jb.m01 = in[0][1];
+    jb.m02 = in[0][2];
+    jb.m12 = in[1][2];
     jb.run();
     double r = jb.eig[0];
     if (jb.eig[1] < r) r = jb.eig[1];

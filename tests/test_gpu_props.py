@@ -134,6 +134,43 @@ def test_props_other_epoch_and_definitions(restatement):
     check(restatement, cat, defs=("m200c", "vir", "178b", "1000c", "200b"))
 
 
+@pytest.mark.parametrize("n_halos,lo,hi", [
+    (1, 257, 257),       # one window of each kind
+    (33, 60, 70),        # around 64 bound records
+    (65, 250, 300),      # around 256 records: windows end inside a group of 256
+    (130, 2, 5),         # fewer than 3 records or bound ones
+    (12, 2040, 2200),    # around the 2,048 records of a tile
+    (3, 17_000, 20_000),  # more than eight tiles: two reads of the tiles' sums
+])
+def test_props_window_edges(restatement, n_halos, lo, hi):
+    check(restatement, catalog.small_batch(seed=75, n_halos=n_halos, lo=lo, hi=hi))
+
+
+def test_props_more_windows_than_are_held_at_once(restatement):
+    """206 calls, their bound-pass results repeated to 51,500 calls (103,000
+    windows): every copy has the properties of the first, bit for bit."""
+    cat = catalog.small_batch(seed=76, n_halos=206, lo=2, hi=400)
+    po, halos, want, _ = run_props(cat)
+    k = 250
+    many = np.tile(halos, k)
+    many["first"] += np.repeat(np.arange(k), halos.size).astype(many["first"].dtype) * po.size
+    plan = halopot.Plan(np.ascontiguousarray(many))
+    d_po = DeviceArray.from_numpy(np.ascontiguousarray(np.tile(po, k)))
+    d_h = DeviceArray.from_numpy(np.ascontiguousarray(many))
+    d_p = DeviceArray.zeros(many.size * catalog.PROPS_DTYPE.itemsize)
+    try:
+        plan.props(d_po.address, d_h.address, d_p.address, halopot.mass_definitions(None))
+        synchronize()
+        got = d_p.download(np.empty(many.size, catalog.PROPS_DTYPE))
+    finally:
+        plan.close()
+        for d in (d_po, d_h, d_p):
+            d.free()
+    for f in catalog.PROPS_DTYPE.names:
+        a = got[f].reshape(k, halos.size, -1)
+        np.testing.assert_array_equal(a, np.broadcast_to(want[f].reshape(1, halos.size, -1), a.shape), err_msg=f)
+
+
 def test_props_per_call_plan(restatement):
     cat = catalog.small_batch(seed=73, n_halos=20, lo=5, hi=2000)
     check(restatement, cat, opts=halopot.options(per_call=1))
