@@ -1437,7 +1437,7 @@ struct Engine {
                                                scale_calls.as<ScaleCall>());
             HP_LAUNCHED();
         }
-        k_scale_fit<<<blocks(H, 64), 64, 0, s>>>(fit_list.as<int32_t>(), fit_n.as<int32_t>(),
+        k_scale_fit<<<std::min(blocks(H, kWave / kBinLanes), 4096), kWave, 0, s>>>(fit_list.as<int32_t>(), fit_n.as<int32_t>(),
                                                  pcall.as<PropCall>(), d_props, pa,
                                                  scale_calls.as<ScaleCall>());
         HP_LAUNCHED();
