@@ -387,7 +387,8 @@ struct Engine {
     DevBuf seg_wave_l, seg_block_l, seg_tiles_l, seg_hist, seg_hsum, srt_rv;
     // halo properties
     DevBuf pcnt, pscan, pcall, psums, shape_st, shape_part, shape_cd, scale_calls, r_pe, pe_cnt,
-        fit_list, fit_n, shape_one, shape_pairs, shape_windows;
+        fit_list, fit_n, shape_one, shape_pairs, shape_windows, prop_r2,
+        prop_bound;
     // record assembly
     DevBuf gsegs, gtiles, gcen;
     SubBufs sub;
@@ -487,7 +488,7 @@ struct Engine {
         DevBuf *all[] = {&hfirst, &hcount, &root_tiles, &groups, &direct_blocks,
                          &scan_tiles, &call_tile0, &call_ntiles, &box, &bad, &pot, &rkey, &badlist, &A, &B, &F,
                          &leaf_of, &sides, &nodes, &parent, &fat, &small0, &group0, &groupc, &wave_off, &wave_hsum, &big, &tiles,
-                         &parts, &splitres, &dparts, &counters, &work, &depth_buf, &pcnt, &pscan, &pcall, &psums, &shape_st, &shape_part, &shape_cd, &scale_calls, &r_pe, &pe_cnt, &fit_list, &fit_n, &shape_one, &shape_pairs, &shape_windows, &gsegs, &gtiles, &gcen, &keys0, &keys1, &vals0,
+                         &parts, &splitres, &dparts, &counters, &work, &depth_buf, &pcnt, &pscan, &pcall, &psums, &shape_st, &shape_part, &shape_cd, &scale_calls, &r_pe, &pe_cnt, &fit_list, &fit_n, &shape_one, &shape_pairs, &shape_windows, &prop_r2, &prop_bound, &gsegs, &gtiles, &gcen, &keys0, &keys1, &vals0,
                          &vals1, &hist, &hsum, &srt, &callinfo, &tsum, &tcand, &tile_i32, &rec_call, &strip_cnt, &stage,
                          &seg_wave_l, &seg_block_l, &seg_tiles_l, &seg_hist, &seg_hsum, &srt_rv};
         for (DevBuf *b : all) f(*b);
@@ -1342,6 +1343,8 @@ struct Engine {
         HP_ENSURE(shape_st, sizeof(ShapeState) * 2 * (H + 1));
         HP_ENSURE(shape_part, sizeof(ShapePart) * 2 * (nst + 1));
         HP_ENSURE(shape_cd, sizeof(float4) * (T.nrec + 1));
+        HP_ENSURE(prop_r2, sizeof(float) * (T.nrec + 1));
+        HP_ENSURE(prop_bound, sizeof(uint64_t) * kTileWords * (nst + 1));
         HP_ENSURE(scale_calls, sizeof(ScaleCall) * (H + 1));
         HP_ENSURE(r_pe, sizeof(double) * (H + 1));
         HP_ENSURE(pe_cnt, sizeof(int32_t) * (nst + 1));
@@ -1366,45 +1369,39 @@ struct Engine {
         const ScanTile *tl = scan_tiles.as<ScanTile>();
         const int32_t *t0 = call_tile0.as<int32_t>(), *tn = call_ntiles.as<int32_t>();
         const int64_t *hf = hfirst.as<int64_t>(), *hc = hcount.as<int64_t>();
+        const PropReads pr = {prop_r2.as<float>(), prop_bound.as<uint64_t>(),
+                              shape_cd.as<float4>()};
+        int32_t *cnts = fit_n.as<int32_t>();
+        k_fill_i32<<<1, 64, 0, s>>>(cnts, 0, 1 + kShapeLists);
+        HP_LAUNCHED();
         if (nst > 0) {
             k_props_counts<<<nst, kWave, 0, s>>>(d_po, tl, nst, d_halos, hf, hc,
-                                                 pcnt.as<PropCount>());
+                                                 pcnt.as<PropCount>(), pr);
             HP_LAUNCHED();
         }
         k_props_prefix<<<blocks(H, 256), 256, 0, s>>>(t0, tn, H, pcnt.as<PropCount>());
         HP_LAUNCHED();
         if (nst > 0) {
-            k_props_scan<<<nst, kWave, 0, s>>>(d_po, tl, nst, d_halos, hf, hc,
+            k_props_scan<<<nst, kWave, 0, s>>>(pr, tl, nst, d_halos, hf, hc,
                                                pcnt.as<PropCount>(), pa, pscan.as<PropScan>());
             HP_LAUNCHED();
         }
-        k_props_calls<<<blocks(H, 256), 256, 0, s>>>(t0, tn, H, d_halos, hc,
-                                                     pscan.as<PropScan>(), pcall.as<PropCall>());
+        k_props_calls<<<blocks(H, 64), 64, 0, s>>>(t0, tn, H, d_halos, hc, pscan.as<PropScan>(),
+                                                   pcall.as<PropCall>());
         HP_LAUNCHED();
         if (nst > 0) {
             k_props_sums<<<nst, kWave, 0, s>>>(d_po, tl, nst, d_halos, hf, pcnt.as<PropCount>(),
                                                pcall.as<PropCall>(), pa, psums.as<PropSums>());
             HP_LAUNCHED();
         }
-        k_props_final<<<blocks(H, 256), 256, 0, s>>>(d_po, t0, tn, H, d_halos, hf,
-                                                     pcall.as<PropCall>(), psums.as<PropSums>(),
-                                                     pa, d_props);
-        HP_LAUNCHED();
-        // calc_shape in both windows, SHAPE_ITERATIONS rounds
         ShapeState *ss = shape_st.as<ShapeState>();
-        k_shape_init<<<blocks(H, 256), 256, 0, s>>>(H, d_halos, hc, pcall.as<PropCall>(), d_props,
-                                                    pa, ss);
+        k_props_final<<<blocks(H, 64), 64, 0, s>>>(
+            pr, pcnt.as<PropCount>(), t0, tn, H, d_halos, hf, pcall.as<PropCall>(),
+            psums.as<PropSums>(), pa, d_props, ss, scale_calls.as<ScaleCall>(),
+            fit_list.as<int32_t>(), fit_n.as<int32_t>());
         HP_LAUNCHED();
-        if (nst > 0) {
-            k_shape_prep<<<nst, kWave, 0, s>>>(d_po, tl, nst, d_halos, hf, ss,
-                                               shape_cd.as<float4>());
-            HP_LAUNCHED();
-        }
-        // the windows of few records in one launch, the large ones an
-        // iteration at a time
-        int32_t *cnts = fit_n.as<int32_t>();
-        k_fill_i32<<<1, 64, 0, s>>>(cnts, 0, 1 + kShapeLists);
-        HP_LAUNCHED();
+        // calc_shape in both windows, SHAPE_ITERATIONS rounds: the small windows
+        // in one launch, the large ones an iteration at a time
         if (nst > 0) {
             const ShapeLists sl = {shape_one.as<int32_t>(), shape_pairs.as<int32_t>(),
                                    shape_windows.as<int32_t>(), cnts + 1};
@@ -1427,13 +1424,8 @@ struct Engine {
             }
         }
         // calc_scale_radius and the pseudo-evolution masses
-        k_scale_init<<<blocks(H, 256), 256, 0, s>>>(H, d_po, hf, t0, tn, pcall.as<PropCall>(),
-                                                    psums.as<PropSums>(),
-                                                    scale_calls.as<ScaleCall>(),
-                                                    fit_list.as<int32_t>(), fit_n.as<int32_t>());
-        HP_LAUNCHED();
         if (nst > 0) {
-            k_scale_bins<<<nst, kWave, 0, s>>>(d_po, tl, nst, hf, pcnt.as<PropCount>(),
+            k_scale_bins<<<nst, kWave, 0, s>>>(pr, tl, nst, hf, pcnt.as<PropCount>(),
                                                scale_calls.as<ScaleCall>());
             HP_LAUNCHED();
         }
@@ -1446,7 +1438,7 @@ struct Engine {
                                                   r_pe.as<double>(), d_props);
         HP_LAUNCHED();
         if (nst > 0) {
-            k_pe_tiles<<<nst, kWave, 0, s>>>(d_po, tl, nst, d_halos, hf, hc, r_pe.as<double>(),
+            k_pe_tiles<<<nst, kWave, 0, s>>>(pr, tl, nst, d_halos, hf, hc, r_pe.as<double>(),
                                              pe_cnt.as<int32_t>());
             HP_LAUNCHED();
         }

@@ -129,28 +129,59 @@ __device__ __forceinline__ void wave_arg_better(double &v, int32_t &j) {
     }
 }
 
+// words of bound flags per tile, a word per 64 records
+constexpr int kTileWords = kScanTile / kWave;
+
+// What the passes over all records read, taken from the records once: r2 (4
+// bytes), the bound flags (a bit, 1: !(pe < ke)) and the float offsets from
+// the centre with the flag (16 bytes, the shapes).  The passes went through
+// the records' 48 bytes each for themselves, six times.
+struct PropReads {
+    float *r2;
+    uint64_t *bound;  // kTileWords per tile
+    float4 *cd;
+};
+
 __global__ __launch_bounds__(kWave) void k_props_counts(const struct potential *__restrict__ srt,
                                                         const ScanTile *__restrict__ tiles,
                                                         int32_t ntiles,
                                                         const hp_halo *__restrict__ halos,
                                                         const int64_t *__restrict__ hfirst,
                                                         const int64_t *__restrict__ hcount,
-                                                        PropCount *__restrict__ cnt) {
+                                                        PropCount *__restrict__ cnt,
+                                                        PropReads out) {
     const int32_t t = blockIdx.x;
     if (t >= ntiles) return;
     const ScanTile st = tiles[t];
     const int64_t first = hfirst[st.call];
     const int32_t end = min(st.off + kScanTile, call_kept(halos, hcount, st.call));
+    const float c0 = halos[st.call].pos[0], c1 = halos[st.call].pos[1], c2 = halos[st.call].pos[2];
     int32_t nb = 0, ns = 0;
-    for (int32_t j = st.off + lane_id(); j < end; j += kWave) {
-        const double pe = srt[first + j].pe;
-        const float ke = srt[first + j].ke;
-        nb += !(pe < (double)ke) ? 1 : 0;
-        ns += pe > (double)ke ? 1 : 0;
+    uint64_t *word = out.bound + (int64_t)kTileWords * t;
+    for (int32_t base = st.off; base < end; base += kWave, word++) {
+        const int32_t j = base + lane_id();
+        bool b = false, sb = false;
+        if (j < end) {
+            const struct potential &r = srt[first + j];
+            b = !(r.pe < (double)r.ke);
+            sb = r.pe > (double)r.ke;
+            out.r2[first + j] = r.r2;
+            out.cd[first + j] =
+                make_float4(r.pos[0] - c0, r.pos[1] - c1, r.pos[2] - c2, b ? 1.0f : 0.0f);
+        }
+        const uint64_t m = ballot(b);
+        if (lane_id() == 0) *word = m;
+        nb += __popcll(m);
+        ns += __popcll(ballot(sb));
     }
-    nb = wave_sum(nb);
-    ns = wave_sum(ns);
     if (lane_id() == 0) cnt[t] = PropCount{nb, ns};
+}
+
+// set bits of m up to this lane's
+__device__ __forceinline__ int32_t count_to_lane(uint64_t m) {
+    return (int32_t)__builtin_amdgcn_mbcnt_hi(
+               (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0)) +
+           (int32_t)((m >> lane_id()) & 1);
 }
 
 // per call: exclusive prefix of the tile counts, in tile order
@@ -158,18 +189,46 @@ __global__ void k_props_prefix(const int32_t *__restrict__ call_tile0,
                                const int32_t *__restrict__ call_ntiles, int32_t nh,
                                PropCount *__restrict__ cnt) {
     const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    int32_t nb = 0, ns = 0;
-    for (int32_t t = call_tile0[h]; t < call_tile0[h] + call_ntiles[h]; t++) {
-        const PropCount c = cnt[t];
-        cnt[t] = PropCount{nb, ns};
-        nb += c.nb;
-        ns += c.ns;
+    const int32_t t0 = h < nh ? call_tile0[h] : 0, nt = h < nh ? call_ntiles[h] : 0;
+    if (nt <= kFewTiles) {
+        int32_t nb = 0, ns = 0;
+        for (int32_t t = t0; t < t0 + nt; t++) {
+            const PropCount c = cnt[t];
+            cnt[t] = PropCount{nb, ns};
+            nb += c.nb;
+            ns += c.ns;
+        }
     }
+    for_large_calls(t0, nt, [&](int32_t first, int32_t n, bool) {
+        int32_t nb = 0, ns = 0;
+        for (int32_t base = 0; base < n; base += kWave) {
+            const bool in = base + lane_id() < n;
+            PropCount c = {0, 0};
+            if (in) c = cnt[first + base + lane_id()];
+            const int32_t b = wave_scan_add(c.nb), e = wave_scan_add(c.ns);
+            if (in) cnt[first + base + lane_id()] = PropCount{nb + b - c.nb, ns + e - c.ns};
+            nb += read_lane(b, kWave - 1);
+            ns += read_lane(e, kWave - 1);
+        }
+    });
+}
+
+// bound records among a call's first n, from the tile counts before each tile
+// and the flags
+__device__ __forceinline__ int32_t bound_before(int32_t n, int32_t tile0,
+                                                const PropCount *__restrict__ pre,
+                                                const uint64_t *__restrict__ bound) {
+    if (n <= 0) return 0;
+    const int32_t t = tile0 + (n - 1) / kScanTile, k = (n - 1) % kScanTile + 1;
+    const uint64_t *w = bound + (int64_t)kTileWords * t;
+    int32_t c = pre[t].nb;
+    for (int32_t i = 0; i < k / kWave; i++) c += __popcll(w[i]);
+    if (k % kWave) c += __popcll(w[k / kWave] & ((1ull << (k % kWave)) - 1));
+    return c;
 }
 
 // walk 1 (src/properties.c:402-431), one wavefront per tile
-__global__ __launch_bounds__(kWave) void k_props_scan(const struct potential *__restrict__ srt,
+__global__ __launch_bounds__(kWave) void k_props_scan(const PropReads in,
                                                       const ScanTile *__restrict__ tiles,
                                                       int32_t ntiles,
                                                       const hp_halo *__restrict__ halos,
@@ -198,16 +257,12 @@ __global__ __launch_bounds__(kWave) void k_props_scan(const struct potential *__
     for (int32_t base = st.off; base < end; base += kWave) {
         const int32_t j = base + lane;
         const bool v = j < end;
-        float r2 = 0.0f, ke = 0.0f;
-        double pe = 0.0;
-        if (v) {
-            r2 = srt[first + j].r2;
-            pe = srt[first + j].pe;
-            ke = srt[first + j].ke;
-        }
-        const bool b = v && !(pe < (double)ke);
-        const int32_t n = wave_scan_add(b ? 1 : 0) + carry;
-        carry = read_lane(n, kWave - 1);
+        float r2 = 0.0f;
+        if (v) r2 = in.r2[first + j];
+        const uint64_t mb = in.bound[(int64_t)kTileWords * t + (base - st.off) / kWave];
+        const bool b = (mb >> lane) & 1;
+        const int32_t n = count_to_lane(mb) + carry;
+        carry += __popcll(mb);
         const double r = prop_radius(r2, pa.force_res);
         const double r3 = r * r * r;
         if (v && (double)(j + 1) / r3 > pa.dens_thresh) s.last_all = j;
@@ -256,35 +311,74 @@ __global__ void k_props_calls(const int32_t *__restrict__ call_tile0,
                               const int64_t *__restrict__ hcount,
                               const PropScan *__restrict__ ts, PropCall *__restrict__ pc) {
     const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    const int32_t t0 = call_tile0[h], t1 = t0 + call_ntiles[h];
+    const bool v = h < nh;
+    const int32_t t0 = v ? call_tile0[h] : 0, nt = v ? call_ntiles[h] : 0;
     PropCall c;
-    c.kept = call_kept(halos, hcount, h);
-    int32_t last_all = -1, last0 = -1, n0 = 0, tfirst = -1;
-    double pe_b = 0.0;
+    int32_t last_all = -1, last0 = -1, n0 = 0;
     for (int k = 0; k < 4; k++) c.alt[k] = 0;
     c.vir = 0;
-    for (int32_t t = t0; t < t1; t++) {
-        const PropScan &s = ts[t];
-        last_all = max(last_all, s.last_all);
-        if (s.last0 >= 0) {
-            if (tfirst < 0) tfirst = t;
-            last0 = s.last0;
-            n0 = s.n0;
-        }
-        for (int k = 0; k < 4; k++) c.alt[k] = max(c.alt[k], ts[t].alt[k]);
-        c.vir = max(c.vir, s.vir);
-        pe_b = s.pe_b > pe_b ? s.pe_b : pe_b;
-    }
-    c.pe_b = pe_b;
-    // vmax counts from the first index above dens_thresh on: the part of
-    // that tile after it, then whole tiles
+    c.pe_b = 0.0;
     double vm = -1.0;
     int32_t jm = INT32_MAX;
-    if (tfirst >= 0) {
-        arg_better(vm, jm, ts[tfirst].v_after, ts[tfirst].j_after);
-        for (int32_t t = tfirst + 1; t < t1; t++) arg_better(vm, jm, ts[t].v_all, ts[t].j_all);
+    // vmax counts from the first index above dens_thresh on: the part of
+    // that tile after it, then whole tiles
+    if (nt <= kFewTiles) {
+        for (int32_t t = t0; t < t0 + nt; t++) {
+            const PropScan &s = ts[t];
+            last_all = max(last_all, s.last_all);
+            if (last0 >= 0) arg_better(vm, jm, s.v_all, s.j_all);
+            else if (s.last0 >= 0) arg_better(vm, jm, s.v_after, s.j_after);
+            if (s.last0 >= 0) {
+                last0 = s.last0;
+                n0 = s.n0;
+            }
+            for (int k = 0; k < 4; k++) c.alt[k] = max(c.alt[k], s.alt[k]);
+            c.vir = max(c.vir, s.vir);
+            c.pe_b = s.pe_b > c.pe_b ? s.pe_b : c.pe_b;
+        }
     }
+    // every field of a tile is monotone over the tiles: maxima over the lanes
+    for_large_calls(t0, nt, [&](int32_t a, int32_t n, bool mine) {
+        int32_t all = -1, l0 = -1, n_0 = 0, vir = 0, alt[4] = {0, 0, 0, 0}, j = INT32_MAX;
+        double best = -1.0, pe_b = 0.0;
+        bool seen = false;
+        for (int32_t base = 0; base < n; base += kWave) {
+            const bool in = base + lane_id() < n;
+            const PropScan &s = ts[a + base + (in ? lane_id() : 0)];
+            const uint64_t above = ballot(in && s.last0 >= 0);
+            if (in) {
+                all = max(all, s.last_all);
+                l0 = max(l0, s.last0);
+                n_0 = max(n_0, s.n0);
+                for (int k = 0; k < 4; k++) alt[k] = max(alt[k], s.alt[k]);
+                vir = max(vir, s.vir);
+                pe_b = s.pe_b > pe_b ? s.pe_b : pe_b;
+                const uint64_t before = above & ((1ull << lane_id()) - 1);
+                if (seen || before) arg_better(best, j, s.v_all, s.j_all);
+                else if (s.last0 >= 0) arg_better(best, j, s.v_after, s.j_after);
+            }
+            seen = seen || above != 0;
+        }
+        all = wave_max(all);
+        l0 = wave_max(l0);
+        n_0 = wave_max(n_0);
+        for (int k = 0; k < 4; k++) alt[k] = wave_max(alt[k]);
+        vir = wave_max(vir);
+        pe_b = wave_max(pe_b);
+        wave_arg_better(best, j);
+        if (mine) {
+            last_all = all;
+            last0 = l0;
+            n0 = n_0;
+            for (int k = 0; k < 4; k++) c.alt[k] = alt[k];
+            c.vir = vir;
+            c.pe_b = pe_b;
+            vm = best;
+            jm = j;
+        }
+    });
+    if (!v) return;
+    c.kept = call_kept(halos, hcount, h);
     c.n_all = last_all + 1;
     c.n0 = n0;
     c.dens_tot = last0 >= 0 ? last0 : 0;
@@ -322,10 +416,12 @@ __global__ __launch_bounds__(kWave) void k_props_sums(const struct potential *__
         if (v) rec = srt[first + j];
         const bool b = v && !(rec.pe < (double)rec.ke);
         const bool sb = v && rec.pe > (double)rec.ke;
-        const int32_t n = wave_scan_add(b ? 1 : 0) + carry_b;
-        const int32_t ns = wave_scan_add(sb ? 1 : 0) + carry_s;  // inclusive
-        carry_b = read_lane(n, kWave - 1);
-        carry_s = read_lane(ns, kWave - 1);
+        const uint64_t mb = ballot(b), ms = ballot(sb);
+        const int32_t n = count_to_lane(mb) + carry_b;
+        const int32_t ns = count_to_lane(ms) + carry_s;  // inclusive
+        carry_b += __popcll(mb);
+        carry_s += __popcll(ms);
+        nb_tile += __popcll(mb);
         if (b) {
             const float *x = rec.pos;
             // src/properties.c:127-137: float differences and products
@@ -342,7 +438,6 @@ __global__ __launch_bounds__(kWave) void k_props_sums(const struct potential *__
                 acc[6 + k] += dv;
                 acc[9 + k] += dv * dv;
             }
-            nb_tile++;
             if (j >= 1 && 2 * (int64_t)n >= (int64_t)c.n0) half = min(half, j);
         }
         if (sb) {
@@ -362,94 +457,9 @@ __global__ __launch_bounds__(kWave) void k_props_sums(const struct potential *__
     s.ke = wave_sum(acc[12]);
     s.phi_i = wave_sum(acc[13]);
     s.phi_c = wave_sum(acc[14]);
-    s.n = wave_sum(nb_tile);
+    s.n = nb_tile;
     s.half = wave_min(half);
     if (lane == 0) out[t] = s;
-}
-
-__global__ void k_props_final(const struct potential *__restrict__ srt,
-                              const int32_t *__restrict__ call_tile0,
-                              const int32_t *__restrict__ call_ntiles, int32_t nh,
-                              const hp_halo *__restrict__ halos,
-                              const int64_t *__restrict__ hfirst,
-                              const PropCall *__restrict__ pc, const PropSums *__restrict__ ts,
-                              PropArgs pa, hp_halo_props *__restrict__ props) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    const hp_halo &hh = halos[h];
-    const int64_t first = hfirst[h];
-    const PropCall c = pc[h];
-    const double PM = pa.particle_mass;
-    const float scale_now = pa.scale_now;
-    double L[3] = {0, 0, 0}, sx[3] = {0, 0, 0}, sv[3] = {0, 0, 0}, sv2[3] = {0, 0, 0};
-    double ke = 0, phi = 0;
-    int64_t n = 0;
-    int32_t half = INT32_MAX;
-    for (int32_t t = call_tile0[h]; t < call_tile0[h] + call_ntiles[h]; t++) {
-        const PropSums &s = ts[t];
-        for (int k = 0; k < 3; k++) {
-            L[k] += s.L[k];
-            sx[k] += s.sx[k];
-            sv[k] += s.sv[k];
-            sv2[k] += s.sv2[k];
-        }
-        ke += s.ke;
-        phi += s.phi_i + s.phi_c;
-        n += s.n;
-        half = min(half, s.half);
-    }
-    hp_halo_props o;
-    const double m = (double)c.n0 * PM;
-    o.m = (float)((double)c.n_all * PM);
-    o.mgrav = (float)m;
-    // src/properties.c:460-475: float fields accumulated from double terms
-    float xoff = 0.0f, voff = 0.0f;
-    double vr = 0.0;
-    for (int k = 0; k < 3; k++) {
-        // the reference's running means start at 0 and stay there with no
-        // record averaged
-        const double dsx = n > 0 ? sx[k] / (double)n : -(double)hh.pos[k];
-        const double dsv = n > 0 ? sv[k] / (double)n : -(double)hh.pos[k + 3];
-        xoff = (float)((double)xoff + dsx * dsx);
-        voff = (float)((double)voff + dsv * dsv);
-        vr += n > 0 ? (sv2[k] - sv[k] * sv[k] / (double)n) / (double)n : 0.0;
-    }
-    for (int k = 0; k < 4; k++) o.alt_m[k] = (float)((double)c.alt[k] * PM);
-    o.Xoff = (float)(sqrt((double)xoff) * 1e3);
-    o.Voff = (float)sqrt((double)voff);
-    o.vrms = (float)sqrt(vr);
-    o.vmax = (float)(kVmaxConst * sqrt(c.vmax * (PM / (double)scale_now)));
-    o.rvmax = c.j_vmax >= 0
-                  ? (float)(prop_radius(srt[first + c.j_vmax].r2, pa.force_res) * 1e3)
-                  : 0.0f;
-    const int32_t ih = half == INT32_MAX ? 0 : half;
-    o.halfmass_radius = c.kept > 0 ? (float)(sqrt((double)srt[first + ih].r2) * 1e3) : 0.0f;
-    o.r = (float)(cbrt((3.0 / (4.0 * M_PI)) * (double)c.n0 / pa.thresh0) * 1e3);
-    const double rvir = cbrt((3.0 / (4.0 * M_PI)) * (double)c.vir / pa.rvir_dens) * 1e3;
-    const double mvir = (double)c.vir * PM;
-    o.rvir = (float)rvir;
-    for (int k = 0; k < 3; k++) o.J[k] = (float)(PM * (double)scale_now * L[k]);
-    // src/properties.c:328-349
-    const double total_phi = phi / 2.0;
-    o.kin_to_pot = total_phi != 0.0 ? (float)(ke / total_phi) : 0.0f;
-    o.energy = (float)((ke - total_phi) * PM * kGc / (double)scale_now);
-    const double Jh = PM * (double)scale_now * sqrt(L[0] * L[0] + L[1] * L[1] + L[2] * L[2]);
-    o.spin = (float)(m > 0 ? Jh * sqrt(fabs((double)o.energy)) / (kGc * pow(m, 2.5))
-                           : 0.0);
-    o.bullock_spin = (float)(m > 0 ? Jh / (mvir * sqrt(2.0 * kGc * mvir * rvir *
-                                                        (double)scale_now / 1e3))
-                                   : 0.0);
-    // filled by the shape, scale-radius and pseudo-evolution kernels
-    o.rs = o.klypin_rs = o.chi2 = 0.0f;
-    o.b_to_a = o.c_to_a = o.b_to_a2 = o.c_to_a2 = 0.0f;
-    for (int k = 0; k < 3; k++) o.A[k] = o.A2[k] = 0.0f;
-    for (int k = 0; k < 6; k++) o.inertia_tensor[k] = o.inertia_tensor2[k] = 0.0f;
-    o.m_pe_b = o.m_pe_d = 0.0f;
-    o.n_mdelta = c.n0;
-    o.dens_tot = c.dens_tot;
-    o.n_vir = c.vir;
-    o.n_half = ih;
-    props[h] = o;
 }
 
 // ------------------------------------------------------------- shapes
@@ -486,64 +496,30 @@ struct ShapePart {
     double v[8];       // weight, xx, yy, zz, yx, zx, zy, unused
 };
 
-__global__ void k_shape_init(int32_t nh, const hp_halo *__restrict__ halos,
-                             const int64_t *__restrict__ hcount, const PropCall *__restrict__ pc,
-                             const hp_halo_props *__restrict__ props, PropArgs pa,
-                             ShapeState *__restrict__ st) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    const PropCall c = pc[h];
+// the windows' first ellipsoids (spheres) and their bound records
+__device__ __forceinline__ void shape_init(const PropCall &c, int32_t tile0, float r,
+                                           const PropCount *__restrict__ pre,
+                                           const uint64_t *__restrict__ bound,
+                                           const PropArgs &pa, ShapeState *__restrict__ st) {
     for (int w = 0; w < 2; w++) {
-        ShapeState s;
-        s.r = w == 0 ? (float)(cbrt((3.0 / (4.0 * M_PI)) * (double)c.alt[2] / pa.thresh3) * 1e3)
-                     : props[h].r;
+        ShapeState &s = st[w];
+        const float wr =
+            w == 0 ? (float)(cbrt((3.0 / (4.0 * M_PI)) * (double)c.alt[2] / pa.thresh3) * 1e3) : r;
+        s.r = wr;
         s.n = min(w == 0 ? c.alt[2] : c.dens_tot, c.kept);
         float min_r = (float)(pa.force_res * pa.force_res);
-        min_r *= 1e6 / (s.r * s.r);
+        min_r *= 1e6 / (wr * wr);
         s.min_r = min_r;
         s.b_to_a = s.c_to_a = 0.0f;
         for (int k = 0; k < 3; k++) s.A[k] = 0.0f;
         for (int k = 0; k < 6; k++) s.inertia[k] = 0.0f;
         for (int k = 0; k < 3; k++) {
             for (int l = 0; l < 3; l++) s.orth[k][l] = k == l ? 1.0 : 0.0;
-            s.eig[k] = (double)(s.r * s.r) * 1e-6;
+            s.eig[k] = (double)(wr * wr) * 1e-6;
         }
-        s.done = !(s.r > 0) || s.n <= 0;
+        s.done = !(wr > 0) || s.n <= 0;
         s.assigned = 0;
-        s.nbound = 0;
-        st[2 * h + w] = s;
-    }
-}
-
-// x, y, z offsets from the centre and the bound flag of the records the
-// windows cover; each window's bound records are counted
-__global__ __launch_bounds__(kWave) void k_shape_prep(const struct potential *__restrict__ srt,
-                                                      const ScanTile *__restrict__ tiles,
-                                                      int32_t ntiles,
-                                                      const hp_halo *__restrict__ halos,
-                                                      const int64_t *__restrict__ hfirst,
-                                                      ShapeState *__restrict__ st,
-                                                      float4 *__restrict__ cd) {
-    const int32_t t = blockIdx.x;
-    if (t >= ntiles) return;
-    const ScanTile tl = tiles[t];
-    const int32_t n0 = st[2 * tl.call].n, n1 = st[2 * tl.call + 1].n;
-    const int32_t n = max(n0, n1);
-    const int64_t first = hfirst[tl.call];
-    const float c0 = halos[tl.call].pos[0], c1 = halos[tl.call].pos[1], c2 = halos[tl.call].pos[2];
-    int32_t b0 = 0, b1 = 0;
-    for (int32_t j = tl.off + lane_id(); j < min(tl.off + kScanTile, n); j += kWave) {
-        const struct potential &r = srt[first + j];
-        const bool b = !(r.pe < (double)r.ke);
-        cd[first + j] = make_float4(r.pos[0] - c0, r.pos[1] - c1, r.pos[2] - c2, b ? 1.0f : 0.0f);
-        b0 += (b && j < n0) ? 1 : 0;
-        b1 += (b && j < n1) ? 1 : 0;
-    }
-    b0 = wave_sum(b0);
-    b1 = wave_sum(b1);
-    if (lane_id() == 0) {
-        if (b0) atomicAdd(&st[2 * tl.call].nbound, b0);
-        if (b1) atomicAdd(&st[2 * tl.call + 1].nbound, b1);
+        s.nbound = bound_before(s.n, tile0, pre, bound);
     }
 }
 
@@ -1034,44 +1010,160 @@ struct ScaleCall {
     float klypin, rs, chi2;  // results for the fitted calls
 };
 
-// src/nfw.c:134-152: the bound records of [0, dens_tot - 1) and the bin size
-__global__ void k_scale_init(int32_t nh, const struct potential *__restrict__ srt,
-                             const int64_t *__restrict__ hfirst,
-                             const int32_t *__restrict__ call_tile0,
-                             const int32_t *__restrict__ call_ntiles,
-                             const PropCall *__restrict__ pc, const PropSums *__restrict__ ts,
-                             ScaleCall *__restrict__ sc, int32_t *__restrict__ fit_list,
-                             int32_t *__restrict__ fit_n) {
+// per call: the halo fields, and where its shape windows and its fit start
+__global__ void k_props_final(const PropReads in, const PropCount *__restrict__ pre,
+                              const int32_t *__restrict__ call_tile0,
+                              const int32_t *__restrict__ call_ntiles, int32_t nh,
+                              const hp_halo *__restrict__ halos,
+                              const int64_t *__restrict__ hfirst,
+                              const PropCall *__restrict__ pc, const PropSums *__restrict__ ts,
+                              PropArgs pa, hp_halo_props *__restrict__ props,
+                              ShapeState *__restrict__ shapes, ScaleCall *__restrict__ scales,
+                              int32_t *__restrict__ fit_list, int32_t *__restrict__ fit_n) {
     const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    const PropCall c = pc[h];
-    int64_t nb = 0;  // bound records in [0, dens_tot)
-    for (int32_t t = call_tile0[h]; t < call_tile0[h] + call_ntiles[h]; t++) nb += ts[t].n;
-    const int32_t end = c.dens_tot - 1;
-    if (end >= 0) {
-        const struct potential &r = srt[hfirst[h] + end];
-        if (!(r.pe < (double)r.ke)) nb--;
+    const bool v = h < nh;
+    const int32_t t0 = v ? call_tile0[h] : 0, nt = v ? call_ntiles[h] : 0;
+    double L[3] = {0, 0, 0}, sx[3] = {0, 0, 0}, sv[3] = {0, 0, 0}, sv2[3] = {0, 0, 0};
+    double ke = 0, phi = 0;
+    int32_t n = 0, half = INT32_MAX;
+    auto add = [&](const PropSums &s) {
+        for (int k = 0; k < 3; k++) {
+            L[k] += s.L[k];
+            sx[k] += s.sx[k];
+            sv[k] += s.sv[k];
+            sv2[k] += s.sv2[k];
+        }
+        ke += s.ke;
+        phi += s.phi_i + s.phi_c;
+        n += s.n;
+        half = min(half, s.half);
+    };
+    if (nt <= kFewTiles)
+        for (int32_t t = t0; t < t0 + nt; t++) add(ts[t]);
+    for_large_calls(t0, nt, [&](int32_t a, int32_t k, bool mine) {
+        // lane c < 15 adds up component c, in tile order
+        static_assert(offsetof(PropSums, n) == 15 * sizeof(double), "fifteen sums, then counts");
+        const int c = min(lane_id(), 14);
+        double x = 0.0;
+        int32_t m = 0, hf = INT32_MAX;
+        for (int32_t t = a; t < a + k; t++) x += reinterpret_cast<const double *>(ts + t)[c];
+        for (int32_t t = a + lane_id(); t < a + k; t += kWave) {
+            m += ts[t].n;
+            hf = min(hf, ts[t].half);
+        }
+        m = wave_sum(m);
+        hf = wave_min(hf);
+        if (mine) {
+            n = m;
+            half = hf;
+        }
+        for (int q = 0; q < 3; q++) {
+            const double l = read_lane(x, q), y = read_lane(x, 3 + q), z = read_lane(x, 6 + q),
+                         z2 = read_lane(x, 9 + q);
+            if (mine) {
+                L[q] = l;
+                sx[q] = y;
+                sv[q] = z;
+                sv2[q] = z2;
+            }
+        }
+        const double e = read_lane(x, 12), p = read_lane(x, 13) + read_lane(x, 14);
+        if (mine) {
+            ke = e;
+            phi = p;
+        }
+    });
+    // src/nfw.c:134-152: a fit takes 100 bound records of [0, dens_tot - 1)
+    const PropCall c = v ? pc[h] : PropCall{};
+    int64_t nfit = 0;
+    if (v) {
+        const int32_t end = c.dens_tot - 1;
+        nfit = n;
+        if (end >= 0)
+            nfit -= (in.bound[(int64_t)kTileWords * (t0 + end / kScanTile) + end % kScanTile / kWave] >>
+                     (end % kWave)) & 1;
     }
-    ScaleCall s;
-    s.end = end;
-    s.pad = 0;
-    s.nbins = 0;
-    s.ppbin = 0;
-    if (nb >= kMinScale) {
-        int64_t pp = (int64_t)ceil((double)nb / (double)kScaleBins);
-        if (pp < kMinPerBin) pp = nb / (nb / kMinPerBin);
-        s.ppbin = (int32_t)pp;
-        s.nbins = (int32_t)(nb / pp);
-        fit_list[atomicAdd(fit_n, 1)] = h;  // the fits run one call per lane, together
+    const bool fits = nfit >= kMinScale;
+    const uint64_t mf = ballot(fits);  // the fits run together
+    if (mf) {
+        int32_t at = 0;
+        if (lane_id() == 0) at = atomicAdd(fit_n, __popcll(mf));
+        at = uniform(at) + __popcll(mf & ((1ull << lane_id()) - 1));
+        if (fits) fit_list[at] = h;
     }
-    for (int k = 0; k <= kScaleBins; k++) s.bin_r[k] = 0.0f;
-    s.klypin = s.rs = s.chi2 = 0.0f;
-    sc[h] = s;
+    if (!v) return;
+    const hp_halo &hh = halos[h];
+    const int64_t first = hfirst[h];
+    const double PM = pa.particle_mass;
+    const float scale_now = pa.scale_now;
+    hp_halo_props o;
+    const double m = (double)c.n0 * PM;
+    o.m = (float)((double)c.n_all * PM);
+    o.mgrav = (float)m;
+    // src/properties.c:460-475: float fields accumulated from double terms
+    float xoff = 0.0f, voff = 0.0f;
+    double vr = 0.0;
+    for (int k = 0; k < 3; k++) {
+        // the reference's running means start at 0 and stay there with no
+        // record averaged
+        const double dsx = n > 0 ? sx[k] / (double)n : -(double)hh.pos[k];
+        const double dsv = n > 0 ? sv[k] / (double)n : -(double)hh.pos[k + 3];
+        xoff = (float)((double)xoff + dsx * dsx);
+        voff = (float)((double)voff + dsv * dsv);
+        vr += n > 0 ? (sv2[k] - sv[k] * sv[k] / (double)n) / (double)n : 0.0;
+    }
+    for (int k = 0; k < 4; k++) o.alt_m[k] = (float)((double)c.alt[k] * PM);
+    o.Xoff = (float)(sqrt((double)xoff) * 1e3);
+    o.Voff = (float)sqrt((double)voff);
+    o.vrms = (float)sqrt(vr);
+    o.vmax = (float)(kVmaxConst * sqrt(c.vmax * (PM / (double)scale_now)));
+    o.rvmax = c.j_vmax >= 0
+                  ? (float)(prop_radius(in.r2[first + c.j_vmax], pa.force_res) * 1e3)
+                  : 0.0f;
+    const int32_t ih = half == INT32_MAX ? 0 : half;
+    o.halfmass_radius = c.kept > 0 ? (float)(sqrt((double)in.r2[first + ih]) * 1e3) : 0.0f;
+    o.r = (float)(cbrt((3.0 / (4.0 * M_PI)) * (double)c.n0 / pa.thresh0) * 1e3);
+    const double rvir = cbrt((3.0 / (4.0 * M_PI)) * (double)c.vir / pa.rvir_dens) * 1e3;
+    const double mvir = (double)c.vir * PM;
+    o.rvir = (float)rvir;
+    for (int k = 0; k < 3; k++) o.J[k] = (float)(PM * (double)scale_now * L[k]);
+    // src/properties.c:328-349
+    const double total_phi = phi / 2.0;
+    o.kin_to_pot = total_phi != 0.0 ? (float)(ke / total_phi) : 0.0f;
+    o.energy = (float)((ke - total_phi) * PM * kGc / (double)scale_now);
+    const double Jh = PM * (double)scale_now * sqrt(L[0] * L[0] + L[1] * L[1] + L[2] * L[2]);
+    o.spin = (float)(m > 0 ? Jh * sqrt(fabs((double)o.energy)) / (kGc * pow(m, 2.5))
+                           : 0.0);
+    o.bullock_spin = (float)(m > 0 ? Jh / (mvir * sqrt(2.0 * kGc * mvir * rvir *
+                                                        (double)scale_now / 1e3))
+                                   : 0.0);
+    // filled by the shape, scale-radius and pseudo-evolution kernels
+    o.rs = o.klypin_rs = o.chi2 = 0.0f;
+    o.b_to_a = o.c_to_a = o.b_to_a2 = o.c_to_a2 = 0.0f;
+    for (int k = 0; k < 3; k++) o.A[k] = o.A2[k] = 0.0f;
+    for (int k = 0; k < 6; k++) o.inertia_tensor[k] = o.inertia_tensor2[k] = 0.0f;
+    o.m_pe_b = o.m_pe_d = 0.0f;
+    o.n_mdelta = c.n0;
+    o.dens_tot = c.dens_tot;
+    o.n_vir = c.vir;
+    o.n_half = ih;
+    props[h] = o;
+    shape_init(c, t0, o.r, pre, in.bound, pa, shapes + 2 * h);
+    ScaleCall &sc = scales[h];
+    sc.end = c.dens_tot - 1;
+    int64_t pp = 0;
+    if (fits) {
+        pp = (int64_t)ceil((double)nfit / (double)kScaleBins);
+        if (pp < kMinPerBin) pp = nfit / (nfit / kMinPerBin);
+    }
+    sc.ppbin = (int32_t)pp;
+    sc.nbins = fits ? (int32_t)(nfit / pp) : 0;
+    sc.bin_r[0] = 0.0f;
 }
 
 // src/nfw.c:153-162: the outer edge of bin k is between the k * ppbin-th
 // bound record and the record after it
-__global__ __launch_bounds__(kWave) void k_scale_bins(const struct potential *__restrict__ srt,
+__global__ __launch_bounds__(kWave) void k_scale_bins(const PropReads in,
                                                       const ScanTile *__restrict__ tiles,
                                                       int32_t ntiles,
                                                       const int64_t *__restrict__ hfirst,
@@ -1086,14 +1178,13 @@ __global__ __launch_bounds__(kWave) void k_scale_bins(const struct potential *__
     int32_t carry = pre[t].nb;
     for (int32_t base = tl.off; base < end; base += kWave) {
         const int32_t j = base + lane_id();
-        const bool v = j < end;
-        bool b = false;
-        if (v) b = !(srt[first + j].pe < (double)srt[first + j].ke);
-        const int32_t n = wave_scan_add(b ? 1 : 0) + carry;
-        carry = read_lane(n, kWave - 1);
-        if (b && n % pp == 0 && n / pp <= kScaleBins) {
-            const float r = (float)(1e3 * 0.5 * (sqrt((double)srt[first + j].r2) +
-                                                 sqrt((double)srt[first + j + 1].r2)));
+        uint64_t mb = in.bound[(int64_t)kTileWords * t + (base - tl.off) / kWave];
+        if (end - base < kWave) mb &= (1ull << (end - base)) - 1;
+        const int32_t n = count_to_lane(mb) + carry;
+        carry += __popcll(mb);
+        if (((mb >> lane_id()) & 1) && n % pp == 0 && n / pp <= kScaleBins) {
+            const float r = (float)(1e3 * 0.5 * (sqrt((double)in.r2[first + j]) +
+                                                 sqrt((double)in.r2[first + j + 1])));
             sc[tl.call].bin_r[n / pp] = r;
         }
     }
@@ -1315,7 +1406,7 @@ __global__ void k_props_late(int32_t nh, const PropCall *__restrict__ pc,
 }
 
 // bound records with r < r_pe_d per tile
-__global__ __launch_bounds__(kWave) void k_pe_tiles(const struct potential *__restrict__ srt,
+__global__ __launch_bounds__(kWave) void k_pe_tiles(const PropReads in,
                                                     const ScanTile *__restrict__ tiles,
                                                     int32_t ntiles,
                                                     const hp_halo *__restrict__ halos,
@@ -1330,11 +1421,11 @@ __global__ __launch_bounds__(kWave) void k_pe_tiles(const struct potential *__re
     const double lim = r_pe[tl.call];
     const int32_t end = min(tl.off + kScanTile, call_kept(halos, hcount, tl.call));
     int32_t n = 0;
-    for (int32_t j = tl.off + lane_id(); j < end; j += kWave) {
-        const struct potential &r = srt[first + j];
-        n += !(r.pe < (double)r.ke) && sqrt((double)r.r2) < lim ? 1 : 0;
+    for (int32_t base = tl.off; base < end; base += kWave) {
+        const int32_t j = base + lane_id();
+        const uint64_t mb = in.bound[(int64_t)kTileWords * t + (base - tl.off) / kWave];
+        n += __popcll(ballot(j < end && sqrt((double)in.r2[first + j]) < lim) & mb);
     }
-    n = wave_sum(n);
     if (lane_id() == 0) cnt[t] = n;
 }
 
@@ -1343,10 +1434,17 @@ __global__ void k_pe_calls(int32_t nh, const int32_t *__restrict__ call_tile0,
                            const int32_t *__restrict__ cnt, PropArgs pa,
                            hp_halo_props *__restrict__ props) {
     const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    int64_t n = 0;
-    for (int32_t t = call_tile0[h]; t < call_tile0[h] + call_ntiles[h]; t++) n += cnt[t];
-    props[h].m_pe_d = (float)((double)n * pa.particle_mass);
+    const int32_t t0 = h < nh ? call_tile0[h] : 0, nt = h < nh ? call_ntiles[h] : 0;
+    int32_t n = 0;  // a call's records are counted in 32 bits
+    if (nt <= kFewTiles)
+        for (int32_t t = t0; t < t0 + nt; t++) n += cnt[t];
+    for_large_calls(t0, nt, [&](int32_t a, int32_t k, bool mine) {
+        int32_t m = 0;
+        for (int32_t t = a + lane_id(); t < a + k; t += kWave) m += cnt[t];
+        m = wave_sum(m);
+        if (mine) n = m;
+    });
+    if (h < nh) props[h].m_pe_d = (float)((double)n * pa.particle_mass);
 }
 
 }  // namespace hp
