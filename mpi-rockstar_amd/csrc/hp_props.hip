@@ -473,7 +473,7 @@ __global__ __launch_bounds__(kWave) void k_props_sums(const struct potential *__
 // launch (k_shape_small); the others take two launches an iteration, a
 // window that has stopped being skipped.  On 50,000 calls (6.7M records) ten
 // tile passes over everything and their per-window steps were 1.67 ms; now
-// 0.68 ms in the one launch and 0.24 in the twenty.  The records' offsets from the centre (float
+// 0.58 ms in the one launch and 0.23 in the twenty.  The records' offsets from the centre (float
 // differences, as the reference takes them) and bound flags are compacted
 // once into 16 bytes per record.
 
@@ -791,48 +791,78 @@ __device__ __forceinline__ bool shape_step(ShapeRun &s, const double (&sum)[7],
 // in one launch.  A workgroup holds 64 windows at a time of a range of its
 // own; a window that stops makes room for the range's next one, so that the
 // steps stay full though windows take 1 to 10 iterations.  Every iteration
-//   * the windows' records are laid end to end and gone through 256 at a
-//     time, a thread per record: windows hold 25 records on average, and a
-//     wavefront per window left most lanes idle;
+//   * a thread takes a record; a round takes as many records of each window
+//     that has some left as 256 threads allow (4 of 64 windows, all 256 of
+//     the last one), so that in the sums all windows run at once (0.58 ms
+//     against 0.61 with the windows laid end to end, some five to a round);
 //   * each window's seven sums are added up in record order by four lanes,
 //     from the terms in LDS (0 for a record outside the ellipsoid: the
 //     running sums start at 0, so they never are -0 and keep their bits);
 //   * one lane per window takes the step.
 // What bounds it is the chain through the three, above all the last: some
 // 2,000 dependent double instructions of the Jacobi rotations, on one of the
-// four wavefronts (53% of the cycles hold a vector instruction).  So as many
-// workgroups as fit are kept on a compute unit: what a window carries from
-// step to step is held down to a few registers, and six workgroups with a few
-// registers spilled are 0.68 ms against 0.73 with four.
+// four wavefronts (a vector instruction in half of the cycles, the rest in
+// the tail: 10 iterations are a chain of 0.2 ms for a workgroup on its own).
+// So as many workgroups as fit are kept on a compute unit: what a window
+// carries from step to step is held down to a few registers, and six
+// workgroups with some registers spilled are 0.58 ms against 0.65 with four.
 constexpr int kShapeWindows = 64;
 constexpr int kShapeThreads = 4 * kShapeWindows;
 constexpr int kShapeResident = 6;                     // workgroups on a compute unit
 constexpr int kComputeUnits = 256;
 constexpr int kShapeGroups = kComputeUnits * kShapeResident;  // all that run at once
 
-// The first kOneTileGroups workgroups take the one-tile windows instead, a
-// wavefront each through all of its iterations: both kinds are chains of
-// dependent double operations and fill each other's waits.
+// The first kOneTileGroups workgroups take the one-tile windows instead, 16
+// each at a time: a wavefront sums a window, and the windows' steps are taken
+// together as above (each on a wavefront of its own cost as much as the
+// sums).  Both kinds are chains of dependent double operations and fill each
+// other's waits.
 constexpr int kOneTileGroups = 256;
+constexpr int kOneTileSlots = 16;
 
-// ell: 12 doubles in LDS of this wavefront's own; every lane writes and reads
-// the same values
-__device__ void shape_one_tile(const int32_t *__restrict__ list, int32_t n, int32_t first,
-                               int32_t stride, const int64_t *__restrict__ hfirst,
-                               const float4 *__restrict__ cd, ShapeState *__restrict__ st,
-                               double *ell) {
-    for (int32_t i = first; i < n; i += stride) {
-        const int32_t sw = uniform(list[i]);
-        const ShapeState &s = st[sw];
-        ShapeRun run = {s.r, s.b_to_a, s.c_to_a, 0, kShapeIterations};
-        for (int k = 0; k < 9; k++) ell[k] = s.orth[k / 3][k % 3];
-        for (int k = 0; k < 3; k++) ell[9 + k] = s.eig[k];
-        const float4 *rec = cd + hfirst[sw >> 1];
-        const int32_t end = s.n;
-        const double min_r = (double)s.min_r;
-        double sum[7];
-        do shape_sums(ell, ell + 9, min_r, rec, 0, end, sum);
-        while (shape_step(run, sum, st + sw, ell, ell + 9));
+__device__ __forceinline__ void shape_one_tile(const int32_t *__restrict__ list, int32_t n,
+                                               const int64_t *__restrict__ hfirst,
+                                               const float4 *__restrict__ cd,
+                                               ShapeState *__restrict__ st, double (*s_ell)[13],
+                                               double (*s_sum)[7], int64_t *s_first,
+                                               int32_t *s_n) {
+    const int32_t tid = threadIdx.x, wave = uniform(tid / kWave);
+    for (int32_t i0 = blockIdx.x; i0 < n; i0 += kOneTileGroups * kOneTileSlots) {
+        // slot k: window i0 + k kOneTileGroups of the list
+        const int32_t i = i0 + tid * kOneTileGroups;
+        ShapeRun run = {};
+        int32_t sw = -1;
+        if (tid < kOneTileSlots) {
+            if (i < n) {
+                sw = list[i];
+                const ShapeState &s = st[sw];
+                run = ShapeRun{s.r, s.b_to_a, s.c_to_a, 0, kShapeIterations};
+                s_first[tid] = hfirst[sw >> 1];
+                for (int k = 0; k < 9; k++) s_ell[tid][k] = s.orth[k / 3][k % 3];
+                for (int k = 0; k < 3; k++) s_ell[tid][9 + k] = s.eig[k];
+                s_ell[tid][12] = (double)s.min_r;
+            }
+            s_n[tid] = sw < 0 ? 0 : st[sw].n;
+        }
+        while (__syncthreads_or(tid < kOneTileSlots && sw >= 0)) {
+            for (int k = wave; k < kOneTileSlots; k += kShapeThreads / kWave) {
+                const int32_t nk = uniform(s_n[k]);
+                if (nk == 0) continue;
+                double sum[7];
+                shape_sums(s_ell[k], s_ell[k] + 9, s_ell[k][12], cd + s_first[k], 0, nk, sum);
+                if (lane_id() == 0)
+                    for (int q = 0; q < 7; q++) s_sum[k][q] = sum[q];
+            }
+            __syncthreads();
+            if (tid < kOneTileSlots && sw >= 0) {
+                double sum[7];
+                for (int q = 0; q < 7; q++) sum[q] = s_sum[tid][q];
+                if (!shape_step(run, sum, st + sw, s_ell[tid], s_ell[tid] + 9)) {
+                    sw = -1;
+                    s_n[tid] = 0;
+                }
+            }
+        }
     }
 }
 
@@ -847,11 +877,8 @@ __global__ __launch_bounds__(kShapeThreads, kShapeResident) void k_shape_small(
     __shared__ int64_t s_first[kShapeWindows];
     __shared__ int32_t s_n[kShapeWindows];       // records; 0: no window
     const int32_t tid = threadIdx.x, lane = lane_id();
-    const uint32_t wave0 = (uint32_t)uniform(tid & ~(kWave - 1));
-    constexpr int kWaves = kShapeThreads / kWave;
     if (blockIdx.x < kOneTileGroups) {
-        shape_one_tile(one, *none, blockIdx.x * kWaves + uniform(tid / kWave),
-                       kOneTileGroups * kWaves, hfirst, cd, st, s_ell[tid / kWave]);
+        shape_one_tile(one, *none, hfirst, cd, st, s_ell, s_sum, s_first, s_n);
         return;
     }
     const int64_t groups = gridDim.x - kOneTileGroups;
@@ -887,58 +914,65 @@ __global__ __launch_bounds__(kShapeThreads, kShapeResident) void k_shape_small(
             }
         }
         __syncthreads();
-        // lane l of every wavefront: the end of window l's records
-        const uint32_t nl = (uint32_t)s_n[lane];
-        const uint32_t ends = (uint32_t)wave_scan_add((int32_t)nl);
-        const uint32_t total = (uint32_t)read_lane((int32_t)ends, kWave - 1);
-        if (total == 0) break;  // the same in every wavefront
-        const uint32_t hi = (uint32_t)__shfl((int32_t)ends, task, 64);
-        const uint32_t lo = hi - (uint32_t)__shfl((int32_t)nl, task, 64);
+        // Rounds over the windows that still have records, every one taking
+        // the same number `per` of them from `pos` on: lane l of every
+        // wavefront holds window l's count, and a round's k-th running
+        // window has the threads and terms [k per, k per + per).
+        const int32_t nl = s_n[lane], n_task = s_n[task];
+        if (ballot(nl > 0) == 0) break;  // the same in every wavefront
+        int32_t pos = 0, per = 0, w = 0;
+        uint64_t act = 0;
+        float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        // the round's record of this thread (flag 0: none), read a round ahead
+        auto read = [&]() {
+            act = ballot(nl > pos);
+            q.w = 0.0f;
+            if (act == 0) return;
+            per = kShapeThreads / __popcll(act);
+            // tid / per, exact for both below 256
+            const int32_t k = (int32_t)((uint32_t)tid * (65536u / (uint32_t)per + 1u) >> 16);
+            const int32_t i = pos + tid - k * per;
+            const int32_t rank = __popcll(act & ((1ull << lane) - 1));
+            const bool run_l = nl > pos;
+            // window of rank k: lane k takes the lane number of the k-th one
+            const int32_t kth =
+                __builtin_amdgcn_ds_permute(4 * (run_l ? rank : kWave - 1), run_l ? lane : 0);
+            w = __shfl(kth, k, 64);
+            const int32_t n_w = __shfl(nl, w, 64);
+            if (k < __popcll(act) && i < n_w) q = cd[s_first[w] + i];
+        };
+        read();
         double acc = 0.0, acc2 = 0.0;
-        for (uint32_t base = 0;; base += kShapeThreads) {
-            const uint32_t f0 = base + wave0;  // of this wavefront
-            if (f0 < total) {
-                const uint32_t f = f0 + (uint32_t)lane;
-                // the window of f: those ended by f0, and by each end after it
-                int32_t w = __popcll(ballot(ends <= f0));
-                uint64_t m = ballot(ends > f0 && ends - f0 < (uint32_t)kWave);
-                while (m) {
-                    const int b = __builtin_ctzll(m);
-                    m &= m - 1;
-                    w += f >= (uint32_t)read_lane((int32_t)ends, b) ? 1 : 0;
+        while (act != 0) {
+            double v[7] = {0, 0, 0, 0, 0, 0, 0};
+            if (q.w != 0.0f) {
+                const double *e = s_ell[w];
+                const double d[3] = {(double)q.x, (double)q.y, (double)q.z};
+                double r = 0;
+                for (int k = 0; k < 3; k++) {
+                    double dr = 0;
+                    for (int l = 0; l < 3; l++) dr += e[3 * k + l] * d[l];
+                    r += dr * dr / e[9 + k];
                 }
-                const uint32_t w_lo = (uint32_t)__shfl((int32_t)(ends - nl), w, 64);
-                if (f < total) {
-                    const float4 q = cd[s_first[w] + (int64_t)(f - w_lo)];
-                    double v[7] = {0, 0, 0, 0, 0, 0, 0};
-                    if (q.w != 0.0f) {
-                        const double *e = s_ell[w];
-                        const double d[3] = {(double)q.x, (double)q.y, (double)q.z};
-                        double r = 0;
-                        for (int k = 0; k < 3; k++) {
-                            double dr = 0;
-                            for (int l = 0; l < 3; l++) dr += e[3 * k + l] * d[l];
-                            r += dr * dr / e[9 + k];
-                        }
-                        if (!shape_terms(r, e[12], d, v))
-                            for (int k = 0; k < 7; k++) v[k] = 0.0;
-                    }
-                    for (int k = 0; k < 7; k++) s_term[tid][k] = v[k];
-                }
+                if (!shape_terms(r, e[12], d, v))
+                    for (int k = 0; k < 7; k++) v[k] = 0.0;
             }
+            for (int k = 0; k < 7; k++) s_term[tid][k] = v[k];
+            const int32_t a = __popcll(act & ((1ull << task) - 1)) * per;
+            const int32_t b = a + min(per, n_task - pos);  // below a: not running
+            pos += per;
+            read();
             __syncthreads();
-            const int32_t a = lo > base ? (int32_t)min(lo - base, (uint32_t)kShapeThreads) : 0;
-            const int32_t b = hi > base ? (int32_t)min(hi - base, (uint32_t)kShapeThreads) : 0;
             int32_t i = a;
-            for (; i + 8 <= b; i += 8) {
-                double v[8], v2[8];
-                for (int k = 0; k < 8; k++) {
-                    v[k] = s_term[i + k][comp];
-                    v2[k] = s_term[i + k][comp2];
+            for (; i + 4 <= b; i += 4) {
+                double x[4], x2[4];
+                for (int k = 0; k < 4; k++) {
+                    x[k] = s_term[i + k][comp];
+                    x2[k] = s_term[i + k][comp2];
                 }
-                for (int k = 0; k < 8; k++) {
-                    acc += v[k];
-                    acc2 += v2[k];
+                for (int k = 0; k < 4; k++) {
+                    acc += x[k];
+                    acc2 += x2[k];
                 }
             }
             for (; i < b; i++) {
@@ -946,7 +980,6 @@ __global__ __launch_bounds__(kShapeThreads, kShapeResident) void k_shape_small(
                 acc2 += s_term[i][comp2];
             }
             __syncthreads();
-            if (total - base <= kShapeThreads) break;
         }
         s_sum[task][comp] = acc;
         if (comp < 6) s_sum[task][comp2] = acc2;
