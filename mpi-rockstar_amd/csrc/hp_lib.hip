@@ -390,7 +390,7 @@ struct Engine {
         fit_list, fit_n, shape_one, shape_pairs, shape_windows, prop_r2,
         prop_bound;
     // record assembly
-    DevBuf gsegs, gtiles, gcen;
+    DevBuf gsegs;
     SubBufs sub;
     int64_t cap_nodes = 0, cap_small = 0, cap_group = 0, cap_big = 0, cap_tiles = 0, cap_fat = 0;
     std::vector<int32_t> depth_end;  // node count after each depth's level
@@ -488,7 +488,7 @@ struct Engine {
         DevBuf *all[] = {&hfirst, &hcount, &root_tiles, &groups, &direct_blocks,
                          &scan_tiles, &call_tile0, &call_ntiles, &box, &bad, &pot, &rkey, &badlist, &A, &B, &F,
                          &leaf_of, &sides, &nodes, &parent, &fat, &small0, &group0, &groupc, &wave_off, &wave_hsum, &big, &tiles,
-                         &parts, &splitres, &dparts, &counters, &work, &depth_buf, &pcnt, &pscan, &pcall, &psums, &shape_st, &shape_part, &shape_cd, &scale_calls, &r_pe, &pe_cnt, &fit_list, &fit_n, &shape_one, &shape_pairs, &shape_windows, &prop_r2, &prop_bound, &gsegs, &gtiles, &gcen, &keys0, &keys1, &vals0,
+                         &parts, &splitres, &dparts, &counters, &work, &depth_buf, &pcnt, &pscan, &pcall, &psums, &shape_st, &shape_part, &shape_cd, &scale_calls, &r_pe, &pe_cnt, &fit_list, &fit_n, &shape_one, &shape_pairs, &shape_windows, &prop_r2, &prop_bound, &gsegs, &keys0, &keys1, &vals0,
                          &vals1, &hist, &hsum, &srt, &callinfo, &tsum, &tcand, &tile_i32, &rec_call, &strip_cnt, &stage,
                          &seg_wave_l, &seg_block_l, &seg_tiles_l, &seg_hist, &seg_hsum, &srt_rv};
         for (DevBuf *b : all) f(*b);
@@ -1623,7 +1623,7 @@ static Engine *thread_engine(int *err) {
 // to the first child is an error (src/groupies.c:254).
 static int plan_gather(const hp_tree_halo *tree, int64_t nh, const int64_t *base, int64_t nbase,
                        int64_t nparticles, double ratio, std::vector<GatherSeg> &segs,
-                       std::vector<float> &cen, hp_halo *calls, int64_t *total) {
+                       hp_halo *calls, int64_t *total) {
     struct Frame {
         int64_t h, child;
         int64_t steps;      // sibling steps taken (a list longer than the tree is a cycle)
@@ -1634,7 +1634,6 @@ static int plan_gather(const hp_tree_halo *tree, int64_t nh, const int64_t *base
     std::vector<int64_t> path;
     int64_t pos = 0;
     segs.clear();
-    cen.clear();
     for (int64_t b = 0; b < nbase; b++) {
         const int64_t bh = base[b];
         if (bh < 0 || bh >= nh)
@@ -1658,8 +1657,10 @@ static int plan_gather(const hp_tree_halo *tree, int64_t nh, const int64_t *base
             int32_t flags = h == bh ? 1 : 0;
             if (!potential_only && (double)t.num_p < small) flags = 2;
             if (t.num_p > 0)
-                segs.push_back(GatherSeg{t.p_start, pos, (int32_t)t.num_p, (int32_t)b, flags,
-                                         potential_only});
+                segs.push_back(GatherSeg{t.p_start, (int32_t)pos,
+                                         flags | (potential_only ? kGatherPotential : 0),
+                                         {tree[bh].pos[0], tree[bh].pos[1], tree[bh].pos[2]},
+                                         0});
             pos += t.num_p;
             if (pos > INT32_MAX / 2)
                 return set_error(HP_EINVAL, "hp_gather_calls: more than %d records", INT32_MAX / 2);
@@ -1704,7 +1705,6 @@ static int plan_gather(const hp_tree_halo *tree, int64_t nh, const int64_t *base
             path.pop_back();
             st.pop_back();
         }
-        for (int k = 0; k < 3; k++) cen.push_back(tree[bh].pos[k]);
         hp_halo &hc = calls[b];
         memset(&hc, 0, sizeof hc);
         hc.first = first;
@@ -2151,9 +2151,8 @@ __attribute__((visibility("default"))) int hp_gather_calls(
         (nbase > 0 && (!tree || !base || !calls)) || (nparticles > 0 && !d_particles))
         return set_error(HP_EINVAL, "hp_gather_calls: bad arguments");
     std::vector<GatherSeg> segs;
-    std::vector<float> cen;
     int64_t total = 0;
-    int r = plan_gather(tree, nhalos, base, nbase, nparticles, include_host_ratio, segs, cen,
+    int r = plan_gather(tree, nhalos, base, nbase, nparticles, include_host_ratio, segs,
                         calls, &total);
     if (r) return r;
     if (total > cap_records)
@@ -2162,20 +2161,13 @@ __attribute__((visibility("default"))) int hp_gather_calls(
     if (total > 0 && !d_po) return set_error(HP_EINVAL, "hp_gather_calls: bad arguments");
     *nrecords = total;
     if (segs.empty()) return HP_OK;
-    std::vector<GatherTile> tiles;
-    for (size_t i = 0; i < segs.size(); i++)
-        for (int32_t off = 0; off < segs[i].n; off += kGatherTile)
-            tiles.push_back(GatherTile{(int32_t)i, off});
     Engine *e = thread_engine(&r);
     if (!e) return r;
     HP_TRY(hipSetDevice(e->device));
-    if ((r = e->upload(e->gsegs, segs)) || (r = e->upload(e->gtiles, tiles)) ||
-        (r = e->upload(e->gcen, cen)))
-        return r;
-    const int32_t nt = (int32_t)tiles.size();
-    k_gather_records<<<std::min(nt, 8192), 256, 0, e->stream>>>(
+    if ((r = e->upload(e->gsegs, segs))) return r;
+    k_gather_records<<<Engine::blocks(total, kGatherGroup), kGatherThreads, 0, e->stream>>>(
         reinterpret_cast<const GParticle *>(d_particles), e->gsegs.as<GatherSeg>(),
-        e->gtiles.as<GatherTile>(), nt, e->gcen.as<float>(), d_po);
+        (int32_t)segs.size(), (int32_t)total, d_po);
     HP_TRY(hipGetLastError());
     HP_TRY(hipStreamSynchronize(e->stream));
     return HP_OK;

@@ -197,6 +197,37 @@ def test_gpu_gather_matches_restatement(restatement, groups):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("sizes,offset", [
+    ([1], 0),
+    ([1] * 1025, 8),               # as many segments as records in a group, and one more
+    ([1024, 1024, 63], 0),         # segments that end with a group
+    ([1023, 1, 0, 2, 5000, 65], 8),
+    ([3] * 4200, 0),               # more segments than two steps of 64 tell apart
+])
+def test_gpu_gather_segment_edges(restatement, sizes, offset):
+    """Halos without links, records at an 8-byte aligned address."""
+    from halopot.hipmem import DeviceArray
+
+    npart = int(np.sum(sizes))
+    parts = _particles(npart)
+    t = _tree([(n, -1, []) for n in sizes], npart)
+    t["num_child_particles"] = t["num_p"]
+    d_parts = DeviceArray.from_numpy(parts)
+    d_po = DeviceArray.zeros(npart * 48 + offset)
+    try:
+        calls, n = halopot.gather_calls(t, np.arange(len(sizes)), d_parts.address, npart,
+                                        d_po.address + offset, npart)
+        raw = d_po.download(np.empty(npart * 48 + offset, np.uint8))
+    finally:
+        d_parts.free()
+        d_po.free()
+    assert n == npart and not raw[:offset].any()
+    want = b"".join(restatement.particle_radii(parts, t, b, 0.3, npart).tobytes()
+                    for b in range(len(sizes)))
+    assert raw[offset:].tobytes() == want
+
+
+@pytest.mark.gpu
 def test_gpu_gathered_batch_through_the_bound_pass(restatement, groups):
     """Gather on the device, then the bound pass on the gathered records: the
     kept counts are the records that are not potential-only, and the result
