@@ -398,7 +398,8 @@ struct Engine {
     // last run
     hp_stats st{};
 
-    int init() {
+    // `graphs`: with the streams that recorded steps branch to
+    int init(bool graphs = true) {
         if (stream) return HP_OK;
         int n = 0;
         if (hipGetDeviceCount(&n) != hipSuccess || n < 1) {
@@ -431,7 +432,7 @@ struct Engine {
         else
             (void)hipGetLastError();
         for (auto &e : ev) HP_TRY(hipEventCreate(&e));
-        for (int b = 0; b < 3; b++) {
+        for (int b = 0; b < 3 && graphs; b++) {
             HP_TRY(hipStreamCreateWithFlags(&side[b], hipStreamDefault));
             HP_TRY(hipEventCreateWithFlags(&join_ev[b], hipEventDisableTiming));
         }
@@ -469,10 +470,26 @@ struct Engine {
     int32_t host_counters[kNumCounters] = {};
     unsigned long long host_work[4] = {};
 
+    // An engine that serves one call (hp_bound_pass_host) carves its buffers
+    // from one allocation of its own, sized by a first go through reserve()
+    // and load_tables() that only adds up what they ask for; a buffer that
+    // they don't name is allocated as elsewhere.
+    bool counting = false;
+    size_t counted = 0;
+    DevBuf arena;
+
     int grab(DevBuf &b, size_t n) {
-        if (!carve) return b.ensure(n);
+        if (!carve && !counting) return b.ensure(n);
         if (b.carved && b.bytes >= n) return HP_OK;
         const size_t a = (n + 255) & ~(size_t)255;
+        if (counting) {
+            counted += a;
+            return HP_OK;
+        }
+        if (carve_off + a > carve_cap && arena.p) {
+            if (b.carved) b.release();
+            return b.ensure(n);
+        }
         if (carve_off + a > carve_cap)
             return set_error(HP_EINVAL, "scratch of %zu bytes is too small (%zu more needed)",
                              carve_cap, carve_off + a - carve_cap);
@@ -492,6 +509,19 @@ struct Engine {
                          &vals1, &hist, &hsum, &srt, &callinfo, &tsum, &tcand, &tile_i32, &rec_call, &strip_cnt, &stage,
                          &seg_wave_l, &seg_block_l, &seg_tiles_l, &seg_hist, &seg_hsum, &srt_rv};
         for (DevBuf *b : all) f(*b);
+    }
+
+    // One allocation for reserve(T, true), load_tables(T) and `extra` bytes in
+    // `nextra` more buffers.
+    int take_arena(const Tables &T, size_t extra, int nextra) {
+        counting = true;
+        int r = reserve(T, true);
+        if (!r) r = load_tables(T);
+        counting = false;
+        if (r || (r = arena.ensure(counted + extra + 256 * (size_t)nextra))) return r;
+        carve = arena.as<uint8_t>();
+        carve_cap = arena.bytes;
+        return HP_OK;
     }
 
     // Every buffer is carved again from the start of the region.
@@ -542,6 +572,7 @@ struct Engine {
             (void)hipStreamSynchronize(stream);
             drop_graphs();
             for_each_buf([](DevBuf &b) { b.release(); });
+            arena.release();
             sub.release();
             for (auto &e : ev)
                 if (e) (void)hipEventDestroy(e);
@@ -567,7 +598,7 @@ struct Engine {
     template <typename T>
     int upload(DevBuf &b, const std::vector<T> &v) {
         HP_GRAB(b, sizeof(T) * (v.size() ? v.size() : 1));
-        if (!v.empty())
+        if (!v.empty() && !counting)
             HP_TRY(hipMemcpyAsync(b.p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice, stream));
         return HP_OK;
     }
@@ -1893,9 +1924,10 @@ __attribute__((visibility("default"))) void compute_kinetic_energy(struct potent
     }
 }
 
-__attribute__((visibility("default"))) int hp_plan_create(hp_plan **out, const hp_halo *halos,
-                                                          int64_t nhalos,
-                                                          const hp_options *opt) {
+// hp_plan_create; with `one_call`, the plan of a call that ends with it: its
+// buffers, and 1 + nextra more of extra bytes, come from one allocation.
+static int plan_create(hp_plan **out, const hp_halo *halos, int64_t nhalos, const hp_options *opt,
+                       bool one_call, size_t extra, int nextra) {
     if (!out || (nhalos > 0 && !halos) || nhalos < 0)
         return set_error(HP_EINVAL, "hp_plan_create: bad arguments");
     if (opt && ((uint32_t)opt->accumulate > HP_ACC_F64 || (uint32_t)opt->method > HP_METHOD_AUTO ||
@@ -1910,7 +1942,8 @@ __attribute__((visibility("default"))) int hp_plan_create(hp_plan **out, const h
         c[h] = halos[h].count;
     }
     int r = make_tables(p->T, f.data(), c.data(), nhalos, p->opt.method, true);
-    if (!r) r = p->eng.init();
+    if (!r) r = p->eng.init(!one_call || p->opt.use_graph);
+    if (!r && one_call && !p->opt.per_call) r = p->eng.take_arena(p->T, extra, nextra);
     if (!r) {
         p->first = f;
         p->count = c;
@@ -1938,6 +1971,12 @@ __attribute__((visibility("default"))) int hp_plan_create(hp_plan **out, const h
     }
     *out = p;
     return HP_OK;
+}
+
+__attribute__((visibility("default"))) int hp_plan_create(hp_plan **out, const hp_halo *halos,
+                                                          int64_t nhalos,
+                                                          const hp_options *opt) {
+    return plan_create(out, halos, nhalos, opt, false, 0, 0);
 }
 
 // Makes `t` the plan's launch setting (graphs are recorded again on the next
@@ -2678,8 +2717,15 @@ __attribute__((visibility("default"))) int hp_bound_pass_host(struct potential *
                                                               int64_t nrecords, hp_halo *halos,
                                                               int64_t nhalos, uint8_t *bound,
                                                               const hp_options *opt) {
+    // The plan lives for this call: one allocation holds its sixty buffers
+    // and the three of the call (allocated and freed one by one they took a
+    // third of a call of 530,000 records).
+    size_t n = 1;  // the records that the calls cover: nrecords, or the call is refused
+    for (int64_t h = 0; halos && h < nhalos; h++) n += (size_t)std::max<int64_t>(halos[h].count, 0);
+    const size_t npo = sizeof(struct potential) * n,
+                 nh = sizeof(hp_halo) * (size_t)(nhalos > 0 ? nhalos + 1 : 1), nb = n;
     hp_plan *p = nullptr;
-    int r = hp_plan_create(&p, halos, nhalos, opt);
+    int r = plan_create(&p, halos, nhalos, opt, true, npo + nh + nb, 3);
     if (r) return r;
     if (p->T.nrec != nrecords) {
         hp_plan_destroy(p);
@@ -2687,9 +2733,9 @@ __attribute__((visibility("default"))) int hp_bound_pass_host(struct potential *
                          (long long)nrecords);
     }
     DevBuf dpo, dh, db;
-    r = dpo.ensure(sizeof(struct potential) * (nrecords + 1));
-    if (!r) r = dh.ensure(sizeof(hp_halo) * (nhalos + 1));
-    if (!r) r = db.ensure(nrecords + 1);
+    r = p->eng.grab(dpo, npo);
+    if (!r) r = p->eng.grab(dh, nh);
+    if (!r) r = p->eng.grab(db, nb);
     hipStream_t s = p->eng.stream;
     if (!r && (hipMemcpyAsync(dpo.p, po, sizeof(struct potential) * nrecords,
                               hipMemcpyHostToDevice, s) != hipSuccess ||
