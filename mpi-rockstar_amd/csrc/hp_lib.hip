@@ -2400,7 +2400,7 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
     const SubTile *dt = B.tiles.as<SubTile>();
     int32_t *cnt = B.counters.as<int32_t>();
     SParticle *parts = reinterpret_cast<SParticle *>(d_particles);
-    k_fill_i32<<<1, 64, 0, s>>>(cnt, 0, kSfCounters);
+    k_fill_i32<<<Engine::blocks(kSfCounters, 256), 256, 0, s>>>(cnt, 0, kSfCounters);
     HP_LAUNCHED();
     k_fill_i32<<<Engine::blocks(ng, 256), 256, 0, s>>>(B.gerr.as<int32_t>(), 0, ng);
     HP_LAUNCHED();
@@ -2435,39 +2435,48 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
     k_sub_roots<<<Engine::blocks(ng, 64), 64, 0, s>>>((int32_t)ng, dg, B.pbox.as<float>(),
                                               B.nodes.as<Node6>(), act, act_big, cnt, fused);
     HP_LAUNCHED();
-    for (int level = 0;; level++) {
-        int32_t na[kSfCounters];
+    // The host reads the counts, then queues levels for as long as the
+    // workgroups they might need are few (a workgroup without a node leaves
+    // at once): a level doubles the nodes at most, and M points make fewer
+    // than M / kFuseMaxNode nodes to split.  On one group of 5,003 particles
+    // the reads between levels were a fifth of the call.
+    constexpr int64_t kBlind = 2048;
+    int32_t na[kSfCounters];
+    auto read_counts = [&]() -> int {
         HP_TRY(hipMemcpyAsync(na, cnt, sizeof na, hipMemcpyDeviceToHost, s));
         HP_TRY(hipStreamSynchronize(s));
-        const int32_t ns_ = na[kSfActive], nb_ = na[kSfActiveBig];
+        return HP_OK;
+    };
+    for (int level = 0;;) {
+        if ((r = read_counts())) return r;
+        int64_t nb_ = na[kSfTree + 2 * level], ns_ = na[kSfTree + 2 * level + 1];
         if (!ns_ && !nb_) break;
         if (level > 4 * 64) return set_error(HP_EHIP, "hp_find_subfofs: tree too deep");
-        k_fill_i32<<<1, 1, 0, s>>>(cnt + kSfActive, 0, 1);
-        HP_LAUNCHED();
-        k_fill_i32<<<1, 1, 0, s>>>(cnt + kSfActiveBig, 0, 1);
-        HP_LAUNCHED();
-        if (nb_) {
-            k_sub_split<1024><<<(uint32_t)nb_, 1024, 0, s>>>(
-                B.nodes.as<Node6>(), act_big, B.w.as<SParticle>(), B.w2.as<SParticle>(),
-                B.rk.as<int32_t>(), B.bpos.as<int32_t>(), B.spos.as<int32_t>(), nxt, nxt_big,
-                cnt, (int32_t)node_cap, fused);
-            HP_LAUNCHED();
-        }
-        if (ns_) {
-            k_sub_split<kSfThreads><<<(uint32_t)ns_, kSfThreads, 0, s>>>(
-                B.nodes.as<Node6>(), act, B.w.as<SParticle>(), B.w2.as<SParticle>(),
-                B.rk.as<int32_t>(), B.bpos.as<int32_t>(), B.spos.as<int32_t>(), nxt, nxt_big,
-                cnt, (int32_t)node_cap, fused);
-            HP_LAUNCHED();
-        }
-        std::swap(act, nxt);
-        std::swap(act_big, nxt_big);
+        do {
+            if (nb_) {
+                k_sub_split<1024><<<(uint32_t)nb_, 1024, 0, s>>>(
+                    B.nodes.as<Node6>(), act_big, B.w.as<SParticle>(), B.w2.as<SParticle>(),
+                    B.rk.as<int32_t>(), B.bpos.as<int32_t>(), B.spos.as<int32_t>(), nxt, nxt_big,
+                    cnt, level, (int32_t)node_cap, fused);
+                HP_LAUNCHED();
+            }
+            if (ns_) {
+                k_sub_split<kSfThreads><<<(uint32_t)ns_, kSfThreads, 0, s>>>(
+                    B.nodes.as<Node6>(), act, B.w.as<SParticle>(), B.w2.as<SParticle>(),
+                    B.rk.as<int32_t>(), B.bpos.as<int32_t>(), B.spos.as<int32_t>(), nxt, nxt_big,
+                    cnt, level, (int32_t)node_cap, fused);
+                HP_LAUNCHED();
+            }
+            std::swap(act, nxt);
+            std::swap(act_big, nxt_big);
+            level++;
+            ns_ = std::min(2 * (ns_ + nb_), M / (kFuseMaxNode + 1));
+            nb_ = std::min(2 * nb_, M / (kSfBigNode + 1));
+        } while (ns_ + nb_ <= kBlind && ns_ + nb_ > 0 && level % 6 && level <= 4 * 64);
     }
     {
         // the nodes of at most kFuseMax points, each finished by one workgroup
-        int32_t nf = 0;
-        HP_TRY(hipMemcpyAsync(&nf, cnt + kSfFused, sizeof nf, hipMemcpyDeviceToHost, s));
-        HP_TRY(hipStreamSynchronize(s));
+        const int32_t nf = na[kSfFused];
         if (nf > 0) {
             k_sub_fused<<<(uint32_t)nf, kSfThreads, 0, s>>>(B.nodes.as<Node6>(), fused,
                                                            B.w.as<SParticle>(),
@@ -2475,13 +2484,16 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
                                                            (int32_t)node_cap);
             HP_LAUNCHED();
         }
-        int32_t nn = 0;
-        HP_TRY(hipMemcpyAsync(&nn, cnt + kSfNodes, sizeof nn, hipMemcpyDeviceToHost, s));
-        HP_TRY(hipStreamSynchronize(s));
+        // the nodes there are, or, of few points, could be
+        int32_t nn = (int32_t)node_cap;
+        if (node_cap > 8 * kBlind) {
+            HP_TRY(hipMemcpyAsync(&nn, cnt + kSfNodes, sizeof nn, hipMemcpyDeviceToHost, s));
+            HP_TRY(hipStreamSynchronize(s));
+        }
         nn = (int32_t)std::min<int64_t>(nn, node_cap);
         if (nn > 0) {
             k_sub_collect<<<(uint32_t)nn, kWave, 0, s>>>(B.nodes.as<Node6>(), B.w.as<SParticle>(),
-                                                         B.w2.as<SParticle>(),
+                                                         B.w2.as<SParticle>(), cnt,
                                                          B.slot_leaf.as<int32_t>());
             HP_LAUNCHED();
         }
@@ -2583,44 +2595,42 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
         // partition_sort_particles, level by level
         SortRange *ra = B.rng0.as<SortRange>(), *rb = B.rng1.as<SortRange>();
         SortRange *rs = B.rsmall.as<SortRange>();
-        k_fill_i32<<<1, 64, 0, s>>>(cnt + kSfRange, 0, 3);
-        HP_LAUNCHED();
         k_sort_roots<<<Engine::blocks(ng, 64), 64, 0, s>>>((int32_t)ng, dg, ra, rs, cnt,
                                                    (int32_t)cap_rng, (int32_t)cap_rsmall);
         HP_LAUNCHED();
         int32_t nsmall = 0;
-        for (int level = 0;; level++) {
-            int32_t na[kSfCounters];
-            HP_TRY(hipMemcpyAsync(na, cnt, sizeof na, hipMemcpyDeviceToHost, s));
-            HP_TRY(hipStreamSynchronize(s));
+        for (int level = 0;;) {
+            if ((r = read_counts())) return r;
             if (na[kSfErr])
                 return set_error(HP_EHIP, "hp_find_subfofs: scratch overflow (%d)", na[kSfErr]);
-            const int32_t nr = na[kSfRange], nm = na[kSfRangeMid];
+            int64_t nr = na[kSfSort + 2 * level], nm = na[kSfSort + 2 * level + 1];
             nsmall = na[kSfRangeSmall];
             if (!nr && !nm) break;
             // each level halves the value span of every range it splits
             if (level > 40) return set_error(HP_EHIP, "hp_find_subfofs: output sort too deep");
-            k_fill_i32<<<1, 1, 0, s>>>(cnt + kSfRange, 0, 1);
-            HP_LAUNCHED();
-            k_fill_i32<<<1, 1, 0, s>>>(cnt + kSfRangeMid, 0, 1);
-            HP_LAUNCHED();
-            if (nr) {
-                k_sort_split<kSortThreads1><<<(uint32_t)nr, kSortThreads1, 0, s>>>(
-                    ra, v0, v1, x0, x1, B.rk.as<int32_t>(), B.bpos.as<int32_t>(),
-                    B.spos.as<int32_t>(), rb, rs, cnt, (int32_t)cap_rng, (int32_t)cap_rsmall);
-                HP_LAUNCHED();
-            }
-            if (nm) {
-                k_sort_split<kSortThreads2><<<(uint32_t)nm, kSortThreads2, 0, s>>>(
-                    ra + 2 * cap_rng - 1, v0, v1, x0, x1, B.rk.as<int32_t>(),
-                    B.bpos.as<int32_t>(), B.spos.as<int32_t>(), rb, rs, cnt, (int32_t)cap_rng,
-                    (int32_t)cap_rsmall);
-                HP_LAUNCHED();
-            }
-            std::swap(ra, rb);
+            do {
+                if (nr) {
+                    k_sort_split<kSortThreads1><<<(uint32_t)nr, kSortThreads1, 0, s>>>(
+                        ra, v0, v1, x0, x1, B.rk.as<int32_t>(), B.bpos.as<int32_t>(),
+                        B.spos.as<int32_t>(), rb, rs, cnt, level, (int32_t)cap_rng,
+                        (int32_t)cap_rsmall);
+                    HP_LAUNCHED();
+                }
+                if (nm) {
+                    k_sort_split<kSortThreads2><<<(uint32_t)nm, kSortThreads2, 0, s>>>(
+                        ra + 2 * cap_rng - 1, v0, v1, x0, x1, B.rk.as<int32_t>(),
+                        B.bpos.as<int32_t>(), B.spos.as<int32_t>(), rb, rs, cnt, level,
+                        (int32_t)cap_rng, (int32_t)cap_rsmall);
+                    HP_LAUNCHED();
+                }
+                std::swap(ra, rb);
+                level++;
+                nm = std::min(2 * (nr + nm), M / (kSortSmall + 1));
+                nr = std::min(2 * nr, M / (kSortMid + 1));
+            } while (nr + nm <= kBlind && nr + nm > 0 && level % 6 && level <= 40);
         }
         if (nsmall > 0) {
-            k_sort_small<<<(uint32_t)nsmall, kWave, 0, s>>>(rs, v0, v1, x0, x1);
+            k_sort_small<<<(uint32_t)nsmall, kWave, 0, s>>>(rs, cnt, v0, v1, x0, x1);
             HP_LAUNCHED();
         }
         k_sub_emit<<<Engine::blocks(M, 256), 256, 0, s>>>(

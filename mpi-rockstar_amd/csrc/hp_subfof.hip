@@ -78,16 +78,20 @@ static_assert(sizeof(Node6) == 80, "node layout");
 
 enum SfCounter {
     kSfNodes = 0,
-    kSfActive = 1,     // nodes to split next level with kSfThreads
-    kSfEmit = 2,
-    kSfErr = 3,
-    kSfActiveBig = 4,  // nodes above kSfBigNode points: split with 1024 threads
-    kSfFused = 5,      // nodes of at most kFuseMax points: finished by k_sub_fused
-    kSfEdges = 6,      // 64-bit (6 and 7): pairs the linking walk listed
-    kSfRange = 8,      // output-order ranges above kSortMid values to split next level
-    kSfRangeSmall = 9, // output-order ranges finished by one wavefront
-    kSfRangeMid = 10,  // output-order ranges of at most kSortMid values to split next level
-    kSfCounters = 11
+    kSfEmit = 1,
+    kSfErr = 2,
+    kSfFused = 3,      // nodes of at most kFuseMax points: finished by k_sub_fused
+    kSfEdges = 4,      // 64-bit (4 and 5): pairs the linking walk listed
+    kSfRangeSmall = 6, // output-order ranges finished by one wavefront
+    // per level, what the level splits: the tree's nodes above kSfBigNode
+    // points and the others, then the output order's ranges above kSortMid
+    // values and the others.  A level's kernels read their counts here, so
+    // that levels can follow each other without the host.
+    kSfTree = 8,
+    kSfTreeLevels = 258,
+    kSfSort = kSfTree + 2 * kSfTreeLevels,
+    kSfSortLevels = 42,
+    kSfCounters = kSfSort + 2 * kSfSortLevels
 };
 constexpr int kSfBigNode = 8192;
 
@@ -289,11 +293,12 @@ __global__ __launch_bounds__(kWave) void k_sub_scale(const SubGroup *__restrict_
 constexpr int kFuseMaxNode = 1024;  // kFuseMax, declared with its kernel below
 __device__ __forceinline__ void push_active(int32_t id, int32_t n, int32_t *__restrict__ small,
                                             int32_t *__restrict__ big,
-                                            int32_t *__restrict__ counters,
+                                            int32_t *__restrict__ counters, int32_t level,
                                             int32_t *__restrict__ fused) {
+    int32_t *count = counters + kSfTree + 2 * level;
     if (n <= kFuseMaxNode) fused[atomicAdd(&counters[kSfFused], 1)] = id;
-    else if (n > kSfBigNode) big[atomicAdd(&counters[kSfActiveBig], 1)] = id;
-    else small[atomicAdd(&counters[kSfActive], 1)] = id;
+    else if (n > kSfBigNode) big[atomicAdd(&count[0], 1)] = id;
+    else small[atomicAdd(&count[1], 1)] = id;
 }
 
 __global__ void k_sub_roots(int32_t ng, const SubGroup *__restrict__ groups,
@@ -322,7 +327,7 @@ __global__ void k_sub_roots(int32_t ng, const SubGroup *__restrict__ groups,
     nd.left = nd.right = nd.parent = nd.skip = -1;
     nd.where = 0;
     nodes[gi] = nd;
-    if (g.n > kLeaf6) push_active(gi, g.n, active, active_big, counters, fused);
+    if (g.n > kLeaf6) push_active(gi, g.n, active, active_big, counters, 0, fused);
 }
 
 // ------------------------------------------------------------- tree build
@@ -384,8 +389,10 @@ __global__ __launch_bounds__(NT) void k_sub_split(
     Node6 *__restrict__ nodes, const int32_t *__restrict__ active, SParticle *__restrict__ wa,
     SParticle *__restrict__ wb, int32_t *__restrict__ rk, int32_t *__restrict__ bpos,
     int32_t *__restrict__ spos, int32_t *__restrict__ next, int32_t *__restrict__ next_big,
-    int32_t *__restrict__ counters, int32_t node_cap, int32_t *__restrict__ fused) {
+    int32_t *__restrict__ counters, int32_t level, int32_t node_cap,
+    int32_t *__restrict__ fused) {
     constexpr int NW = NT / kWave;
+    if ((int32_t)blockIdx.x >= counters[kSfTree + 2 * level + (NT == 1024 ? 0 : 1)]) return;
     __shared__ int s_w[NW];
     __shared__ int32_t s_k[2];
     __shared__ float s_box[NW][24];
@@ -515,8 +522,8 @@ __global__ __launch_bounds__(NT) void k_sub_split(
     me_n.left = l;
     me_n.right = l + 1;
     nodes[me] = me_n;
-    if (L.n > kLeaf6) push_active(l, L.n, next, next_big, counters, fused);
-    if (R.n > kLeaf6) push_active(l + 1, R.n, next, next_big, counters, fused);
+    if (L.n > kLeaf6) push_active(l, L.n, next, next_big, counters, level + 1, fused);
+    if (R.n > kLeaf6) push_active(l + 1, R.n, next, next_big, counters, level + 1, fused);
 }
 
 // A node of at most kFuseMax points is split down to its leaves by one
@@ -558,6 +565,7 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
     __shared__ int s_w[kSfThreads / kWave];
     __shared__ int32_t s_cnt[2], s_g0;
     const int tid = threadIdx.x;
+    if ((int32_t)blockIdx.x >= counters[kSfFused]) return;
     const int32_t root = roots[blockIdx.x];
     const Node6 rn = nodes[root];
     const int32_t s0 = rn.start, N = rn.n;
@@ -797,7 +805,9 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
 __global__ __launch_bounds__(kWave) void k_sub_collect(const Node6 *__restrict__ nodes,
                                                        SParticle *__restrict__ wa,
                                                        const SParticle *__restrict__ wb,
+                                                       const int32_t *__restrict__ counters,
                                                        int32_t *__restrict__ slot_leaf) {
+    if ((int32_t)blockIdx.x >= counters[kSfNodes]) return;
     const Node6 nd = nodes[blockIdx.x];
     if (nd.div >= 0) return;
     for (int32_t p = lane_id(); p < nd.n; p += kWave) {
@@ -1855,14 +1865,15 @@ struct SortRange {
 // from 0 and the mid-sized ones from cap_next down
 __device__ __forceinline__ void push_range(SortRange r, SortRange *__restrict__ next,
                                            SortRange *__restrict__ small,
-                                           int32_t *__restrict__ counters, int32_t cap_next,
-                                           int32_t cap_small) {
+                                           int32_t *__restrict__ counters, int32_t level,
+                                           int32_t cap_next, int32_t cap_small) {
+    int32_t *count = counters + kSfSort + 2 * level;
     if (r.n > kSortMid) {
-        const int32_t k = atomicAdd(&counters[kSfRange], 1);
+        const int32_t k = atomicAdd(&count[0], 1);
         if (k < cap_next) next[k] = r;
         else atomicOr(&counters[kSfErr], 4);
     } else if (r.n > kSortSmall) {
-        const int32_t k = atomicAdd(&counters[kSfRangeMid], 1);
+        const int32_t k = atomicAdd(&count[1], 1);
         if (k < cap_next) next[2 * cap_next - 1 - k] = r;
         else atomicOr(&counters[kSfErr], 4);
     } else {
@@ -1879,7 +1890,8 @@ __global__ void k_sort_roots(int32_t ng, const SubGroup *__restrict__ groups,
     if (gi >= ng) return;
     const SubGroup g = groups[gi];
     if (g.n >= 2)
-        push_range(SortRange{g.off, g.n, 0, 1, 0, 0}, next, small, counters, cap_next, cap_small);
+        push_range(SortRange{g.off, g.n, 0, 1, 0, 0}, next, small, counters, 0, cap_next,
+                   cap_small);
 }
 
 // exclusive prefix sum over the workgroup's threads, and the total
@@ -1926,9 +1938,10 @@ __global__ __launch_bounds__(NT) void k_sort_split(
     const SortRange *__restrict__ ranges, int32_t *__restrict__ v0, int32_t *__restrict__ v1,
     int32_t *__restrict__ x0, int32_t *__restrict__ x1, int32_t *__restrict__ rk,
     int32_t *__restrict__ bpos, int32_t *__restrict__ spos, SortRange *__restrict__ next,
-    SortRange *__restrict__ small, int32_t *__restrict__ counters, int32_t cap_next,
-    int32_t cap_small) {
+    SortRange *__restrict__ small, int32_t *__restrict__ counters, int32_t level,
+    int32_t cap_next, int32_t cap_small) {
     static_assert(NT == 1024 || NT == 256, "launch shapes");
+    if ((int32_t)blockIdx.x >= counters[kSfSort + 2 * level + (NT == 1024 ? 0 : 1)]) return;
     __shared__ int s_w[4 * (NT / kWave)];
     __shared__ int32_t s_k[1];
     const SortRange sr = NT == 1024 ? ranges[blockIdx.x] : *(ranges - blockIdx.x);
@@ -2031,7 +2044,7 @@ __global__ __launch_bounds__(NT) void k_sort_split(
     const SortRange L{s0, nsmall, wh, llo, lhi, 0}, R{s0 + nsmall, n - nsmall, wh, rlo, rhi, 0};
     for (const SortRange &c : {L, R}) {
         if (c.n >= 2) {
-            push_range(c, next, small, counters, cap_next, cap_small);
+            push_range(c, next, small, counters, level + 1, cap_next, cap_small);
         } else if (c.n == 1 && wh) {
             v0[c.start] = v1[c.start];
             x0[c.start] = x1[c.start];
@@ -2042,12 +2055,14 @@ __global__ __launch_bounds__(NT) void k_sort_split(
 // a range of at most kSortSmall: the reference's loop itself, by one lane,
 // on a copy in LDS; the result to the first buffer
 __global__ __launch_bounds__(kWave) void k_sort_small(const SortRange *__restrict__ ranges,
+                                                      const int32_t *__restrict__ counters,
                                                       int32_t *__restrict__ v0,
                                                       int32_t *__restrict__ v1,
                                                       int32_t *__restrict__ x0,
                                                       int32_t *__restrict__ x1) {
     __shared__ int32_t s_v[kSortSmall], s_x[kSortSmall];
     __shared__ int2 s_stack[kSortSmall];
+    if ((int32_t)blockIdx.x >= counters[kSfRangeSmall]) return;
     const SortRange sr = ranges[blockIdx.x];
     const int32_t s0 = sr.start, n = min(sr.n, kSortSmall);
     const int32_t *__restrict__ vs = sr.where ? v1 : v0;
