@@ -365,8 +365,8 @@ __device__ void partition_ks(const int32_t *__restrict__ bpos, const int32_t *__
     *S = (lo < nbig && bpos[lo] < rK) ? bpos[lo] + 1 : rK;
 }
 
-// The same by a whole wavefront, in every lane: 64 candidates a step (one at a
-// time the dependent reads were half of a level of 5,000 points).
+// The same by a whole wavefront, in every lane: 64 candidates a step (a level
+// of 16,000 points 15.5 us against 18.6 by halves, each a dependent read).
 __device__ void partition_ks_wave(const int32_t *__restrict__ bpos,
                                   const int32_t *__restrict__ spos,
                                   int32_t n, int32_t nbig, int32_t nsmall, int32_t *K, int32_t *S) {
@@ -1245,8 +1245,18 @@ __device__ __forceinline__ uint64_t slot_bits(int32_t base, int32_t lo, int32_t 
     return from & to;
 }
 
-// fast3tree_find_next_closest_distance (src/fast3tree.c:992-1030) for 64
-// sampled particles per wavefront, neighbours in the tree order.
+// Queries of a wavefront in the searches: all 64 lanes, or, where the batch
+// has too few tiles to give every SIMD a wavefront, one row of 16.  A
+// wavefront's time is its chain through the chunks near any of its rows: on
+// one group of 15,985 particles (250 tiles) the searches take 123 and 102 us,
+// where with 64 queries they took 190 and 168.
+constexpr int32_t kFewQueryTiles = 512;
+__host__ __device__ constexpr int32_t query_lanes(int64_t tiles64) {
+    return tiles64 < kFewQueryTiles ? 16 : kWave;
+}
+
+// fast3tree_find_next_closest_distance (src/fast3tree.c:992-1030) for the
+// sampled particles of a tile, a lane each, neighbours in the tree order.
 //
 // The reference's answer depends on its visiting order only through
 // rounding: a leaf that improves nothing returns sqrt(r * r) = r (exact for
@@ -1264,12 +1274,12 @@ __global__ __launch_bounds__(kWave) void k_sub_next_closest(
     const SParticle *__restrict__ w, const Node6 *__restrict__ nodes,
     const int32_t *__restrict__ slot_leaf, const PackPoint *__restrict__ pk,
     const Box6 *__restrict__ chunks,
-    const Box6 *__restrict__ blocks, float *__restrict__ dist, int ordered) {
+    const Box6 *__restrict__ blocks, float *__restrict__ dist, int ordered, int32_t lanes) {
     __shared__ PairLds L;
     const SubTile tl = qtiles[blockIdx.x];
     const SubGroup g = groups[tl.group];
     const int32_t q = tl.off + lane_id();
-    const bool valid = q < g.nsample;
+    const bool valid = lane_id() < lanes && q < g.nsample;
     const int32_t root = tl.group;
     float c[6] = {0, 0, 0, 0, 0, 0};
     int32_t skip = -1, s_lo = 0, s_hi = 0, slot = g.off;
@@ -1491,13 +1501,14 @@ __global__ __launch_bounds__(kWave) void k_sub_link(const SubGroup *__restrict__
                                                     const Box6 *__restrict__ blocks,
                                                     EdgeRec *__restrict__ edges, int64_t cap_edges,
                                                     int32_t *__restrict__ deg,
-                                                    int32_t *__restrict__ counters) {
+                                                    int32_t *__restrict__ counters,
+                                                    int32_t lanes) {
     __shared__ PairLds L;
     __shared__ EdgeRec s_e[kLinkStage];
     const SubTile tl = ltiles[blockIdx.x];
     const SubGroup g = groups[tl.group];
     const int32_t i = g.off + tl.off + lane_id(), end = g.off + g.n;
-    const bool valid = i < end;
+    const bool valid = lane_id() < lanes && i < end;
     const float r = target[tl.group];
     const float r2 = r * r;
     float c[6] = {0, 0, 0, 0, 0, 0};
