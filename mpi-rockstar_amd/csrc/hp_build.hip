@@ -1673,7 +1673,7 @@ __device__ void level_done(int32_t *c, int32_t *lv, int32_t level) {
     big[level + 1] = stop ? big[level] : c[kBigNext];
     tile[level + 1] = stop ? tile[level] : c[kTileNext];
     c[kGlobalNodes] = nodes;
-    c[kLevel] = level + 1;
+    if (level == 0 || c[kActive]) c[kLevel] = level + 1;  // a level with nothing to split adds no depth
     c[kActive] = big[level + 1] > big[level] ? 1 : 0;
 }
 __global__ void k_levels_init(int32_t *__restrict__ c, int32_t *__restrict__ lv) {

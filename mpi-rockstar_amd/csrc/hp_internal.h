@@ -125,7 +125,7 @@ enum Counter {
     // level state, advanced on the device between levels
     kGlobalNodes = 9, // nodes made by the split levels (subtree nodes follow)
     // 10-13 unused (the split levels' ranges are in the level buffer)
-    kLevel = 14,      // levels advanced so far
+    kLevel = 14,      // 1 + the levels that had a node to split so far
     kActive = 15,     // the current level has big tasks
     kBadRoots = 16,   // calls with non-finite points, listed for their own pass
     kGroupNext = 17,  // workgroup subtree tasks (wave_max < n <= big_threshold), append-only

@@ -1049,13 +1049,18 @@ struct Engine {
     }
 
     // Runs split levels from `level` until the level state is inactive,
-    // checking every kLevelBatch levels.  Returns the next level index.
+    // checking after every batch.  The first batch holds the levels that the
+    // largest call takes at least, halving at best, and kLevelSlack more; a
+    // level with nothing to split costs its three launches (12 us), a check a
+    // copy and a wait (20 us).  Returns the next level index.
     int finish_levels(int level, int *next) {
-        constexpr int kLevelBatch = 8;
+        constexpr int kLevelBatch = 4, kLevelSlack = 3;
+        int n = kLevelSlack;
+        for (int64_t m = max_count; m > std::max(big_min(), 1); m /= 2) n++;
         int r;
-        for (;;) {
-            if ((r = enqueue_levels(level, kLevelBatch))) return r;
-            level += kLevelBatch;
+        for (;; n = kLevelBatch) {
+            if ((r = enqueue_levels(level, n))) return r;
+            level += n;
             if ((r = read_counters())) return r;
             if (!h_counters[kActive] || h_counters[kErrFlags]) break;
             if (level > kMaxLevels - kLevelBatch)
