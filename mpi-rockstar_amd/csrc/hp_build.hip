@@ -347,14 +347,13 @@ __device__ __forceinline__ void write_node(Node *nd, const float *lo, const floa
 // for k_roots_bad; every other call gets its root node here, its points in
 // tree order when it is a single leaf, and its root queued as a task.  The
 // subtree-task slots of a wavefront's calls are taken with one atomic.
-__global__ __launch_bounds__(256) void k_roots(const int64_t *__restrict__ hfirst,
-                                               const int64_t *__restrict__ hcount,
-                                               const int32_t *__restrict__ box,
-                                               const int32_t *__restrict__ bad,
-                                               const float4 *__restrict__ A,
-                                               int32_t *__restrict__ badlist, int nhalos,
-                                               BuildArgs a) {
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void root_of_call(int h, const int64_t *__restrict__ hfirst,
+                                             const int64_t *__restrict__ hcount,
+                                             const int32_t *__restrict__ box,
+                                             const int32_t *__restrict__ bad,
+                                             const float4 *__restrict__ A,
+                                             int32_t *__restrict__ badlist, int nhalos,
+                                             const BuildArgs &a) {
     const bool v = h < nhalos;
     int32_t first = 0, nfin = 0, bucket = 0;
     bool isbad = false;
@@ -417,19 +416,29 @@ __global__ __launch_bounds__(256) void k_roots(const int64_t *__restrict__ hfirs
     else if (gsmall) push_group_at(a, gslot0 + rank_below(mg), h, lo, hi, 0, first, nfin);
 }
 
+__global__ __launch_bounds__(256) void k_roots(const int64_t *__restrict__ hfirst,
+                                               const int64_t *__restrict__ hcount,
+                                               const int32_t *__restrict__ box,
+                                               const int32_t *__restrict__ bad,
+                                               const float4 *__restrict__ A,
+                                               int32_t *__restrict__ badlist, int nhalos,
+                                               BuildArgs a) {
+    root_of_call(blockIdx.x * blockDim.x + threadIdx.x, hfirst, hcount, box, bad, A, badlist,
+                 nhalos, a);
+}
+
 // The listed calls with non-finite points, one workgroup each: removal of
 // the non-finite records to the tail in the order of the reference's swap
 // loop (src/fast3tree.c:875-887), root node, root queued or finished as a
 // leaf.
-__global__ __launch_bounds__(256) void k_roots_bad(const int64_t *__restrict__ hfirst,
+__device__ __forceinline__ void roots_of_bad_calls(const int64_t *__restrict__ hfirst,
                                                    const int64_t *__restrict__ hcount,
                                                    const int32_t *__restrict__ box,
                                                    const int32_t *__restrict__ bad,
                                                    float4 *__restrict__ A,
                                                    const int32_t *__restrict__ badlist,
-                                                   BuildArgs a) {
+                                                   int32_t nlist, const BuildArgs &a) {
     __shared__ int s_cnt[2][4];
-    const int32_t nlist = a.counters[kBadRoots];
     for (int32_t li = blockIdx.x; li < nlist; li += gridDim.x) {
         const int h = badlist[li];
         const int32_t first = (int32_t)hfirst[h];
@@ -508,6 +517,35 @@ __global__ __launch_bounds__(256) void k_roots_bad(const int64_t *__restrict__ h
         }
         __syncthreads();
     }
+}
+__global__ __launch_bounds__(256) void k_roots_bad(const int64_t *__restrict__ hfirst,
+                                                   const int64_t *__restrict__ hcount,
+                                                   const int32_t *__restrict__ box,
+                                                   const int32_t *__restrict__ bad,
+                                                   float4 *__restrict__ A,
+                                                   const int32_t *__restrict__ badlist,
+                                                   BuildArgs a) {
+    roots_of_bad_calls(hfirst, hcount, box, bad, A, badlist, a.counters[kBadRoots], a);
+}
+
+// k_roots, k_roots_bad and k_levels_init of a single call, in one launch of
+// one workgroup (a call of 134 records is bound by its launches).
+__device__ void level_done(int32_t *c, int32_t *lv, int32_t level);
+__device__ void levels_init(int32_t *c, int32_t *lv);
+__global__ __launch_bounds__(256) void k_root_one(const int64_t *__restrict__ hfirst,
+                                                  const int64_t *__restrict__ hcount,
+                                                  const int32_t *__restrict__ box,
+                                                  const int32_t *__restrict__ bad,
+                                                  float4 *__restrict__ A,
+                                                  int32_t *__restrict__ badlist,
+                                                  int32_t *__restrict__ lv, BuildArgs a) {
+    root_of_call(threadIdx.x, hfirst, hcount, box, bad, A, badlist, 1, a);
+    __threadfence();
+    __syncthreads();
+    if (bad[0] > 0) roots_of_bad_calls(hfirst, hcount, box, bad, A, badlist, 1, a);
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) levels_init(a.counters, lv);
 }
 
 // ------------------------------------------------------------ small tasks
@@ -874,10 +912,8 @@ __device__ __forceinline__ void wave_subtree(const BuildArgs &a, WaveTree &W, fl
 // Each task also gets its node ids here, 2n - 2 for n points (the most a
 // subtree can need; ids it does not use are never referenced), the first
 // kept in tile0: one atomic per wavefront instead of one per subtree.
-__global__ __launch_bounds__(256) void k_group_classes(const Task *__restrict__ in, BuildArgs a,
-                                                       Task *__restrict__ out) {
-    const int32_t n = min(a.counters[kGroupNext], a.cap_group);
-    const int32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void group_class(int32_t k, int32_t n, const Task *__restrict__ in,
+                                            const BuildArgs &a, Task *__restrict__ out) {
     if (k - lane_id() >= n) return;  // whole wavefronts past the list
     Task t;
     int c = -1;
@@ -900,6 +936,11 @@ __global__ __launch_bounds__(256) void k_group_classes(const Task *__restrict__ 
         base = __shfl(base, 0, 64);
         if (c == q) out[(int64_t)q * a.cap_group + base + rank_below(m)] = t;
     }
+}
+__global__ __launch_bounds__(256) void k_group_classes(const Task *__restrict__ in, BuildArgs a,
+                                                       Task *__restrict__ out) {
+    group_class(blockIdx.x * blockDim.x + threadIdx.x, min(a.counters[kGroupNext], a.cap_group), in,
+                a, out);
 }
 
 // A node of more than kPart points of the workgroup's current level.
@@ -1676,11 +1717,13 @@ __device__ void level_done(int32_t *c, int32_t *lv, int32_t level) {
     if (level == 0 || c[kActive]) c[kLevel] = level + 1;  // a level with nothing to split adds no depth
     c[kActive] = big[level + 1] > big[level] ? 1 : 0;
 }
-__global__ void k_levels_init(int32_t *__restrict__ c, int32_t *__restrict__ lv) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__device__ void levels_init(int32_t *c, int32_t *lv) {
     lvl_big(lv)[0] = 0;
     lvl_tile(lv)[0] = 0;
     level_done(c, lv, 0);
+}
+__global__ void k_levels_init(int32_t *__restrict__ c, int32_t *__restrict__ lv) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) levels_init(c, lv);
 }
 
 // --------------------------------------------------------------- multipoles

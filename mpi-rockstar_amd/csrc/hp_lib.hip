@@ -797,6 +797,14 @@ struct Engine {
                 rkey.as<uint64_t>());
             HP_LAUNCHED();
         }
+        if (H == 1) {
+            k_root_one<<<1, 256, 0, s>>>(hfirst.as<int64_t>(), hcount.as<int64_t>(),
+                                         box.as<int32_t>(), bad.as<int32_t>(), A.as<float4>(),
+                                         badlist.as<int32_t>(), depth_buf.as<int32_t>(),
+                                         build_args(small0.as<Task>()));
+            HP_LAUNCHED();
+            return HP_OK;
+        }
         if (H > 0) {
             k_roots<<<blocks(H, 256), 256, 0, s>>>(hfirst.as<int64_t>(), hcount.as<int64_t>(),
                                                    box.as<int32_t>(), bad.as<int32_t>(),
@@ -863,19 +871,20 @@ struct Engine {
         // and the largest call.  Largest first: the big subtrees hold most
         // points and the fewest workgroups per CU.
         const int64_t gmax = std::min<int64_t>(max_count, big_max());
-        if (gmax > kWaveMin) {
-            k_group_classes<<<blocks(cap_group, 256), 256, 0, s>>>(group0.as<Task>(), ba,
-                                                                   groupc.as<Task>());
-            HP_LAUNCHED();
-        }
         {  // the wavefront subtrees' node ids: exclusive scan of 2n - 2 over the list
             const int32_t m = (int32_t)cap_small + 1;
             const int32_t nbk = (m + kScanBlock - 1) / kScanBlock;
             int32_t *off = wave_off.as<int32_t>();
             if (nbk == 1) {
-                k_wave_ids_one<<<1, 1024, 0, s>>>(small0.as<Task>(), ba, off, m);
+                k_task_ids_one<<<1, 1024, 0, s>>>(gmax > kWaveMin ? group0.as<Task>() : nullptr,
+                                                  groupc.as<Task>(), small0.as<Task>(), ba, off, m);
                 HP_LAUNCHED();
             } else {
+                if (gmax > kWaveMin) {
+                    k_group_classes<<<blocks(cap_group, 256), 256, 0, s>>>(group0.as<Task>(), ba,
+                                                                           groupc.as<Task>());
+                    HP_LAUNCHED();
+                }
                 k_wave_need<<<std::min(blocks(m, 256), 4096), 256, 0, s>>>(small0.as<Task>(), ba,
                                                                            off, m);
                 HP_LAUNCHED();

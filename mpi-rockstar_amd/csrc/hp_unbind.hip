@@ -146,11 +146,20 @@ __global__ __launch_bounds__(1024) void k_scan_add(int32_t *__restrict__ v, int3
         if (base + k < m) v[base + k] += add;
 }
 
-// The wavefront subtrees' node ids (k_wave_need, the scan and k_wave_base)
-// in one launch, for a list of at most kScanBlock entries (a small batch or
-// one call): off[k] = the ids of the tasks before k.
-__global__ __launch_bounds__(1024) void k_wave_ids_one(const Task *__restrict__ tasks, BuildArgs a,
+// k_group_classes (with `group`), then the wavefront subtrees' node ids
+// (k_wave_need, the scan and k_wave_base) in one launch, for a wavefront list
+// of at most kScanBlock entries (a small batch or one call): off[k] = the ids
+// of the tasks before k.
+__global__ __launch_bounds__(1024) void k_task_ids_one(const Task *__restrict__ group,
+                                                       Task *__restrict__ groupc,
+                                                       const Task *__restrict__ tasks, BuildArgs a,
                                                        int32_t *__restrict__ off, int32_t m) {
+    if (group) {
+        const int32_t n = min(a.counters[kGroupNext], a.cap_group);
+        for (int32_t k = threadIdx.x; k - lane_id() < n; k += 1024) group_class(k, n, group, a, groupc);
+        __threadfence();
+        __syncthreads();
+    }
     const int32_t ntasks = min(a.counters[kSmallNext], a.cap_small);
     const int32_t base = threadIdx.x * 4;
     int32_t x[4], s = 0;
@@ -166,7 +175,9 @@ __global__ __launch_bounds__(1024) void k_wave_ids_one(const Task *__restrict__ 
         o += x[k];
     }
     if (threadIdx.x == 0) {
-        const int32_t base0 = a.counters[kNodeCount];
+        // (the classes' ids are taken by then, by atomics of this launch)
+        const int32_t base0 = __hip_atomic_load(a.counters + kNodeCount, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
         a.counters[kWaveIdBase] = base0;
         a.counters[kNodeCount] = base0 + tot;
     }
