@@ -2501,10 +2501,10 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
         // the nodes of at most kFuseMax points, each finished by one workgroup
         const int32_t nf = na[kSfFused];
         if (nf > 0) {
-            k_sub_fused<<<(uint32_t)nf, kSfThreads, 0, s>>>(B.nodes.as<Node6>(), fused,
-                                                           B.w.as<SParticle>(),
-                                                           B.w2.as<SParticle>(), cnt,
-                                                           (int32_t)node_cap);
+            k_sub_fused<<<(uint32_t)nf, kFuseThreads, 0, s>>>(B.nodes.as<Node6>(), fused,
+                                                             B.w.as<SParticle>(),
+                                                             B.w2.as<SParticle>(), cnt,
+                                                             (int32_t)node_cap);
             HP_LAUNCHED();
         }
         // the nodes there are, or, of few points, could be

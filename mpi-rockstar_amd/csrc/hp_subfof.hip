@@ -351,8 +351,9 @@ __device__ __forceinline__ int block_rank(bool b, int *total, int *s_w) {
 
 // K and S of the closed form (file header) for one partition; b and r are
 // the positions of the bigs in order and of the smalls in order
-__device__ void partition_ks(const int32_t *__restrict__ bpos, const int32_t *__restrict__ spos,
-                             int32_t n, int32_t nbig, int32_t nsmall, int32_t *K, int32_t *S) {
+template <class T>
+__device__ void partition_ks(const T *__restrict__ bpos, const T *__restrict__ spos, int32_t n,
+                             int32_t nbig, int32_t nsmall, int32_t *K, int32_t *S) {
     // b_k = bpos[k - 1]; r_k = spos[nsmall - k]; b_k < r_k holds for k <= K
     int32_t lo = 0, hi = min(nbig, nsmall);
     while (lo < hi) {
@@ -386,10 +387,11 @@ __device__ void partition_ks_wave(const int32_t *__restrict__ bpos,
 
 // destination of the element at p (class big, rank among its class) in the
 // closed form
+template <class T>
 __device__ __forceinline__ int32_t partition_dest(int32_t p, bool big, int32_t rank, int32_t n,
                                                   int32_t nsmall, int32_t S,
-                                                  const int32_t *__restrict__ bpos,
-                                                  const int32_t *__restrict__ spos) {
+                                                  const T *__restrict__ bpos,
+                                                  const T *__restrict__ spos) {
     // the clamps never bind for a partition the form describes; they keep
     // every read inside the node's lists whatever the input
     if (p < S) {
@@ -545,16 +547,30 @@ __global__ __launch_bounds__(NT) void k_sub_split(
     if (R.n > kLeaf6) push_active(l + 1, R.n, next, next_big, counters, level + 1, fused);
 }
 
+// v reduced over the lane's row of 16 (the row's lanes active)
+template <typename T, typename Op>
+__device__ __forceinline__ T row_reduce(T v, Op op) {
+    v = op(v, dpp_move<0xB1>(v));   // quad_perm [1, 0, 3, 2]
+    v = op(v, dpp_move<0x4E>(v));   // quad_perm [2, 3, 0, 1]
+    v = op(v, dpp_move<0x141>(v));  // row_half_mirror
+    return op(v, dpp_move<0x140>(v));  // row_mirror
+}
+
 // A node of at most kFuseMax points is split down to its leaves by one
 // workgroup, in LDS, all nodes of a level at once: the coordinates stay in
 // place and a permutation of local positions moves; one block-wide scan
-// ranks every node's points, one thread per node finds its K and S, the
-// children's boxes come from atomic min/max on order-preserving keys.  The
-// same splits as k_sub_split, node for node; the particles are written once,
-// to the other buffer, at the end.
+// ranks every node's points, one thread per node finds its K and S.  The
+// children's boxes come from atomic min/max on order-preserving keys, over
+// the points in their new order: there a row of 16 lanes mostly lies in one
+// child, and its lanes are reduced before one of them goes to the atomics
+// (twelve atomics a point took 2.78 ms on 7.2M particles; with 512 threads and
+// the entries compacted by a wavefront too, now 1.29).  The same splits as
+// k_sub_split, node for node; the particles are written once, to the other
+// buffer, at the end.
 constexpr int kFuseMax = kFuseMaxNode;
 constexpr int kFuseList = 2 * (kFuseMax / (kLeaf6 + 1)) + 2;  // nodes of one level
-constexpr int kFusePer = kFuseMax / kSfThreads;                // positions per thread
+constexpr int kFuseThreads = 512;
+constexpr int kFusePer = kFuseMax / kFuseThreads;              // positions per thread
 constexpr uint8_t kFuseDone = 0xff;
 static_assert(kFuseList < kFuseDone, "level entries fit a byte");
 
@@ -568,20 +584,20 @@ struct FuseNode {
     int32_t child;     // first of the children's entries in the next list, -1: none
 };
 
-__global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ nodes,
-                                                          const int32_t *__restrict__ roots,
-                                                          SParticle *__restrict__ wa,
-                                                          SParticle *__restrict__ wb,
-                                                          int32_t *__restrict__ counters,
-                                                          int32_t node_cap) {
+__global__ __launch_bounds__(kFuseThreads) void k_sub_fused(Node6 *__restrict__ nodes,
+                                                            const int32_t *__restrict__ roots,
+                                                            SParticle *__restrict__ wa,
+                                                            SParticle *__restrict__ wb,
+                                                            int32_t *__restrict__ counters,
+                                                            int32_t node_cap) {
     __shared__ float X[6][kFuseMax];
     __shared__ int16_t I[2][kFuseMax];
     __shared__ uint8_t NO[2][kFuseMax];
-    __shared__ int32_t SC[kFuseMax + 1];
-    __shared__ int32_t BP[kFuseMax], SP[kFuseMax];
+    __shared__ int16_t SC[kFuseMax + 1];
+    __shared__ int16_t BP[kFuseMax], SP[kFuseMax];
     __shared__ FuseNode E[2][kFuseList];
-    __shared__ int32_t BK[kFuseList][2][12];
-    __shared__ int s_w[kSfThreads / kWave];
+    __shared__ int32_t BK[kFuseList][12];  // by child entry
+    __shared__ int s_w[kFuseThreads / kWave];
     __shared__ int32_t s_cnt[2], s_g0;
     const int tid = threadIdx.x;
     if ((int32_t)blockIdx.x >= counters[kSfFused]) return;
@@ -591,7 +607,7 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
     const SParticle *__restrict__ src = rn.where ? wb : wa;
     SParticle *__restrict__ dst = rn.where ? wa : wb;
     const int32_t wnew = 1 - rn.where;  // the buffer the subtree's points end in
-    for (int32_t p = tid; p < N; p += kSfThreads) {
+    for (int32_t p = tid; p < N; p += kFuseThreads) {
         const SParticle q = src[s0 + p];
         for (int k = 0; k < 6; k++) X[k][p] = q.pos[k];
         I[0][p] = (int16_t)p;
@@ -632,8 +648,8 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
             e.child = -1;
         }
         if (tid == 0) s_cnt[nxt] = 0;
-        for (int x = tid; x < kFuseList * 24; x += kSfThreads)
-            (&BK[0][0][0])[x] = (x % 12) < 6 ? 0x7fffffff : (int32_t)0x80000000;
+        for (int x = tid; x < kFuseList * 12; x += kFuseThreads)
+            (&BK[0][0])[x] = (x % 12) < 6 ? 0x7fffffff : (int32_t)0x80000000;
         __syncthreads();
         // 2. classes and one scan of the bigs over every position
         int32_t cnt_local = 0;
@@ -660,10 +676,10 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
         int32_t run = off + incl - cnt_local;
         for (int r = 0; r < kFusePer; r++) {
             const int32_t p = tid * kFusePer + r;
-            if (p < N) SC[p] = run;
+            if (p < N) SC[p] = (int16_t)run;
             run += bigv[r] ? 1 : 0;
         }
-        if (tid == kSfThreads - 1) SC[N] = run;  // the last thread ends with the total
+        if (tid == kFuseThreads - 1) SC[N] = (int16_t)run;  // the last thread ends with the total
         __syncthreads();
         // 3. ranks within the node and the two position lists
         for (int r = 0; r < kFusePer; r++) {
@@ -675,8 +691,8 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
             if (e.dim < 0) continue;
             const int32_t rel = p - e.start;
             const int32_t rb = SC[p] - SC[e.start];
-            if (bigv[r]) BP[e.start + rb] = rel;
-            else SP[e.start + (rel - rb)] = rel;
+            if (bigv[r]) BP[e.start + rb] = (int16_t)rel;
+            else SP[e.start + (rel - rb)] = (int16_t)rel;
         }
         __syncthreads();
         // 4. each node: K and S, its children's entries and global ids
@@ -702,9 +718,9 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
             }
         }
         __syncthreads();
-        // 5. every position of a splitting node to its place, the children's
-        //    boxes; the level's children take their global ids with one atomic
-        //    (child slot c is node s_g0 + c)
+        // 5. every position of a splitting node to its place; the level's
+        //    children take their global ids with one atomic (child slot c is
+        //    node s_g0 + c)
         if (tid == 0) {
             const int32_t nc = s_cnt[nxt];
             int32_t g0 = nc ? atomicAdd(&counters[kSfNodes], nc) : 0;
@@ -741,14 +757,34 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
                 NO[nxt][q] = kFuseDone;
                 continue;
             }
-            const int side = d < e.nsmall ? 0 : 1;
-            const int32_t ce = e.child + side;
-            const int32_t cn = side ? e.n - e.nsmall : e.nsmall;
-            NO[nxt][q] = cn > kLeaf6 ? (uint8_t)ce : kFuseDone;
-            for (int k = 0; k < 6; k++) {
-                const int32_t key = float_key(X[k][id]);
-                atomicMin(&BK[en][side][k], key);
-                atomicMax(&BK[en][side][6 + k], key);
+            NO[nxt][q] = (uint8_t)(e.child + (d < e.nsmall ? 0 : 1));
+        }
+        __syncthreads();
+        // the children's boxes
+        for (int r = 0; r < kFusePer; r++) {
+            const int32_t p = r * kFuseThreads + tid;
+            const int32_t ce = p < N ? NO[nxt][p] : kFuseDone;
+            const bool in = ce != kFuseDone;
+            int32_t key[6];
+            if (in) {
+                const int16_t id = I[nxt][p];
+                for (int k = 0; k < 6; k++) key[k] = float_key(X[k][id]);
+            }
+            const uint64_t same = ballot(in && ce == dpp_move<0x150>(ce));  // as the row's lane 0
+            if ((uint16_t)(same >> (lane_id() & 48)) == 0xffff) {
+                for (int k = 0; k < 6; k++) {
+                    const int32_t lo = row_reduce(key[k], [](int32_t a, int32_t b) { return min(a, b); });
+                    const int32_t hi = row_reduce(key[k], [](int32_t a, int32_t b) { return max(a, b); });
+                    if ((lane_id() & 15) == 0) {
+                        atomicMin(&BK[ce][k], lo);
+                        atomicMax(&BK[ce][6 + k], hi);
+                    }
+                }
+            } else if (in) {
+                for (int k = 0; k < 6; k++) {
+                    atomicMin(&BK[ce][k], key[k]);
+                    atomicMax(&BK[ce][6 + k], key[k]);
+                }
             }
         }
         __syncthreads();
@@ -765,8 +801,8 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
                 for (int c = 0; c < 2; c++) {
                     FuseNode &ce = E[nxt][e.child + c];
                     for (int k = 0; k < 6; k++) {
-                        ce.lo[k] = key_float(BK[tid][c][k]);
-                        ce.hi[k] = key_float(BK[tid][c][6 + k]);
+                        ce.lo[k] = key_float(BK[e.child + c][k]);
+                        ce.hi[k] = key_float(BK[e.child + c][6 + k]);
                         C[c].lo[k] = ce.lo[k];
                         C[c].hi[k] = ce.hi[k];
                     }
@@ -792,22 +828,28 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
         __syncthreads();
         // the next level holds only the children of more than kLeaf6 points:
         // compact the entries, renumbering the positions' entries
-        if (tid == 0) {
-            int32_t m = 0;
+        if (tid < kWave) {
+            static_assert(kFuseList <= kWave, "a lane per entry");
             const int32_t nn2 = s_cnt[nxt];
-            for (int32_t c = 0; c < nn2; c++) {
-                if (E[nxt][c].n > kLeaf6 && s_g0 >= 0) {
-                    if (m != c) E[nxt][m] = E[nxt][c];
-                    BP[c] = m;  // old entry -> new entry (BP is free here)
-                    m++;
-                } else {
-                    BP[c] = -1;
-                }
+            constexpr int kWords = sizeof(FuseNode) / 4;
+            int32_t e[kWords];
+            const int32_t *from = reinterpret_cast<const int32_t *>(&E[nxt][min(tid, kFuseList - 1)]);
+#pragma unroll
+            for (int k = 0; k < kWords; k++) e[k] = from[k];
+            const bool keep = tid < nn2 && E[nxt][tid].n > kLeaf6 && s_g0 >= 0;
+            const uint64_t m = ballot(keep);
+            const int32_t to = rank_below(m);
+            if (tid < nn2) BP[tid] = (int16_t)(keep ? to : -1);  // old entry -> new (BP is free here)
+            wave_sync();
+            int32_t *into = reinterpret_cast<int32_t *>(&E[nxt][to]);
+            if (keep) {
+#pragma unroll
+                for (int k = 0; k < kWords; k++) into[k] = e[k];
             }
-            s_cnt[nxt] = m;
+            if (tid == 0) s_cnt[nxt] = __popcll(m);
         }
         __syncthreads();
-        for (int32_t p = tid; p < N; p += kSfThreads) {
+        for (int32_t p = tid; p < N; p += kFuseThreads) {
             const uint8_t en = NO[nxt][p];
             if (en != kFuseDone) NO[nxt][p] = (uint8_t)BP[en];
         }
@@ -815,7 +857,7 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_fused(Node6 *__restrict__ no
         cur = nxt;
     }
     // the particles in their final order, to the other buffer
-    for (int32_t k = tid; k < N; k += kSfThreads) dst[s0 + k] = src[s0 + I[cur][k]];
+    for (int32_t k = tid; k < N; k += kFuseThreads) dst[s0 + k] = src[s0 + I[cur][k]];
 }
 
 // after the build: the leaves whose points the last write left in the
@@ -1055,15 +1097,6 @@ __device__ __forceinline__ float box_gap2(const Box6 &x, const float *lo, const 
         d += e * e;
     }
     return d;
-}
-
-// v reduced over the lane's row of 16 (all lanes active)
-template <typename T, typename Op>
-__device__ __forceinline__ T row_reduce(T v, Op op) {
-    v = op(v, dpp_move<0xB1>(v));   // quad_perm [1, 0, 3, 2]
-    v = op(v, dpp_move<0x4E>(v));   // quad_perm [2, 3, 0, 1]
-    v = op(v, dpp_move<0x141>(v));  // row_half_mirror
-    return op(v, dpp_move<0x140>(v));  // row_mirror
 }
 
 // A wavefront's queries: four rows of 16 lanes, one per column tile of the
