@@ -166,16 +166,25 @@ template <int CTRL>
 __device__ __forceinline__ int dpp_i32(int v) {
     return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
 }
+// the same into the rows of ROWS only; the others get 0
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_rows_i32(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
 
-template <int CTRL, typename T>
+template <int CTRL, int ROWS = 0xf, typename T>
 __device__ __forceinline__ T dpp_move(T v) {
     static_assert(sizeof(T) == 4 || sizeof(T) == 8, "32- or 64-bit lanes");
+    auto move = [](int x) {
+        if constexpr (ROWS == 0xf) return dpp_i32<CTRL>(x);
+        else return dpp_rows_i32<CTRL, ROWS>(x);
+    };
     if constexpr (sizeof(T) == 4) {
-        return __builtin_bit_cast(T, dpp_i32<CTRL>(__builtin_bit_cast(int, v)));
+        return __builtin_bit_cast(T, move(__builtin_bit_cast(int, v)));
     } else {
         const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        const uint32_t lo = (uint32_t)dpp_i32<CTRL>((int)(uint32_t)u);
-        const uint32_t hi = (uint32_t)dpp_i32<CTRL>((int)(uint32_t)(u >> 32));
+        const uint32_t lo = (uint32_t)move((int)(uint32_t)u);
+        const uint32_t hi = (uint32_t)move((int)(uint32_t)(u >> 32));
         return __builtin_bit_cast(T, ((uint64_t)hi << 32) | lo);
     }
 }
@@ -202,24 +211,17 @@ __device__ __forceinline__ T wave_reduce(T v, Op op) {
 }
 
 // Inclusive prefix sum over the lanes of a wavefront, on DPP moves: row_shr
-// 1, 2, 4, 8 within rows of 16, then row_bcast 15 and 31 across rows.  Call
-// with all 64 lanes active.
+// 1, 2, 4, 8 within rows of 16, then row_bcast 15 and 31 across rows.  A lane
+// without a source adds 0 (so a sum of -0 alone comes out as 0): no selects.
+// Call with all 64 lanes active.
 template <typename T>
 __device__ __forceinline__ T wave_scan_add(T v) {
-    const int lane = lane_id(), r = lane & 15;
-    T u;
-    u = dpp_move<0x111>(v);
-    if (r >= 1) v = v + u;
-    u = dpp_move<0x112>(v);
-    if (r >= 2) v = v + u;
-    u = dpp_move<0x114>(v);
-    if (r >= 4) v = v + u;
-    u = dpp_move<0x118>(v);
-    if (r >= 8) v = v + u;
-    u = dpp_move<0x142>(v);  // row_bcast:15, rows 1 and 3
-    if ((lane >> 4) & 1) v = v + u;
-    u = dpp_move<0x143>(v);  // row_bcast:31, rows 2 and 3
-    if (lane >= 32) v = v + u;
+    v = v + dpp_move<0x111>(v);
+    v = v + dpp_move<0x112>(v);
+    v = v + dpp_move<0x114>(v);
+    v = v + dpp_move<0x118>(v);
+    v = v + dpp_move<0x142, 0xa>(v);  // row_bcast:15, rows 1 and 3
+    v = v + dpp_move<0x143, 0xc>(v);  // row_bcast:31, rows 2 and 3
     return v;
 }
 
