@@ -28,9 +28,9 @@
 // by the scalar unit.
 //
 // What bounds it: issue.  Of the cycles of a 6.7M-record batch's walk 92% hold
-// a vector instruction (33 a node visit) and 77% a scalar one or a branch (29
-// a visit), of 93% and 79% before the accumulator and the loop's state were
-// kept in place (36 and 33 a visit, 1.64 ms; now 1.51).  Both units count: an
+// a vector instruction (31 a node visit) and 77% a scalar one (24 a visit) or a
+// branch, of 93% and 79% before the accumulator and the loop's state were kept
+// in place (36 and 26 a visit, 1.64 ms; now 1.51).  Both units count: an
 // acceptance test in float with a scalar fallback (3 vector instructions
 // less, 8 scalar ones more) and a scalar test of the node's range (2 less, 4
 // more) made the walk 7 and 6% slower.
