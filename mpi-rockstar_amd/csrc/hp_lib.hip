@@ -2538,13 +2538,31 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
             B.pk.as<PackPoint>(), B.chunks.as<Box6>(), B.cblocks.as<Box6>(),
             B.dist.as<float>(), cfg.ordered_search, qlanes);
         HP_LAUNCHED();
-        HP_TRY(hipMemcpyAsync(B.sel.p, B.dist.p, sizeof(float) * S, hipMemcpyDeviceToDevice, s));
     }
-    k_sub_median<<<(uint32_t)ng, kSfThreads, 0, s>>>(dg, thresh, B.sel.as<float>(),
-                                                      B.sel2.as<float>(), B.rk.as<int32_t>(),
-                                                      B.bpos.as<int32_t>(), B.spos.as<int32_t>(),
-                                                      B.target.as<float>());
-    HP_LAUNCHED();
+    int32_t nsmin = INT32_MAX, nsmax = 0;
+    for (const SubGroup &sg : G) {
+        nsmin = std::min(nsmin, sg.nsample);
+        nsmax = std::max(nsmax, sg.nsample);
+    }
+    if (nsmin <= kMedSmall) {
+        k_sub_median_lds<256, kMedSmall><<<(uint32_t)ng, 256, 0, s>>>(
+            dg, 0, B.dist.as<float>(), B.target.as<float>());
+        HP_LAUNCHED();
+    }
+    if (nsmax > kMedSmall) {
+        k_sub_median_lds<1024, kMedLarge><<<(uint32_t)ng, 1024, 0, s>>>(
+            dg, kMedSmall, B.dist.as<float>(), B.target.as<float>());
+        HP_LAUNCHED();
+    }
+    if (nsmax > kMedLarge) {
+        HP_TRY(hipMemcpyAsync(B.sel.p, B.dist.p, sizeof(float) * S, hipMemcpyDeviceToDevice, s));
+        k_sub_median<<<(uint32_t)ng, kSfThreads, 0, s>>>(dg, thresh, B.sel.as<float>(),
+                                                          B.sel2.as<float>(), B.rk.as<int32_t>(),
+                                                          B.bpos.as<int32_t>(),
+                                                          B.spos.as<int32_t>(),
+                                                          B.target.as<float>());
+        HP_LAUNCHED();
+    }
     // the linking, the reference's numbers and roots, then its output order
     if (M) {
         const int32_t m = (int32_t)M;

@@ -368,9 +368,9 @@ __device__ void partition_ks(const T *__restrict__ bpos, const T *__restrict__ s
 
 // The same by a whole wavefront, in every lane: 64 candidates a step (a level
 // of 16,000 points 15.5 us against 18.6 by halves, each a dependent read).
-__device__ void partition_ks_wave(const int32_t *__restrict__ bpos,
-                                  const int32_t *__restrict__ spos,
-                                  int32_t n, int32_t nbig, int32_t nsmall, int32_t *K, int32_t *S) {
+template <class T>
+__device__ void partition_ks_wave(const T *__restrict__ bpos, const T *__restrict__ spos, int32_t n,
+                                  int32_t nbig, int32_t nsmall, int32_t *K, int32_t *S) {
     // b_k = bpos[k - 1]; r_k = spos[nsmall - k]; b_k < r_k holds for k <= K
     int32_t lo = 0, hi = min(nbig, nsmall);
     while (lo < hi) {
@@ -1375,10 +1375,133 @@ __global__ __launch_bounds__(kWave) void k_sub_next_closest(
 
 // ------------------------------------------------------ linking length
 
+// exclusive prefix sum over the workgroup's threads, and the total
+template <int NT>
+__device__ __forceinline__ int block_excl_scan(int x, int *total, int *s_w) {
+    constexpr int NW = NT / kWave;
+    const int incl = wave_scan_add(x);
+    const int wv = threadIdx.x / kWave;
+    if (lane_id() == kWave - 1) s_w[wv] = incl;
+    __syncthreads();
+    int off = 0, tot = 0;
+    for (int j = 0; j < NW; j++) {
+        off += j < wv ? s_w[j] : 0;
+        tot += s_w[j];
+    }
+    __syncthreads();
+    *total = tot;
+    return off + incl - x;
+}
+
 // find_median_r (src/groupies.c:744-786) per group, one workgroup: the
 // reference's quickselect step by step, each rad_partition evaluated in
-// parallel with the closed form; buf holds the distances (a copy), buf2,
-// rk, bpos and spos are scratch of the same extent
+// parallel with the closed form.  A sample of at most CAP values (and more
+// than `above`) is held in LDS, each thread's share of the range in
+// registers while a partition moves it: a step is a scan, a search of K and a
+// scatter in LDS.  With the lists in global memory the 10,000 values of one
+// group took 110 us; now 54.
+constexpr int kMedSmall = 2048;
+constexpr int kMedLarge = 10240;
+static_assert(kSampleMax <= kMedLarge, "a drawn sample fits");
+template <int NT, int CAP>
+__global__ __launch_bounds__(NT) void k_sub_median_lds(const SubGroup *__restrict__ groups,
+                                                       int32_t above,
+                                                       const float *__restrict__ dist,
+                                                       float *__restrict__ target) {
+    constexpr int kPer = CAP / NT;
+    static_assert(kPer * NT == CAP && CAP <= 65536, "shares of the range; 16-bit positions");
+    __shared__ float v[CAP];
+    __shared__ uint16_t bp[CAP], sp[CAP];
+    __shared__ int s_w[NT / kWave];
+    __shared__ int32_t s_v[4];
+    __shared__ float s_piv;
+    const SubGroup g = groups[blockIdx.x];
+    const int32_t ns = g.nsample, tid = threadIdx.x;
+    if (ns < 1 && above == 0 && tid == 0) target[blockIdx.x] = 0.0f;
+    if (ns <= above || ns > CAP) return;
+    for (int32_t p = tid; p < ns; p += NT) v[p] = dist[g.sample_off + p];
+    __syncthreads();
+    const int32_t k = g.k;
+    uint32_t seed = g.seed;  // thread 0's copy is the live one
+    int32_t left = 0, right = ns;
+    while (ns > 1) {
+        if (tid == 0) {
+            const float u = (float)(rand_r_glibc(&seed) % 2147483647) / (float)2147483647;
+            const float at_f = (float)left + u * (float)(right - left);
+            // u rounds to 1.0f for the top 63 of 2^31 draws; the reference
+            // then reads one past the range, here the last slot is taken
+            const int32_t at = min((int32_t)at_f, right - 1);
+            const float pv = v[at];
+            v[at] = v[right - 1];
+            v[right - 1] = pv;
+            s_piv = pv;
+        }
+        __syncthreads();
+        const float pv = s_piv;
+        const int32_t m = right - 1 - left;  // the loop's range [left, right - 1)
+        const int32_t per = (m + NT - 1) / NT, p0 = tid * per;
+        float x[kPer];
+        uint32_t big = 0;
+#pragma unroll
+        for (int j = 0; j < kPer; j++) {
+            const bool in = j < per && p0 + j < m;
+            x[j] = in ? v[left + p0 + j] : 0.0f;
+            big |= in && x[j] > pv ? 1u << j : 0u;
+        }
+        int nbig;
+        const int32_t run0 = block_excl_scan<NT>(__popc(big), &nbig, s_w);
+        const int32_t nsmall = m - nbig;
+        int32_t run = run0;  // bigs before the position
+#pragma unroll
+        for (int j = 0; j < kPer; j++) {
+            const int32_t p = p0 + j;
+            if (j >= per || p >= m) break;
+            if (big >> j & 1) bp[run++] = (uint16_t)p;
+            else sp[p - run] = (uint16_t)p;
+        }
+        __syncthreads();
+        if (tid < kWave) {
+            int32_t K, S;
+            partition_ks_wave(bp, sp, m, nbig, nsmall, &K, &S);
+            s_v[0] = S;
+        }
+        __syncthreads();
+        const int32_t S = s_v[0];
+        run = run0;
+#pragma unroll
+        for (int j = 0; j < kPer; j++) {
+            const int32_t p = p0 + j;
+            if (j >= per || p >= m) break;
+            const bool b = big >> j & 1;
+            v[left + partition_dest(p, b, b ? run : p - run, m, nsmall, S, bp, sp)] = x[j];
+            run += b ? 1 : 0;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            // rad_partition's end: the pivot moves to the first slot above it
+            const int32_t si = left + nsmall;
+            const float t = v[right - 1];
+            v[right - 1] = v[si];
+            v[si] = t;
+            int32_t done = 0;
+            if (k == si || v[left] == v[right - 1]) done = 1;
+            else if (k < si) right = si;
+            else left = si + 1;
+            s_v[1] = done;
+            s_v[2] = left;
+            s_v[3] = right;
+        }
+        __syncthreads();
+        if (s_v[1]) break;
+        left = s_v[2];
+        right = s_v[3];
+    }
+    if (tid == 0) target[blockIdx.x] = ns > 1 ? v[k] : v[0];
+}
+
+// The same for a larger sample (every particle of a group, exact_ll_calc), in
+// global memory; buf holds the distances (a copy), buf2, rk, bpos and spos
+// are scratch of the same extent.
 __global__ __launch_bounds__(kSfThreads) void k_sub_median(
     const SubGroup *__restrict__ groups, float frac, float *__restrict__ buf,
     float *__restrict__ buf2, int32_t *__restrict__ rk, int32_t *__restrict__ bpos,
@@ -1388,17 +1511,10 @@ __global__ __launch_bounds__(kSfThreads) void k_sub_median(
     __shared__ float s_piv;
     const SubGroup g = groups[blockIdx.x];
     const int32_t ns = g.nsample;
-    if (ns < 1) {
-        if (threadIdx.x == 0) target[blockIdx.x] = 0.0f;
-        return;
-    }
+    if (ns <= kMedLarge) return;  // k_sub_median_lds
     float *v = buf + g.sample_off;
     float *v2 = buf2 + g.sample_off;
     int32_t *rko = rk + g.sample_off, *bp = bpos + g.sample_off, *sp = spos + g.sample_off;
-    if (ns < 2) {
-        if (threadIdx.x == 0) target[blockIdx.x] = v[0];
-        return;
-    }
     const int32_t k = g.k;
     uint32_t seed = g.seed;  // thread 0's copy is the live one
     int32_t left = 0, right = ns;
@@ -1955,24 +2071,6 @@ __global__ void k_sort_roots(int32_t ng, const SubGroup *__restrict__ groups,
     if (g.n >= 2)
         push_range(SortRange{g.off, g.n, 0, 1, 0, 0}, next, small, counters, 0, cap_next,
                    cap_small);
-}
-
-// exclusive prefix sum over the workgroup's threads, and the total
-template <int NT>
-__device__ __forceinline__ int block_excl_scan(int x, int *total, int *s_w) {
-    constexpr int NW = NT / kWave;
-    const int incl = wave_scan_add(x);
-    const int wv = threadIdx.x / kWave;
-    if (lane_id() == kWave - 1) s_w[wv] = incl;
-    __syncthreads();
-    int off = 0, tot = 0;
-    for (int j = 0; j < NW; j++) {
-        off += j < wv ? s_w[j] : 0;
-        tot += s_w[j];
-    }
-    __syncthreads();
-    *total = tot;
-    return off + incl - x;
 }
 
 template <int NT>

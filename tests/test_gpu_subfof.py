@@ -214,6 +214,26 @@ def test_gpu_subfof_chunk_edges(restatement, spread):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("exact_ll,sizes", [
+    (0, (1, 2, 3, 0, 2047, 2048, 2049, 10000, 10001)),  # every particle, or 10,000 drawn
+    (1, (10240, 10241, 2048, 257)),                     # every particle
+])
+def test_gpu_subfof_sample_sizes(restatement, exact_ll, sizes):
+    """find_median_r's samples at the sizes between which it is done in other
+    ways; half of the points on a lattice, so that distances repeat."""
+    rng = np.random.default_rng(12)
+    plist = []
+    for n in sizes:
+        x = rng.normal(size=(n, 6))
+        x[: n // 2] = rng.integers(-3, 4, (n // 2, 6)) * 0.25
+        p = np.zeros(n, catalog.PARTICLE_DTYPE)
+        p["id"] = np.arange(n)
+        p["pos"] = np.round(x * 4096) / 4096
+        plist.append(p)
+    _check_batch(restatement, plist, exact_ll=exact_ll)
+
+
+@pytest.mark.gpu
 def test_gpu_subfof_exact_ll_and_lower_levels(restatement):
     fg = catalog.fof_groups(seed=5, n_groups=6, lo=300, hi=12000)
     plist = [fg.particles[f:f + n].copy() for f, n in fg.groups]
