@@ -1732,7 +1732,9 @@ __global__ __launch_bounds__(kWave) void k_sub_link(const SubGroup *__restrict__
 }
 
 // the lists in place (off: exclusive scan of the counts) and each
-// particle's earliest earlier neighbour
+// particle's earliest earlier neighbour.  kmin only falls, so a step that does
+// not lie below the value read, however old, needs no atomic; the list is
+// nearly in step order, and few need one (4,000 groups 0.66 to 0.505 ms).
 __global__ void k_sub_adjacent(int64_t ne, const EdgeRec *__restrict__ edges,
                                const int32_t *__restrict__ off, int32_t *__restrict__ adj,
                                int32_t *__restrict__ kmin) {
@@ -1740,7 +1742,8 @@ __global__ void k_sub_adjacent(int64_t ne, const EdgeRec *__restrict__ edges,
     if (e >= ne) return;
     const EdgeRec r = edges[e];
     adj[off[r.i] + r.rank] = r.j;
-    atomicMin(kmin + r.j, r.i);
+    if (__hip_atomic_load(kmin + r.j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > r.i)
+        atomicMin(kmin + r.j, r.i);
 }
 
 // the step whose small FOF each particle takes (-1: never listed; a creating
@@ -1797,6 +1800,11 @@ __global__ void k_sub_label(int32_t m, int32_t *__restrict__ par,
 }
 
 constexpr int32_t kEventDedup = 64;
+// list entries whose neighbours' steps and numbers are read at once: a thread
+// waits for one read of the list and two of the particles per 8 entries
+// instead of per entry (4,000 groups 0.734 ms entry by entry, 0.486 by fours,
+// 0.460 by eights)
+constexpr int kEventAhead = 8;
 
 // The pairs of step i that can merge, (i's number, x's number) for each
 // listed x numbered before step i under another number, in list order.  A
@@ -1817,16 +1825,26 @@ __global__ void k_sub_events(int32_t m, const int32_t *__restrict__ off,
     int32_t k = 0;
     if (e1 > e0) {
         const int32_t f = lab[i];
-        for (int32_t e = e0; e < e1; e++) {
-            const int32_t x = adj[e];
-            if (kmin[x] >= i) continue;
-            const int32_t lx = lab[x];
-            if (lx == f) continue;
-            // checked against the step's first kEventDedup pairs only: a
-            // repeat kept past them is one more pair that cannot merge
-            bool seen = false;
-            for (int32_t q = 0; q < min(k, kEventDedup) && !seen; q++) seen = stage[e0 + q].y == lx;
-            if (!seen) stage[e0 + k++] = make_int2(f, lx);
+        int32_t last = f;  // (f itself is no pair)
+        for (int32_t e = e0; e < e1; e += kEventAhead) {
+            int32_t kx[kEventAhead], lx[kEventAhead];
+#pragma unroll
+            for (int t = 0; t < kEventAhead; t++) {
+                const int32_t x = adj[min(e + t, e1 - 1)];
+                kx[t] = kmin[x];
+                lx[t] = lab[x];
+            }
+#pragma unroll
+            for (int t = 0; t < kEventAhead; t++) {
+                if (e + t >= e1 || kx[t] >= i || lx[t] == f || lx[t] == last) continue;
+                last = lx[t];
+                // checked against the step's first kEventDedup pairs only: a
+                // repeat kept past them is one more pair that cannot merge
+                bool seen = false;
+                for (int32_t q = 0; q < min(k, kEventDedup) && !seen; q++)
+                    seen = stage[e0 + q].y == lx[t];
+                if (!seen) stage[e0 + k++] = make_int2(f, lx[t]);
+            }
         }
     }
     ecnt[i] = k;
