@@ -1346,12 +1346,10 @@ __global__ __launch_bounds__(kWave) void k_sub_next_closest(
                     const int t = __builtin_ctzll(may);
                     may &= may - 1;
                     const float d = dist6(c, w[base + t]);
-                    if (d < m1) {
-                        m2 = m1;
-                        m1 = d;
-                    } else if (d > m1 && d < m2) {
-                        m2 = d;
-                    }
+                    // selects: as branches the two went to scratch memory
+                    const bool less = d < m1;
+                    m2 = less ? m1 : d > m1 && d < m2 ? d : m2;
+                    m1 = less ? d : m1;
                 }
             }
             const float was = thr;
