@@ -1022,6 +1022,7 @@ constexpr float kPairUnit = 8192.0f;       // |b|^2 / kPairUnit fits a half
 struct PackPoint {
     half8 hi, lo;
 };
+static_assert(sizeof(PackPoint) == 2 * sizeof(half8), "read as an array of half8");
 
 // a box of points; the boxes of each 64 slots and of each 64 such chunks
 struct Box6 {
@@ -1099,6 +1100,12 @@ __device__ __forceinline__ float box_gap2(const Box6 &x, const float *lo, const 
     return d;
 }
 
+// The searches of 4,000 groups (7.2M particles) are bound by vector
+// instructions (about 79% of the cycles; the matrix cores are busy for 34%).
+// With a lane's bits in one word, the next points read into the registers of
+// the last, chunks without a hit left before the bits are read, and a chunk's
+// address kept scalar, they took 3.53 -> 3.21 and 3.35 -> 3.18 ms.
+//
 // A wavefront's queries: four rows of 16 lanes, one per column tile of the
 // products, each with its box and its largest squared radius (consecutive
 // slots share leaves, so a row's box is about a leaf's).
@@ -1106,7 +1113,7 @@ constexpr int kRows = kWave / 16;
 struct PairLds {
     float lo[kRows][6], hi[kRows][6], far[kRows];
     int32_t t[kWave];
-    uint32_t may[kWave][2], sure[kWave][2];  // per query, a bit per point of the chunk
+    alignas(8) uint16_t may[kWave][4], sure[kWave][4];  // per query, a bit per point of the chunk
 };
 
 struct PairSearch {
@@ -1132,8 +1139,8 @@ struct PairSearch {
                 L.hi[q][k] = hi;
             }
         }
-        L.may[lane][0] = L.may[lane][1] = 0;
-        L.sure[lane][0] = L.sure[lane][1] = 0;
+        take(L.may[lane]);
+        take(L.sure[lane]);
         L.t[lane] = slot;
         __syncthreads();
 #pragma unroll
@@ -1166,24 +1173,41 @@ struct PairSearch {
         for (int t = 0; t < kRows; t++) sure[t] = L.t[16 * t + col];
     }
 
+    // a query's bits, cleared for the next chunk
+    static __device__ __forceinline__ uint64_t take(uint16_t (&x)[4]) {
+        uint64_t m;
+        const uint64_t none = 0;
+        __builtin_memcpy(&m, x, sizeof(m));
+        __builtin_memcpy(x, &none, sizeof(m));
+        return m;
+    }
+
+    // Row `col` of product r is point 16 * (col / 4) + 4 * r + col % 4 of the
+    // chunk, so that a lane's results of the four products (rows 4 * q + i)
+    // are the 16 neighbouring points from 16 * q on: one word of the bits.
     __device__ __forceinline__ void points(const PackPoint *__restrict__ pk, int32_t k,
                                            half8 (&x)[4]) const {
         const int lane = lane_id(), col = lane & 15, q = lane >> 4;
+        // the chunk's address is the wavefront's, the lane's offset in it fixed
+        const half8 *p = &pk[(int64_t)k * kWave].hi;
+        p += 2 * (16 * (col >> 2) + (col & 3)) + (q >> 1);
 #pragma unroll
-        for (int r = 0; r < 4; r++) x[r] = (&pk[k * kWave + 16 * r + col].hi)[q >> 1];
+        for (int r = 0; r < 4; r++) x[r] = p[8 * r];
     }
 
     // The slots of chunk k against the queries of the rows in `rows`: per
     // query the bits of the points that may be, and that certainly are,
-    // closer.  The points of chunk `next` are read meanwhile.
+    // closer; false (and no bits) if no query has any, as for most chunks.
+    // The points of chunk `next` are read after the last product, into the
+    // same registers: the other wavefronts cover what the caller's work on the
+    // bits does not.
     template <bool SURE>
-    __device__ __forceinline__ void chunk(const PackPoint *__restrict__ pk, int32_t k, int32_t next,
+    __device__ __forceinline__ bool chunk(const PackPoint *__restrict__ pk, int32_t k, int32_t next,
                                           uint32_t rows, PairLds &L, uint64_t &m_may,
                                           uint64_t &m_sure) {
         const int lane = lane_id(), col = lane & 15, q = lane >> 4;
         if (have != k) points(pk, k, a);
-        half8 ahead[4];
-        points(pk, next, ahead);
+        bool any = false;
 #pragma unroll
         for (int t = 0; t < kRows; t++) {
             if (!(rows >> t & 1)) continue;
@@ -1192,38 +1216,37 @@ struct PairSearch {
 #pragma unroll
             for (int r = 0; r < 4; r++)
                 v[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[r], b[t], zero, 0, 0, 0);
-            int32_t low[4];
+            int32_t low = INT32_MAX;
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                low[r] = min(min(min(__float_as_int(v[r][0]), __float_as_int(v[r][1])),
-                                 __float_as_int(v[r][2])), __float_as_int(v[r][3]));
-            if (!ballot(min(min(low[0], low[1]), min(low[2], low[3])) < may[t])) continue;
+                low = min(min(min(min(low, __float_as_int(v[r][0])), __float_as_int(v[r][1])),
+                              __float_as_int(v[r][2])), __float_as_int(v[r][3]));
+            if (!ballot(low < may[t])) continue;
+            any = true;
+            // the sign of the saturated difference is the comparison
+            // (saturated: a threshold of INT32_MIN takes none)
+            uint32_t nm = 0, ns = 0;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                if (!ballot(low[r] < may[t])) continue;
-                uint32_t nm = 0, ns = 0;
+            for (int r = 3; r >= 0; r--) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    nm |= __float_as_int(v[r][i]) < may[t] ? 1u << i : 0u;
-                    if constexpr (SURE) ns |= __float_as_int(v[r][i]) < sure[t] ? 1u << i : 0u;
-                }
-                const int sh = 16 * (r & 1) + 4 * q;
-                if (nm) {
-                    atomicOr(&L.may[16 * t + col][r >> 1], nm << sh);
-                    if constexpr (SURE) atomicOr(&L.sure[16 * t + col][r >> 1], ns << sh);
+                for (int i = 3; i >= 0; i--) {
+                    const int32_t x = __float_as_int(v[r][i]);
+                    nm = __builtin_amdgcn_alignbit(nm, __builtin_elementwise_sub_sat(x, may[t]), 31);
+                    if constexpr (SURE)
+                        ns = __builtin_amdgcn_alignbit(ns, __builtin_elementwise_sub_sat(x, sure[t]), 31);
                 }
             }
+            L.may[16 * t + col][q] = (uint16_t)nm;
+            if constexpr (SURE) L.sure[16 * t + col][q] = (uint16_t)ns;
         }
-        __syncthreads();
-        m_may = ((uint64_t)L.may[lane][1] << 32) | L.may[lane][0];
-        L.may[lane][0] = L.may[lane][1] = 0;
-        m_sure = 0;
-        if constexpr (SURE) {
-            m_sure = ((uint64_t)L.sure[lane][1] << 32) | L.sure[lane][0];
-            L.sure[lane][0] = L.sure[lane][1] = 0;
-        }
-        for (int r = 0; r < 4; r++) a[r] = ahead[r];
+        if (next != k) points(pk, next, a);
         have = next;
+        if (!any) return false;
+        __syncthreads();
+        m_may = take(L.may[lane]);
+        m_sure = 0;
+        if constexpr (SURE) m_sure = take(L.sure[lane]);
+        return true;
     }
 };
 
@@ -1281,8 +1304,8 @@ __device__ __forceinline__ uint64_t slot_bits(int32_t base, int32_t lo, int32_t 
 // Queries of a wavefront in the searches: all 64 lanes, or, where the batch
 // has too few tiles to give every SIMD a wavefront, one row of 16.  A
 // wavefront's time is its chain through the chunks near any of its rows: on
-// one group of 15,985 particles (250 tiles) the searches take 123 and 102 us,
-// where with 64 queries they took 190 and 168.
+// one group of 15,985 particles (250 tiles) the searches took 123 and 102 us,
+// where with 64 queries they took 190 and 168 (95 and 83 now).
 constexpr int32_t kFewQueryTiles = 512;
 __host__ __device__ constexpr int32_t query_lanes(int64_t tiles64) {
     return tiles64 < kFewQueryTiles ? 16 : kWave;
@@ -1336,7 +1359,7 @@ __global__ __launch_bounds__(kWave) void k_sub_next_closest(
                     [&](int32_t k, int32_t next, uint32_t rows) {
             const int32_t base = k * kWave;
             uint64_t may, sure;
-            P.chunk<false>(pk, k, next, rows, L, may, sure);
+            if (!P.chunk<false>(pk, k, next, rows, L, may, sure)) return;
             // the group's slots outside the skipped subtree
             may &= slot_bits(base, g.off, g.off + g.n) & ~slot_bits(base, s_lo, s_hi);
             if (!valid) may = 0;
@@ -1684,7 +1707,7 @@ __global__ __launch_bounds__(kWave) void k_sub_link(const SubGroup *__restrict__
                 [&](int32_t k, int32_t next, uint32_t rows) {
         const int32_t base = k * kWave;
         uint64_t may, hit;
-        P.chunk<true>(pk, k, next, rows, L, may, hit);
+        if (!P.chunk<true>(pk, k, next, rows, L, may, hit)) return;
         const uint64_t later = valid ? slot_bits(base, i + 1, end) : 0ull;
         hit &= later;
         uint64_t amb = may & later & ~hit;
