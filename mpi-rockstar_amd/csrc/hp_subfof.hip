@@ -1159,6 +1159,9 @@ struct PairSearch {
         const float s2 = (r2 * S) * S;
         const float room = 3.0f * kPairEps * na + 1.0e-3f * sqrtf(na) + 1.5f;
         const float up = s2 * 1.001f + room, dn = s2 * 0.999f - room;
+        // a squared radius past the largest float takes no pair for certain:
+        // the float distance of a pair may be infinite too, and not below it
+        const bool sure_ok = valid && dn > 0.0f && r2 < __builtin_inff();
         const float f = row_reduce(valid ? r2 : 0.0f, [](float a, float b) { return b > a ? b : a; });
         __syncthreads();
         if (col == 0) L.far[q] = f;
@@ -1167,7 +1170,7 @@ struct PairSearch {
 #pragma unroll
         for (int t = 0; t < kRows; t++) may[t] = L.t[16 * t + col];
         __syncthreads();
-        L.t[lane] = valid && dn > 0.0f ? __float_as_int(dn) : INT32_MIN;
+        L.t[lane] = sure_ok ? __float_as_int(dn) : INT32_MIN;
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < kRows; t++) sure[t] = L.t[16 * t + col];

@@ -234,6 +234,27 @@ def test_gpu_subfof_sample_sizes(restatement, exact_ll, sizes):
 
 
 @pytest.mark.gpu
+def test_gpu_subfof_infinite_linking_length(restatement):
+    """A group so thin along z that norm_sd makes coordinates of 1e22 of the
+    others: their squared distances are infinite, and so is the linking
+    length's square.  No infinite distance is below that (src/fast3tree.c:437),
+    so only pairs of equal x and y are linked.  Coordinates of few bits and
+    counts that are powers of two, so that norm_sd's sums are exact in any
+    order."""
+    rng = np.random.default_rng(3)
+    plist = []
+    for n in (64, 256, 1024):
+        p = np.zeros(n, catalog.PARTICLE_DTYPE)
+        p["id"] = np.arange(n)
+        x = np.round(rng.normal(size=(n, 6)) * 64) / 64
+        x[:, 2] = np.ldexp(x[:, 2], -73)
+        p["pos"] = x
+        plist.append(p)
+    g, _, _ = _check_batch(restatement, plist, min_p=2)
+    assert np.isinf(g["target_r"]).all()
+
+
+@pytest.mark.gpu
 def test_gpu_subfof_exact_ll_and_lower_levels(restatement):
     fg = catalog.fof_groups(seed=5, n_groups=6, lo=300, hi=12000)
     plist = [fg.particles[f:f + n].copy() for f, n in fg.groups]
