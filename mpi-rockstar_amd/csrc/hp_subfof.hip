@@ -1017,6 +1017,7 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr float kPairEps = 1.5258789e-5f;  // 2^-16
+constexpr int kPairScaleMax = 64;         // exponent of the largest scale
 constexpr float kPairUnit = 8192.0f;       // |b|^2 / kPairUnit fits a half
 
 struct PackPoint {
@@ -1030,13 +1031,16 @@ struct Box6 {
 };
 
 // The power of two that brings a group's largest coordinate into [4096,
-// 8192), so that twice a coordinate fits a half.
+// 8192), so that twice a coordinate fits a half; at most 2^64.  Squared
+// distances below the normal floats are rounded to multiples of 2^-149, which
+// are 2^-21 at that scale, far less than the room around a radius: with a
+// larger one they decide pairs that the products would decide otherwise.
 __device__ __forceinline__ float pair_scale(const Node6 &root) {
     float m = 0.0f;
     for (int k = 0; k < 6; k++)
         m = fmaxf(m, fmaxf(__builtin_fabsf(root.lo[k]), __builtin_fabsf(root.hi[k])));
     if (!(m > 0.0f && m < __builtin_inff())) return 1.0f;
-    return __builtin_ldexpf(1.0f, min(13 - __builtin_amdgcn_frexp_expf(m), 100));
+    return __builtin_ldexpf(1.0f, min(13 - __builtin_amdgcn_frexp_expf(m), kPairScaleMax));
 }
 
 // Each slot's vector in halves (as a point: the six dimensions, 1 and |b|^2),

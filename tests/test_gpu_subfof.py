@@ -255,6 +255,24 @@ def test_gpu_subfof_infinite_linking_length(restatement):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("exponent", [-50, -52, -66, -70, -72])
+def test_gpu_subfof_subnormal_squared_distances(restatement, exponent):
+    """Groups without velocities are not scaled (src/groupies.c:827), so that
+    positions of 2^-70 stay and their squared distances are subnormal: a few
+    units in the last place, with many ties at the linking length.  And
+    around 2^-51, where the searches' common scale stops growing."""
+    rng = np.random.default_rng(4)
+    plist = []
+    for n in (64, 256, 1024):
+        p = np.zeros(n, catalog.PARTICLE_DTYPE)
+        p["id"] = np.arange(n)
+        p["pos"][:, :3] = np.ldexp(np.round(rng.normal(size=(n, 3)) * 64) / 64, exponent)
+        plist.append(p)
+    _, subs, _ = _check_batch(restatement, plist, min_p=2)
+    assert subs.shape[0] > 50
+
+
+@pytest.mark.gpu
 def test_gpu_subfof_exact_ll_and_lower_levels(restatement):
     fg = catalog.fof_groups(seed=5, n_groups=6, lo=300, hi=12000)
     plist = [fg.particles[f:f + n].copy() for f, n in fg.groups]
