@@ -1012,6 +1012,7 @@ __global__ __launch_bounds__(kCap, 8) void k_subtree(const float4 *__restrict__ 
                 a.fin[first + tid] = p0;
                 a.leaf_of[first + tid] = t.node;
             }
+            __syncthreads();  // every wavefront has read the entry it is at
             if (tid == 0) S.next = k_after;
             __syncthreads();
             continue;
