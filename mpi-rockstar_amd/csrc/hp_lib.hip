@@ -223,7 +223,9 @@ struct Tables {
     std::vector<Group> groups;          // walk wavefronts, 64 sink points each
     std::vector<int2> direct_blocks;    // direct-kernel workgroups
     std::vector<ScanTile> scan_tiles;
+    // per call; after the counts, the calls of more than kFewTiles tiles
     std::vector<int32_t> call_tile0, call_ntiles;
+    int32_t nlarge() const { return (int32_t)(call_ntiles.size() - call_tile0.size()); }
     std::vector<int32_t> seg_wave, seg_block;  // calls sorted by one wavefront / workgroup
     std::vector<SegTile> seg_tiles;            // tiles of the calls sorted by passes
     int method = HP_METHOD_TREE;
@@ -312,6 +314,8 @@ static int make_tables(Tables &T, const int64_t *first, const int64_t *count, in
                 T.scan_tiles.push_back(ScanTile{(int32_t)h, (int32_t)off});
             T.call_ntiles[h] = (int32_t)(T.scan_tiles.size() - T.call_tile0[h]);
         }
+        for (int64_t h = 0; h < nh; h++)
+            if (T.call_ntiles[h] > kFewTiles) T.call_ntiles.push_back((int32_t)h);
         int64_t big_before = 0;  // records of the pass-sorted calls before this one
         int32_t tiles_before = 0;
         for (int64_t h = 0; h < nh; h++) {
@@ -1383,6 +1387,7 @@ struct Engine {
     int props(const Tables &T, const struct potential *d_po, const hp_halo *d_halos,
               const hp_mass_defs &md, hp_halo_props *d_props) {
         const int32_t H = (int32_t)T.nhalos, nst = (int32_t)T.scan_tiles.size();
+        const int32_t cg = call_groups(H, T.nlarge());
         if (H == 0) return HP_OK;
         HP_ENSURE(pcnt, sizeof(PropCount) * (nst + 1));
         HP_ENSURE(pscan, sizeof(PropScan) * (nst + 1));
@@ -1427,14 +1432,14 @@ struct Engine {
                                                  pcnt.as<PropCount>(), pr);
             HP_LAUNCHED();
         }
-        k_props_prefix<<<blocks(H, 256), 256, 0, s>>>(t0, tn, H, pcnt.as<PropCount>());
+        k_props_prefix<<<cg, kWave, 0, s>>>(t0, tn, H, pcnt.as<PropCount>());
         HP_LAUNCHED();
         if (nst > 0) {
             k_props_scan<<<nst, kWave, 0, s>>>(pr, tl, nst, d_halos, hf, hc,
                                                pcnt.as<PropCount>(), pa, pscan.as<PropScan>());
             HP_LAUNCHED();
         }
-        k_props_calls<<<blocks(H, 64), 64, 0, s>>>(t0, tn, H, d_halos, hc, pscan.as<PropScan>(),
+        k_props_calls<<<cg, kWave, 0, s>>>(t0, tn, H, d_halos, hc, pscan.as<PropScan>(),
                                                    pcall.as<PropCall>());
         HP_LAUNCHED();
         if (nst > 0) {
@@ -1443,7 +1448,7 @@ struct Engine {
             HP_LAUNCHED();
         }
         ShapeState *ss = shape_st.as<ShapeState>();
-        k_props_final<<<blocks(H, 64), 64, 0, s>>>(
+        k_props_final<<<cg, kWave, 0, s>>>(
             pr, pcnt.as<PropCount>(), t0, tn, H, d_halos, hf, pcall.as<PropCall>(),
             psums.as<PropSums>(), pa, d_props, ss, scale_calls.as<ScaleCall>(),
             fit_list.as<int32_t>(), fit_n.as<int32_t>());
@@ -1490,7 +1495,7 @@ struct Engine {
                                              pe_cnt.as<int32_t>());
             HP_LAUNCHED();
         }
-        k_pe_calls<<<blocks(H, 256), 256, 0, s>>>(H, t0, tn, pe_cnt.as<int32_t>(), pa, d_props);
+        k_pe_calls<<<cg, kWave, 0, s>>>(H, t0, tn, pe_cnt.as<int32_t>(), pa, d_props);
         HP_LAUNCHED();
         return HP_OK;
     }
@@ -1594,7 +1599,7 @@ struct Engine {
         k_gather_sorted<<<blocks(N, 256), 256, 0, s>>>(d_po, sorted_vals, (int32_t)N, S, RV);
         HP_LAUNCHED();
         CallInfo *ci = callinfo.as<CallInfo>();
-        const int32_t nst = (int32_t)T.scan_tiles.size();
+        const int32_t nst = (int32_t)T.scan_tiles.size(), cg = call_groups(H, T.nlarge());
         int32_t *ti32 = tile_i32.as<int32_t>();
         k_call_kept<<<blocks(H, 256), 256, 0, s>>>(sorted_keys, hfirst.as<int64_t>(),
                                                    hcount.as<int64_t>(), H, ci);
@@ -1605,11 +1610,11 @@ struct Engine {
                                                    rvir_thresh, ti32, tsum.as<Moments>());
             HP_LAUNCHED();
         }
-        k_rvir_calls<<<blocks(H, 256), 256, 0, s>>>(RV, call_tile0.as<int32_t>(),
+        k_rvir_calls<<<cg, kWave, 0, s>>>(RV, call_tile0.as<int32_t>(),
                                                     call_ntiles.as<int32_t>(), ti32, H, ci);
         HP_LAUNCHED();
         if (nst > 0) {
-            k_vel_prefix<<<blocks(H, 256), 256, 0, s>>>(call_tile0.as<int32_t>(),
+            k_vel_prefix<<<cg, kWave, 0, s>>>(call_tile0.as<int32_t>(),
                                                         call_ntiles.as<int32_t>(), H,
                                                         tsum.as<Moments>());
             HP_LAUNCHED();
@@ -1618,7 +1623,7 @@ struct Engine {
             HP_LAUNCHED();
         }
         const int32_t *flags = counters.as<int32_t>() + kErrFlags;
-        k_vel_finish<<<blocks(H, 256), 256, 0, s>>>(RV, call_tile0.as<int32_t>(),
+        k_vel_finish<<<cg, kWave, 0, s>>>(RV, call_tile0.as<int32_t>(),
                                                     call_ntiles.as<int32_t>(), H, ci,
                                                     tcand.as<Cand>(), d_halos, flags);
         HP_LAUNCHED();
@@ -1638,7 +1643,7 @@ struct Engine {
                                            flags);
             HP_LAUNCHED();
         }
-        k_nbound_calls<<<blocks(H, 256), 256, 0, s>>>(call_tile0.as<int32_t>(),
+        k_nbound_calls<<<cg, kWave, 0, s>>>(call_tile0.as<int32_t>(),
                                                       call_ntiles.as<int32_t>(), ti32, H, d_halos,
                                                       flags);
         HP_LAUNCHED();

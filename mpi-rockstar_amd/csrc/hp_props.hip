@@ -185,10 +185,10 @@ __device__ __forceinline__ int32_t count_to_lane(uint64_t m) {
 }
 
 // per call: exclusive prefix of the tile counts, in tile order
-__global__ void k_props_prefix(const int32_t *__restrict__ call_tile0,
+__global__ __launch_bounds__(kWave) void k_props_prefix(const int32_t *__restrict__ call_tile0,
                                const int32_t *__restrict__ call_ntiles, int32_t nh,
                                PropCount *__restrict__ cnt) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t h = lane_call(nh, call_ntiles);
     const int32_t t0 = h < nh ? call_tile0[h] : 0, nt = h < nh ? call_ntiles[h] : 0;
     if (nt <= kFewTiles) {
         int32_t nb = 0, ns = 0;
@@ -199,7 +199,7 @@ __global__ void k_props_prefix(const int32_t *__restrict__ call_tile0,
             ns += c.ns;
         }
     }
-    for_large_calls(t0, nt, [&](int32_t first, int32_t n, bool) {
+    for_large_call(t0, nt, [&](int32_t first, int32_t n, bool) {
         int32_t nb = 0, ns = 0;
         for (int32_t base = 0; base < n; base += kWave) {
             const bool in = base + lane_id() < n;
@@ -305,12 +305,12 @@ __global__ __launch_bounds__(kWave) void k_props_scan(const PropReads in,
     if (lane == 0) out[t] = s;
 }
 
-__global__ void k_props_calls(const int32_t *__restrict__ call_tile0,
+__global__ __launch_bounds__(kWave) void k_props_calls(const int32_t *__restrict__ call_tile0,
                               const int32_t *__restrict__ call_ntiles, int32_t nh,
                               const hp_halo *__restrict__ halos,
                               const int64_t *__restrict__ hcount,
                               const PropScan *__restrict__ ts, PropCall *__restrict__ pc) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t h = lane_call(nh, call_ntiles);
     const bool v = h < nh;
     const int32_t t0 = v ? call_tile0[h] : 0, nt = v ? call_ntiles[h] : 0;
     PropCall c;
@@ -338,7 +338,7 @@ __global__ void k_props_calls(const int32_t *__restrict__ call_tile0,
         }
     }
     // every field of a tile is monotone over the tiles: maxima over the lanes
-    for_large_calls(t0, nt, [&](int32_t a, int32_t n, bool mine) {
+    for_large_call(t0, nt, [&](int32_t a, int32_t n, bool mine) {
         int32_t all = -1, l0 = -1, n_0 = 0, vir = 0, alt[4] = {0, 0, 0, 0}, j = INT32_MAX;
         double best = -1.0, pe_b = 0.0;
         bool seen = false;
@@ -1044,7 +1044,7 @@ struct ScaleCall {
 };
 
 // per call: the halo fields, and where its shape windows and its fit start
-__global__ void k_props_final(const PropReads in, const PropCount *__restrict__ pre,
+__global__ __launch_bounds__(kWave) void k_props_final(const PropReads in, const PropCount *__restrict__ pre,
                               const int32_t *__restrict__ call_tile0,
                               const int32_t *__restrict__ call_ntiles, int32_t nh,
                               const hp_halo *__restrict__ halos,
@@ -1053,7 +1053,7 @@ __global__ void k_props_final(const PropReads in, const PropCount *__restrict__ 
                               PropArgs pa, hp_halo_props *__restrict__ props,
                               ShapeState *__restrict__ shapes, ScaleCall *__restrict__ scales,
                               int32_t *__restrict__ fit_list, int32_t *__restrict__ fit_n) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t h = lane_call(nh, call_ntiles);
     const bool v = h < nh;
     const int32_t t0 = v ? call_tile0[h] : 0, nt = v ? call_ntiles[h] : 0;
     double L[3] = {0, 0, 0}, sx[3] = {0, 0, 0}, sv[3] = {0, 0, 0}, sv2[3] = {0, 0, 0};
@@ -1073,7 +1073,7 @@ __global__ void k_props_final(const PropReads in, const PropCount *__restrict__ 
     };
     if (nt <= kFewTiles)
         for (int32_t t = t0; t < t0 + nt; t++) add(ts[t]);
-    for_large_calls(t0, nt, [&](int32_t a, int32_t k, bool mine) {
+    for_large_call(t0, nt, [&](int32_t a, int32_t k, bool mine) {
         // lane c < 15 adds up component c, in tile order
         static_assert(offsetof(PropSums, n) == 15 * sizeof(double), "fifteen sums, then counts");
         const int c = min(lane_id(), 14);
@@ -1462,16 +1462,16 @@ __global__ __launch_bounds__(kWave) void k_pe_tiles(const PropReads in,
     if (lane_id() == 0) cnt[t] = n;
 }
 
-__global__ void k_pe_calls(int32_t nh, const int32_t *__restrict__ call_tile0,
+__global__ __launch_bounds__(kWave) void k_pe_calls(int32_t nh, const int32_t *__restrict__ call_tile0,
                            const int32_t *__restrict__ call_ntiles,
                            const int32_t *__restrict__ cnt, PropArgs pa,
                            hp_halo_props *__restrict__ props) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t h = lane_call(nh, call_ntiles);
     const int32_t t0 = h < nh ? call_tile0[h] : 0, nt = h < nh ? call_ntiles[h] : 0;
     int32_t n = 0;  // a call's records are counted in 32 bits
     if (nt <= kFewTiles)
         for (int32_t t = t0; t < t0 + nt; t++) n += cnt[t];
-    for_large_calls(t0, nt, [&](int32_t a, int32_t k, bool mine) {
+    for_large_call(t0, nt, [&](int32_t a, int32_t k, bool mine) {
         int32_t m = 0;
         for (int32_t t = a + lane_id(); t < a + k; t += kWave) m += cnt[t];
         m = wave_sum(m);

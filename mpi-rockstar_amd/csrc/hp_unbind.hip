@@ -672,38 +672,49 @@ __device__ __forceinline__ int32_t block_sum_i32(int32_t v) {
     return m;
 }
 
-// The per-call kernels run a thread per call.  A thread goes through at most
-// kFewTiles tiles by itself; the calls with more are taken one after another
-// by the whole wavefront, f(first tile, tiles, whether it is this lane's
-// call), a lane per tile: on a call of 2.1M records (1,115 tiles) the loops
-// of dependent reads were 74 to 288 us a kernel.  Called with all lanes
-// active.
+// The per-call kernels run a thread per call of at most kFewTiles tiles, 64 to
+// a workgroup, and a workgroup of one wavefront per larger call; those are
+// listed after the tile counts.  By one thread the 1,115 tiles of a call of
+// 2.1M records were a loop of dependent reads, 74 to 288 us a kernel; by the
+// wavefront that held the call's thread, 64 calls of 17,000 records waited for
+// each other, 0.8 us each a kernel: 342 us of the bound pass's last phase, 138
+// with a wavefront each (of 64 x 40,000 and 60,000 small ones, a batch sorted
+// by size, 627 and 467).
 constexpr int32_t kFewTiles = 8;
+__host__ __device__ constexpr int32_t call_groups(int32_t nh, int32_t nlarge) {
+    return nlarge + (nh + kWave - 1) / kWave;
+}
+// this lane's call, nh where it has none; a large one is in lane 0
+__device__ __forceinline__ int32_t lane_call(int32_t nh, const int32_t *__restrict__ ntiles) {
+    const int32_t nlarge = (int32_t)gridDim.x - (nh + kWave - 1) / kWave;
+    const int32_t w = (int32_t)blockIdx.x - nlarge;
+    if (w < 0) return lane_id() == 0 ? ntiles[nh + (int32_t)blockIdx.x] : nh;
+    const int32_t h = w * kWave + lane_id();
+    return h < nh && ntiles[h] <= kFewTiles ? h : nh;
+}
+// f(first tile, tiles, whether this is the call's lane) for a large call, with
+// all lanes active
 template <class F>
-__device__ __forceinline__ void for_large_calls(int32_t t0, int32_t nt, F &&f) {
-    uint64_t large = ballot(nt > kFewTiles);
-    while (large) {
-        const int l = __builtin_ctzll(large);
-        large &= large - 1;
-        f(__builtin_amdgcn_readlane(t0, l), __builtin_amdgcn_readlane(nt, l), lane_id() == l);
-    }
+__device__ __forceinline__ void for_large_call(int32_t t0, int32_t nt, F &&f) {
+    const int32_t n = uniform(nt);
+    if (n > kFewTiles) f(uniform(t0), n, lane_id() == 0);
 }
 
 // rvir_max (src/properties.c:173-177): the largest j < kept with
 // j^2 > r2_j^3 (4pi/3 rho_vir)^2, r2^3 in float, the rest in double.
 // Per tile (k_rvir_vel_tiles, below), then per call.
-__global__ void k_rvir_calls(const float4 *__restrict__ rv,
+__global__ __launch_bounds__(kWave) void k_rvir_calls(const float4 *__restrict__ rv,
                              const int32_t *__restrict__ call_tile0,
                              const int32_t *__restrict__ call_ntiles,
                              const int32_t *__restrict__ tile_rvir, int32_t nh,
                              CallInfo *__restrict__ ci) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t h = lane_call(nh, call_ntiles);
     const bool v = h < nh;
     const int32_t t0 = v ? call_tile0[h] : 0, nt = v ? call_ntiles[h] : 0;
     int32_t rvm = -1;
     if (nt <= kFewTiles)
         for (int32_t t = t0; t < t0 + nt; t++) rvm = max(rvm, tile_rvir[t]);
-    for_large_calls(t0, nt, [&](int32_t a, int32_t n, bool mine) {
+    for_large_call(t0, nt, [&](int32_t a, int32_t n, bool mine) {
         int32_t m = -1;
         for (int32_t t = a + lane_id(); t < a + n; t += kWave) m = max(m, tile_rvir[t]);
         m = wave_max(m);
@@ -773,10 +784,10 @@ __global__ __launch_bounds__(kWave) void k_rvir_vel_tiles(const float4 *__restri
     }
 }
 
-__global__ void k_vel_prefix(const int32_t *__restrict__ call_tile0,
+__global__ __launch_bounds__(kWave) void k_vel_prefix(const int32_t *__restrict__ call_tile0,
                              const int32_t *__restrict__ call_ntiles, int32_t nh,
                              Moments *__restrict__ tsum) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t h = lane_call(nh, call_ntiles);
     const int32_t t0 = h < nh ? call_tile0[h] : 0, nt = h < nh ? call_ntiles[h] : 0;
     if (nt <= kFewTiles) {
         double a[6] = {0, 0, 0, 0, 0, 0};
@@ -790,7 +801,7 @@ __global__ void k_vel_prefix(const int32_t *__restrict__ call_tile0,
             for (int k = 0; k < 6; k++) a[k] += b[k];
         }
     }
-    for_large_calls(t0, nt, [&](int32_t first, int32_t n, bool) {
+    for_large_call(t0, nt, [&](int32_t first, int32_t n, bool) {
         double run[6] = {0, 0, 0, 0, 0, 0};
         for (int32_t base = 0; base < n; base += kWave) {
             const bool in = base + lane_id() < n;
@@ -930,12 +941,12 @@ __device__ __forceinline__ Cand small_prefix(const float4 *__restrict__ rv, int3
 }
 
 // one thread per call: final selection, halo fields
-__global__ void k_vel_finish(const float4 *__restrict__ rv,
+__global__ __launch_bounds__(kWave) void k_vel_finish(const float4 *__restrict__ rv,
                              const int32_t *__restrict__ call_tile0,
                              const int32_t *__restrict__ call_ntiles, int32_t nh,
                              const CallInfo *__restrict__ ci, const Cand *__restrict__ tcand,
                              hp_halo *__restrict__ halos, const int32_t *__restrict__ flags) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t h = lane_call(nh, call_ntiles);
     if (*flags & kErrDeep) return;
     const bool v = h < nh;
     CallInfo c;
@@ -958,7 +969,7 @@ __global__ void k_vel_finish(const float4 *__restrict__ rv,
             take(a, tcand[2 * t]);
             take(b, tcand[2 * t + 1]);
         }
-    for_large_calls(t0, nt, [&](int32_t first, int32_t n, bool mine) {
+    for_large_call(t0, nt, [&](int32_t first, int32_t n, bool mine) {
         Cand x = no_cand(), y = no_cand();
         for (int32_t t = first + lane_id(); t < first + n; t += kWave) {
             take(x, tcand[2 * t]);
@@ -1080,17 +1091,17 @@ __global__ void k_bound_tail(const int64_t *__restrict__ hfirst, const int64_t *
     for (int64_t j = c.kept + threadIdx.x; j < hcount[h]; j += blockDim.x) bound[hfirst[h] + j] = 0;
 }
 
-__global__ void k_nbound_calls(const int32_t *__restrict__ call_tile0,
+__global__ __launch_bounds__(kWave) void k_nbound_calls(const int32_t *__restrict__ call_tile0,
                                const int32_t *__restrict__ call_ntiles,
                                const int32_t *__restrict__ tile_nb, int32_t nh,
                                hp_halo *__restrict__ halos, const int32_t *__restrict__ flags) {
-    const int32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t h = lane_call(nh, call_ntiles);
     if (*flags & kErrDeep) return;
     const int32_t t0 = h < nh ? call_tile0[h] : 0, nt = h < nh ? call_ntiles[h] : 0;
     int32_t n = 0;
     if (nt <= kFewTiles)
         for (int32_t t = t0; t < t0 + nt; t++) n += tile_nb[t];
-    for_large_calls(t0, nt, [&](int32_t first, int32_t m, bool mine) {
+    for_large_call(t0, nt, [&](int32_t first, int32_t m, bool mine) {
         int32_t x = 0;
         for (int32_t t = first + lane_id(); t < first + m; t += kWave) x += tile_nb[t];
         x = wave_sum(x);

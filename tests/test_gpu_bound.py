@@ -148,3 +148,29 @@ def test_bound_sort_inside_calls_at_every_size(restatement):
             assert np.unique(got["r2"]).size < k  # the case has ties
         np.testing.assert_array_equal(got["flags"], po_o["flags"][f:f + k],
                                       err_msg=f"call {h} of {n}")
+
+
+@pytest.mark.parametrize("counts", [
+    [16_384, 16_385],                          # 8 tiles and 9: the most a thread takes, and one more
+    [20_000] + [7] * 70 + [17_000, 16_384, 17_000],  # large ones first, last and beside each other
+    [3] * 63 + [18_000] + [5],                 # the 64th call, and one more
+])
+def test_bound_large_calls_among_small_ones(restatement, counts):
+    """Calls of more than eight tiles have wavefronts of their own in the
+    kernels that run a thread per call: the bound pass and the properties."""
+    import test_gpu_props
+
+    parts = [catalog.small_batch(seed=300 + i, n_halos=1, lo=n, hi=n + 1, contam=0.0)
+             for i, n in enumerate(counts)]
+    cat = parts[0].copy()
+    size = [p.n_records for p in parts]
+    cat.po = np.zeros(sum(size), cat.po.dtype)  # (concatenating would drop the records' padding)
+    cat.halos = np.zeros(len(parts), cat.halos.dtype)
+    first = np.cumsum([0] + size)
+    for i, p in enumerate(parts):
+        cat.po[first[i]:first[i + 1]] = p.po
+        cat.halos[i] = p.halos[0]
+        cat.halos["first"][i] = first[i]
+    assert [int(c) for c in cat.halos["count"]] == counts
+    _check_batch(restatement, cat)
+    test_gpu_props.check(restatement, cat)
