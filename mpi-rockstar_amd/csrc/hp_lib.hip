@@ -1218,7 +1218,7 @@ struct Engine {
 
     struct Graphs {
         hipGraphExec_t step = nullptr;  // the whole hp_plan_run, one launch
-        int levels = 0;  // split levels recorded in `step`
+        int levels = 0;  // split levels recorded in `step`, or that it has to be recorded with
         const void *po = nullptr, *halos = nullptr, *bound = nullptr;
         Config cfg{};    // the globals the graphs were recorded with
         bool ok = false;
@@ -1259,6 +1259,7 @@ struct Engine {
     // before, between and after the phases (events recorded inside a graph
     // are not usable for elapsed times once the graph is recorded again).
     static constexpr int kLevelMargin = 2;
+    int step_levels() const { return (int)st.levels + 1 + kLevelMargin; }
     int capture_all(const Tables &T, struct potential *d_po, hp_halo *d_halos, uint8_t *d_bound,
                     const hp_options &o, int levels) {
         drop_graphs();
@@ -1316,13 +1317,17 @@ struct Engine {
                    const hp_options &o) {
         hipStream_t s = stream;
         int r;
-        if (!g.ok || g.po != d_po || g.halos != d_halos || g.bound != d_bound ||
-            !(g.cfg == Config::now())) {
-            // learn the depth eagerly, then record
+        const bool same = g.step && g.po == d_po && g.halos == d_halos && g.bound == d_bound &&
+                          g.cfg == Config::now();
+        if (!g.ok || !same) {
+            // learn the depth eagerly, then record (no shallower than trees
+            // that the recorded step was too short for: batches of trees more
+            // than the margin apart, in turn, would be recorded each time)
             if ((r = potential(T, d_po, o))) return r;
             if ((r = enqueue_unbind(T, d_po, d_halos, d_bound))) return r;
             HP_TRY(hipStreamSynchronize(s));
-            return capture_all(T, d_po, d_halos, d_bound, o, (int)st.levels + 1 + kLevelMargin);
+            return capture_all(T, d_po, d_halos, d_bound, o,
+                               std::max(step_levels(), same ? g.levels : 0));
         }
         st = hp_stats();
         st.records = T.nrec;
@@ -1332,6 +1337,7 @@ struct Engine {
         if (h_counters[kErrFlags] & kErrDeep) {
             g.ok = false;
             if ((r = potential(T, d_po, o))) return r;
+            g.levels = std::max(g.levels, step_levels());
             if ((r = enqueue_unbind(T, d_po, d_halos, d_bound))) return r;
             HP_TRY(hipStreamSynchronize(s));
             return HP_OK;

@@ -102,6 +102,44 @@ def test_graph_deeper_tree_falls_back():
         plan.close()
 
 
+def test_graph_of_trees_in_turn_is_recorded_once():
+    """Batches of trees far more than the recorded margin apart, in turn on
+    one plan's buffers: the step is recorded for the deepest ones and
+    replayed from then on (a replay's phase times are set without `timing`,
+    an eager run's are 0)."""
+    base = catalog.small_batch(seed=42, n_halos=6, lo=2000, hi=4000)
+    base.po["flags"] = np.arange(base.n_records, dtype=np.int32)
+    deep = base.copy()
+    f, c = int(deep.halos["first"][0]), int(deep.halos["count"][0])
+    k = np.arange(c)
+    cen = deep.halos["pos"][0, :3]
+    deep.po["pos"][f:f + c, 0] = cen[0] + (0.5 ** (k % 40)) * 0.3
+    deep.po["pos"][f:f + c, 1] = cen[1] + (k % 7) * 1e-3
+    deep.po["pos"][f:f + c, 2] = cen[2] + (k % 5) * 1e-3
+    wants = {0: _eager(base), 1: _eager(deep)}
+    halopot.set_config(base.params)
+    plan = halopot.Plan(base.halos, halopot.options(use_graph=1))
+    d_po = DeviceArray.from_numpy(base.po)
+    d_h = DeviceArray.from_numpy(base.halos)
+    d_b = DeviceArray.zeros(base.n_records)
+    replayed = []
+    try:
+        for which in (0, 1, 0, 1, 0, 1):
+            cat = (base, deep)[which]
+            d_po.upload(cat.po)
+            d_h.upload(cat.halos)
+            plan.run(d_po.address, d_h.address, d_b.address)
+            synchronize()
+            got = (d_po.download(np.empty_like(cat.po)), d_h.download(np.empty_like(cat.halos)),
+                   d_b.download(np.empty(cat.n_records, np.uint8)))
+            _same(got, wants[which])
+            replayed.append(plan.stats()["ms_total"] > 0)
+    finally:
+        plan.close()
+    # recorded, too shallow, recorded again, then replays
+    assert replayed == [False, False, False, True, True, True]
+
+
 def test_graph_rerecords_on_config_change():
     cat = catalog.small_batch(seed=43, n_halos=30, lo=5, hi=5000, potential_only=0.1)
     cat.po["flags"] = np.arange(cat.n_records, dtype=np.int32)
