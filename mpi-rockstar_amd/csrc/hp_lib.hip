@@ -484,13 +484,14 @@ struct Engine {
 
     int grab(DevBuf &b, size_t n) {
         if (!carve && !counting) return b.ensure(n);
-        if (b.carved && b.bytes >= n) return HP_OK;
+        if (b.p && b.bytes >= n) return HP_OK;
         const size_t a = (n + 255) & ~(size_t)255;
         if (counting) {
             counted += a;
             return HP_OK;
         }
-        if (carve_off + a > carve_cap && arena.p) {
+        // a buffer that has an allocation of its own keeps to one
+        if (arena.p && (carve_off + a > carve_cap || (b.p && !b.carved))) {
             if (b.carved) b.release();
             return b.ensure(n);
         }
