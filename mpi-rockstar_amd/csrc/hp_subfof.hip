@@ -1308,6 +1308,47 @@ __device__ __forceinline__ uint64_t slot_bits(int32_t base, int32_t lo, int32_t 
     return from & to;
 }
 
+// f(t, squared distance in float) for the slots of chunk k that a lane's bits
+// name, in order; r2: the squared radius that f's pairs have to be below.
+// Mostly a lane has one or two of a chunk's 64.  But particles far out (10,000
+// standard deviations) take the bits of the group's common scale from the
+// others, whose pairs are then all left to the float distance: where a lane
+// has more than kManyBits, the lanes that the chunk's box is near to take the
+// group's slots [lo, hi) of it together, each point read once at a uniform
+// address.  50 groups of 5,000 with a particle at 10^6: 6.42 ms by tree walks,
+// 9.75 with a read a lane and bit, now 6.08; at 10^4 6.36, 7.02 and 5.65.
+constexpr int kManyBits = 16, kPairBatch = 8;
+template <class F>
+__device__ __forceinline__ void pair_distances(uint64_t bits, int32_t k, int32_t lo, int32_t hi,
+                                               const float (&c)[6], float r2,
+                                               const SParticle *__restrict__ w,
+                                               const Box6 *__restrict__ chunks, F &&f) {
+    const int32_t base = k * kWave;
+    if (ballot(__popcll(bits) > kManyBits) && !(box_gap2(load_const(chunks + k), c, c) < r2))
+        bits = 0;
+    if (ballot(__popcll(bits) > kManyBits)) {
+        const int32_t end = min(hi - base, kWave);
+        for (int32_t t = max(lo - base, 0); t < end; t += kPairBatch) {
+            SParticle p[kPairBatch];
+#pragma unroll
+            for (int i = 0; i < kPairBatch; i++) p[i] = load_const(w + base + min(t + i, end - 1));
+#pragma unroll
+            for (int i = 0; i < kPairBatch; i++) {
+                const float d = dist6(c, p[i]);
+                if (t + i < end && (bits >> (t + i) & 1)) f(t + i, d);
+            }
+        }
+        return;
+    }
+    while (ballot(bits != 0)) {
+        if (bits) {
+            const int t = __builtin_ctzll(bits);
+            bits &= bits - 1;
+            f(t, dist6(c, w[base + t]));
+        }
+    }
+}
+
 // Queries of a wavefront in the searches: all 64 lanes, or, where the batch
 // has too few tiles to give every SIMD a wavefront, one row of 16.  A
 // wavefront's time is its chain through the chunks near any of its rows: on
@@ -1371,17 +1412,12 @@ __global__ __launch_bounds__(kWave) void k_sub_next_closest(
             may &= slot_bits(base, g.off, g.off + g.n) & ~slot_bits(base, s_lo, s_hi);
             if (!valid) may = 0;
             if (!ballot(may != 0)) return;
-            while (ballot(may != 0)) {
-                if (may) {
-                    const int t = __builtin_ctzll(may);
-                    may &= may - 1;
-                    const float d = dist6(c, w[base + t]);
-                    // selects: as branches the two went to scratch memory
-                    const bool less = d < m1;
-                    m2 = less ? m1 : d > m1 && d < m2 ? d : m2;
-                    m1 = less ? d : m1;
-                }
-            }
+            pair_distances(may, k, g.off, g.off + g.n, c, thr, w, chunks, [&](int, float d) {
+                // selects: as branches the two went to scratch memory
+                const bool less = d < m1;
+                m2 = less ? m1 : d > m1 && d < m2 ? d : m2;
+                m1 = less ? d : m1;
+            });
             const float was = thr;
             if (m1 < thr) thr = fminf(thr, m1 * 1.000002f);
             if (ballot(thr < was)) P.radius(thr, valid, L);
@@ -1717,15 +1753,11 @@ __global__ __launch_bounds__(kWave) void k_sub_link(const SubGroup *__restrict__
         if (!P.chunk<true>(pk, k, next, rows, L, may, hit)) return;
         const uint64_t later = valid ? slot_bits(base, i + 1, end) : 0ull;
         hit &= later;
-        uint64_t amb = may & later & ~hit;
+        const uint64_t amb = may & later & ~hit;
         if (!ballot((hit | amb) != 0)) return;
-        while (ballot(amb != 0)) {
-            if (amb) {
-                const int t = __builtin_ctzll(amb);
-                amb &= amb - 1;
-                if (dist6(c, w[base + t]) < r2) hit |= 1ull << t;
-            }
-        }
+        pair_distances(amb, k, g.off, end, c, r2, w, chunks, [&](int t, float d) {
+            if (d < r2) hit |= 1ull << t;
+        });
         // the chunk's pairs: lanes in order, each lane's in order, staged in
         // LDS (appended directly when they alone overfill it)
         const int32_t nh = __popcll(hit);
