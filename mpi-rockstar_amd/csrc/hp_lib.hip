@@ -672,6 +672,10 @@ struct Engine {
     // A call has split levels when it holds more points than its bucket's
     // threshold (the device splits on its finite points, never more).
     int layout_walk(const Tables &T) {
+        if (counting) {  // not made, its size bounded: a part's lists differ by a piece at most
+            const size_t n = T.groups.size();
+            return grab(groups, sizeof(Group) * (n + n / 8 + 2 * (size_t)xcds));
+        }
         std::vector<Group> lv, rest;
         for (const Group &x : T.groups) {
             const int64_t n = T.count[(size_t)x.root];
@@ -2270,6 +2274,17 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
     int64_t ndrawn = 0;
     std::vector<std::pair<int64_t, int64_t>> ranges;
     int64_t M = 0, S = 0;
+    // the searches' wavefronts, those of the largest groups first: they go
+    // through the most chunks, and the last ones started bound the launch.
+    // Sizes are told apart to a quarter of a power of two, the groups counted
+    // into classes (a sort of 100,000 groups of 12 took 9 of 15 ms)
+    constexpr int kSizeClasses = 128;
+    auto size_class = [](int32_t n) {  // the largest first
+        const int e = 31 - __builtin_clz((uint32_t)n | 1u);
+        return kSizeClasses - 1 - (n < 4 ? n : 4 * e + (n >> (e - 2) & 3));
+    };
+    int64_t place[kSizeClasses + 1] = {}, l64 = 0, q64 = 0;  // l64, q64: tiles of 64
+    int32_t nsmin = INT32_MAX, nsmax = 0;
     for (int64_t g = 0; g < ngroups; g++) {
         const int64_t n = groups[g].num_p, f = groups[g].first;
         if (n < 0 || f < 0 || f + n > nparticles)
@@ -2306,23 +2321,26 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
         for (int64_t off = 0; off < n; off += kSubTile)
             tiles.push_back(SubTile{(int32_t)g, (int32_t)off});
         sg.ntiles = (int32_t)(tiles.size() - sg.tile0);
+        place[size_class(sg.n) + 1]++;
+        l64 += (n + kWave - 1) / kWave;
+        q64 += (ns + kWave - 1) / kWave;
+        nsmin = std::min(nsmin, sg.nsample);
+        nsmax = std::max(nsmax, sg.nsample);
         M += n;
         S += ns;
     }
-    // the searches' wavefronts, those of the largest groups first: they go
-    // through the most chunks, and the last ones started bound the launch
-    std::vector<int32_t> by_size((size_t)ngroups);
-    for (int64_t g = 0; g < ngroups; g++) by_size[(size_t)g] = (int32_t)g;
-    std::stable_sort(by_size.begin(), by_size.end(), [&](int32_t a, int32_t b) {
-        return G[(size_t)a].n > G[(size_t)b].n;
-    });
-    int64_t l64 = 0, q64 = 0;
-    for (const SubGroup &sg : G) {
-        l64 += (sg.n + kWave - 1) / kWave;
-        q64 += (sg.nsample + kWave - 1) / kWave;
+    std::vector<int32_t> by_size;
+    if (l64 > ngroups) {  // (else none has more than one tile)
+        by_size.resize((size_t)ngroups);
+        for (int k = 1; k <= kSizeClasses; k++) place[k] += place[k - 1];
+        for (int64_t g = 0; g < ngroups; g++)
+            by_size[(size_t)place[size_class(G[(size_t)g].n)]++] = (int32_t)g;
     }
     const int32_t llanes = query_lanes(l64), qlanes = query_lanes(q64);
-    for (int32_t g : by_size) {
+    ltiles.reserve((size_t)(llanes == kWave ? l64 : 4 * l64));
+    qtiles.reserve((size_t)(qlanes == kWave ? q64 : 4 * q64));
+    for (int64_t k = 0; k < ngroups; k++) {
+        const int32_t g = by_size.empty() ? (int32_t)k : by_size[(size_t)k];
         const SubGroup &sg = G[(size_t)g];
         for (int32_t off = 0; off < sg.n; off += llanes) ltiles.push_back(SubTile{g, off});
         for (int32_t off = 0; off < sg.nsample; off += qlanes) qtiles.push_back(SubTile{g, off});
@@ -2550,11 +2568,6 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
             B.pk.as<PackPoint>(), B.chunks.as<Box6>(), B.cblocks.as<Box6>(),
             B.dist.as<float>(), cfg.ordered_search, qlanes);
         HP_LAUNCHED();
-    }
-    int32_t nsmin = INT32_MAX, nsmax = 0;
-    for (const SubGroup &sg : G) {
-        nsmin = std::min(nsmin, sg.nsample);
-        nsmax = std::max(nsmax, sg.nsample);
     }
     if (nsmin <= kMedSmall) {
         k_sub_median_lds<256, kMedSmall><<<(uint32_t)ng, 256, 0, s>>>(

@@ -1399,7 +1399,9 @@ __global__ __launch_bounds__(kWave) void k_sub_next_closest(
     }
     float m1 = __builtin_inff(), m2 = __builtin_inff();
     float thr = valid ? T : 0.0f;  // nothing at or above T is ever taken
-    if (!ordered) {
+    // (a group of one leaf has no slots outside the skipped subtree)
+    const bool others = valid && (s_lo > g.off || s_hi < g.off + g.n);
+    if (!ordered && ballot(others)) {
         PairSearch P;
         P.init(slot, valid, c, pair_scale(nodes[root]), pk, L);
         P.radius(thr, valid, L);
