@@ -672,7 +672,10 @@ struct Engine {
     // A call has split levels when it holds more points than its bucket's
     // threshold (the device splits on its finite points, never more).
     int layout_walk(const Tables &T) {
-        if (counting) {  // not made, its size bounded: a part's lists differ by a piece at most
+        // Not made while counting, but its size bounded: an XCD has at most a
+        // piece more than its share.  (Made twice, the lists of 1,000,000 calls
+        // of 3 records took a tenth of hp_bound_pass_host.)
+        if (counting) {
             const size_t n = T.groups.size();
             return grab(groups, sizeof(Group) * (n + n / 8 + 2 * (size_t)xcds));
         }
@@ -2284,7 +2287,7 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
         return kSizeClasses - 1 - (n < 4 ? n : 4 * e + (n >> (e - 2) & 3));
     };
     int64_t place[kSizeClasses + 1] = {}, l64 = 0, q64 = 0;  // l64, q64: tiles of 64
-    int32_t nsmin = INT32_MAX, nsmax = 0;
+    int32_t nsmin = INT32_MAX, nsmax = 0, nmax = 0;
     for (int64_t g = 0; g < ngroups; g++) {
         const int64_t n = groups[g].num_p, f = groups[g].first;
         if (n < 0 || f < 0 || f + n > nparticles)
@@ -2324,13 +2327,14 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
         place[size_class(sg.n) + 1]++;
         l64 += (n + kWave - 1) / kWave;
         q64 += (ns + kWave - 1) / kWave;
+        nmax = std::max(nmax, sg.n);
         nsmin = std::min(nsmin, sg.nsample);
         nsmax = std::max(nsmax, sg.nsample);
         M += n;
         S += ns;
     }
     std::vector<int32_t> by_size;
-    if (l64 > ngroups) {  // (else none has more than one tile)
+    if (nmax > kWave) {  // (else no group has more than one tile)
         by_size.resize((size_t)ngroups);
         for (int k = 1; k <= kSizeClasses; k++) place[k] += place[k - 1];
         for (int64_t g = 0; g < ngroups; g++)
