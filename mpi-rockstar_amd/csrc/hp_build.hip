@@ -1839,7 +1839,12 @@ __global__ void k_internal_com(Node *__restrict__ nodes, const int32_t *__restri
 }
 
 // Tile partials of dmin for big nodes (every big task of every level), then
-// one thread per big node sums its tiles in order.
+// k_dmin_big combines each node's.  The reference adds the points' distances
+// in tree order; here a tile's are added across its threads and the tiles'
+// across a wavefront's lanes, in another order but always the same.  The sums
+// are f64, of terms of one sign (some 1e-15 of the sum apart), and dmin is
+// rounded to a float: it moves by its last bit where the value is as near to a
+// rounding boundary as that.
 __global__ __launch_bounds__(kTileThreads) void k_dmin_tiles(const Node *__restrict__ nodes,
                                                              const float4 *__restrict__ fin,
                                                              const int2 *__restrict__ tiles,

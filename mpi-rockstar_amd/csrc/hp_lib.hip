@@ -368,6 +368,7 @@ struct Engine {
     int32_t big_max() const { return *std::max_element(bucket_big, bucket_big + kTuneBuckets); }
     int32_t big_min() const { return *std::min_element(bucket_big, bucket_big + kTuneBuckets); }
     int xcds = 1;             // XCDs of the device (each with its own L2)
+    int cus = 1;              // its compute units
     int32_t walk_groups = 0;  // entries of the loaded walk table (XCD layout)
     // The walk table holds the wavefronts of the calls with split levels
     // first (walk_groups_lv entries), then the others, each part laid out on
@@ -457,6 +458,7 @@ struct Engine {
         sub_grid[2] = std::max(1, per_cu) * prop.multiProcessorCount;
         HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree_wave, kWave, 0));
         wave_grid = std::max(1, per_cu) * prop.multiProcessorCount;
+        cus = prop.multiProcessorCount;
         if (const char *s = getenv("HALOPOT_BIG_THRESHOLD")) {
             const int32_t bt = std::min(std::max(atoi(s), kLeafPoints), kSmallMax);
             for (int b = 0; b < kTuneBuckets; b++) bucket_big[b] = bt;
@@ -564,6 +566,7 @@ struct Engine {
         sub_grid[2] = std::max(1, per_cu) * prop.multiProcessorCount;
         HP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_subtree_wave, kWave, 0));
         wave_grid = std::max(1, per_cu) * prop.multiProcessorCount;
+        cus = prop.multiProcessorCount;
         carve = static_cast<uint8_t *>(region);
         carve_cap = bytes;
         own_stream = false;
@@ -1475,7 +1478,7 @@ struct Engine {
             k_shape_list<<<blocks(nst, kListThreads), kListThreads, 0, s>>>(tl, nst, ss, sl);
             HP_LAUNCHED();
             // few windows: four to a workgroup, so that they spread over the GPU
-            k_shape_small<<<kOneTileGroups + std::min<int>(blocks(2 * (int64_t)H, 4), kShapeGroups),
+            k_shape_small<<<kOneTileGroups + std::min<int>(blocks(2 * (int64_t)H, 4), cus * kShapeResident),
                             kShapeThreads, 0, s>>>(H, hf, shape_cd.as<float4>(), sl.one,
                                                    sl.counts + kOneTile, ss);
             HP_LAUNCHED();
@@ -2585,11 +2588,9 @@ __attribute__((visibility("default"))) int hp_find_subfofs(struct particle *d_pa
     }
     if (nsmax > kMedLarge) {
         HP_TRY(hipMemcpyAsync(B.sel.p, B.dist.p, sizeof(float) * S, hipMemcpyDeviceToDevice, s));
-        k_sub_median<<<(uint32_t)ng, kSfThreads, 0, s>>>(dg, thresh, B.sel.as<float>(),
-                                                          B.sel2.as<float>(), B.rk.as<int32_t>(),
-                                                          B.bpos.as<int32_t>(),
-                                                          B.spos.as<int32_t>(),
-                                                          B.target.as<float>());
+        k_sub_median<<<(uint32_t)ng, kSfThreads, 0, s>>>(
+            dg, B.sel.as<float>(), B.sel2.as<float>(), B.rk.as<int32_t>(), B.bpos.as<int32_t>(),
+            B.spos.as<int32_t>(), B.target.as<float>());
         HP_LAUNCHED();
     }
     // the linking, the reference's numbers and roots, then its output order

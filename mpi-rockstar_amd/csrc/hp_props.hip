@@ -809,8 +809,6 @@ __device__ __forceinline__ bool shape_step(ShapeRun &s, const double (&sum)[7],
 constexpr int kShapeWindows = 64;
 constexpr int kShapeThreads = 4 * kShapeWindows;
 constexpr int kShapeResident = 6;                     // workgroups on a compute unit
-constexpr int kComputeUnits = 256;
-constexpr int kShapeGroups = kComputeUnits * kShapeResident;  // all that run at once
 
 // The first kOneTileGroups workgroups take the one-tile windows instead, 16
 // each at a time: a wavefront sums a window, and the windows' steps are taken

@@ -999,6 +999,9 @@ __device__ float nc_ordered(const float (&c)[6], int32_t root, int32_t skip, flo
 // The error of that value is below kPairEps (|a|^2 + |b|^2) (2^-22 of each
 // product for the split, 32 sums in FP32, each to 2^-23) plus 1.5e-4 (2 |a| +
 // |b|) + 1 for lo parts below the smallest normal half, 2^-14, taken as zero.
+// (Measured against f64 on twelve kinds of coordinates, scales 2^-39 to
+// 2^64, skewed, clumped and with outliers: at most 0.042 of that, and 6.7e-7
+// (|a|^2 + |b|^2).)
 // With |b| <= |a| + d the thresholds leave that much room on both sides of a
 // radius: a pair above `may` is certainly not closer, one below `sure`
 // certainly is, and the few between are decided by the reference's own float
@@ -1569,9 +1572,9 @@ __global__ __launch_bounds__(NT) void k_sub_median_lds(const SubGroup *__restric
 // global memory; buf holds the distances (a copy), buf2, rk, bpos and spos
 // are scratch of the same extent.
 __global__ __launch_bounds__(kSfThreads) void k_sub_median(
-    const SubGroup *__restrict__ groups, float frac, float *__restrict__ buf,
-    float *__restrict__ buf2, int32_t *__restrict__ rk, int32_t *__restrict__ bpos,
-    int32_t *__restrict__ spos, float *__restrict__ target) {
+    const SubGroup *__restrict__ groups, float *__restrict__ buf, float *__restrict__ buf2,
+    int32_t *__restrict__ rk, int32_t *__restrict__ bpos, int32_t *__restrict__ spos,
+    float *__restrict__ target) {
     __shared__ int s_w[kSfThreads / kWave];
     __shared__ int32_t s_v[4];
     __shared__ float s_piv;
