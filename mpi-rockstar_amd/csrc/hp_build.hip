@@ -979,7 +979,11 @@ struct SubLds {
 
 // One workgroup per task of the list `cls` (nodes of at most kCap points), a
 // thread per point.  Bound by the latency of a task: LDS (77 KB at 1,024
-// points) and registers leave 8 wavefronts per SIMD at every size.
+// points) and registers leave 8 wavefronts per SIMD at every size.  At the 64
+// registers of that a thread spills some 100 bytes (734 MB of HBM traffic a
+// launch of the 1,024-point size on the one-GPU catalogue, against 315 MB for
+// the kernel with 256 threads); with more registers and fewer wavefronts it was
+// slower (1,162 us against 731).
 template <int kCap>
 __global__ __launch_bounds__(kCap, 8) void k_subtree(const float4 *__restrict__ A,
                                                      const float4 *__restrict__ B,

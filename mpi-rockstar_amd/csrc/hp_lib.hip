@@ -1163,8 +1163,13 @@ struct Engine {
                 build_checked = false;
             }
             if (timing) HP_TRY(hipEventRecord(ev[1], s));
-            // the subtree sizes beside each other: 530,000 records 0.91 -> 0.84
-            // ms; on one call of 11,000 the events cost what they save
+            // The subtree sizes beside each other, where the batch is large
+            // enough that they gain more than the events cost.  Below the
+            // line: one call of 11,000 438 us alone, 440 so; 40 of 800 220 and
+            // 250, 20 of 1,600 304 and 392, 8 of 4,000 416 and 403.  Above: 40
+            // of 1,100 436 and 405, batches of 51,000 554 and 476, of 175,000
+            // 574 and 483, of 464,000 994 and 910; single calls within 3%
+            // either way (60,000 781 and 748, 100,000 834 and 852).
             if ((r = enqueue_multipole((int)st.levels, max_count > 512 && loaded_n > 32768)))
                 return r;
         } else if (timing) {
